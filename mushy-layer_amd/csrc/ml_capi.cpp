@@ -318,6 +318,7 @@ int ml_hc_op_create(ml_ctx ctx, int dim, const int lo[], const int hi[], double 
   op->params = *params;
   op->cp = {params->stefan, params->compositionRatio, params->waterDistributionCoeff, params->specificHeatRatio,
             params->thetaEutectic, params->ThetaEutectic};
+  ml::closure_prepare(op->cp);
   std::memcpy(op->bc.type, bc->type, sizeof(bc->type));
   std::memcpy(op->bc.val, bc->val, sizeof(bc->val));
   op->bc.apply = bc->apply;

@@ -4,9 +4,11 @@
 // reference configures (AMRFASMultiGrid driving AMRNonLinearMultiCompOp,
 // srcSubcycle/AMRLevelMushyLayerInit.cpp:989-1022; driver specification in
 // host/FASMultiGrid.H), with kernels fused per level:
-//   tiled levels:   relax(nu1) | restrict phi, phi0 and rhs-L(phi) in one
-//                   kernel | rhs_c += L_c(phi_c) | ... | prolong fused into
-//                   the first post-smoothing launch | relax(nu2)
+//   tiled levels:   rhs += L(phi) | relax(nu1) | restrict phi, phi0 and
+//                   rhs-L(phi), one launch on 2D levels up to 512^2 cells and
+//                   three above and in 3D | ... | prolong fused into the
+//                   first post-smoothing launch | relax(nu2), on such a level
+//                   0 with the residual norm and the stopping rule
 //   coarse levels:  one single-workgroup kernel for the whole sub-cycle,
 //                   including the 40-iteration relax bottom solve.
 // Norms accumulate into per-iteration slots zeroed once per solve.
@@ -40,6 +42,7 @@ HCEngine::~HCEngine() {
     if (m_phi[l]) hipFree(m_phi[l]);
     if (m_rhs[l]) hipFree(m_rhs[l]);
     if (m_phi0[l]) hipFree(m_phi0[l]);
+    if (m_res[l]) hipFree(m_res[l]);
   }
   for (double* q : m_alt)
     if (q) hipFree(q);
@@ -65,6 +68,7 @@ int HCEngine::init() {
   m_phi.assign(m_L, nullptr);
   m_rhs.assign(m_L, nullptr);
   m_phi0.assign(m_L, nullptr);
+  m_res.assign(m_L, nullptr);
   for (int l = 1; l < m_L; ++l) {
     const size_t bytes = sizeof(double) * 2 * m_op->lev[l].g.ncell;
     void* p = nullptr;
@@ -77,6 +81,11 @@ int HCEngine::init() {
     ML_HIP(ctx, vec_set(2 * m_op->lev[l].g.ncell, m_phi[l], 0.0, ctx->stream));
     ML_HIP(ctx, vec_set(2 * m_op->lev[l].g.ncell, m_rhs[l], 0.0, ctx->stream));
     ML_HIP(ctx, vec_set(2 * m_op->lev[l].g.ncell, m_phi0[l], 0.0, ctx->stream));
+    if (l < m_lc && hc_fuses(m_op->lev[l].g)) {
+      ML_HIP(ctx, hipMalloc(&p, bytes));
+      m_res[l] = static_cast<double*>(p);
+      ML_HIP(ctx, vec_set(2 * m_op->lev[l].g.ncell, m_res[l], 0.0, ctx->stream));
+    }
   }
   // relax ping-pong partners: every level relaxed by the tiled kernels
   // (above m_lc, or all levels when none fits one workgroup) and level 0
@@ -166,7 +175,7 @@ int HCEngine::upload_desc(double* phi0, const double* rhs0, const ml_solve_opts&
   return ML_OK;
 }
 
-int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, const int* skip) {
+int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, const int* skip, int slot, bool* fused) {
   ml_ctx ctx = m_op->ctx;
   hipStream_t s = ctx->stream;
   auto P = [&](int l) { return cur(l, phi); };
@@ -177,7 +186,11 @@ int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, con
     return A;
   };
   double* B[2];
+  *fused = false;
   const int ltiles = m_lc < m_L ? m_lc : m_L - 1;   // tiled levels above the coarse kernel
+  // fused levels: the restriction (and the operator on the level's own
+  // state, which completes its FAS right-hand side) rides on the relaxation
+  auto fuses = [&](int l) { return o.nu1 > 0 && l < ltiles && hc_fuses(m_op->lev[l].g); };
   if (m_lc >= m_L && m_L == 1) {
     // a single level too large for one workgroup: relax bottom with tiles
     bufs(0, phi, B);
@@ -187,10 +200,18 @@ int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, con
   for (int l = 0; l < ltiles; ++l) {
     const HCArgs<double> A = args(l);
     bufs(l, phi, B);
-    ML_HIP(ctx, hc_relax<double>(A, B, &m_cur[l], R(l), 2 * o.nu1, 0, s));
-    ML_HIP(ctx, hc_restrict_all<double>(A, m_op->lev[l + 1].g, P(l), R(l), R(l + 1), P(l + 1), m_phi0[l + 1], 0,
-                                        s));
-    if (l + 1 < m_lc) ML_HIP(ctx, hc_apply_op<double>(args(l + 1), P(l + 1), R(l + 1), R(l + 1), 0, s));
+    // a fused coarser level adds L(phi) to the restricted residual itself
+    const bool next = l + 1 < m_lc && fuses(l + 1) && m_res[l + 1];
+    double* resc = next ? m_res[l + 1] : R(l + 1);
+    if (fuses(l)) {
+      const bool add = l > 0 && m_res[l];
+      ML_HIP(ctx, hc_relax_restrict<double>(A, B, &m_cur[l], add ? m_res[l] : R(l), add ? R(l) : nullptr, 2 * o.nu1,
+                                            m_op->lev[l + 1].g, resc, P(l + 1), m_phi0[l + 1], s));
+    } else {
+      ML_HIP(ctx, hc_relax<double>(A, B, &m_cur[l], R(l), 2 * o.nu1, 0, s));
+      ML_HIP(ctx, hc_restrict_all<double>(A, m_op->lev[l + 1].g, P(l), R(l), resc, P(l + 1), m_phi0[l + 1], 0, s));
+    }
+    if (l + 1 < m_lc && !next) ML_HIP(ctx, hc_apply_op<double>(args(l + 1), P(l + 1), R(l + 1), R(l + 1), 0, s));
   }
   if (m_lc < m_L) {
     ML_HIP(ctx, hc_coarse_vcycle<double>(m_desc, m_op->dim, m_lc > 0 ? 1 : 0, s));
@@ -204,6 +225,12 @@ int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, con
     const HCArgs<double> A = args(l);
     const Geom gc = m_op->lev[l + 1].g;
     bufs(l, phi, B);
+    if (l == 0 && o.nu2 > 0 && hc_fuses(m_op->lev[0].g)) {
+      ML_HIP(ctx, hc_relax_final<double>(A, B, &m_cur[0], rhs, 2 * o.nu2, &gc, P(1), m_phi0[1], m_slots + slot,
+                                         CtlFuse{m_ctl, m_slots, m_arrive, 0}, s));
+      *fused = true;
+      continue;
+    }
     ML_HIP(ctx, hc_relax_tiles<double>(A, B, &m_cur[l], R(l), 2 * o.nu2, 0, &gc, P(l + 1), m_phi0[l + 1], s));
   }
   return ML_OK;
@@ -244,11 +271,13 @@ int HCEngine::solve(double* phi, const double* rhs, const ml_solve_opts& o, ml_s
   for (;;) {
     for (int b = 0; b < batch && launched < o.max_iter; ++b) {
       const int before = m_cur[0];
-      if ((rc = vcycle(phi, rhs, o, skip))) return rc;
-      if (flip0 < 0) flip0 = m_cur[0] != before ? 1 : 0;
       ++launched;
-      // the residual kernel's last workgroup applies the stopping rule
-      if ((rc = residual_norm(cur(0, phi), rhs, launched, skip, true))) return rc;
+      bool fused = false;
+      if ((rc = vcycle(phi, rhs, o, skip, launched, &fused))) return rc;
+      if (flip0 < 0) flip0 = m_cur[0] != before ? 1 : 0;
+      // the last workgroup of the kernel that takes the norm applies the
+      // stopping rule
+      if (!fused && (rc = residual_norm(cur(0, phi), rhs, launched, skip, true))) return rc;
     }
     if ((rc = read_ctl(&c))) return rc;
     if (c.done || launched >= o.max_iter) break;

@@ -10,6 +10,8 @@
 // bit for bit.
 #include <hip/hip_ext.h>
 
+#include <type_traits>
+
 #include "ml_common.h"
 #include "ml_kernels.h"
 #include "ml_tile.h"
@@ -207,6 +209,416 @@ __global__ __launch_bounds__(NT) void hc_relax_tile_kernel(HCArgs<T> A, TileIO<T
     if (!r.owner) continue;
     io.phi_out[r.q] = sphi[r.e];
     io.phi_out[r.q + g.ncell] = sphi[E + r.e];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// 2D red/black relaxation over regions of 32 x 32 positions: the core of
+// 32 - 2H cells a side that the workgroup owns and a halo of H cells (H = the
+// colour passes, one more where a result of the relaxed state follows).  The
+// passes and values are those of hc_relax_tile_kernel.
+//
+// A pass is bound by its chain of some 170 FP64 instructions (stencil and
+// closure), so no lane may idle in it: each of the 512 threads holds the two
+// cells of an x pair, one of each colour (slot m: the cell of parity m), and
+// a pass runs one slot with every lane at work, where one cell per lane
+// leaves half of them waiting.  State, closure, right-hand side, lambda and
+// faces of both cells stay in registers; LDS holds only the closure, which
+// the neighbours read (16 KB).  Rows are 256 B apart and a row's active cells
+// alternate with the next row's, so the 32 lanes of an 8-byte LDS access
+// cover every bank once.
+//
+// What a launch costs besides its passes is fetching its code and arguments,
+// both cold: so the arguments are one small struct (not the operator's
+// geometry), the tile is the 2D workgroup index (no divisions), the faces,
+// right-hand side and state of a pair come as 16-byte loads with 32-bit
+// offsets, and the closure of the incoming state is one loop for both cells.
+//
+//   RB_PLAIN     the relaxed state
+//   RB_RESTRICT  ... and the FAS restriction of its residual and itself
+//   RB_NORM      ... and the max-norm of its residual with the stopping rule
+// With rhs_out the right-hand side first receives L(phi) of the incoming
+// state.  Measured (events around the launch, 256^2 mushy state): 8 passes
+// 14.4 us, 21.2 us with one cell per lane (32x8 tiles, 512 threads); at 512^2
+// 34.7 against 74.3 us; on the way down one launch of 10.5 us replaces
+// relaxation, restriction and operator (9.0 + 7.3 + 8.4 us).  GEN: any grid -- a periodic length below 32 or odd (equal colours
+// then meet at its seam: a pass looks at both slots, and reads neighbours as
+// of its start), arrays beyond 32-bit byte offsets.
+enum : int { RB_PLAIN = 0, RB_RESTRICT = 1, RB_NORM = 2 };
+constexpr int kRB = 32;            // positions per side
+constexpr int kRBThreads = kRB * kRB / 2;
+
+template <typename T>
+struct PairArgs {
+  const int* skip;
+  const T *phi, *rhs, *b0, *b1, *a;    // a nullable
+  int nx, ny, sy, npass, first, per0, per1, ntx;
+  unsigned ncell;
+  long long nf0, nf1;
+  T alpha, beta, dxinv;
+  T *phi_out, *rhs_out;
+  const T *pc, *pc0;                   // prolongation source (nullable)
+  T *out, *phic, *phic0;
+  int cnx, cny, csy;                   // the coarse level of pc or of out
+  unsigned cncell;
+  unsigned long long* norm;
+  CtlFuse fuse;
+  ClosureP<T> cp;
+  T gs[2][2][2], gb[2][2][2];          // GhostForm
+};
+
+// linear prolongation (prolong_value) of the correction pc - pc0 to fine cell
+// (i, j); the outer coarse neighbour is at most one cell beyond the coarse
+// level, so it wraps or clamps without a division
+template <typename T, typename Off>
+__device__ __forceinline__ void prolong_pair2(const PairArgs<T>& A, int i, int j, T* p) {
+  constexpr T fx1 = T(3) / T(16), fx2 = T(9) / T(16), f0 = T(1) / T(16);
+  const int ic = i >> 1, jc = j >> 1;
+  int X1 = ic + ((i & 1) ? 1 : -1), Y1 = jc + ((j & 1) ? 1 : -1);
+  if (X1 < 0) X1 = A.per0 ? A.cnx - 1 : 0;
+  if (X1 >= A.cnx) X1 = A.per0 ? 0 : A.cnx - 1;
+  if (Y1 < 0) Y1 = A.per1 ? A.cny - 1 : 0;
+  if (Y1 >= A.cny) Y1 = A.per1 ? 0 : A.cny - 1;
+  const Off r0 = Off(1) + Off(A.csy) * Off(jc + 1), r1 = Off(1) + Off(A.csy) * Off(Y1 + 1);
+  const Off q[4] = {(r0 + Off(ic)) * Off(sizeof(T)), (r1 + Off(X1)) * Off(sizeof(T)), (r0 + Off(X1)) * Off(sizeof(T)),
+                    (r1 + Off(ic)) * Off(sizeof(T))};
+  auto ld = [](const T* b, Off o) { return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(b) + o); };
+  T v[2][4];
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[n][c] = ld(A.pc + (n ? A.cncell : 0u), q[c]);
+  if (A.pc0) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) v[n][c] = v[n][c] - ld(A.pc0 + (n ? A.cncell : 0u), q[c]);
+  }
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    p[n] = p[n] + fx2 * v[n][0] + f0 * v[n][1];
+    p[n] = p[n] + fx1 * (v[n][2] + v[n][3]);
+  }
+}
+
+// two values at any 8-byte alignment in one load
+typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <typename T, int MODE, bool GEN>
+__global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T> A) {
+  using Off = typename std::conditional<GEN, unsigned long long, unsigned>::type;
+  constexpr int NP = kRB * kRB;
+  constexpr Off W = sizeof(T);
+  __shared__ T sl[2 * NP];                                  // closure
+  __shared__ T sr[MODE == RB_RESTRICT ? 2 * NP : 1];        // restriction scratch
+  const int nx = A.nx, ny = A.ny, npass = A.npass;
+  const int H = npass + (MODE == RB_PLAIN ? 0 : 1);
+  const int core = kRB - 2 * H;
+  // GEN: the workgroups of all tiles in one dimension
+  const int by = GEN ? int(blockIdx.x / unsigned(A.ntx)) : int(blockIdx.y);
+  const int bx = GEN ? int(blockIdx.x) - by * A.ntx : int(blockIdx.x);
+  const int x0 = bx * core, y0 = by * core;
+  const int ey = threadIdx.x >> 4, ex0 = 2 * (threadIdx.x & 15);
+  const int ux0 = x0 - H + ex0, uy = y0 - H + ey;
+  const bool per0 = A.per0 != 0, per1 = A.per1 != 0;
+  auto wrap = [](int v, int n) {
+    if (GEN) {
+      v %= n;
+      return v < 0 ? v + n : v;
+    }
+    return v < 0 ? v + n : (v >= n ? v - n : v);   // n >= 32: at most one length away
+  };
+  const bool iny = uy >= 0 && uy < ny;
+  const bool oky = iny || per1;
+  const int gj = oky ? wrap(uy, ny) : 0;
+  // distance from the core
+  auto beyond = [&](int e) {
+    const int lo = H - e, hi = e - (H + core) + 1;
+    const int d = lo > hi ? lo : hi;
+    return d > 0 ? d : 0;
+  };
+  const int dy = beyond(ey);
+  const int swap = (ux0 + uy) & 1;   // parity of the pair's first cell
+  const int wy = per1 ? 0 : ((gj == 0 ? 4 : 0) | (gj == ny - 1 ? 8 : 0));
+  // cells of the pair in x order: c = 0, 1; slot m holds cell m ^ swap
+  const bool in0 = ux0 >= 0 && ux0 < nx, in1 = ux0 >= -1 && ux0 + 1 < nx;
+  const bool ok0 = oky && (in0 || per0), ok1 = oky && (in1 || per0);
+  const int gx0 = ok0 ? wrap(ux0, nx) : 0, gx1 = ok1 ? wrap(ux0 + 1, nx) : 0;
+  const Off row = Off(A.sy) * Off(gj + 1) + Off(1);
+  const Off q0 = (row + Off(gx0)) * W, q1 = (row + Off(gx1)) * W;   // byte offsets
+
+  auto ld = [](const T* b, Off o) { return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(b) + o); };
+  T ph[2][2], rr[2][2], aa[2][2], lam[2][2], pl[2][2];
+  CellFaces<T, 2> F[2];
+  const Off fx0 = (Off(gx0) + Off(nx + 1) * Off(gj)) * W, fx1 = (Off(gx1) + Off(nx + 1) * Off(gj)) * W;
+  const Off fy0 = (Off(gx0) + Off(nx) * Off(gj)) * W, fy1 = (Off(gx1) + Off(nx) * Off(gj)) * W;
+  if (ok0 && ok1 && gx1 == gx0 + 1) {
+    auto ld2 = [](const T* b, Off o) { return *reinterpret_cast<const dbl2u*>(reinterpret_cast<const char*>(b) + o); };
+    dbl2u vp[2], vr[2], vx[2], vl[2], vh[2];
+    T vz[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) vp[n] = ld2(A.phi + (n ? A.ncell : 0u), q0);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      vr[n] = ld2(A.rhs + (n ? A.ncell : 0u), q0);
+      const T *bx = A.b0 + (n ? A.nf0 : 0), *by = A.b1 + (n ? A.nf1 : 0);
+      vx[n] = ld2(bx, fx0);
+      vz[n] = ld(bx + 2, fx0);
+      vl[n] = ld2(by, fy0);
+      vh[n] = ld2(by + nx, fy0);
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        const bool second = (m ^ swap) != 0;
+        ph[m][n] = second ? vp[n].y : vp[n].x;
+        rr[m][n] = second ? vr[n].y : vr[n].x;
+        F[m].v[n][0] = second ? vx[n].y : vx[n].x;
+        F[m].v[n][1] = second ? vz[n] : vx[n].y;
+        F[m].v[n][2] = second ? vl[n].y : vl[n].x;
+        F[m].v[n][3] = second ? vh[n].y : vh[n].x;
+      }
+  } else {
+    // a pair across the periodic seam or beside a wall
+#pragma unroll 1
+    for (int m = 0; m < 2; ++m) {
+      const bool second = (m ^ swap) != 0;
+      if (!(second ? ok1 : ok0)) continue;
+      const Off qm = second ? q1 : q0, fx = second ? fx1 : fx0, fy = second ? fy1 : fy0;
+      T v[2][6];
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const T *bx = A.b0 + (n ? A.nf0 : 0), *by = A.b1 + (n ? A.nf1 : 0);
+        v[n][0] = ld(A.phi + (n ? A.ncell : 0u), qm);
+        v[n][1] = ld(A.rhs + (n ? A.ncell : 0u), qm);
+        v[n][2] = ld(bx, fx);
+        v[n][3] = ld(bx + 1, fx);
+        v[n][4] = ld(by, fy);
+        v[n][5] = ld(by + nx, fy);
+      }
+      auto take = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          ph[k][n] = v[n][0];
+          rr[k][n] = v[n][1];
+#pragma unroll
+          for (int f = 0; f < 4; ++f) F[k].v[n][f] = v[n][2 + f];
+        }
+      };
+      if (m == 0)
+        take(0);
+      else
+        take(1);
+    }
+  }
+  // (the loads above are in bounds in any case)
+  if (A.skip && *A.skip) return;
+  int e[2], lim[2], gi[2], wall[2];
+  Off q[2];
+  bool cell[2], owner[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const bool second = (m ^ swap) != 0;
+    const int ex = ex0 + (second ? 1 : 0);
+    e[m] = ey * kRB + ex;
+    cell[m] = second ? ok1 : ok0;
+    gi[m] = second ? gx1 : gx0;
+    q[m] = second ? q1 : q0;
+    const int dx = beyond(ex);
+    const int dist = dx > dy ? dx : dy;
+    owner[m] = (second ? in1 : in0) && iny && dist == 0;
+    lim[m] = cell[m] ? H - 1 - dist : -1;   // last pass that updates the cell
+    wall[m] = wy | (per0 ? 0 : ((gi[m] == 0 ? 1 : 0) | (gi[m] == nx - 1 ? 2 : 0)));
+    aa[m][0] = aa[m][1] = T(1);
+    if (A.a && cell[m]) {
+      aa[m][0] = ld(A.a, q[m]);
+      aa[m][1] = ld(A.a + A.ncell, q[m]);
+    }
+  }
+  if (A.pc) {
+#pragma unroll 1
+    for (int m = 0; m < 2; ++m) {
+      if (!(m ? cell[1] : cell[0])) continue;
+      T v[2] = {m ? ph[1][0] : ph[0][0], m ? ph[1][1] : ph[0][1]};
+      prolong_pair2<T, Off>(A, m ? gi[1] : gi[0], gj, v);
+      if (m == 0) {
+        ph[0][0] = v[0];
+        ph[0][1] = v[1];
+      } else {
+        ph[1][0] = v[0];
+        ph[1][1] = v[1];
+      }
+    }
+  }
+  // one copy of the closure for both cells
+#pragma unroll 1
+  for (int m = 0; m < 2; ++m) {
+    T th, cl;
+    closure<T>(m ? ph[1][0] : ph[0][0], m ? ph[1][1] : ph[0][1], A.cp, th, cl);
+    if (m ? cell[1] : cell[0]) {
+      sl[m ? e[1] : e[0]] = th;
+      sl[NP + (m ? e[1] : e[0])] = cl;
+    }
+    if (m == 0) {
+      pl[0][0] = th;
+      pl[0][1] = cl;
+    } else {
+      pl[1][0] = th;
+      pl[1][1] = cl;
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    lam[m][0] = lambda_of<T, 2>(F[m], 0, aa[m][0], A.alpha, A.beta, A.dxinv);
+    lam[m][1] = lambda_of<T, 2>(F[m], 1, aa[m][1], A.alpha, A.beta, A.dxinv);
+  }
+  __syncthreads();
+  // L(phi) of slot m; a neighbour beyond a wall is the ghost of the cell's
+  // own closure (computeDiffusedVar's BC)
+  auto lof = [&](auto M, T(&out)[2]) __attribute__((always_inline)) {
+    constexpr int m = decltype(M)::value;
+    T st[2][5];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const T* s = sl + n * NP + e[m];
+      st[n][0] = pl[m][n];
+      st[n][1] = s[1];
+      st[n][2] = s[-1];
+      st[n][3] = s[kRB];
+      st[n][4] = s[-kRB];
+    }
+    if (wall[m]) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+          const int k = 1 + 2 * (f >> 1) + (1 - (f & 1));
+          const T gh = fma(A.gs[f >> 1][f & 1][n], st[n][0], A.gb[f >> 1][f & 1][n]);
+          st[n][k] = ((wall[m] >> f) & 1) ? gh : st[n][k];
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      out[n] = lof_of<T, 2>(F[m], n, st[n], aa[m][n], ph[m][n], A.alpha, A.beta, A.dxinv);
+  };
+  auto st = [](T* b, Off o, T v) { *reinterpret_cast<T*>(reinterpret_cast<char*>(b) + o) = v; };
+  if (A.rhs_out) {
+    auto add = [&](auto M) __attribute__((always_inline)) {
+      constexpr int m = decltype(M)::value;
+      if (lim[m] < 0) return;
+      T lf[2];
+      lof(M, lf);
+      rr[m][0] = rr[m][0] + lf[0];
+      rr[m][1] = rr[m][1] + lf[1];
+      if (owner[m]) {
+        st(A.rhs_out, q[m], rr[m][0]);
+        st(A.rhs_out + A.ncell, q[m], rr[m][1]);
+      }
+    };
+    add(IC<0>{});
+    add(IC<1>{});
+    __syncthreads();   // the passes below overwrite the closure just read
+  }
+  auto runs = [&](int m, int p, int colour) {
+    return p <= lim[m] && (!GEN || ((gi[m] + gj) & 1) == colour);
+  };
+  auto put = [&](int m) __attribute__((always_inline)) {
+    sl[e[m]] = pl[m][0];
+    sl[NP + e[m]] = pl[m][1];
+  };
+  auto update = [&](auto M, int p, int colour) __attribute__((always_inline)) {
+    constexpr int m = decltype(M)::value;
+    if (!runs(m, p, colour)) return;
+    T lf[2];
+    lof(M, lf);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) ph[m][n] = ph[m][n] - lam[m][n] * (lf[n] - rr[m][n]);
+    closure<T>(ph[m][0], ph[m][1], A.cp, pl[m][0], pl[m][1]);
+    if (!GEN) put(m);
+  };
+#pragma unroll 1
+  for (int p = 0; p < npass; ++p) {
+    const int colour = (A.first + p) & 1;
+    if (GEN || colour == 0) update(IC<0>{}, p, colour);
+    if (GEN || colour == 1) update(IC<1>{}, p, colour);
+    if constexpr (GEN) {
+      __syncthreads();
+      if (runs(0, p, colour)) put(0);
+      if (runs(1, p, colour)) put(1);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    if (!owner[m]) continue;
+    st(A.phi_out, q[m], ph[m][0]);
+    st(A.phi_out + A.ncell, q[m], ph[m][1]);
+  }
+  if constexpr (MODE == RB_NORM) {
+    T mx = T(0);
+    int nan = 0;
+    auto res = [&](auto M) __attribute__((always_inline)) {
+      constexpr int m = decltype(M)::value;
+      if (!owner[m]) return;
+      T lf[2];
+      lof(M, lf);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        const T ar = fabs(rr[m][n] - lf[n]);
+        if (ar != ar) nan = 1;
+        else if (ar > mx) mx = ar;
+      }
+    };
+    res(IC<0>{});
+    res(IC<1>{});
+    block_max_atomic<T>(mx, nan, A.norm, A.fuse);
+  }
+  if constexpr (MODE == RB_RESTRICT) {
+    // RESTRICTRESNLVC / RESTRICT (src/AMRNonLinearMultiCompOpF.ChF:452-585):
+    // (rhs - L phi)/4 and phi/4 per fine cell, child sums in Fortran order
+    T tr[2][2];
+    auto res = [&](auto M) __attribute__((always_inline)) {
+      constexpr int m = decltype(M)::value;
+      if (!owner[m]) return;
+      T lf[2];
+      lof(M, lf);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        tr[m][n] = (rr[m][n] - lf[n]) / T(4);
+        sr[n * NP + e[m]] = ph[m][n] / T(4);
+      }
+    };
+    res(IC<0>{});
+    res(IC<1>{});
+    __syncthreads();   // every closure has been read
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (!owner[m]) continue;
+      sl[e[m]] = tr[m][0];
+      sl[NP + e[m]] = tr[m][1];
+    }
+    __syncthreads();
+    // coarse cells of the core (at most 13 a side), 16 threads a row
+    const int cy = threadIdx.x >> 4, cx = threadIdx.x & 15;
+    const int I = x0 / 2 + cx, J = y0 / 2 + cy;
+    if (cx >= core / 2 || cy >= core / 2 || I >= A.cnx || J >= A.cny) return;
+    const Off qc = (Off(I + 1) + Off(A.csy) * Off(J + 1)) * W;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      T s = T(0), sp = T(0);
+#pragma unroll
+      for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+        for (int ii = 0; ii < 2; ++ii) {
+          const int f = n * NP + (2 * cy + jj + H) * kRB + 2 * cx + ii + H;
+          s = s + sl[f];
+          sp = sp + sr[f];
+        }
+      st(A.out + (n ? A.cncell : 0u), qc, s);
+      st(A.phic + (n ? A.cncell : 0u), qc, sp);
+      st(A.phic0 + (n ? A.cncell : 0u), qc, sp);
+    }
   }
 }
 
@@ -1061,23 +1473,13 @@ static hipError_t launch_tile(const HCArgs<T>& A, TileIO<T> io, hipStream_t s) {
   return hipGetLastError();
 }
 
-// Passes per relax launch: small grids are latency bound, so up to four
-// red/black sweeps share one launch (halo 8); large grids use one sweep per
-// launch (halo 2) to keep the redundant halo work small.
-constexpr int kTilesForDeepHalo = 1024;
+// Colour passes of one 2D relaxation launch: up to 512^2 cells the launches
+// are latency-bound and four sweeps share one (core 16^2 of the 32^2 region;
+// at 512^2 34.7 us against four launches of 13.9 us); larger levels, where
+// the halo's work counts, take one sweep (core 28^2).
+constexpr long long kDeepHaloCells = 512 * 512;
 
-template <typename T, int DIM>
-static int relax_passes_per_launch(const Geom& g) {
-  int ntx, nty;
-  const int nt = tiles_of<T, DIM>(g, ntx, nty);
-  return (DIM == 2 && nt <= kTilesForDeepHalo) ? 8 : 2;
-}
-
-// tiles of the one-sweep 2D relaxation launch on large levels (measured
-// best of 5 shapes at 2048^2)
-struct HCRelaxWide2 {
-  static constexpr int TX = 32, TY = 8, TZ = 1, NT = 256;
-};
+static int relax_passes_per_launch(const Geom& g) { return g.dim == 2 && g.nvalid() <= kDeepHaloCells ? 8 : 2; }
 
 // tiles of the 3D relaxation launch (measured best of 5 shapes at 128^3;
 // the others spill registers)
@@ -1085,53 +1487,101 @@ struct HCRelaxTile3 {
   static constexpr int TX = 16, TY = 8, TZ = 4, NT = 512;
 };
 
-template <typename T, int DIM>
-static hipError_t launch_relax_tile(const HCArgs<T>& A, TileIO<T> io, hipStream_t s, const LaunchTimer* tm) {
-  using D = TileDims<T, DIM>;
-  using DW = HCRelaxWide2;
+// algorithmic bytes of a relaxation launch: state (2 comps) in and out, rhs,
+// a, faces (2 comps) once each; the coarse state (and its initial copy) when
+// prolonged on load
+template <typename T>
+static double relax_bytes(const HCArgs<T>& A, const TileIO<T>& io) {
+  const double cells = double(A.g.nvalid());
+  double faces = 0;
+  for (int d = 0; d < A.g.dim; ++d) faces += double(A.g.nface[d]);
+  double b = 2 * cells + 2 * cells + (A.a ? 2 * cells : 0) + 2 * faces + 2 * cells;
+  if (io.pc) b += 2 * io.gc.nvalid() * (io.pc0 ? 2 : 1);
+  return b * sizeof(T);
+}
+
+template <typename T, int MODE>
+static hipError_t launch_relax_pair(const HCArgs<T>& A, const TileIO<T>& io, hipStream_t s, const LaunchTimer* tm) {
+  const int H = io.npass + (MODE == RB_PLAIN ? 0 : 1);
+  if (io.npass < 1 || H > 9) return hipErrorInvalidValue;
+  const Geom& g = A.g;
+  PairArgs<T> P{};
+  P.skip = A.skip;
+  P.phi = io.phi;
+  P.rhs = io.rhs;
+  P.b0 = A.b[0];
+  P.b1 = A.b[1];
+  P.a = A.a;
+  P.nx = g.n[0];
+  P.ny = g.n[1];
+  P.sy = int(g.sy);
+  P.npass = io.npass;
+  P.first = io.first;
+  P.per0 = g.periodic[0];
+  P.per1 = g.periodic[1];
+  P.ncell = unsigned(g.ncell);
+  P.nf0 = g.nface[0];
+  P.nf1 = g.nface[1];
+  P.alpha = A.alpha;
+  P.beta = A.beta;
+  P.dxinv = T(1) / (T(g.dx) * T(g.dx));
+  P.phi_out = io.phi_out;
+  P.rhs_out = io.rhs_out;
+  P.pc = io.pc;
+  P.pc0 = io.pc0;
+  P.out = io.out;
+  P.phic = io.phic;
+  P.phic0 = io.phic0;
+  P.cnx = io.gc.n[0];
+  P.cny = io.gc.n[1];
+  P.csy = int(io.gc.sy);
+  P.cncell = unsigned(io.gc.ncell);
+  P.norm = io.norm;
+  P.fuse = io.fuse;
+  P.cp = A.cp;
+  const GhostForm<T> gf = ghost_form<T>(A.bc, T(g.dx));
+  for (int d = 0; d < 2; ++d)
+    for (int sd = 0; sd < 2; ++sd)
+      for (int n = 0; n < 2; ++n) {
+        P.gs[d][sd][n] = gf.s[d][sd][n];
+        P.gb[d][sd][n] = gf.b[d][sd][n];
+      }
+  const int core = kRB - 2 * H;
+  const int ntx = (g.n[0] + core - 1) / core, nty = (g.n[1] + core - 1) / core;
+  if (g.ncell >= (1LL << 32)) return hipErrorInvalidValue;   // (32-bit component stride)
+  P.ntx = ntx;
+  // GEN where a grid needs it: more than 2^16 - 1 tiles along y included
+  bool gen = nty > 65535 || 8 * (g.ncell > g.nface[0] + g.nface[1] ? g.ncell : g.nface[0] + g.nface[1]) >= (1LL << 32);
+  for (int d = 0; d < 2; ++d) gen = gen || (g.periodic[d] && (g.n[d] < kRB || (g.n[d] & 1)));
+  const bool timed = tm && *tm->n < tm->cap;
+  if (tm && !timed) ++*tm->missed;
+  auto kern = gen ? hc_relax_pair_kernel<T, MODE, true> : hc_relax_pair_kernel<T, MODE, false>;
+  hipExtLaunchKernelGGL(kern, gen ? dim3(unsigned(ntx) * unsigned(nty)) : dim3(ntx, nty), dim3(kRBThreads), 0, s, timed ? tm->start[*tm->n] : nullptr,
+                        timed ? tm->stop[*tm->n] : nullptr, 0, P);
+  const hipError_t err = hipGetLastError();
+  if (err == hipSuccess && timed) {
+    *tm->bytes += relax_bytes(A, io);
+    ++*tm->n;
+  }
+  return err;
+}
+
+template <typename T>
+static hipError_t launch_relax_tile3(const HCArgs<T>& A, TileIO<T> io, hipStream_t s, const LaunchTimer* tm) {
   using D3 = HCRelaxTile3;
-  int nt = tiles_of<T, DIM>(A.g, io.ntx, io.nty);
-  const int pmax = relax_passes_per_launch<T, DIM>(A.g);
-  if (io.npass < 1 || io.npass > pmax) return hipErrorInvalidValue;
-  size_t lds = tile_lds<T, DIM>(io.npass, false);
-  if (DIM == 2 && pmax == 2) {
-    io.ntx = (A.g.n[0] + DW::TX - 1) / DW::TX;
-    io.nty = (A.g.n[1] + DW::TY - 1) / DW::TY;
-    nt = io.ntx * io.nty;
-    lds = 4 * size_t(DW::TX + 2 * io.npass) * (DW::TY + 2 * io.npass) * sizeof(T);
-  }
-  if (DIM == 3) {
-    io.ntx = (A.g.n[0] + D3::TX - 1) / D3::TX;
-    io.nty = (A.g.n[1] + D3::TY - 1) / D3::TY;
-    nt = io.ntx * io.nty * ((A.g.n[2] + D3::TZ - 1) / D3::TZ);
-    lds = 4 * size_t(D3::TX + 2 * io.npass) * (D3::TY + 2 * io.npass) * (D3::TZ + 2 * io.npass) * sizeof(T);
-  }
+  if (io.npass < 1 || io.npass > 2) return hipErrorInvalidValue;
+  io.ntx = (A.g.n[0] + D3::TX - 1) / D3::TX;
+  io.nty = (A.g.n[1] + D3::TY - 1) / D3::TY;
+  const int nt = io.ntx * io.nty * ((A.g.n[2] + D3::TZ - 1) / D3::TZ);
+  const size_t lds = 4 * size_t(D3::TX + 2 * io.npass) * (D3::TY + 2 * io.npass) * (D3::TZ + 2 * io.npass) * sizeof(T);
   if (lds > kMaxLds) return hipErrorInvalidValue;
   const bool timed = tm && *tm->n < tm->cap;
   if (tm && !timed) ++*tm->missed;
-  hipEvent_t e0 = timed ? tm->start[*tm->n] : nullptr, e1 = timed ? tm->stop[*tm->n] : nullptr;
-  if constexpr (DIM == 2) {
-    if (pmax == 8)
-      hipExtLaunchKernelGGL((hc_relax_tile_kernel<T, DIM, D::TX, D::TY, D::TZ, 8, 512>), dim3(nt), dim3(512), lds,
-                            s, e0, e1, 0, A, io);
-    else
-      hipExtLaunchKernelGGL((hc_relax_tile_kernel<T, DIM, DW::TX, DW::TY, DW::TZ, 2, DW::NT>), dim3(nt), dim3(DW::NT),
-                            lds, s, e0, e1, 0, A, io);
-  } else {
-    hipExtLaunchKernelGGL((hc_relax_tile_kernel<T, DIM, D3::TX, D3::TY, D3::TZ, 2, D3::NT>), dim3(nt), dim3(D3::NT),
-                          lds, s, e0, e1, 0, A, io);
-  }
+  hipExtLaunchKernelGGL((hc_relax_tile_kernel<T, 3, D3::TX, D3::TY, D3::TZ, 2, D3::NT>), dim3(nt), dim3(D3::NT), lds,
+                        s, timed ? tm->start[*tm->n] : nullptr, timed ? tm->stop[*tm->n] : nullptr, 0, A, io);
   const hipError_t err = hipGetLastError();
   if (err == hipSuccess && timed) {
-    // algorithmic bytes: state (2 comps) in and out, rhs, a, faces (2 comps)
-    // once each; the coarse state (and its initial copy) when prolonged on
-    // load
-    const double cells = double(A.g.nvalid());
-    double faces = 0;
-    for (int d = 0; d < DIM; ++d) faces += double(A.g.nface[d]);
-    double b = 2 * cells + 2 * cells + (A.a ? 2 * cells : 0) + 2 * faces + 2 * cells;
-    if (io.pc) b += 2 * io.gc.nvalid() * (io.pc0 ? 2 : 1);
-    *tm->bytes += b * sizeof(T);
+    *tm->bytes += relax_bytes(A, io);
     ++*tm->n;
   }
   return err;
@@ -1236,7 +1686,7 @@ hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T
   if (!pc && npass > 0 && hc_streams(A.g))
     return A.g.dim == 2 ? hc_relax_stream<T, 2>(A, buf, cur, rhs, npass, first, s, tm)
                         : hc_relax_stream<T, 3>(A, buf, cur, rhs, npass, first, s, tm);
-  const int pmax = A.g.dim == 2 ? relax_passes_per_launch<T, 2>(A.g) : relax_passes_per_launch<T, 3>(A.g);
+  const int pmax = relax_passes_per_launch(A.g);
   int done = 0;
   while (done < npass) {
     TileIO<T> io{};
@@ -1250,7 +1700,7 @@ hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T
       io.pc = pc;
       io.pc0 = pc0;
     }
-    hipError_t e = A.g.dim == 2 ? launch_relax_tile<T, 2>(A, io, s, tm) : launch_relax_tile<T, 3>(A, io, s, tm);
+    hipError_t e = A.g.dim == 2 ? launch_relax_pair<T, RB_PLAIN>(A, io, s, tm) : launch_relax_tile3<T>(A, io, s, tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += io.npass;
@@ -1267,6 +1717,68 @@ hipError_t hc_relax(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs,
                     hipStream_t s, const LaunchTimer* tm) {
   if (npass <= 0) return hipSuccess;
   return hc_relax_tiles<T>(A, buf, cur, rhs, npass, first, nullptr, nullptr, nullptr, s, tm);
+}
+
+bool hc_fuses(const Geom& g) { return g.dim == 2 && !hc_streams(g); }
+
+template <typename T>
+hipError_t hc_relax_restrict(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, T* rhs_out, int npass,
+                             const Geom& gc, T* resc, T* phic, T* phic0, hipStream_t s) {
+  if (npass < 1 || rhs_out == rhs) return hipErrorInvalidValue;
+  const int pmax = relax_passes_per_launch(A.g);
+  for (int done = 0; done < npass;) {
+    TileIO<T> io{};
+    io.phi = buf[*cur];
+    io.phi_out = buf[1 - *cur];
+    io.rhs = done && rhs_out ? rhs_out : rhs;
+    io.rhs_out = done ? nullptr : rhs_out;
+    io.npass = (npass - done) < pmax ? (npass - done) : pmax;
+    io.first = done & 1;
+    const bool end = done + io.npass == npass;
+    if (end) {
+      io.gc = gc;
+      io.out = resc;
+      io.phic = phic;
+      io.phic0 = phic0;
+    }
+    const hipError_t e = end ? launch_relax_pair<T, RB_RESTRICT>(A, io, s, nullptr)
+                             : launch_relax_pair<T, RB_PLAIN>(A, io, s, nullptr);
+    if (e != hipSuccess) return e;
+    *cur = 1 - *cur;
+    done += io.npass;
+  }
+  return hipSuccess;
+}
+
+template <typename T>
+hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, const Geom* gc,
+                          const T* pc, const T* pc0, unsigned long long* norm, const CtlFuse& fuse, hipStream_t s) {
+  if (npass < 1) return hipErrorInvalidValue;
+  const int pmax = relax_passes_per_launch(A.g);
+  for (int done = 0; done < npass;) {
+    TileIO<T> io{};
+    io.phi = buf[*cur];
+    io.phi_out = buf[1 - *cur];
+    io.rhs = rhs;
+    io.npass = (npass - done) < pmax ? (npass - done) : pmax;
+    io.first = done & 1;
+    if (done == 0 && pc) {
+      io.gc = *gc;
+      io.pc = pc;
+      io.pc0 = pc0;
+    }
+    const bool end = done + io.npass == npass;
+    if (end) {
+      io.norm = norm;
+      io.fuse = fuse;
+    }
+    const hipError_t e =
+        end ? launch_relax_pair<T, RB_NORM>(A, io, s, nullptr) : launch_relax_pair<T, RB_PLAIN>(A, io, s, nullptr);
+    if (e != hipSuccess) return e;
+    *cur = 1 - *cur;
+    done += io.npass;
+  }
+  return hipSuccess;
 }
 
 template <typename T>
@@ -1360,6 +1872,11 @@ template hipError_t hc_relax<double>(const HCArgs<double>&, double* const[2], in
 template hipError_t hc_relax_tiles<double>(const HCArgs<double>&, double* const[2], int*, const double*, int, int,
                                            const Geom*, const double*, const double*, hipStream_t,
                                            const LaunchTimer*);
+template hipError_t hc_relax_restrict<double>(const HCArgs<double>&, double* const[2], int*, const double*, double*,
+                                              int, const Geom&, double*, double*, double*, hipStream_t);
+template hipError_t hc_relax_final<double>(const HCArgs<double>&, double* const[2], int*, const double*, int,
+                                           const Geom*, const double*, const double*, unsigned long long*,
+                                           const CtlFuse&, hipStream_t);
 template hipError_t hc_coarse_vcycle<double>(const CoarseDesc<double>*, int, int, hipStream_t);
 template hipError_t hc_residual<double>(const HCArgs<double>&, double*, const double*, double*,
                                         unsigned long long*, int, hipStream_t, const CtlFuse&);

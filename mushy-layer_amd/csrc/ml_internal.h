@@ -159,7 +159,9 @@ class HCEngine {
 
  private:
   int init();
-  int vcycle(double* phi, const double* rhs, const ml_solve_opts& o, const int* skip);
+  // one V-cycle; *fused: its last launch also took the residual norm of
+  // level 0 into `slot` and applied the stopping rule
+  int vcycle(double* phi, const double* rhs, const ml_solve_opts& o, const int* skip, int slot, bool* fused);
   int residual_norm(double* phi, const double* rhs, int slot, const int* skip, bool check);
   int read_norm(int slot, double* out);
   int read_ctl(SolveCtl* out);
@@ -191,6 +193,7 @@ class HCEngine {
   ml_hc_op m_op;
   int m_L = 0, m_lc = 0;
   std::vector<double*> m_phi, m_rhs, m_phi0;   // per level (level 0: caller's arrays)
+  std::vector<double*> m_res;                  // restricted residual of the fused tiled levels (FAS rhs less L(phi))
   std::vector<double*> m_alt;                  // relax ping-pong partners (tiled levels, and level 0)
   std::vector<int> m_cur;                      // which of the pair holds the state
   double* m_rhs_be = nullptr;                   // backward-Euler rhs of level 0

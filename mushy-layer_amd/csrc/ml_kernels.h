@@ -162,6 +162,7 @@ struct TileIO {
   const T* pc;    // prolongation-on-load: coarse state ...
   const T* pc0;   // ... minus its initial value (nullable)
   int npass, first, homog, ntx, nty;
+  T* rhs_out;     // relax: rhs += L(phi) before the first pass, written here (nullable; != rhs)
 };
 
 // grid-stride indices: of a plain launch, or of workgroup b of the nb that
@@ -529,6 +530,20 @@ hipError_t hc_relax(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs,
 template <typename T>
 hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                           const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm = nullptr);
+// whether the two launches below serve level g (else the caller runs the
+// relaxation, restriction, operator and residual kernels one by one)
+bool hc_fuses(const Geom& g);
+// the way down of one FAS level: with rhs_out, rhs_out = rhs + L(phi) first
+// (the FAS right-hand side; rhs_out != rhs) and that is the equation relaxed;
+// npass >= 1 colour passes; then the restriction of hc_restrict_all
+template <typename T>
+hipError_t hc_relax_restrict(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, T* rhs_out, int npass,
+                             const Geom& gc, T* resc, T* phic, T* phic0, hipStream_t s);
+// hc_relax_tiles (npass >= 1) and the residual of the relaxed state: its
+// max-norm into *norm, with the stopping rule
+template <typename T>
+hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, const Geom* gc,
+                          const T* pc, const T* pc0, unsigned long long* norm, const CtlFuse& fuse, hipStream_t s);
 template <typename T>
 hipError_t hc_coarse_vcycle(const CoarseDesc<T>* dev_desc, int dim, int apply_first, hipStream_t s);
 template <typename T>

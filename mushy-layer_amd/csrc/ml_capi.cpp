@@ -328,11 +328,33 @@ int ml_hc_op_create(ml_ctx ctx, int dim, const int lo[], const int hi[], double 
     return fail(ctx, ML_ENOTSUP, "odd periodic length on a level of at most 1024 cells that does not coarsen");
   ml::Geom g0 = ml::make_geom(dim, n, periodic, dx);
   op->lev.resize(depth);
+  op->lc = depth;
+  for (int l = 0; l < depth; ++l) {
+    op->lev[l].g = l == 0 ? g0 : ml::coarsen_geom(g0, 1 << l);
+    if (op->lc == depth && op->lev[l].g.nvalid() <= ml::hc_coarse_cells()) op->lc = l;
+    if (l >= op->lc)
+      for (int d = 0; d < dim; ++d) op->ncfaces += 2 * size_t(op->lev[l].g.nface[d]);
+  }
+  if (op->lc < depth) {
+    void* p = nullptr;
+    op->ncfaces += op->ncfaces & 1;
+    if (hipMalloc(&p, sizeof(double) * op->ncfaces) != hipSuccess) {
+      ml_hc_op_destroy(op.release());
+      return fail(ctx, ML_ENOMEM, "hipMalloc bCoef");
+    }
+    op->cfaces = static_cast<double*>(p);
+    ml::vec_set((long long)op->ncfaces, op->cfaces, 0.0, ctx->stream);
+  }
+  double* cf = op->cfaces;
   for (int l = 0; l < depth; ++l) {
     ml::HCLevel& L = op->lev[l];
-    L.g = l == 0 ? g0 : ml::coarsen_geom(g0, 1 << l);
     for (int d = 0; d < dim; ++d) {
       void* p = nullptr;
+      if (l >= op->lc) {
+        L.b[d] = cf;
+        cf += 2 * L.g.nface[d];
+        continue;
+      }
       if (hipMalloc(&p, sizeof(double) * 2 * L.g.nface[d]) != hipSuccess) {
         ml_hc_op_destroy(op.release());
         return fail(ctx, ML_ENOMEM, "hipMalloc bCoef");
@@ -348,12 +370,14 @@ int ml_hc_op_create(ml_ctx ctx, int dim, const int lo[], const int hi[], double 
 int ml_hc_op_destroy(ml_hc_op op) {
   if (!op) return ML_EINVAL;
   if (op->ctx) hipStreamSynchronize(op->ctx->stream);
-  for (auto& L : op->lev) {
+  for (int l = 0; l < int(op->lev.size()); ++l) {
+    ml::HCLevel& L = op->lev[l];
     for (int d = 0; d < 3; ++d)
-      if (L.b[d]) hipFree(L.b[d]);
+      if (L.b[d] && l < op->lc) hipFree(L.b[d]);
     if (L.a) hipFree(L.a);
     if (L.tmp) hipFree(L.tmp);
   }
+  if (op->cfaces) hipFree(op->cfaces);
   if (op->adv) hipFree(op->adv);
   delete op;
   return ML_OK;

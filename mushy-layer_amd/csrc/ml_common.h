@@ -66,15 +66,15 @@ __host__ __device__ inline Geom coarsen_geom(const Geom& f, int ratio) {
 }
 
 // Closure constants (src/MushyLayerParams.h), and what the closure takes from
-// them once (closure_prepare; left as they are here, the closure divides
-// everywhere).
+// them once (closure_prepare; left as they are here, tolr sends every cell to
+// the divisions).
 template <typename T>
 struct ClosureP {
   T St, CR, pc, c, te, Te;
   T hs = T(0);           // solidus enthalpy where Theta is a number (c, pc > 0)
   T hes = T(0), hek = T(0);   // eutectic enthalpy ~ (CR + Theta)*hes + hek
   T tolr = T(NAN), tolk = T(0);   // ... which decides a regime further than |.|*tolr + tolk from it
-  T a2 = T(0), r2a = T(0);    // the porosity quadratic's 2a and its reciprocal (0: divide)
+  T a2 = T(0), r2a = T(0);    // the porosity quadratic's 2a and its reciprocal
   T a4 = T(0), kb = T(0), k1 = T(0), kc = T(0), kp = T(0);   // its 4a, CR(1-2c), 1-pc, c-1, pc*St
 };
 
@@ -109,7 +109,7 @@ __host__ __device__ inline T porosity_mush(T C, T H, const ClosureP<T>& p) {
   return (-b - sqrt(b * b - T(4) * a * q)) / (T(2) * a);
 }
 
-// porosity_mush with the prepared products (r2a != 0)
+// porosity_mush with the prepared products
 template <typename T>
 __host__ __device__ inline T porosity_mush_prepared(T C, T H, const ClosureP<T>& p) {
   const T validC = (C >= -p.CR) ? C : -p.CR;
@@ -127,26 +127,23 @@ __host__ __device__ inline T porosity_mush_prepared(T C, T H, const ClosureP<T>&
 __host__ inline void closure_prepare(ClosureP<double>& p) {
   auto moderate = [](double x) { return x == 0.0 || (fabs(x) > 1e-30 && fabs(x) < 1e30); };
   const double k1 = p.St + p.te * (1.0 - p.c), cre = p.CR + p.Te;
-  const bool ok = moderate(p.St) && moderate(p.CR) && moderate(p.pc) && moderate(p.c) && moderate(p.te) &&
-                  moderate(p.Te) && moderate(k1) && moderate(cre) && cre != 0.0;
-  if (!ok) return;
-  if (p.c > 0.0 && p.pc > 0.0) {
-    p.hs = p.te * p.c;
-    p.hes = k1 / cre;
-    p.hek = p.c * p.te;
-    p.tolr = 1e-14;
-    p.tolk = 1e-14 * fabs(p.hek) + 1e-290;
-  }
   const double a = p.CR * (p.c - 1.0) + p.St * (p.pc - 1.0);
-  if (moderate(a) && a != 0.0 && p.St != 0.0) {
-    p.a2 = 2.0 * a;
-    p.r2a = 1.0 / p.a2;
-    p.a4 = 4.0 * a;
-    p.kb = p.CR * (1.0 - 2.0 * p.c);
-    p.k1 = 1.0 - p.pc;
-    p.kc = p.c - 1.0;
-    p.kp = p.pc * p.St;
-  }
+  const bool ok = moderate(p.St) && moderate(p.CR) && moderate(p.pc) && moderate(p.c) && moderate(p.te) &&
+                  moderate(p.Te) && moderate(k1) && moderate(cre) && cre != 0.0 && moderate(a) && a != 0.0 &&
+                  p.St != 0.0 && p.c > 0.0 && p.pc > 0.0;
+  if (!ok) return;
+  p.hs = p.te * p.c;
+  p.hes = k1 / cre;
+  p.hek = p.c * p.te;
+  p.tolr = 1e-14;
+  p.tolk = 1e-14 * fabs(p.hek) + 1e-290;
+  p.a2 = 2.0 * a;
+  p.r2a = 1.0 / p.a2;
+  p.a4 = 4.0 * a;
+  p.kb = p.CR * (1.0 - 2.0 * p.c);
+  p.k1 = 1.0 - p.pc;
+  p.kc = p.c - 1.0;
+  p.kp = p.pc * p.St;
 }
 
 // CALCULATE_BOUNDING_ENERGY (src/EnthalpyVariablesF.ChF:657-698) followed by
@@ -159,10 +156,19 @@ __host__ inline void closure_prepare(ClosureP<double>& p) {
 template <typename T>
 __host__ __device__ inline void closure(T H, T C, const ClosureP<T>& p, T& theta, T& Cl) {
   const T hl = p.St - C + p.te + p.Te;
-  T hs = p.hs;
   const T pr = (p.CR + C) * p.hes;
   T he = pr + p.hek;
-  if (__builtin_expect(!(fabs(H - he) > fabs(pr) * p.tolr + p.tolk), 0)) {
+  const bool sure = fabs(H - he) > fabs(pr) * p.tolr + p.tolk;
+  // (one condition for the mush: a branch costs as much as four operations)
+  if (sure && H > he && H < hl && H > p.hs) {
+    const T chi = porosity_mush_prepared(C, H, p);
+    // one division: (-x)/y and -(x/y) are the same IEEE value
+    Cl = (C + p.CR * (T(1) - chi)) / (chi + p.pc * (T(1) - chi));
+    theta = -Cl;
+    return;
+  }
+  T hs = p.hs;
+  if (!sure) {
     if (C < -p.CR)
       hs = T(0);
     else
@@ -173,20 +179,18 @@ __host__ __device__ inline void closure(T H, T C, const ClosureP<T>& p, T& theta
     he = chie * (p.St + p.te * (T(1) - p.c)) + p.c * p.te;
   }
   const bool solid = H <= hs, eut = !solid && H > hs && H <= he;
-  if (!solid && !eut && H > he && H < hl) {
-    // (H and C are finite here, H between two numbers)
-    const T chi = p.r2a != T(0) ? porosity_mush_prepared(C, H, p) : porosity_mush(C, H, p);
-    // one division: (-x)/y and -(x/y) are the same IEEE value
+  if (!sure && !solid && !eut && H > he && H < hl) {
+    const T chi = porosity_mush(C, H, p);
     Cl = (C + p.CR * (T(1) - chi)) / (chi + p.pc * (T(1) - chi));
     theta = -Cl;
-  } else {
-    const bool liquid = H >= hl;
-    theta = eut ? p.te : (liquid ? H - p.St : T(NAN));
-    Cl = eut ? p.Te : (liquid ? C : T(NAN));
-    if (solid) {
-      theta = p.c == T(1) ? H : H / p.c;
-      Cl = p.Te;
-    }
+    return;
+  }
+  const bool liquid = H >= hl;
+  theta = eut ? p.te : (liquid ? H - p.St : T(NAN));
+  Cl = eut ? p.Te : (liquid ? C : T(NAN));
+  if (solid) {
+    theta = p.c == T(1) ? H : H / p.c;
+    Cl = p.Te;
   }
 }
 

@@ -26,7 +26,6 @@
 namespace ml {
 
 namespace {
-constexpr int kSmallCells = 1024;
 constexpr int kMaxHalvings = 6;   // FP32-refined step-length backtracking
 }
 
@@ -37,7 +36,6 @@ HCEngine::~HCEngine() {
   if (m_lindesc) hipFree(m_lindesc);
   if (m_hlindesc) hipHostFree(m_hlindesc);
   m_stage_lin.release();
-  m_stage_fas.release();
   for (size_t l = 1; l < m_phi.size(); ++l) {
     if (m_phi[l]) hipFree(m_phi[l]);
     if (m_rhs[l]) hipFree(m_rhs[l]);
@@ -49,8 +47,6 @@ HCEngine::~HCEngine() {
   if (m_rhs_be) hipFree(m_rhs_be);
   if (m_slots) hipFree(m_slots);
   if (m_hslots) hipHostFree(m_hslots);
-  if (m_desc) hipFree(m_desc);
-  if (m_hdesc) hipHostFree(m_hdesc);
   if (m_ctl) hipFree(m_ctl);
   if (m_arrive) hipFree(m_arrive);
   if (m_hctl) hipHostFree(m_hctl);
@@ -59,12 +55,7 @@ HCEngine::~HCEngine() {
 int HCEngine::init() {
   ml_ctx ctx = m_op->ctx;
   m_L = int(m_op->lev.size());
-  m_lc = m_L;
-  for (int l = 0; l < m_L; ++l)
-    if (m_op->lev[l].g.nvalid() <= kSmallCells) {
-      m_lc = l;
-      break;
-    }
+  m_lc = m_op->lc;
   m_phi.assign(m_L, nullptr);
   m_rhs.assign(m_L, nullptr);
   m_phi0.assign(m_L, nullptr);
@@ -106,10 +97,6 @@ int HCEngine::init() {
   m_slots = static_cast<unsigned long long*>(p);
   ML_HIP(ctx, hipHostMalloc(&p, sizeof(unsigned long long) * m_nslots, hipHostMallocDefault));
   m_hslots = static_cast<unsigned long long*>(p);
-  ML_HIP(ctx, hipMalloc(&p, sizeof(CoarseDesc<double>)));
-  m_desc = static_cast<CoarseDesc<double>*>(p);
-  ML_HIP(ctx, hipHostMalloc(&p, sizeof(CoarseDesc<double>), hipHostMallocDefault));
-  m_hdesc = static_cast<CoarseDesc<double>*>(p);
   ML_HIP(ctx, hipMalloc(&p, sizeof(SolveCtl)));
   m_ctl = static_cast<SolveCtl*>(p);
   ML_HIP(ctx, hipMalloc(&p, sizeof(unsigned int)));
@@ -147,34 +134,6 @@ int HCEngine::write_ctl(const SolveCtl& c) {
 
 // ------------------------------------------------------------------------
 // FP64 FAS.
-int HCEngine::upload_desc(double* phi0, const double* rhs0, const ml_solve_opts& o) {
-  ml_ctx ctx = m_op->ctx;
-  CoarseDesc<double> D;
-  std::memset(&D, 0, sizeof(D));
-  D.l0 = m_lc;
-  D.nlev = m_L;
-  D.nu1 = o.nu1;
-  D.nu2 = o.nu2;
-  D.bottom = o.bottom;
-  D.cp = m_op->cp;
-  D.bc = m_op->bc;
-  D.alpha = m_op->alpha;
-  D.beta = m_op->beta;
-  D.skip = &m_ctl->done;
-  for (int l = 0; l < m_L; ++l) {
-    LevelDesc<double>& L = D.lev[l];
-    L.g = m_op->lev[l].g;
-    L.phi = l == 0 ? phi0 : m_phi[l];
-    L.rhs = l == 0 ? const_cast<double*>(rhs0) : m_rhs[l];
-    L.phi0 = m_phi0[l];
-    L.tmp = nullptr;
-    L.a = m_op->lev[l].a;
-    for (int d = 0; d < 3; ++d) L.b[d] = m_op->lev[l].b[d];
-  }
-  ML_HIP(ctx, m_stage_fas.put(m_desc, m_hdesc, &D, sizeof(D), ctx->stream));
-  return ML_OK;
-}
-
 int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, const int* skip, int slot, bool* fused) {
   ml_ctx ctx = m_op->ctx;
   hipStream_t s = ctx->stream;
@@ -214,7 +173,22 @@ int HCEngine::vcycle(double* phi, const double* rhs, const ml_solve_opts& o, con
     if (l + 1 < m_lc && !next) ML_HIP(ctx, hc_apply_op<double>(args(l + 1), P(l + 1), R(l + 1), R(l + 1), 0, s));
   }
   if (m_lc < m_L) {
-    ML_HIP(ctx, hc_coarse_vcycle<double>(m_desc, m_op->dim, m_lc > 0 ? 1 : 0, s));
+    HCCoarse<double> C{};
+    C.skip = skip;
+    C.phi = m_lc == 0 ? phi : m_phi[m_lc];
+    C.rhs = R(m_lc);
+    C.faces = m_op->cfaces;
+    C.nfaces = int(m_op->ncfaces);
+    C.nl = m_L - m_lc;
+    for (int l = m_lc; l < m_L; ++l) C.a[l - m_lc] = m_op->lev[l].a;
+    C.nu1 = o.nu1;
+    C.nu2 = o.nu2;
+    C.bottom = o.bottom;
+    C.add_first = m_lc > 0 ? 1 : 0;
+    C.alpha = m_op->alpha;
+    C.beta = m_op->beta;
+    C.cp = m_op->cp;
+    ML_HIP(ctx, hc_coarse_vcycle<double>(m_op->lev[m_lc].g, m_op->bc, C, s));
   } else {
     // no level small enough for one workgroup: the coarsest tiled level is
     // the bottom
@@ -252,8 +226,7 @@ int HCEngine::solve(double* phi, const double* rhs, const ml_solve_opts& o, ml_s
   if (o.precision == ML_PRECISION_FP32_REFINED) return solve_refined(phi, rhs, o, st);
   if (o.max_iter + 1 > m_nslots) return fail(ctx, ML_EINVAL, "max_iter too large");
   if (o.nu1 < 0 || o.nu2 < 0 || o.bottom < 0) return fail(ctx, ML_EINVAL, "negative smoothing count");
-  int rc = upload_desc(phi, rhs, o);
-  if (rc) return rc;
+  int rc = 0;
   // the level-0 partner starts as a full copy (ghost cells included) so
   // that a state ending in it can be copied back whole
   const size_t bytes0 = sizeof(double) * 2 * m_op->lev[0].g.ncell;

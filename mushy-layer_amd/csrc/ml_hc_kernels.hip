@@ -21,8 +21,7 @@ namespace ml {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kWGThreads = 1024;   // single-workgroup kernel: one thread per cell ...
-constexpr int kWGCells = 1024;     // ... of the largest level it holds
+constexpr int kWGCells = 1024;   // largest level of the single-workgroup kernel
 
 enum : int { kResid = 1, kApply = 2, kRestrict = 3 };
 
@@ -754,364 +753,417 @@ __global__ __launch_bounds__(kThreads) void hc_apply_batch_kernel(const HCApplyJ
 }
 
 // ---------------------------------------------------------------------------
-// Single-workgroup V-cycle over the small levels (at most kWGCells cells):
-// thread t owns cell t of the current level; phi and phi_l of that level live
-// in LDS; neighbours are found by periodic wrap or the derived-variable wall
-// rule.  A relaxation pass updates one colour and recomputes the closure of
-// exactly the cells it updated (the other colour's phi_l is unchanged since
-// its own update), so each pass needs a single barrier and half the closures
-// of a full recomputation, with the same values.
-// The level's geometry is copied into registers: reads through the
-// descriptor pointer would be repeated after every barrier or wavefront fence
-// of the relaxation passes.
-template <typename T, int DIM>
-struct WGLevel {
-  const LevelDesc<T>* L;
-  int N, nx, nxy;
-  int n[3], per[3];
-  T dx;
-  long long ncell;
-  int c, i, j, k;
-  long long q;
-  bool own;
-  __device__ inline void init(const LevelDesc<T>* lv) {
-    L = lv;
-    const Geom& g = L->g;
-    for (int d = 0; d < 3; ++d) {
-      n[d] = g.n[d];
-      per[d] = g.periodic[d];
-    }
-    dx = T(g.dx);
-    ncell = g.ncell;
-    nx = n[0];
-    nxy = n[0] * n[1];
-    N = nxy * (DIM == 3 ? n[2] : 1);
-    c = threadIdx.x;
-    own = c < N;
-    int r, kk;
-    divmod_pos(c, nx, r, i);
-    divmod_pos(r, n[1], kk, j);
-    k = DIM == 3 ? kk : 0;
-    q = own ? g.ci(i, j, k) : 0;
-  }
-};
+// Single-workgroup FAS V-cycle over the small levels (at most kWGCells cells
+// and everything below).  All levels' state, right-hand side, initial state,
+// lambda and faces live in LDS for the whole cycle (at most 156 KB over all
+// shapes; the faces come as one contiguous block), so a level visit waits for
+// no global memory.
+//
+// A wavefront alone on its SIMD issues an operation every 8 cycles whether it
+// depends on the last one or not, and a branch costs four of them: the count
+// of instructions along a visit is what bounds it.  So each thread owns one
+// cell of each colour (an x pair; cells t and t + 512 where rows are odd)
+// with its faces, lambda, state and closure in registers; a wall's ghost is
+// written by its cell's owner with each update, into a slot that the stencil
+// reads like any neighbour; offsets come from the host; nothing is divided.
+// Levels whose pairs fit one wavefront are visited by wave 0 alone with
+// wavefront-scope syncs.  The visits are one runtime loop: every launch
+// fetches the code it runs.  Measured at 256^2 (levels 32^2 to 2^2): 65 us a
+// launch, 84 us with one cell per lane and the levels' data in global memory;
+// 3D (12x8x6 down) 87 against 180 us.
+//
+// A pass updates one colour and recomputes the closure of exactly the cells
+// it updated (the other colour's is unchanged since its own update).  The
+// bottom relaxation ends after the first red/black iteration that leaves
+// every cell's state unchanged to the bit: each later one would repeat it.
+constexpr int kHCWG = 512;
 
-// The descriptor's scalars that every pass uses, in registers for the same
-// reason.
-template <typename T>
-struct WGConst {
-  const BCDesc* bc;   // read at wall cells only
-  ClosureP<T> cp;
-  T alpha, beta;
-  __device__ inline void init(const CoarseDesc<T>& D) {
-    bc = &D.bc;
-    cp = D.cp;
-    alpha = D.alpha;
-    beta = D.beta;
-  }
-};
-
-template <typename T, int DIM>
-__device__ inline void wg_stencil(const WGLevel<T, DIM>& W, const BCDesc& bc, const T* pl, int n, T* p) {
-  // without branches on the cell's position: the cells of one colour lie on
-  // different sides of the walls, so branches would diverge in a wavefront.
-  // Across a wall the load reads the cell itself and the ghost formula's
-  // result is selected; the values are those of the branching form.
-  const int c = W.c;
-  const int iv[3] = {W.i, W.j, W.k};
-  const T x0 = pl[c];
-  p[0] = x0;
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    const int nd = W.n[d];
-    const int st = d == 0 ? 1 : (d == 1 ? W.nx : W.nxy);
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int v = iv[d] + (s ? 1 : -1);
-      const bool inside = v >= 0 && v < nd;
-      const bool wall = !inside && !W.per[d];
-      const int off = inside ? (s ? st : -st) : (wall ? 0 : (s ? -(nd - 1) * st : (nd - 1) * st));
-      const T nb = pl[c + off];
-      const T gh = bc_ghost<T>(bc.type[d][s][n], T(bc.val[d][s][n]), x0, s ? 1 : -1, W.dx);
-      p[1 + 2 * d + (s ? 0 : 1)] = (wall && bc.apply) ? gh : nb;
-    }
-  }
-}
-
-// closure of the thread's own cell from its LDS state
-template <typename T, int DIM>
-__device__ inline void wg_closure_own(const ClosureP<T>& cp, const WGLevel<T, DIM>& W, const T* sphi, T* sphl) {
-  if (!W.own) return;
-  T th, cl;
-  closure<T>(sphi[W.c], sphi[W.N + W.c], cp, th, cl);
-  sphl[W.c] = th;
-  sphl[W.N + W.c] = cl;
-}
-
-template <typename T, int DIM>
-__device__ inline void wg_faces(const LevelDesc<T>* L, int i, int j, int k, CellFaces<T, DIM>& F, T* aq) {
-  load_faces<T, DIM>(L->g, L->b, i, j, k, F);
-  const long long q = L->g.ci(i, j, k);
-  aq[0] = L->a ? L->a[q] : T(1);
-  aq[1] = L->a ? L->a[q + L->g.ncell] : T(1);
-}
-
-// L(phi) of the thread's cell (both components) from phi/phi_l in LDS
-template <typename T, int DIM>
-__device__ inline void wg_lof(const WGConst<T>& K, const WGLevel<T, DIM>& W, const CellFaces<T, DIM>& F,
-                              const T* aq, const T* sphi, const T* sphl, T* lof) {
-  const T dxinv = T(1) / (W.dx * W.dx);
-#pragma unroll
-  for (int n = 0; n < 2; ++n) {
-    T st[7];
-    wg_stencil<T, DIM>(W, *K.bc, sphl + n * W.N, n, st);
-    lof[n] = lof_of<T, DIM>(F, n, st, aq[n], sphi[n * W.N + W.c], K.alpha, K.beta, dxinv);
-  }
-}
-
-// Per-level operator data of the thread's cell, held in registers.
-template <typename T, int DIM>
-struct WGCellOp {
-  CellFaces<T, DIM> F;
-  T aq[2], lam[2];
-  __device__ inline void load(const WGConst<T>& K, const WGLevel<T, DIM>& W) {
-    if (!W.own) return;
-    wg_faces<T, DIM>(W.L, W.i, W.j, W.k, F, aq);
-    const T scale = T(1) / (W.dx * W.dx);
-    lam[0] = lambda_of<T, DIM>(F, 0, aq[0], K.alpha, K.beta, scale);
-    lam[1] = lambda_of<T, DIM>(F, 1, aq[1], K.alpha, K.beta, scale);
-  }
-};
-
-// npass colour passes (first colour red) on the level whose phi is staged in
-// sphi and whose phi_l (closure of sphi) is staged in sphl; rr = rhs of the
-// thread's cell.  Leaves sphi/sphl consistent and writes phi to global memory.
-// With fixed_stop, the passes end after the first red/black iteration that
-// leaves every cell's state unchanged to the bit: each later iteration would
-// start from the same state and repeat it exactly, so the result is that of
-// all npass passes.
-template <typename T, int DIM>
-__device__ void wg_relax(const WGConst<T>& K, const WGLevel<T, DIM>& W, const WGCellOp<T, DIM>& O,
-                         const T* rr, T* sphi, T* sphl, int npass, bool fixed_stop = false) {
-  bool changed = false;
-  auto pass = [&](int p) {
-    if (W.own && !((W.i + W.j + W.k + p) & 1)) {
-      T lof[2];
-      wg_lof<T, DIM>(K, W, O.F, O.aq, sphi, sphl, lof);
-      const int c = W.c;
-      const T h0 = sphi[c], t0 = sphi[W.N + c];
-      const T h = h0 - O.lam[0] * (lof[0] - rr[0]);
-      const T t = t0 - O.lam[1] * (lof[1] - rr[1]);
-      changed = changed || bits_of(h) != bits_of(h0) || bits_of(t) != bits_of(t0);
-      sphi[c] = h;
-      sphi[W.N + c] = t;
-      T th, cl;
-      closure<T>(h, t, K.cp, th, cl);
-      sphl[c] = th;
-      sphl[W.N + c] = cl;
-    }
+// linear prolongation from LDS: e(x, y, z) the coarse correction
+template <typename T, int DIM, class E>
+__device__ __forceinline__ T prolong_lds(const int* nc, const int* per, int i, int j, int k, E e, T p) {
+  const T den = T(1) / (DIM == 3 ? T(64) : T(16));
+  const T fx1 = T(3) * den, fx2 = T(9) * den, fx3 = T(27) * den, f0 = T(1) * den;
+  auto outer = [&](int v, int d) {
+    const int c = v >> 1, o = c + ((v & 1) ? 1 : -1), n = nc[d];
+    return o < 0 ? (per[d] ? n - 1 : 0) : (o >= n ? (per[d] ? 0 : n - 1) : o);
   };
-  if (W.N <= 64) {
-    // every cell is owned by wave 0: it runs the passes alone, synchronising
-    // at wavefront scope; the other waves wait once
-    if (threadIdx.x < 64)
-      for (int p = 0; p < npass; ++p) {
-        pass(p);
-        wave_sync();
-        if (fixed_stop && (p & 1)) {
-          if (!__any(changed)) break;
-          changed = false;
-        }
-      }
-    __syncthreads();
+  const int X0 = i >> 1, Y0 = j >> 1, Z0 = DIM == 3 ? k >> 1 : 0;
+  const int X1 = outer(i, 0), Y1 = outer(j, 1), Z1 = DIM == 3 ? outer(k, 2) : 0;
+  if (DIM == 2) {
+    p = p + fx2 * e(X0, Y0, 0) + f0 * e(X1, Y1, 0);
+    p = p + fx1 * (e(X1, Y0, 0) + e(X0, Y1, 0));
   } else {
-    for (int p = 0; p < npass; ++p) {
-      pass(p);
-      if (fixed_stop && (p & 1)) {
-        if (!__syncthreads_or(changed)) break;
-        changed = false;
-      } else {
-        __syncthreads();
-      }
-    }
+    p = p + fx3 * e(X0, Y0, Z0) + f0 * e(X1, Y1, Z1);
+    p = p + fx2 * (e(X1, Y0, Z0) + e(X0, Y1, Z0) + e(X0, Y0, Z1));
+    p = p + fx1 * (e(X1, Y1, Z0) + e(X0, Y1, Z1) + e(X1, Y0, Z1));
   }
-  if (W.own) {
-    W.L->phi[W.q] = sphi[W.c];
-    W.L->phi[W.q + W.ncell] = sphi[W.N + W.c];
-  }
+  return p;
 }
 
-// stage the thread's (phi) into LDS and compute every closure
 template <typename T, int DIM>
-__device__ inline void wg_stage(const WGConst<T>& K, const WGLevel<T, DIM>& W, const T* ph, T* sphi, T* sphl) {
-  if (W.own) {
-    sphi[W.c] = ph[0];
-    sphi[W.N + W.c] = ph[1];
-  }
-  __syncthreads();
-  wg_closure_own<T, DIM>(K.cp, W, sphi, sphl);
-  __syncthreads();
-}
-
-// Coarse part of the FAS V-cycle (levels l0 .. nlev-1) in one workgroup:
-//   rhs_l0 += L(phi_l0) when apply_first (the restriction into l0 was done by
-//   the finer level's kernel); then for l = l0 .. nlev-2: relax nu1; restrict
-//   phi and rhs - L phi; rhs_{l+1} += L(phi_{l+1}); bottom relax; then back
-//   up: phi_l += P(phi_{l+1} - phi0_{l+1}); relax nu2.
-// Levels are visited with their state in registers/LDS; global memory keeps
-// phi, rhs and phi0 of every level for the way back up and for the finer
-// tiled levels.
-template <typename T, int DIM>
-__global__ __launch_bounds__(kWGThreads) void hc_coarse_vcycle_kernel(const CoarseDesc<T>* __restrict__ Dp,
-                                                                      int apply_first) {
+__global__ __launch_bounds__(kHCWG) void hc_coarse_vcycle_kernel(HCCoarse<T> A) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
-  const CoarseDesc<T>& D = *Dp;
-  if (D.skip && *D.skip) return;
-  WGConst<T> K;
-  K.init(D);
-  const int nu1 = D.nu1, nu2 = D.nu2, bottom = D.bottom;
-  T* sphi = reinterpret_cast<T*>(smem_raw);   // 2*kWGCells
-  T* sphl = sphi + 2 * kWGCells;              // 2*kWGCells
-  T* se = sphl + 2 * kWGCells;                // coarse correction, 2*kWGCells/4
-  const int l0 = D.l0, L = D.nlev;
-  const T denom = DIM == 3 ? T(8) : T(4);
-
-  // state of the current level's cell in registers
-  T ph[2] = {T(0), T(0)}, rr[2] = {T(0), T(0)};
-  // `staged`: sphi/sphl already hold the current level's state and closures
-  // and `Oc` its operator data (loaded with its FAS right-hand side), so the
-  // level visit that follows neither reloads nor restages them
-  WGCellOp<T, DIM> Oc;
-  bool staged = false;
-  {
-    WGLevel<T, DIM> W;
-    W.init(&D.lev[l0]);
-    if (W.own) {
-      ph[0] = W.L->phi[W.q];
-      ph[1] = W.L->phi[W.q + W.L->g.ncell];
-      rr[0] = W.L->rhs[W.q];
-      rr[1] = W.L->rhs[W.q + W.L->g.ncell];
-    }
-    if (apply_first) {
-      Oc.load(K, W);
-      wg_stage<T, DIM>(K, W, ph, sphi, sphl);
-      if (W.own) {
-        T lof[2];
-        wg_lof<T, DIM>(K, W, Oc.F, Oc.aq, sphi, sphl, lof);
-        rr[0] = rr[0] + lof[0];
-        rr[1] = rr[1] + lof[1];
-        W.L->rhs[W.q] = rr[0];
-        W.L->rhs[W.q + W.L->g.ncell] = rr[1];
-      }
-      __syncthreads();
-      staged = true;
-    }
-  }
-
-  for (int l = l0; l < L - 1; ++l) {
-    WGLevel<T, DIM> W;
-    W.init(&D.lev[l]);
-    if (!staged) {
-      Oc.load(K, W);
-      wg_stage<T, DIM>(K, W, ph, sphi, sphl);
-    }
-    const WGCellOp<T, DIM>& O = Oc;   // reloaded below for the coarser level after its last use
-    wg_relax<T, DIM>(K, W, O, rr, sphi, sphl, 2 * nu1);
-    // restriction (RESTRICTRESNLVC / RESTRICT): each fine cell's
-    // (rhs - L phi)/2^d and phi/2^d, then child sums in Fortran order
-    T tr[2] = {T(0), T(0)}, tp[2] = {T(0), T(0)};
-    if (W.own) {
-      T lof[2];
-      wg_lof<T, DIM>(K, W, O.F, O.aq, sphi, sphl, lof);
-      tr[0] = (rr[0] - lof[0]) / denom;
-      tr[1] = (rr[1] - lof[1]) / denom;
-      tp[0] = sphi[W.c] / denom;
-      tp[1] = sphi[W.N + W.c] / denom;
-    }
-    __syncthreads();
-    if (W.own) {
-      sphl[W.c] = tr[0];
-      sphl[W.N + W.c] = tr[1];
-      sphi[W.c] = tp[0];
-      sphi[W.N + W.c] = tp[1];
-    }
-    __syncthreads();
-    WGLevel<T, DIM> Wc;
-    Wc.init(&D.lev[l + 1]);
-    if (Wc.own) {
-      T s[2] = {T(0), T(0)}, sp[2] = {T(0), T(0)};
-      for (int kk = 0; kk < (DIM == 3 ? 2 : 1); ++kk)
-        for (int jj = 0; jj < 2; ++jj)
-          for (int ii = 0; ii < 2; ++ii) {
-            const int fc = (2 * Wc.i + ii) + W.nx * (2 * Wc.j + jj) + W.nxy * (DIM == 3 ? 2 * Wc.k + kk : 0);
+  typedef T vec2 __attribute__((ext_vector_type(2)));
+  const int tid = threadIdx.x;
+  const int nl = A.nl, tot = A.tot, N0 = A.off[1], tot1 = tot - N0;
+  T* P = reinterpret_cast<T*>(smem_raw);   // state [2][tot]
+  T* R = P + 2 * tot;                       // right-hand side [2][tot]
+  T* P0 = R + 2 * tot;                      // initial state of the levels below the first [2][tot1]
+  T* SL = P0 + 2 * tot1;                    // closure of the level [2][kWGCells], then ...
+  constexpr int CS = kWGCells;              // (component stride of both)
+  T* SX = SL + 2 * CS;                      // ... wall ghosts of the owners' cells, or the restriction terms
+  T* FC = SX + 2 * CS;                      // faces, as the block holds them
+  T* LM = FC + A.nfaces;                    // lambda [2][tot], kept for the way up (nl > 1)
+  // ghost rule of every wall face f = 2d + s on the first level: s, b per
+  // component; one more entry of zeros for cells without a wall
+  __shared__ T GT[2 * DIM + 1][4];
+  // first level's state and right-hand side, and the faces: loads first
+  const long long sy = A.n[0] + 2, sz = sy * (A.n[1] + 2), nc0 = sz * (DIM == 3 ? A.n[2] + 2 : 1);
+  auto level_of = [&](int l) __attribute__((always_inline)) {
+    CLev L;
+    for (int d = 0; d < 3; ++d) L.n[d] = d < DIM ? A.n[d] >> l : 1;
+    L.nx = L.n[0];
+    L.nxy = L.n[0] * L.n[1];
+    L.off = A.off[l];
+    L.N = A.off[l + 1] - L.off;
+    return L;
+  };
+  const CLev L0 = level_of(0);
 #pragma unroll
-            for (int n = 0; n < 2; ++n) {
-              s[n] = s[n] + sphl[n * W.N + fc];
-              sp[n] = sp[n] + sphi[n * W.N + fc];
-            }
-          }
-      const long long qc = Wc.q;
-      const long long ncc = Wc.L->g.ncell;
+  for (int f = 0; f <= 2 * DIM; ++f)
+    if (tid == f) {
 #pragma unroll
       for (int n = 0; n < 2; ++n) {
-        Wc.L->phi[qc + n * ncc] = sp[n];
-        Wc.L->phi0[qc + n * ncc] = sp[n];
+        GT[f][2 * n] = f < 2 * DIM ? A.gs[f >> 1][f & 1][n] : T(0);
+        GT[f][2 * n + 1] = f < 2 * DIM ? A.gb[f >> 1][f & 1][n] : T(0);
       }
-      ph[0] = sp[0];
-      ph[1] = sp[1];
-      rr[0] = s[0];
-      rr[1] = s[1];
     }
-    __syncthreads();
-    // FAS coarse right-hand side rhs_{l+1} += L(phi_{l+1})
-    {
-      Oc.load(K, Wc);
-      wg_stage<T, DIM>(K, Wc, ph, sphi, sphl);
-      if (Wc.own) {
-        T lof[2];
-        wg_lof<T, DIM>(K, Wc, Oc.F, Oc.aq, sphi, sphl, lof);
-        rr[0] = rr[0] + lof[0];
-        rr[1] = rr[1] + lof[1];
-        Wc.L->rhs[Wc.q] = rr[0];
-        Wc.L->rhs[Wc.q + Wc.L->g.ncell] = rr[1];
-      }
-      __syncthreads();
-      staged = true;
+  long long q0[2];
+  T h0[2][2], r0[2][2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int c = tid + m * kHCWG;
+    if (c >= N0) continue;
+    int i, j, k;
+    clev_coords(L0, c, i, j, k);
+    q0[m] = (i + 1) + sy * (j + 1) + (DIM == 3 ? sz * (k + 1) : 0);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      h0[m][n] = A.phi[q0[m] + n * nc0];
+      r0[m][n] = A.rhs[q0[m] + n * nc0];
     }
   }
   {
-    WGLevel<T, DIM> W;
-    W.init(&D.lev[L - 1]);
-    if (!staged) {
-      Oc.load(K, W);
-      wg_stage<T, DIM>(K, W, ph, sphi, sphl);
+    constexpr int KF = 6;
+    const vec2* src = reinterpret_cast<const vec2*>(A.faces);
+    vec2* dst = reinterpret_cast<vec2*>(FC);
+    const int n2 = A.nfaces >> 1;
+#pragma unroll 1
+    for (int base = tid; base < n2; base += KF * kHCWG) {
+      vec2 v[KF];
+#pragma unroll
+      for (int k = 0; k < KF; ++k)
+        if (base + k * kHCWG < n2) v[k] = src[base + k * kHCWG];
+#pragma unroll
+      for (int k = 0; k < KF; ++k)
+        if (base + k * kHCWG < n2) dst[base + k * kHCWG] = v[k];
     }
-    wg_relax<T, DIM>(K, W, Oc, rr, sphi, sphl, 2 * bottom, true);
   }
-  for (int l = L - 2; l >= l0; --l) {
-    // coarse correction phi_{l+1} - phi0_{l+1} into LDS (compact layout)
-    WGLevel<T, DIM> Wc;
-    Wc.init(&D.lev[l + 1]);
-    if (Wc.own) {
-      const long long ncc = Wc.L->g.ncell;
-      se[Wc.c] = sphi[Wc.c] - Wc.L->phi0[Wc.q];
-      se[Wc.N + Wc.c] = sphi[Wc.N + Wc.c] - Wc.L->phi0[Wc.q + ncc];
+  if (A.skip && *A.skip) return;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int c = tid + m * kHCWG;
+    if (c >= N0) continue;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      P[n * tot + c] = h0[m][n];
+      R[n * tot + c] = r0[m][n];
     }
-    __syncthreads();
-    WGLevel<T, DIM> W;
-    W.init(&D.lev[l]);
-    WGCellOp<T, DIM> O;
-    O.load(K, W);
-    if (W.own) {
-      const long long nc = W.L->g.ncell;
-      rr[0] = W.L->rhs[W.q];
-      rr[1] = W.L->rhs[W.q + nc];
-      ph[0] = prolong_value_lds<T, DIM>(Wc.L->g, W.i, W.j, W.k, se, W.L->phi[W.q]);
-      ph[1] = prolong_value_lds<T, DIM>(Wc.L->g, W.i, W.j, W.k, se + Wc.N, W.L->phi[W.q + nc]);
+  }
+  __syncthreads();
+  const T rdenom = DIM == 3 ? T(0.125) : T(0.25);   // (a division by 2^d is this product)
+
+#pragma unroll 1
+  for (int v = 0; v < 2 * nl - 1; ++v) {
+    const bool up = v >= nl, bot = v == nl - 1, down = v < nl - 1;
+    const int l = up ? 2 * nl - 2 - v : v;
+    const CLev L = level_of(l);
+    const int off = L.off, offc = off + L.N;
+    const bool even = (L.nx & 1) == 0;
+    const bool small = cown_active<kHCWG>(L) <= 64;
+    const int step = small ? 64 : kHCWG;   // threads of this visit
+    const T lsc = T(1 << l);
+    const T dx = A.dx * lsc;
+    const T dxinv = T(1) / (dx * dx);
+    auto sync = [&]() __attribute__((always_inline)) {
+      if (small)
+        wave_sync();
+      else
+        __syncthreads();
+    };
+    int fo[DIM], nf[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) {
+      fo[d] = A.fo[l][d];
+      nf[d] = A.nf[l][d];
     }
-    __syncthreads();
-    wg_stage<T, DIM>(K, W, ph, sphi, sphl);
-    wg_relax<T, DIM>(K, W, O, rr, sphi, sphl, 2 * nu2);
+    if (!small || tid < 64) {
+      // state (on the way up with the prolonged correction) and closure, one
+      // cell per thread
+#pragma unroll 1
+      for (int c = tid; c < L.N; c += step) {
+        T ph[2] = {P[off + c], P[tot + off + c]};
+        if (up) {
+          int i, j, k;
+          clev_coords(L, c, i, j, k);
+          const int nc[3] = {L.n[0] >> 1, L.n[1] >> 1, L.n[2] >> 1};
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            const T* pc = P + n * tot + offc;
+            const T* p0 = P0 + n * tot1 + (offc - N0);
+            auto e = [&](int x, int y, int z) -> T {
+              const int q = x + nc[0] * (y + nc[1] * z);
+              return pc[q] - p0[q];
+            };
+            ph[n] = prolong_lds<T, DIM>(nc, A.per, i, j, k, e, ph[n]);
+            P[n * tot + off + c] = ph[n];
+          }
+        }
+        T th, cl;
+        closure<T>(ph[0], ph[1], A.cp, th, cl);
+        SL[c] = th;
+        SL[CS + c] = cl;
+      }
+      sync();
+      // the thread's cell of each colour: neighbours, faces, lambda, right-
+      // hand side, state, closure
+      COwn o;
+      cown_set<kHCWG>(L, o);
+      int c[2], nb[2][2 * DIM], col[2], wall[2];
+      bool multi[2] = {false, false};
+      CellFaces<T, DIM> F[2];
+      T ph[2][2], pl[2][2], rr[2][2], aa[2][2], lam[2][2], ws[2][2], wb[2][2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        c[m] = 0;
+        if (o.p[m] < 0) continue;
+        int i, j, k;
+        cunpack(o.p[m], i, j, k);
+        c[m] = i + L.nx * j + L.nxy * k;
+        col[m] = (i + j + k) & 1;
+        // the first wall's ghost lives in the owner's slot of SX, rewritten
+        // with each update; further walls of the cell are formed on reading
+        const int slot = 2 * CS + m * kHCWG + tid;
+        const int iv[3] = {i, j, k};
+        int first = 2 * DIM;
+        wall[m] = 0;
+#pragma unroll
+        for (int d = DIM - 1; d >= 0; --d) {
+          const int st = d == 0 ? 1 : (d == 1 ? L.nx : L.nxy);
+          const int nd = L.n[d];
+          const int w = A.per[d] ? 0 : 1;
+          const bool lo = iv[d] == 0, hi = iv[d] == nd - 1;
+          nb[m][2 * d] = lo ? (w ? slot : c[m] + (nd - 1) * st) : c[m] - st;
+          nb[m][2 * d + 1] = hi ? (w ? slot : c[m] - (nd - 1) * st) : c[m] + st;
+          if (w && (lo || hi)) {
+            wall[m] |= (lo ? 1 << (2 * d) : 0) | (hi ? 2 << (2 * d) : 0);
+            first = lo ? 2 * d : 2 * d + 1;
+          }
+        }
+        wall[m] &= wall[m] - 1;   // (first is the lowest)
+        multi[m] = wall[m] != 0;
+        const T lsw = lsc;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          ws[m][n] = GT[first][2 * n];
+          const T b = GT[first][2 * n + 1];
+          wb[m][n] = ws[m][n] < T(0) ? b : b * lsw;   // a Neumann constant scales with dx
+        }
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) {
+          const int fx = L.n[0] + (d == 0), fy = L.n[1] + (d == 1);
+          const int at = fo[d] + i + fx * (j + (DIM == 3 ? fy * k : 0));
+          const int st = d == 0 ? 1 : (d == 1 ? fx : fx * fy);
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            F[m].v[n][2 * d] = FC[at + n * nf[d]];
+            F[m].v[n][2 * d + 1] = FC[at + n * nf[d] + st];
+          }
+        }
+        aa[m][0] = aa[m][1] = T(1);
+        if (A.a[l]) {
+          const long long lsy = L.n[0] + 2, lsz = lsy * (L.n[1] + 2);
+          const long long q = (i + 1) + lsy * (j + 1) + (DIM == 3 ? lsz * (k + 1) : 0);
+          aa[m][0] = A.a[l][q];
+          aa[m][1] = A.a[l][q + lsz * (DIM == 3 ? L.n[2] + 2 : 1)];
+        }
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          if (up) {
+            lam[m][n] = LM[n * tot + off + c[m]];
+          } else {
+            lam[m][n] = lambda_of<T, DIM>(F[m], n, aa[m][n], A.alpha, A.beta, dxinv);
+            if (nl > 1) LM[n * tot + off + c[m]] = lam[m][n];
+          }
+          rr[m][n] = R[n * tot + off + c[m]];
+          ph[m][n] = P[n * tot + off + c[m]];
+          pl[m][n] = SL[n * CS + c[m]];
+          SX[n * CS + m * kHCWG + tid] = fma(ws[m][n], pl[m][n], wb[m][n]);
+        }
+      }
+      // L(phi) of slot m
+      auto lof = [&](auto M, T(&out)[2]) __attribute__((always_inline)) {
+        constexpr int m = decltype(M)::value;
+        T st[2][7];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          st[n][0] = pl[m][n];
+#pragma unroll
+          for (int f = 0; f < 2 * DIM; ++f) st[n][1 + 2 * (f >> 1) + (1 - (f & 1))] = SL[n * CS + nb[m][f]];
+        }
+        if (multi[m]) {
+#pragma unroll
+          for (int f = 1; f < 2 * DIM; ++f)
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+              if ((wall[m] >> f) & 1) {
+                const T s = GT[f][2 * n], b = GT[f][2 * n + 1];
+                st[n][1 + 2 * (f >> 1) + (1 - (f & 1))] = fma(s, pl[m][n], s < T(0) ? b : b * lsc);
+              }
+        }
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+          out[n] = lof_of<T, DIM>(F[m], n, st[n], aa[m][n], ph[m][n], A.alpha, A.beta, dxinv);
+      };
+      if (!up && (v > 0 || A.add_first)) {
+        // FAS right-hand side: rhs += L(phi)
+        auto add = [&](auto M) __attribute__((always_inline)) {
+          constexpr int m = decltype(M)::value;
+          if (o.p[m] < 0) return;
+          T lf[2];
+          lof(M, lf);
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            rr[m][n] = rr[m][n] + lf[n];
+            R[n * tot + off + c[m]] = rr[m][n];
+          }
+        };
+        add(IC<0>{});
+        add(IC<1>{});
+        sync();   // the passes overwrite the closures just read
+      }
+      bool changed = false;
+      auto update = [&](auto M) __attribute__((always_inline)) {
+        constexpr int m = decltype(M)::value;
+        if (o.p[m] < 0) return;
+        T lf[2];
+        lof(M, lf);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          const T nv = ph[m][n] - lam[m][n] * (lf[n] - rr[m][n]);
+          changed = changed || bits_of(nv) != bits_of(ph[m][n]);
+          ph[m][n] = nv;
+        }
+        closure<T>(ph[m][0], ph[m][1], A.cp, pl[m][0], pl[m][1]);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+          SL[n * CS + c[m]] = pl[m][n];
+          SX[n * CS + m * kHCWG + tid] = fma(ws[m][n], pl[m][n], wb[m][n]);
+        }
+      };
+      // the bottom ends at its fixed point
+      auto fixed = [&]() __attribute__((always_inline)) {
+        const bool go = small ? __any(changed) : __syncthreads_or(changed);
+        changed = false;
+        return !go;
+      };
+      const int its = bot ? A.bottom : (up ? A.nu2 : A.nu1);
+      if (even) {
+#pragma unroll 1
+        for (int it = 0; it < its; ++it) {
+          update(IC<0>{});
+          sync();
+          update(IC<1>{});
+          sync();
+          if (bot && fixed()) break;
+        }
+      } else {
+#pragma unroll 1
+        for (int p = 0; p < 2 * its; ++p) {
+          if (o.p[0] >= 0 && col[0] == (p & 1)) update(IC<0>{});
+          if (o.p[1] >= 0 && col[1] == (p & 1)) update(IC<1>{});
+          sync();
+          if (bot && (p & 1) && fixed()) break;
+        }
+      }
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (o.p[m] >= 0) {
+          P[off + c[m]] = ph[m][0];
+          P[tot + off + c[m]] = ph[m][1];
+        }
+      if (down) {
+        // restriction (RESTRICTRESNLVC / RESTRICT): (rhs - L phi)/2^d per
+        // cell, then child sums in Fortran order
+        auto res = [&](auto M) __attribute__((always_inline)) {
+          constexpr int m = decltype(M)::value;
+          if (o.p[m] < 0) return;
+          T lf[2];
+          lof(M, lf);
+          rr[m][0] = (rr[m][0] - lf[0]) * rdenom;
+          rr[m][1] = (rr[m][1] - lf[1]) * rdenom;
+        };
+        res(IC<0>{});
+        res(IC<1>{});
+        sync();   // the ghosts in SX have been read
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (o.p[m] >= 0) {
+            SX[c[m]] = rr[m][0];
+            SX[CS + c[m]] = rr[m][1];
+          }
+        sync();
+        const CLev C = level_of(l + 1);
+#pragma unroll 1
+        for (int cc = tid; cc < C.N; cc += step) {
+          int I, J, K;
+          clev_coords(C, cc, I, J, K);
+          const int f0 = 2 * I + L.nx * (2 * J) + (DIM == 3 ? L.nxy * (2 * K) : 0);
+#pragma unroll
+          for (int n = 0; n < 2; ++n) {
+            T s = T(0), sp = T(0);
+#pragma unroll
+            for (int kk = 0; kk < (DIM == 3 ? 2 : 1); ++kk)
+#pragma unroll
+              for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                for (int ii = 0; ii < 2; ++ii) {
+                  const int f = f0 + ii + L.nx * jj + L.nxy * kk;
+                  s = s + SX[n * CS + f];
+                  sp = sp + P[n * tot + off + f] * rdenom;
+                }
+            R[n * tot + offc + cc] = s;
+            P[n * tot + offc + cc] = sp;
+            P0[n * tot1 + (offc - N0) + cc] = sp;
+          }
+        }
+      }
+    }
+    // the next visit reads what this one wrote: wave 0 alone where both are
+    // small, else the workgroup
+    bool next_small = false;
+    if (small && v + 1 < 2 * nl - 1) next_small = cown_active<kHCWG>(level_of(v + 1 >= nl ? 2 * nl - 3 - v : v + 1)) <= 64;
+    if (!next_small)
+      __syncthreads();
+    else if (tid < 64)
+      wave_sync();
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int c = tid + m * kHCWG;
+    if (c >= N0) continue;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) A.phi[q0[m] + n * nc0] = P[n * tot + c];
   }
 }
 
@@ -1781,13 +1833,40 @@ hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T
   return hipSuccess;
 }
 
+int hc_coarse_cells() { return kWGCells; }
+
 template <typename T>
-hipError_t hc_coarse_vcycle(const CoarseDesc<T>* dev_desc, int dim, int apply_first, hipStream_t s) {
-  const size_t lds = (size_t(4) * kWGCells + size_t(2) * (kWGCells / 4)) * sizeof(T);
-  if (dim == 2)
-    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 2>), dim3(1), dim3(kWGThreads), lds, s, dev_desc, apply_first);
+hipError_t hc_coarse_vcycle(const Geom& g, const BCDesc& bc, HCCoarse<T> A, hipStream_t s) {
+  if (g.nvalid() > kWGCells || A.nl < 1 || A.nl > kHCCoarseLevels) return hipErrorInvalidValue;
+  for (int d = 0; d < 3; ++d) {
+    A.n[d] = g.n[d];
+    A.per[d] = g.periodic[d];
+  }
+  int fo = 0;
+  for (int l = 0; l < A.nl; ++l) {
+    const Geom gl = l == 0 ? g : coarsen_geom(g, 1 << l);
+    A.off[l + 1] = A.off[l] + int(gl.nvalid());
+    for (int d = 0; d < g.dim; ++d) {
+      A.fo[l][d] = fo;
+      A.nf[l][d] = int(gl.nface[d]);
+      fo += 2 * A.nf[l][d];
+    }
+  }
+  A.tot = A.off[A.nl];
+  A.dx = T(g.dx);
+  const GhostForm<T> gf = ghost_form<T>(bc, T(g.dx));
+  for (int d = 0; d < 3; ++d)
+    for (int sd = 0; sd < 2; ++sd)
+      for (int n = 0; n < 2; ++n) {
+        A.gs[d][sd][n] = gf.s[d][sd][n];
+        A.gb[d][sd][n] = gf.b[d][sd][n];
+      }
+  const size_t elems = (A.nl > 1 ? 6 : 4) * size_t(A.tot) + 2 * size_t(A.tot - A.off[1]) + 4 * kWGCells + size_t(A.nfaces);
+  // (at most 147 KB over all shapes of up to 1024 cells)
+  if (g.dim == 2)
+    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 2>), dim3(1), dim3(kHCWG), elems * sizeof(T), s, A);
   else
-    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 3>), dim3(1), dim3(kWGThreads), lds, s, dev_desc, apply_first);
+    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 3>), dim3(1), dim3(kHCWG), elems * sizeof(T), s, A);
   return hipGetLastError();
 }
 
@@ -1877,7 +1956,7 @@ template hipError_t hc_relax_restrict<double>(const HCArgs<double>&, double* con
 template hipError_t hc_relax_final<double>(const HCArgs<double>&, double* const[2], int*, const double*, int,
                                            const Geom*, const double*, const double*, unsigned long long*,
                                            const CtlFuse&, hipStream_t);
-template hipError_t hc_coarse_vcycle<double>(const CoarseDesc<double>*, int, int, hipStream_t);
+template hipError_t hc_coarse_vcycle<double>(const Geom&, const BCDesc&, HCCoarse<double>, hipStream_t);
 template hipError_t hc_residual<double>(const HCArgs<double>&, double*, const double*, double*,
                                         unsigned long long*, int, hipStream_t, const CtlFuse&);
 template hipError_t hc_apply_op<double>(const HCArgs<double>&, double*, double*, const double*, int, hipStream_t);

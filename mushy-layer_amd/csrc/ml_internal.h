@@ -122,6 +122,11 @@ struct ml_hc_op_s {
   ml_params params{};
   double alpha = 0.0, beta = -1.0;   // factory defaults (src/AMRNonLinearMultiCompOp.cpp:1622-1633)
   std::vector<ml::HCLevel> lev;
+  // the faces of the levels from lc (the first of at most hc_coarse_cells()
+  // cells) down are one block, level by level and direction by direction
+  int lc = 0;
+  double* cfaces = nullptr;
+  size_t ncfaces = 0;
   std::unique_ptr<ml::HostDriver, void (*)(ml::HostDriver*)> host_driver{nullptr, nullptr};
   std::unique_ptr<ml::HCEngine, void (*)(ml::HCEngine*)> engine{nullptr, nullptr};
   std::unique_ptr<ml::AdjWork, void (*)(ml::AdjWork*)> adj{nullptr, nullptr};
@@ -166,7 +171,6 @@ class HCEngine {
   int read_norm(int slot, double* out);
   int read_ctl(SolveCtl* out);
   int write_ctl(const SolveCtl& c);
-  int upload_desc(double* phi0, const double* rhs0, const ml_solve_opts& o);
   // FP32-refined form: FP64 defect correction around FP32 linear V-cycles
   int solve_refined(double* phi, const double* rhs, const ml_solve_opts& o, ml_solve_stats* st);
   int init_refined();
@@ -200,9 +204,6 @@ class HCEngine {
   unsigned long long* m_slots = nullptr;       // max-norm accumulators
   unsigned long long* m_hslots = nullptr;      // pinned mirror
   int m_nslots = 0;
-  CoarseDesc<double>* m_desc = nullptr;        // device
-  CoarseDesc<double>* m_hdesc = nullptr;       // pinned host staging
-  StagedDesc m_stage_fas;
   SolveCtl* m_ctl = nullptr;                   // device iteration control
   unsigned int* m_arrive = nullptr;            // workgroup arrival counter of the fused stopping rule
   SolveCtl* m_hctl = nullptr;                  // pinned mirror

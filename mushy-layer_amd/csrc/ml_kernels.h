@@ -220,27 +220,27 @@ struct HCApplyJob {
   TileIO<T> io;
 };
 
-// One MG level as seen by the single-workgroup kernels (device memory).
+// Arguments of the single-workgroup FAS V-cycle (hc_coarse_vcycle fills the
+// geometry): the first level's state (in and out) and right-hand side, and
+// the faces of all its levels as one block (level, direction, component).
+constexpr int kHCCoarseLevels = 6;
 template <typename T>
-struct LevelDesc {
-  Geom g;
-  T* phi;
-  T* rhs;
-  T* phi0;
-  T* tmp;
-  const T* a;
-  const T* b[3];
-};
-
-template <typename T>
-struct CoarseDesc {
-  int l0, nlev;
-  int nu1, nu2, bottom;
-  ClosureP<T> cp;
-  BCDesc bc;
-  T alpha, beta;
+struct HCCoarse {
   const int* skip;   // device flag: the kernel returns at once when set
-  LevelDesc<T> lev[kMaxLevels];
+  T* phi;
+  const T* rhs;
+  const T* faces;
+  const T* a[kHCCoarseLevels];   // aCoef per level (nullptr: 1)
+  int nfaces;                    // values of the block, even
+  int nl, nu1, nu2, bottom;
+  int add_first;                 // rhs += L(phi) on the first level
+  int tot, n[3], per[3];
+  // per level: cells before it, face values before its direction d, faces of
+  // direction d
+  int off[kHCCoarseLevels + 1], fo[kHCCoarseLevels][3], nf[kHCCoarseLevels][3];
+  T dx, alpha, beta;
+  ClosureP<T> cp;
+  T gs[3][2][2], gb[3][2][2];    // GhostForm of the first level
 };
 
 __host__ __device__ inline int wrap_clamp(int v, int n, int periodic) {
@@ -544,8 +544,10 @@ hipError_t hc_relax_restrict(const HCArgs<T>& A, T* const buf[2], int* cur, cons
 template <typename T>
 hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, const Geom* gc,
                           const T* pc, const T* pc0, unsigned long long* norm, const CtlFuse& fuse, hipStream_t s);
+// FAS V-cycle of the levels from g (at most hc_coarse_cells() cells) down
+int hc_coarse_cells();
 template <typename T>
-hipError_t hc_coarse_vcycle(const CoarseDesc<T>* dev_desc, int dim, int apply_first, hipStream_t s);
+hipError_t hc_coarse_vcycle(const Geom& g, const BCDesc& bc, HCCoarse<T> A, hipStream_t s);
 template <typename T>
 hipError_t hc_restrict_all(const HCArgs<T>& A, const Geom& gc, T* phi, const T* rhs, T* resc, T* phic, T* phic0,
                            int homog, hipStream_t s);

@@ -125,3 +125,36 @@ def test_closure_at_regime_edges(ml, gpu_ctx, wl, name):
     ok = ~np.isnan(r)
     assert HC.bitwise_equal(a[ok], r[ok])
     op.close()
+
+
+SMALL = {
+    "odd_rows_walls": dict(n=(31, 20), periodic=[0, 0], bc=WALLS),
+    "thin_walls": dict(n=(2, 400), periodic=[0, 0], bc=WALLS),
+    "one_row": dict(n=(300, 1), periodic=[1, 0], bc=WALLS),
+    "deep": dict(n=(32, 32), periodic=[1, 1]),
+    "long": dict(n=(8, 128)),
+    "3d_odd_walls": dict(n=(9, 7, 5), periodic=[0, 0, 0], bc=WALLS),
+    "3d_column": dict(n=(4, 4, 64), periodic=[1, 0, 0], bc=WALLS),
+    "3d_periodic": dict(n=(16, 8, 8), periodic=[1, 1, 1]),
+    "3d_tiled": dict(n=(24, 16, 12)),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SMALL))
+@pytest.mark.parametrize("bottom,nu1,acoef", [(40, 1, False), (3, 2, True), (0, 0, False)])
+def test_single_workgroup_cycles(ml, gpu_ctx, wl, name, bottom, nu1, acoef):
+    """The V-cycle of one workgroup on every kind of level it holds: odd rows
+    (a thread's two cells may share a colour), cells with two and more walls,
+    one to five levels, a bottom that ends at its fixed point or not at all."""
+    case, g, p, bc, b, a, op = _setup(ml, gpu_ctx, wl, SMALL[name], acoef)
+    n = case["n"]
+    old = case["phi"].copy()
+    new = old.copy()
+    kw = dict(max_iter=3, nu1=nu1, nu2=3, bottom=bottom)
+    so = O.hc_be_step(g, p, bc, a, b, case["dt"], new, old, opts=O.default_opts(**kw))
+    dn = ml.DeviceArray(gpu_ctx, old.shape, host=old)
+    st = op.solve_be(dn, ml.DeviceArray(gpu_ctx, old.shape, host=old), case["dt"], opts=ml.default_opts(**kw))
+    out = dn.get()
+    assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
+    assert HC.bitwise_equal(HC.valid(n, out), HC.valid(n, new))
+    op.close()

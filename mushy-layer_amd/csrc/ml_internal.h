@@ -264,6 +264,8 @@ struct ml_vc_op_s {
   bool has_a = false, has_c = false;
   std::vector<ml::VCLevelStore> lev;
   int lc = 0;                       // first level handled by the single-workgroup kernel
+  double* cfaces = nullptr;         // faces of the levels from lc down, one block
+  size_t ncfaces = 0;
   int nslots = 1024;                // norm slots per workspace (max_iter + 1)
   std::vector<ml::VCWork> work;     // solve workspaces; [0] runs on the context stream
   size_t coarse_lds = 0;            // dynamic LDS of the single-workgroup V-cycle

@@ -686,16 +686,6 @@ struct VCFinal {
   CtlFuse fuse;
 };
 
-template <typename T>
-struct VCLevel {
-  Geom g;
-  const T* a;
-  const T* c;
-  const T* b[3];
-  T* e;   // correction
-  T* r;   // residual right-hand side
-};
-
 // one (instance, level) relaxation of a batched launch (the arguments of
 // vc_relax_tile_kernel)
 template <typename T>
@@ -727,14 +717,26 @@ struct WordsJob {
 };
 constexpr int kWordsChunk = 4096;   // words per workgroup of words_batch
 
+// Descriptor of the single-workgroup V-cycle (vc_desc_geometry fills the
+// geometry): right-hand side and correction of its first level, the faces of
+// all its levels as one block (level by level, direction by direction), a and
+// c per level (nullptr: 1 and no c term).
+constexpr int kVCCoarseLevels = 6;
 template <typename T>
 struct VCDesc {
-  int l0, nlev, nu1, nu2, bottom;
-  int bottom_solver, bottom_imax;   // BiCGStab on the coarsest level after `bottom` relaxations (solver 1)
-  BCDesc bc;
-  T alpha, beta;
   const int* skip;
-  VCLevel<T> lev[kMaxLevels];
+  const T* r;
+  T* e;
+  const T* faces;
+  int nfaces;                       // values of the block, even
+  int nl, nu1, nu2, bottom;
+  int bottom_solver, bottom_imax;   // BiCGStab on the coarsest level after `bottom` relaxations (solver 1)
+  int tot, n[3], per[3];
+  int off[kVCCoarseLevels + 1], fo[kVCCoarseLevels][3];   // cells and faces before each level (and direction)
+  T alpha, beta, dx;
+  T gs[3][2], gb[3][2];             // GhostForm of the homogeneous BC
+  const T* a[kVCCoarseLevels];
+  const T* c[kVCCoarseLevels];
 };
 
 // red/black relaxation of L e = r with homogeneous BCs, ping-ponging between
@@ -766,6 +768,8 @@ hipError_t vc_apply_op(const VCArgs<T>& A, const T* phi, T* lhs, int homog, hipS
 template <typename T>
 hipError_t vc_restrict_residual(const VCArgs<T>& A, const Geom& gc, const T* phi, const T* rhs, T* resc,
                                 hipStream_t s);
+template <typename T>
+void vc_desc_geometry(VCDesc<T>& D, const Geom& g, const BCDesc& bc, int nl);
 template <typename T>
 hipError_t vc_coarse_vcycle(const VCDesc<T>* dev_desc, int dim, size_t lds, hipStream_t s);
 // phi = rhs * lambda on the valid cells (preCond's first step)

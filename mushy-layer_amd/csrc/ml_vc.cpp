@@ -187,26 +187,25 @@ int vc_upload_desc(ml_vc_op op, ml::VCWork& W, const ml_solve_opts& o, hipStream
   ml_ctx ctx = op->ctx;
   ml::VCDesc<double> D;
   std::memset(&D, 0, sizeof(D));
-  D.l0 = op->lc;
-  D.nlev = int(op->lev.size());
   D.nu1 = o.nu1;
   D.nu2 = o.nu2;
   D.bottom = o.bottom;
   D.bottom_solver = o.bottom_solver;
   D.bottom_imax = o.bottom_max_iter;
-  D.bc = op->bc;
   D.alpha = op->alpha;
   D.beta = op->beta;
   D.skip = &W.ctl->done;
-  for (int l = 0; l < D.nlev; ++l) {
-    const ml::VCArgs<double> A = op->args(l);
-    ml::VCLevel<double>& L = D.lev[l];
-    L.g = A.g;
-    L.a = A.a;
-    L.c = A.c;
-    for (int d = 0; d < 3; ++d) L.b[d] = A.b[d];
-    L.e = W.e0[l];
-    L.r = W.r[l];
+  const int L = int(op->lev.size());
+  if (op->lc < L) {
+    ml::vc_desc_geometry<double>(D, op->lev[op->lc].g, op->bc, L - op->lc);
+    D.faces = op->cfaces;
+    D.nfaces = int(op->ncfaces);
+    D.r = W.r[op->lc];
+    D.e = W.e0[op->lc];
+    for (int l = op->lc; l < L; ++l) {
+      D.a[l - op->lc] = op->has_a ? op->lev[l].a : nullptr;
+      D.c[l - op->lc] = op->has_c ? op->lev[l].c : nullptr;
+    }
   }
   ML_HIP(ctx, W.stage.put(W.desc, W.hdesc, &D, sizeof(D), stream ? stream : W.stream));
   return ML_OK;
@@ -530,14 +529,27 @@ int ml_vc_op_create(ml_ctx ctx, int dim, const int lo[], const int hi[], double 
     ml_vc_op_destroy(op.release());
     return rc;
   };
+  int rc;
   for (int l = 0; l < depth; ++l) {
     ml::VCLevelStore& L = raw->lev[l];
     L.g = l == 0 ? g0 : ml::coarsen_geom(g0, 1 << l);
-    int rc;
-    for (int d = 0; d < dim; ++d)
-      if ((rc = vc_alloc(ctx, L.g.nface[d], &L.b[d]))) return bail(rc);
+    for (int d = 0; d < dim; ++d) {
+      if (l >= raw->lc)
+        raw->ncfaces += size_t(L.g.nface[d]);
+      else if ((rc = vc_alloc(ctx, L.g.nface[d], &L.b[d])))
+        return bail(rc);
+    }
   }
-  int rc;
+  if (raw->lc < depth) {
+    raw->ncfaces += raw->ncfaces & 1;
+    if ((rc = vc_alloc(ctx, raw->ncfaces, &raw->cfaces))) return bail(rc);
+    double* cf = raw->cfaces;
+    for (int l = raw->lc; l < depth; ++l)
+      for (int d = 0; d < dim; ++d) {
+        raw->lev[l].b[d] = cf;
+        cf += raw->lev[l].g.nface[d];
+      }
+  }
   if (raw->lc < depth) {
     std::vector<ml::Geom> gs(depth);
     for (int l = 0; l < depth; ++l) gs[l] = raw->lev[l].g;
@@ -564,13 +576,15 @@ int ml_vc_op_destroy(ml_vc_op op) {
     vc_work_free(W);
   }
   op->host_driver.reset();
-  for (auto& L : op->lev) {
+  for (int l = 0; l < int(op->lev.size()); ++l) {
+    ml::VCLevelStore& L = op->lev[l];
     for (int d = 0; d < 3; ++d)
-      if (L.b[d]) hipFree(L.b[d]);
+      if (L.b[d] && l < op->lc) hipFree(L.b[d]);
     if (L.a) hipFree(L.a);
     if (L.c) hipFree(L.c);
     if (L.tmp) hipFree(L.tmp);
   }
+  if (op->cfaces) hipFree(op->cfaces);
   delete op;
   return ML_OK;
 }

@@ -415,188 +415,189 @@ __global__ __launch_bounds__(256) void words_batch_kernel(const WordsJob* __rest
 }
 
 // ---------------------------------------------------------------------------
-// Single-workgroup V-cycle over levels l0.. of a device descriptor.  The
-// correction, right-hand side and operator data (faces, a, c, lambda) of
-// every level live in LDS for the whole cycle (compact, x fastest, levels
-// one after another); the operator data are loaded once at the start.  Each
-// thread owns one cell of each colour of a level (even row length) or the
-// cells t and t + 512, with their coordinates held in registers; levels
-// whose owners fit one wavefront are relaxed by wave 0 alone.
+// Single-workgroup V-cycle over the small levels of a device descriptor.  The
+// correction, right-hand side, lambda, faces, a and c of every level live in
+// LDS for the whole cycle (compact, x fastest, levels one after another;
+// faces as one block, read once).
+//
+// A wavefront alone on its SIMD issues an operation every 8 cycles whether it
+// depends on the last one or not, and a branch costs four of them: the count
+// of instructions along a visit bounds it.  Each thread owns one cell of each
+// colour of a level (even row length) or the cells t and t + 512, with their
+// data in registers; a wall's ghost is written by its cell's owner with each
+// update, into a slot that the stencil reads like any neighbour; offsets come
+// from the host.  Levels whose owners fit one wavefront are visited by wave 0
+// alone.  The visits are one runtime loop: every launch fetches the code it
+// runs.  Measured with BiCGStab bottoms, against per-visit geometry and
+// shuffled dot products: five 2D levels from 32x32 63 -> 46 us a launch, two
+// levels from 44x20 (bottom 22x10) 165 -> 115; a visit is now some 6.5K
+// cycles, half of them its set-up.
 
-constexpr int kVCL = 6;   // levels one launch handles: 1024 cells coarsen to one cell in 6 (2D), 4 (3D)
+constexpr int kVCL = kVCCoarseLevels;   // levels one launch handles: 1024 cells coarsen to one cell in 6 (2D), 4 (3D)
 template <int DIM>
 struct VCLevels {
   static constexpr int n = DIM == 3 ? 4 : kVCL;
 };
 
-// operator data of all levels in LDS; q = level offset + compact cell index
-template <typename T, int DIM>
-struct VCLds {
-  T *se, *sr, *sres;   // corrections, right-hand sides, restriction scratch
-  T *sF, *sA, *sC, *sL;   // faces [2*DIM][tot], a, c, lambda
-  int tot;
-  __device__ inline void faces(int q, Faces1<T, DIM>& F) const {
-#pragma unroll
-    for (int f = 0; f < 2 * DIM; ++f) F.v[f] = sF[f * tot + q];
+// x of lane ^ 2^k, k < 5 (DPP within rows of 16, a row swap)
+template <int K>
+__device__ __forceinline__ int lane_xor32(int x) {
+  if constexpr (K == 0) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xF, 0xF, true);    // quad_perm 1,0,3,2
+  if constexpr (K == 1) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xF, 0xF, true);    // quad_perm 2,3,0,1
+  if constexpr (K == 2)   // half mirror (^7), then reversed quads (^3)
+    return __builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, x, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+  if constexpr (K == 3) return __builtin_amdgcn_update_dpp(0, x, 0x128, 0xF, 0xF, true);   // row rotated by 8
+  return x;
+}
+template <int K>
+__device__ __forceinline__ double lane_add(double s) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(s);
+  const int lo = int(u), hi = int(u >> 32);
+  if constexpr (K < 4) {
+    const unsigned long long o =
+        (unsigned long long)unsigned(lane_xor32<K>(lo)) | ((unsigned long long)unsigned(lane_xor32<K>(hi)) << 32);
+    return s + __longlong_as_double((long long)o);
+  } else {
+    // both halves of each swapped pair in every lane: the same sum everywhere
+    auto swap = [](int x) {
+      if constexpr (K == 4) return __builtin_amdgcn_permlane16_swap(x, x, false, false);
+      else return __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    };
+    const auto a = swap(lo), b = swap(hi);
+    const double p = __longlong_as_double((long long)((unsigned long long)unsigned(a[0]) | ((unsigned long long)unsigned(b[0]) << 32)));
+    const double q = __longlong_as_double((long long)((unsigned long long)unsigned(a[1]) | ((unsigned long long)unsigned(b[1]) << 32)));
+    return p + q;
   }
+}
+// the pairwise tree s_t + s_{t+h}, h = P/2 .. 1, over the first P lanes (P a
+// power of two); the value of lane 0, uniform.  (Each node adds the same two
+// values in either order.)
+__device__ __forceinline__ double lane_tree(double s, int P) {
+  if (P > 32) s = lane_add<5>(s);
+  if (P > 16) s = lane_add<4>(s);
+  if (P > 8) s = lane_add<3>(s);
+  if (P > 4) s = lane_add<2>(s);
+  if (P > 2) s = lane_add<1>(s);
+  if (P > 1) s = lane_add<0>(s);
+  const unsigned long long u = (unsigned long long)__double_as_longlong(s);
+  const unsigned lo = __builtin_amdgcn_readfirstlane(int(u)), hi = __builtin_amdgcn_readfirstlane(int(u >> 32));
+  return __longlong_as_double((long long)((unsigned long long)lo | ((unsigned long long)hi << 32)));
+}
+
+// LDS of the coarse V-cycle in elements: corrections, right-hand sides and
+// lambda of every level, a and c, ghost slots (or restriction terms), faces
+struct VCLdsMap {
+  int e, r, lm, a, c, x, f, end;
+};
+__host__ __device__ inline VCLdsMap vc_lds_map(int tot, int nfaces, bool hasa, bool hasc) {
+  VCLdsMap M;
+  M.e = 0;
+  M.r = tot;
+  M.lm = 2 * tot;
+  M.a = 3 * tot;
+  M.c = M.a + (hasa ? tot : 0);
+  M.x = M.c + (hasc ? tot : 0);
+  M.f = M.x + kVCWGCells;
+  M.end = M.f + nfaces;
+  return M;
+}
+
+// One cell's data of a level: neighbours as LDS indices (a wall's ghost in
+// the owner's slot), faces, alpha*a, beta*c, lambda.
+template <typename T, int DIM>
+struct VCCell {
+  int nb[2 * DIM], wall;   // wall: faces beyond the first wall
+  T ws, wb;                // the first wall's ghost: ws*u + wb
+  Faces1<T, DIM> F;
+  T al, bc, lam;
 };
 
-template <typename T>
-size_t vc_coarse_lds_elems(int dim, long long tot) {
-  return size_t(tot) * (2 + 2 * dim + 3) + kVCWGCells;
-}
-
-// homogeneous wall ghost of component 0 (bit 2d+s of bcm: type != 0)
-template <typename T>
-__device__ __forceinline__ T vc_wall(int bcm, int d, int s, T interior, T dx) {
-  return bc_ghost<T>((bcm >> (2 * d + s)) & 1, T(0), interior, s ? 1 : -1, dx);
-}
-
-// A thread's cells of one level for the duration of a level visit:
-// coordinates, colour, neighbour indices and operator data in registers.
+// lof (vc_lof) of the cell whose value is u, neighbours from sm
 template <typename T, int DIM>
-struct VCCtx {
-  int pk[2], c[2], col[2], wall[2];
-  int nb[2][2 * DIM];
-  Faces1<T, DIM> F[2];
-  T aq[2], cv[2], lam[2], rr[2];
-};
-
-template <typename T, int DIM>
-__device__ __forceinline__ void vcx_build(VCCtx<T, DIM>& X, const CLev& L, const int* per, const VCLds<T, DIM>& S) {
-  COwn o;
-  cown_set<kVCWG>(L, o);
+__device__ __forceinline__ T vccell_lof(const VCCell<T, DIM>& X, const T* sm, T u, bool hasc, const VCDesc<T>& D, T beta,
+                                        T dxinv) {
+  T p[2 * DIM];
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    X.pk[m] = o.p[m];
-    if (o.p[m] < 0) continue;
-    int i, j, k;
-    cunpack(o.p[m], i, j, k);
-    const int c = i + L.nx * j + L.nxy * k;
-    X.c[m] = c;
-    X.col[m] = (i + j + k) & 1;
-    clev_nbrs<DIM>(L, per, i, j, k, X.nb[m], X.wall[m]);
-    const int q = L.off + c;
-    S.faces(q, X.F[m]);
-    X.aq[m] = S.sA[q];
-    X.cv[m] = S.sC[q];
-    X.lam[m] = S.sL[q];
-    X.rr[m] = S.sr[q];
+  for (int f = 0; f < 2 * DIM; ++f) p[f] = sm[X.nb[f]];
+  if (X.wall) {
+#pragma unroll
+    for (int f = 1; f < 2 * DIM; ++f)
+      if ((X.wall >> f) & 1) p[f] = fma(D.gs[f >> 1][f & 1], u, D.gb[f >> 1][f & 1]);
   }
-}
-
-// stencil of cell m of the context from the level's corrections su
-template <typename T, int DIM>
-__device__ __forceinline__ void vcx_stencil(const VCCtx<T, DIM>& X, int m, int bcm, T dx, const T* su, T* p) {
-  p[0] = su[X.c[m]];
-#pragma unroll
-  for (int f = 0; f < 2 * DIM; ++f) {
-    const int d = f >> 1, s = f & 1;
-    T v = su[X.nb[m][f]];
-    if ((X.wall[m] >> f) & 1) v = vc_wall<T>(bcm, d, s, v, dx);
-    p[1 + 2 * d + (1 - s)] = v;
-  }
+  T s = X.F.v[1] * (p[1] - u) - X.F.v[0] * (u - p[0]) + X.F.v[3] * (p[3] - u) - X.F.v[2] * (u - p[2]);
+  if (DIM == 3) s = s + X.F.v[5] * (p[5] - u) - X.F.v[4] * (u - p[4]);
+  T lof = X.al * u;
+  if (hasc) lof = lof - X.bc * u;
+  return lof - beta * s * dxinv;
 }
 
 template <typename T, int DIM>
-__device__ __forceinline__ void vcx_relax(const VCCtx<T, DIM>& X, const CLev& L, int bcm, const VCLds<T, DIM>& S,
-                                          bool hasc, T alpha, T beta, int npass) {
-  const T dx = T(L.dx);
-  const T dxinv = T(1) / (dx * dx);
-  T* se = S.se + L.off;
-  auto pass = [&](int p) {
+__device__ __forceinline__ void vccell_build(VCCell<T, DIM>& X, const VCDesc<T>& D, const VCLdsMap& M, const T* sm,
+                                             const CLev& L, const int* fo, int i, int j, int k, int slot, bool hasa,
+                                             bool hasc, T alpha, T beta, T dxinv, bool up, T* LM) {
+  const int c = L.off + i + L.nx * j + L.nxy * k;
+  const int iv[3] = {i, j, k};
+  X.wall = 0;
+  X.ws = X.wb = T(0);
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      if (X.pk[m] < 0 || X.col[m] != (p & 1)) continue;
-      T st[7];
-      vcx_stencil<T, DIM>(X, m, bcm, dx, se, st);
-      const T lof = vc_lof<T, DIM>(X.F[m], st, X.aq[m], hasc, X.cv[m], alpha, beta, dxinv);
-      se[X.c[m]] = st[0] - X.lam[m] * (lof - X.rr[m]);
-    }
-  };
-  // levels whose owners fit one wavefront: wave 0 alone with wavefront-scope
-  // syncs (small is uniform, so the workgroup barrier is reached by all
-  // waves or by none)
-  const bool small = cown_active<kVCWG>(L) <= 64;
-  if (!small || threadIdx.x < 64) {
-#pragma unroll 1
-    for (int p = 0; p < npass; ++p) {
-      pass(p);
-      if (small)
-        wave_sync();
-      else
-        __syncthreads();
+  for (int d = DIM - 1; d >= 0; --d) {
+    const int st = d == 0 ? 1 : (d == 1 ? L.nx : L.nxy);
+    const int nd = L.n[d];
+    const bool w = D.per[d] == 0;
+    const bool lo = iv[d] == 0, hi = iv[d] == nd - 1;
+    X.nb[2 * d] = M.e + (lo ? c + (nd - 1) * st : c - st);
+    X.nb[2 * d + 1] = M.e + (hi ? c - (nd - 1) * st : c + st);
+    if (w) {
+      if (lo) X.nb[2 * d] = M.x + slot;
+      if (hi) X.nb[2 * d + 1] = M.x + slot;
+      if (lo || hi) {
+        X.ws = lo ? D.gs[d][0] : D.gs[d][1];
+        X.wb = lo ? D.gb[d][0] : D.gb[d][1];
+        X.wall |= (lo ? 1 << (2 * d) : 0) | (hi ? 2 << (2 * d) : 0);
+      }
     }
   }
-  if (small) __syncthreads();
-}
-
-// restricted residual (homogeneous BCs, RESTRICTRESDB order) of level Lf into
-// the right-hand side of level Lc, whose correction starts at zero
-template <typename T, int DIM>
-__device__ __forceinline__ void vcx_restrict(const VCCtx<T, DIM>& X, const CLev& Lf, const CLev& Lc, int bcm,
-                                             const VCLds<T, DIM>& S, bool hasc, T alpha, T beta) {
-  const T dx = T(Lf.dx);
-  const T dxinv = T(1) / (dx * dx);
-  const T denom = DIM == 3 ? T(8) : T(4);
-  const T* se = S.se + Lf.off;
+  X.wall &= X.wall - 1;   // (the first wall is the lowest bit)
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    if (X.pk[m] < 0) continue;
-    T st[7];
-    vcx_stencil<T, DIM>(X, m, bcm, dx, se, st);
-    const T lof = vc_lof<T, DIM>(X.F[m], st, X.aq[m], hasc, X.cv[m], alpha, beta, dxinv);
-    S.sres[X.c[m]] = (X.rr[m] - lof) / denom;
+  for (int d = 0; d < DIM; ++d) {
+    const int fx = L.n[0] + (d == 0), fy = L.n[1] + (d == 1);
+    const int at = M.f + fo[d] + i + fx * (j + (DIM == 3 ? fy * k : 0));
+    X.F.v[2 * d] = sm[at];
+    X.F.v[2 * d + 1] = sm[at + (d == 0 ? 1 : (d == 1 ? fx : fx * fy))];
   }
-  __syncthreads();
-  for (int cc = threadIdx.x; cc < Lc.N; cc += kVCWG) {
-    int I, J, K;
-    clev_coords(Lc, cc, I, J, K);
-    T s = T(0);
-    for (int kk = 0; kk < (DIM == 3 ? 2 : 1); ++kk)
-      for (int jj = 0; jj < 2; ++jj)
-        for (int ii = 0; ii < 2; ++ii)
-          s = s + S.sres[(2 * I + ii) + Lf.nx * (2 * J + jj) + Lf.nxy * (DIM == 3 ? 2 * K + kk : 0)];
-    S.sr[Lc.off + cc] = s;
-    S.se[Lc.off + cc] = T(0);
+  const T aq = hasa ? sm[M.a + c] : T(1), cq = hasc ? sm[M.c + c] : T(0);
+  X.al = alpha * aq;
+  X.bc = beta * cq;
+  if (up) {
+    X.lam = LM[c];
+  } else {
+    X.lam = vc_lambda<T, DIM>(X.F, aq, hasc, cq, alpha, beta, dxinv);
+    LM[c] = X.lam;
   }
-  __syncthreads();
 }
 
-// e_f += e_c(parent) (piecewise-constant prolongation)
+// BiCGStab on the coarsest level L from its relaxed correction: L e = r with
+// homogeneous BCs, preconditioner preCond (e = lambda*r, then two red/black
+// iterations).  Preconditioned BiCGStab with restarts; eps 1e-6, reps 1e-12,
+// hang 1e-8, small 1e-30, 5 restarts, L2 norms.  Dot products in a fixed
+// order: 64 interleaved lane sums over the compact cell index, then the tree
+// of lane_tree over the smallest power of two of lanes >= min(N, 64).
+//
+// Thread t holds cell t (and t + 512) of every vector in registers; only the
+// vector under the operator passes through LDS, with its ghosts.  Up to 64
+// cells wave 0 works alone and a dot product needs no LDS at all (the tree is
+// lane swaps: 18 operations, where six 64-bit shuffles were some 700 cycles);
+// beyond, the products pass through LDS, two buffers used in turn, one
+// barrier each.  One copy of preconditioner and operator serves both halves
+// of an iteration.  sm[z..]: the operator's vector (the level's corrections),
+// sm[dot..]: 2*N values.
 template <typename T, int DIM>
-__device__ __forceinline__ void vcx_prolong(const VCCtx<T, DIM>& X, const CLev& Lf, const CLev& Lc, T* se) {
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    if (X.pk[m] < 0) continue;
-    int i, j, k;
-    cunpack(X.pk[m], i, j, k);
-    const int c = Lf.off + X.c[m];
-    se[c] = se[c] + se[Lc.off + (i / 2) + Lc.nx * (j / 2) + Lc.nxy * (DIM == 3 ? k / 2 : 0)];
-  }
-  __syncthreads();
-}
-
-// BiCGStab on the coarsest level L (held in LDS) from its relaxed
-// correction: L e = r with homogeneous BCs, preconditioner preCond (e =
-// lambda*r, then two red/black iterations).  Preconditioned BiCGStab with
-// restarts; eps 1e-6, reps 1e-12, hang 1e-8, small 1e-30, 5 restarts, L2
-// norms.  Dot products run redundantly in every participating wavefront in a
-// fixed order: 64 interleaved lane sums over the compact cell index, then the
-// pairwise tree s_t + s_{t+h}, h = P/2 .. 1 with P the smallest power of two
-// >= min(N, 64).  Levels whose owners fit one
-// wavefront run on wave 0 alone with wavefront-scope syncs.  wk holds 8
-// vectors of L.N values.
-template <typename T, int DIM>
-__device__ __forceinline__ void vcx_bicgstab(const VCCtx<T, DIM>& X, const CLev& L, int bcm, const VCLds<T, DIM>& S, bool hasc,
-                             T alpha, T beta, int imax, T* wk) {
+__device__ __forceinline__ void vcx_bicgstab(const VCDesc<T>& D, const VCLdsMap& M, T* sm, const CLev& L, const int* fo,
+                                             bool hasa, bool hasc, T alpha, T beta, int imax, int dot0) {
   const int N = L.N;
-  const bool small = cown_active<kVCWG>(L) <= 64 && N <= 64 * 2;
-  if (small && threadIdx.x >= 64) {
-    __syncthreads();
-    return;
-  }
-  const int tid = threadIdx.x, stride = small ? 64 : kVCWG, lane = threadIdx.x & 63;
+  const bool small = N <= 64, two = N > kVCWG;
+  if (small && threadIdx.x >= 64) return;   // (the caller syncs the workgroup)
+  const int tid = threadIdx.x, lane = tid & 63;
   auto sync = [&]() __attribute__((always_inline)) {
     if (small)
       wave_sync();
@@ -605,68 +606,82 @@ __device__ __forceinline__ void vcx_bicgstab(const VCCtx<T, DIM>& X, const CLev&
   };
   const T dx = T(L.dx);
   const T dxinv = T(1) / (dx * dx);
-  T* phi = S.se + L.off;
-  const T* rhs = S.sr + L.off;
-  T *r = wk, *rt = wk + N, *e = wk + 2 * N, *p = wk + 3 * N, *pt = wk + 4 * N, *st = wk + 5 * N, *t = wk + 6 * N,
-    *v = wk + 7 * N;
-  auto lof_of = [&](int m, const T* u) __attribute__((always_inline)) {
-    T stc[7];
-    vcx_stencil<T, DIM>(X, m, bcm, dx, u, stc);
-    return vc_lof<T, DIM>(X.F[m], stc, X.aq[m], hasc, X.cv[m], alpha, beta, dxinv);
-  };
-  auto apply = [&](T* out, const T* u) __attribute__((always_inline)) {
+  T* Z = sm + M.e + L.off;
+  const T* rhs = sm + M.r + L.off;
+  VCCell<T, DIM> X[2];
+  bool own[2];
+  int col[2];
+  T ph[2], r[2], rt[2], e[2], p[2], pt[2], vv[2], f[2];
 #pragma unroll
-    for (int m = 0; m < 2; ++m)
-      if (X.pk[m] >= 0) out[X.c[m]] = lof_of(m, u);
-    sync();
+  for (int m = 0; m < 2; ++m) {
+    const int c = tid + m * kVCWG;
+    own[m] = c < N && (m == 0 || two);
+    ph[m] = r[m] = rt[m] = e[m] = p[m] = pt[m] = vv[m] = f[m] = T(0);
+    col[m] = 0;
+    if (!own[m]) continue;
+    int i, j, k;
+    clev_coords(L, c, i, j, k);
+    col[m] = (i + j + k) & 1;
+    vccell_build<T, DIM>(X[m], D, M, sm, L, fo, i, j, k, c, hasa, hasc, alpha, beta, dxinv, true, sm + M.lm);
+    ph[m] = Z[c];
+    f[m] = rhs[c];
+  }
+  auto put = [&](int m, T v) __attribute__((always_inline)) {
+    Z[tid + m * kVCWG] = v;
+    sm[M.x + tid + m * kVCWG] = fma(X[m].ws, v, X[m].wb);
   };
-  auto residual = [&](T* out, const T* u, const T* f) __attribute__((always_inline)) {
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-      if (X.pk[m] >= 0) out[X.c[m]] = f[X.c[m]] - lof_of(m, u);
-    sync();
-  };
-  auto precond = [&](T* z, const T* f) __attribute__((always_inline)) {
-#pragma unroll
-    for (int m = 0; m < 2; ++m)
-      if (X.pk[m] >= 0) z[X.c[m]] = f[X.c[m]] * X.lam[m];
-    sync();
-#pragma unroll 1
-    for (int pass = 0; pass < 4; ++pass) {
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        if (X.pk[m] < 0 || X.col[m] != (pass & 1)) continue;
-        T stc[7];
-        vcx_stencil<T, DIM>(X, m, bcm, dx, z, stc);
-        const T lof = vc_lof<T, DIM>(X.F[m], stc, X.aq[m], hasc, X.cv[m], alpha, beta, dxinv);
-        z[X.c[m]] = stc[0] - X.lam[m] * (lof - f[X.c[m]]);
-      }
-      sync();
-    }
-  };
-  // tree over the smallest power of two of lanes >= min(N, 64)
   int P2 = 1;
   while (P2 < 64 && P2 < N) P2 <<= 1;
+  int buf = 0;
   auto dot = [&](const T* x, const T* y) __attribute__((always_inline)) {
     T s = T(0);
-    for (int c = lane; c < N; c += 64) s = s + x[c] * y[c];
-    for (int h = P2 >> 1; h >= 1; h >>= 1) s = s + __shfl_down(s, h, 64);
-    return __shfl(s, 0, 64);
+    if (small) {
+      if (own[0]) s = s + x[0] * y[0];
+    } else {
+      T* q = sm + dot0 + buf * N;
+      buf ^= 1;
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (own[m]) q[tid + m * kVCWG] = x[m] * y[m];
+      __syncthreads();
+      for (int c = lane; c < N; c += 64) s = s + q[c];
+    }
+    return lane_tree(s, P2);
   };
   const T eps = T(1e-6), reps = T(1e-12), hang = T(1e-8), tiny = T(1e-30);
-  residual(r, phi, rhs);
-  for (int c = tid; c < N; c += stride) {
-    rt[c] = r[c];
-    e[c] = T(0);
-  }
-  T norm0 = sqrt(dot(r, r)), norm1 = norm0;
-  const T r0 = norm0;
+  T norm0 = T(0), norm1 = T(0), r0 = T(0);
   T rho0 = 0, rho1 = 0, alpha0 = 0, alpha1 = 0, omega0 = 0, omega1 = 0;
-  bool init = true;
-  int restarts = 0, recount = 0, i = 0;
-  sync();
-  while (i < imax && norm0 > eps * norm1 && norm1 > T(0)) {
-    ++i;
+  bool init = true, fresh = true, begin = true;
+  int restarts = 0, recount = 0, it = 0;
+  for (;;) {
+    if (fresh) {
+      // residual of phi (at the start, and after a restart)
+      fresh = false;
+      sync();
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (own[m]) put(m, ph[m]);
+      sync();
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        if (!own[m]) continue;
+        r[m] = f[m] - vccell_lof<T, DIM>(X[m], sm, ph[m], hasc, D, beta, dxinv);
+        rt[m] = r[m];
+        e[m] = T(0);
+      }
+      norm0 = sqrt(dot(r, r));
+      if (begin) {
+        begin = false;
+        norm1 = norm0;
+        r0 = norm0;
+      } else {
+        rho0 = alpha0 = omega0 = T(0);
+        ++restarts;
+        init = true;
+      }
+    }
+    if (!(it < imax && norm0 > eps * norm1 && norm1 > T(0))) break;
+    ++it;
     norm1 = norm0;
     alpha1 = alpha0;
     omega1 = omega0;
@@ -674,47 +689,80 @@ __device__ __forceinline__ void vcx_bicgstab(const VCCtx<T, DIM>& X, const CLev&
     rho0 = dot(rt, r);
     if (rho0 == T(0)) break;
     if (init) {
-      for (int c = tid; c < N; c += stride) p[c] = r[c];
+      p[0] = r[0];
+      p[1] = r[1];
       init = false;
     } else {
       const T bt = (rho0 / rho1) * (alpha1 / omega1);
       const T sv = -bt * omega1;
-      for (int c = tid; c < N; c += stride) {
-        T q = bt * p[c];
-        q = q + sv * v[c];
-        p[c] = q + T(1) * r[c];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        T q = bt * p[m];
+        q = q + sv * vv[m];
+        p[m] = q + T(1) * r[m];
       }
     }
-    sync();
-    precond(pt, p);
-    apply(v, pt);
-    const T m = dot(rt, v);
-    alpha0 = rho0 / m;
-    if (fabs(m) > tiny * fabs(rho0)) {
-      const T na = -alpha0;
-      for (int c = tid; c < N; c += stride) {
-        r[c] = r[c] + na * v[c];
-        e[c] = e[c] + alpha0 * pt[c];
+    // half 0: pt = preCond(p), v = L pt; half 1: st = preCond(r), t = L st
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+      T g[2], z[2], w[2] = {T(0), T(0)};
+      sync();   // the last operator's reads are done
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        g[m] = half ? r[m] : p[m];
+        z[m] = T(0);
+        if (!own[m]) continue;
+        z[m] = g[m] * X[m].lam;
+        put(m, z[m]);
       }
       sync();
-      norm0 = sqrt(dot(r, r));
-    } else {
-      for (int c = tid; c < N; c += stride) r[c] = T(0);
-      sync();
-      norm0 = T(0);
-    }
-    if (norm0 > eps * r0 && norm0 > reps * r0) {
-      precond(st, r);
-      apply(t, st);
-      omega0 = dot(t, r) / dot(t, t);
-      sync();   // every wavefront has read r before it changes
-      const T nw = -omega0;
-      for (int c = tid; c < N; c += stride) {
-        e[c] = e[c] + omega0 * st[c];
-        r[c] = r[c] + nw * t[c];
+#pragma unroll 1
+      for (int pass = 0; pass < 5; ++pass) {
+        // four colour passes, then the operator at every cell
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          if (!own[m] || (pass < 4 && col[m] != (pass & 1))) continue;
+          const T lof = vccell_lof<T, DIM>(X[m], sm, z[m], hasc, D, beta, dxinv);
+          if (pass < 4) {
+            z[m] = z[m] - X[m].lam * (lof - g[m]);
+            put(m, z[m]);
+          } else {
+            w[m] = lof;
+          }
+        }
+        if (pass < 4) sync();
       }
-      sync();
-      norm0 = sqrt(dot(r, r));
+      if (half == 0) {
+        pt[0] = z[0];
+        pt[1] = z[1];
+        vv[0] = w[0];
+        vv[1] = w[1];
+        const T mm = dot(rt, vv);
+        alpha0 = rho0 / mm;
+        if (fabs(mm) > tiny * fabs(rho0)) {
+          const T na = -alpha0;
+#pragma unroll
+          for (int m = 0; m < 2; ++m) {
+            r[m] = r[m] + na * vv[m];
+            e[m] = e[m] + alpha0 * pt[m];
+          }
+          norm0 = sqrt(dot(r, r));
+        } else {
+          r[0] = r[1] = T(0);
+          norm0 = T(0);
+        }
+        if (!(norm0 > eps * r0 && norm0 > reps * r0)) break;
+      } else {
+        const T tr = dot(w, r), tt = dot(w, w);
+        omega0 = tr / tt;
+        const T nw = -omega0;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          e[m] = e[m] + omega0 * z[m];
+          r[m] = r[m] + nw * w[m];
+        }
+        norm0 = sqrt(dot(r, r));
+      }
     }
     if (norm0 <= eps * r0 || norm0 <= reps * r0) break;
     if (omega0 == T(0) || norm0 > (T(1) - hang) * norm1) {
@@ -722,160 +770,236 @@ __device__ __forceinline__ void vcx_bicgstab(const VCCtx<T, DIM>& X, const CLev&
         recount = 1;
       } else {
         recount = 0;
-        for (int c = tid; c < N; c += stride) phi[c] = phi[c] + T(1) * e[c];
+        ph[0] = ph[0] + T(1) * e[0];
+        ph[1] = ph[1] + T(1) * e[1];
         if (restarts == 5) {
-          for (int c = tid; c < N; c += stride) e[c] = T(0);
+          e[0] = e[1] = T(0);
           break;
         }
-        sync();
-        residual(r, phi, rhs);
-        norm0 = sqrt(dot(r, r));
-        rho0 = alpha0 = omega0 = T(0);
-        for (int c = tid; c < N; c += stride) {
-          rt[c] = r[c];
-          e[c] = T(0);
-        }
-        sync();
-        ++restarts;
-        init = true;
+        fresh = true;
       }
     }
   }
   sync();
-  for (int c = tid; c < N; c += stride) phi[c] = phi[c] + T(1) * e[c];
-  __syncthreads();
-}
-
-// one cell's operator data (and right-hand side) read from global memory
-template <typename T, int DIM>
-struct VCPre {
-  Faces1<T, DIM> F;
-  T aq, cv, r;
-};
-
-template <typename T, int DIM>
-__device__ __forceinline__ void vcpre_load(VCPre<T, DIM>& P, const VCLevel<T>& lv, const CLev& L, int c, bool rhs) {
-  if (c >= L.N) return;
-  int i, j, k;
-  clev_coords(L, c, i, j, k);
-  VCArgs<T> A;
-  A.g = lv.g;
-  for (int d = 0; d < 3; ++d) A.b[d] = lv.b[d];
-  load_faces1<T, DIM>(A, i, j, k, P.F);
-  const long long g = lv.g.ci(i, j, k);
-  P.aq = lv.a ? lv.a[g] : T(1);
-  P.cv = lv.c ? lv.c[g] : T(0);
-  if (rhs) P.r = lv.r[g];
-}
-
-template <typename T, int DIM>
-__device__ __forceinline__ void vcpre_store(const VCPre<T, DIM>& P, const VCLds<T, DIM>& S, const CLev& L, int c,
-                                            bool hasc, T alpha, T beta, bool rhs) {
-  if (c >= L.N) return;
-  const int q = L.off + c;
 #pragma unroll
-  for (int f = 0; f < 2 * DIM; ++f) S.sF[f * S.tot + q] = P.F.v[f];
-  S.sA[q] = P.aq;
-  S.sC[q] = P.cv;
-  const T dxinv = T(1) / (T(L.dx) * T(L.dx));
-  S.sL[q] = vc_lambda<T, DIM>(P.F, P.aq, hasc, P.cv, alpha, beta, dxinv);
-  if (rhs) {
-    S.se[q] = T(0);
-    S.sr[q] = P.r;
-  }
+  for (int m = 0; m < 2; ++m)
+    if (own[m]) Z[tid + m * kVCWG] = ph[m] + T(1) * e[m];
 }
 
 template <typename T, int DIM>
 __device__ __forceinline__ void vc_coarse_vcycle_body(const VCDesc<T>* __restrict__ Dp) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   constexpr int LL = VCLevels<DIM>::n;
+  typedef T vec2 __attribute__((ext_vector_type(2)));
   const VCDesc<T>& D = *Dp;
   if (D.skip && *D.skip) return;
-  const int l0 = D.l0, nl = D.nlev - D.l0;
-  const bool hasc = D.lev[l0].c != nullptr;
+  const int tid = threadIdx.x;
+  const int nl = D.nl, tot = D.tot, N0 = D.off[1];
+  const bool hasc = D.c[0] != nullptr, hasa = D.a[0] != nullptr;
   const T alpha = D.alpha, beta = D.beta;
-  int per[3];
-  for (int d = 0; d < 3; ++d) per[d] = D.lev[l0].g.periodic[d];
-  int bcm = 0;
-  for (int d = 0; d < DIM; ++d)
-    for (int sd = 0; sd < 2; ++sd) bcm |= (D.bc.type[d][sd][0] != 0 ? 1 : 0) << (2 * d + sd);
-  CLev G[LL];
-  int tot = 0;
-#pragma unroll
-  for (int l = 0; l < LL; ++l) {
-    if (l >= nl) continue;
-    clev_set(G[l], D.lev[l0 + l].g, tot);
-    tot += G[l].N;
-  }
-  VCLds<T, DIM> S;
-  S.tot = tot;
-  S.se = reinterpret_cast<T*>(smem_raw);
-  S.sr = S.se + tot;
-  S.sF = S.sr + tot;
-  S.sA = S.sF + 2 * DIM * tot;
-  S.sC = S.sA + tot;
-  S.sL = S.sC + tot;
-  S.sres = S.sL + tot;
-  // operator data of every level, and level l0's right-hand side: all
-  // global loads first (level l0: cells t and t + 512, coarser levels: cell
-  // t), then the LDS stores
-  VCPre<T, DIM> P0[2], P1[LL - 1];
-#pragma unroll
-  for (int m = 0; m < 2; ++m) vcpre_load<T, DIM>(P0[m], D.lev[l0], G[0], threadIdx.x + m * kVCWG, true);
-#pragma unroll
-  for (int l = 1; l < LL; ++l)
-    if (l < nl) vcpre_load<T, DIM>(P1[l - 1], D.lev[l0 + l], G[l], threadIdx.x, false);
-#pragma unroll
-  for (int m = 0; m < 2; ++m) vcpre_store<T, DIM>(P0[m], S, G[0], threadIdx.x + m * kVCWG, hasc, alpha, beta, true);
-#pragma unroll
-  for (int l = 1; l < LL; ++l)
-    if (l < nl) vcpre_store<T, DIM>(P1[l - 1], S, G[l], threadIdx.x, hasc, alpha, beta, false);
-  __syncthreads();
-  // The level visits below are runtime loops over one copy of their code
-  // (levels rebuilt from the descriptor, offsets by prefix sum): unrolled
-  // per level, the kernel's code is several times the instruction cache and
-  // a launch spends most of its time fetching it.
-  auto level = [&](int l) __attribute__((always_inline)) {
+  const VCLdsMap M = vc_lds_map(tot, D.nfaces, hasa, hasc);
+  T* sm = reinterpret_cast<T*>(smem_raw);
+  T *E = sm + M.e, *R = sm + M.r, *LM = sm + M.lm, *SX = sm + M.x;
+  auto level_of = [&](int l) __attribute__((always_inline)) {
     CLev L;
-    int off = 0;
-    for (int q = 0; q < l; ++q) off += int(D.lev[l0 + q].g.nvalid());
-    clev_set(L, D.lev[l0 + l].g, off);
+    for (int d = 0; d < 3; ++d) L.n[d] = d < DIM ? D.n[d] >> l : 1;
+    L.nx = L.n[0];
+    L.nxy = L.n[0] * L.n[1];
+    L.off = D.off[l];
+    L.N = D.off[l + 1] - L.off;
+    L.dx = D.dx * double(1 << l);
     return L;
   };
-  // down: pre-smoothing and restriction; the coarsest level gets the bottom
-  // smoothing
-#pragma unroll 1
-  for (int l = 0; l < nl; ++l) {
-    const CLev Ll = level(l);
-    VCCtx<T, DIM> X;
-    vcx_build<T, DIM>(X, Ll, per, S);
-    vcx_relax<T, DIM>(X, Ll, bcm, S, hasc, alpha, beta, 2 * (l == nl - 1 ? D.bottom : D.nu1));
-    if (l + 1 < nl) vcx_restrict<T, DIM>(X, Ll, level(l + 1), bcm, S, hasc, alpha, beta);
-  }
-  // the bottom solver on the coarsest level (after its relaxations)
-  if (D.bottom_solver == 1) {
-    const Geom& gb = D.lev[D.nlev - 1].g;
-    CLev Lb;
-    clev_set(Lb, gb, tot - int(gb.nvalid()));
-    VCCtx<T, DIM> X;
-    vcx_build<T, DIM>(X, Lb, per, S);
-    vcx_bicgstab<T, DIM>(X, Lb, bcm, S, hasc, alpha, beta, D.bottom_imax, S.sres + kVCWGCells);
-  }
-  // up: prolongation and post-smoothing
-#pragma unroll 1
-  for (int l = nl - 2; l >= 0; --l) {
-    const CLev Ll = level(l);
-    VCCtx<T, DIM> X;
-    vcx_build<T, DIM>(X, Ll, per, S);
-    vcx_prolong<T, DIM>(X, Ll, level(l + 1), S.se);
-    vcx_relax<T, DIM>(X, Ll, bcm, S, hasc, alpha, beta, 2 * D.nu2);
-  }
-  const VCLevel<T>& lv = D.lev[l0];
-  for (int c = threadIdx.x; c < G[0].N; c += kVCWG) {
+  const CLev L0 = level_of(0);
+  // right-hand side of the first level, a and c of all levels, the faces: all
+  // global loads first
+  auto fab = [&](const CLev& L, int c) __attribute__((always_inline)) {
     int i, j, k;
-    clev_coords(G[0], c, i, j, k);
-    lv.e[lv.g.ci(i, j, k)] = S.se[c];
+    clev_coords(L, c, i, j, k);
+    const int sy = L.n[0] + 2, sz = sy * (L.n[1] + 2);
+    return (i + 1) + sy * (j + 1) + (DIM == 3 ? sz * (k + 1) : 0);
+  };
+  T r0[2];
+  int q0[2];
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const int c = tid + m * kVCWG;
+    if (c >= N0) continue;
+    q0[m] = fab(L0, c);
+    r0[m] = D.r[q0[m]];
   }
+  if (hasc || hasa) {
+    // level 0: cells t and t + 512; coarser levels: cell t
+    T cv[LL + 1], av[LL + 1];
+#pragma unroll
+    for (int l = 0; l < LL; ++l) {
+      if (l >= nl) continue;
+      const CLev L = level_of(l);
+#pragma unroll
+      for (int m = 0; m < (l ? 1 : 2); ++m) {
+        const int c = tid + m * kVCWG;
+        if (c >= L.N) continue;
+        const int q = l ? fab(L, c) : q0[m];
+        if (hasc) cv[l + (l ? 1 : m)] = D.c[l][q];
+        if (hasa) av[l + (l ? 1 : m)] = D.a[l][q];
+      }
+    }
+#pragma unroll
+    for (int l = 0; l < LL; ++l) {
+      if (l >= nl) continue;
+#pragma unroll
+      for (int m = 0; m < (l ? 1 : 2); ++m) {
+        const int c = tid + m * kVCWG;
+        if (c >= D.off[l + 1] - D.off[l]) continue;
+        if (hasc) sm[M.c + D.off[l] + c] = cv[l + (l ? 1 : m)];
+        if (hasa) sm[M.a + D.off[l] + c] = av[l + (l ? 1 : m)];
+      }
+    }
+  }
+  {
+    constexpr int KF = 4;
+    const vec2* src = reinterpret_cast<const vec2*>(D.faces);
+    T* dst = sm + M.f;
+    const int n2 = D.nfaces >> 1;
+#pragma unroll 1
+    for (int base = tid; base < n2; base += KF * kVCWG) {
+      vec2 v[KF];
+#pragma unroll
+      for (int k = 0; k < KF; ++k)
+        if (base + k * kVCWG < n2) v[k] = src[base + k * kVCWG];
+#pragma unroll
+      for (int k = 0; k < KF; ++k)
+        if (base + k * kVCWG < n2) {
+          dst[2 * (base + k * kVCWG)] = v[k].x;
+          dst[2 * (base + k * kVCWG) + 1] = v[k].y;
+        }
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    if (tid + m * kVCWG < N0) R[tid + m * kVCWG] = r0[m];
+  __syncthreads();
+
+#pragma unroll 1
+  for (int v = 0; v < 2 * nl - 1; ++v) {
+    const bool up = v >= nl, bot = v == nl - 1, down = v < nl - 1;
+    const int l = up ? 2 * nl - 2 - v : v;
+    const CLev L = level_of(l);
+    const int off = L.off, offc = off + L.N;
+    const bool even = (L.nx & 1) == 0;
+    const bool small = cown_active<kVCWG>(L) <= 64;
+    const int step = small ? 64 : kVCWG;   // threads of this visit
+    const T dx = T(L.dx);
+    const T dxinv = T(1) / (dx * dx);
+    auto sync = [&]() __attribute__((always_inline)) {
+      if (small)
+        wave_sync();
+      else
+        __syncthreads();
+    };
+    int fo[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) fo[d] = D.fo[l][d];
+    if (!small || tid < 64) {
+      COwn o;
+      cown_set<kVCWG>(L, o);
+      VCCell<T, DIM> X[2];
+      int c[2], col[2];
+      T u[2], rr[2];
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        c[m] = 0;
+        if (o.p[m] < 0) continue;
+        int i, j, k;
+        cunpack(o.p[m], i, j, k);
+        c[m] = i + L.nx * j + L.nxy * k;
+        col[m] = (i + j + k) & 1;
+        vccell_build<T, DIM>(X[m], D, M, sm, L, fo, i, j, k, m * kVCWG + tid, hasa, hasc, alpha, beta, dxinv, up, LM);
+        rr[m] = R[off + c[m]];
+        // from zero on the way down, e_f + e_c(parent) on the way up
+        u[m] = T(0);
+        if (up)
+          u[m] = E[off + c[m]] +
+                 E[offc + (i >> 1) + (L.nx >> 1) * ((j >> 1) + (DIM == 3 ? (L.n[1] >> 1) * (k >> 1) : 0))];
+      }
+      auto put = [&](int m) __attribute__((always_inline)) {
+        E[off + c[m]] = u[m];
+        SX[m * kVCWG + tid] = fma(X[m].ws, u[m], X[m].wb);
+      };
+#pragma unroll
+      for (int m = 0; m < 2; ++m)
+        if (o.p[m] >= 0) put(m);
+      sync();
+      auto update = [&](auto MM) __attribute__((always_inline)) {
+        constexpr int m = decltype(MM)::value;
+        if (o.p[m] < 0) return;
+        const T lof = vccell_lof<T, DIM>(X[m], sm, u[m], hasc, D, beta, dxinv);
+        u[m] = u[m] - X[m].lam * (lof - rr[m]);
+        put(m);
+      };
+      const int its = bot ? D.bottom : (up ? D.nu2 : D.nu1);
+      if (even) {
+#pragma unroll 1
+        for (int it = 0; it < its; ++it) {
+          update(IC<0>{});
+          sync();
+          update(IC<1>{});
+          sync();
+        }
+      } else {
+#pragma unroll 1
+        for (int p = 0; p < 2 * its; ++p) {
+          if (o.p[0] >= 0 && col[0] == (p & 1)) update(IC<0>{});
+          if (o.p[1] >= 0 && col[1] == (p & 1)) update(IC<1>{});
+          sync();
+        }
+      }
+      if (down) {
+        // restricted residual (homogeneous BCs, RESTRICTRESDB order)
+        const T rdenom = DIM == 3 ? T(0.125) : T(0.25);
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (o.p[m] >= 0) rr[m] = (rr[m] - vccell_lof<T, DIM>(X[m], sm, u[m], hasc, D, beta, dxinv)) * rdenom;
+        sync();   // the ghosts in SX have been read
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+          if (o.p[m] >= 0) SX[c[m]] = rr[m];
+        sync();
+        const CLev C = level_of(l + 1);
+#pragma unroll 1
+        for (int cc = tid; cc < C.N; cc += step) {
+          int I, J, K;
+          clev_coords(C, cc, I, J, K);
+          const int f0 = 2 * I + L.nx * (2 * J) + (DIM == 3 ? L.nxy * (2 * K) : 0);
+          T s = T(0);
+#pragma unroll
+          for (int kk = 0; kk < (DIM == 3 ? 2 : 1); ++kk)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+              for (int ii = 0; ii < 2; ++ii) s = s + SX[f0 + ii + L.nx * jj + L.nxy * kk];
+          R[offc + cc] = s;
+        }
+      }
+    }
+    if (bot && D.bottom_solver == 1) {
+      if (!small) __syncthreads();
+      if (small && L.N > 64) __syncthreads();   // all waves join the solver
+      vcx_bicgstab<T, DIM>(D, M, sm, L, fo, hasa, hasc, alpha, beta, D.bottom_imax, M.end);
+    }
+    // the next visit reads what this one wrote: wave 0 alone where both are
+    // small, else the workgroup
+    bool next_small = false;
+    if (small && !(bot && D.bottom_solver == 1 && L.N > 64) && v + 1 < 2 * nl - 1)
+      next_small = cown_active<kVCWG>(level_of(v + 1 >= nl ? 2 * nl - 3 - v : v + 1)) <= 64;
+    if (!next_small)
+      __syncthreads();
+    else if (tid < 64)
+      wave_sync();
+  }
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    if (tid + m * kVCWG < N0) D.e[q0[m]] = E[tid + m * kVCWG];
 }
 
 template <typename T, int DIM>
@@ -1581,11 +1705,46 @@ hipError_t vc_coarse_batch(int dim, const VCDesc<T>* const* descs, int n, size_t
 
 template <typename T>
 size_t vc_coarse_lds_bytes(const Geom* g, int l0, int nlev, bool bicgstab) {
-  long long tot = 0;
-  for (int l = l0; l < nlev; ++l) tot += g[l].nvalid();
-  // BiCGStab: 8 vectors of the coarsest level after the restriction scratch
-  const size_t extra = bicgstab ? size_t(8 * g[nlev - 1].nvalid()) : 0;
-  return (vc_coarse_lds_elems<T>(g[l0].dim, tot) + extra) * sizeof(T);
+  long long tot = 0, nf = 0;
+  for (int l = l0; l < nlev; ++l) {
+    tot += g[l].nvalid();
+    for (int d = 0; d < g[l].dim; ++d) nf += g[l].nface[d];
+  }
+  // with a and c; BiCGStab above 64 cells: two buffers of products
+  const long long N = g[nlev - 1].nvalid();
+  const size_t extra = bicgstab && N > 64 ? size_t(2 * N) : 0;
+  return (size_t(vc_lds_map(int(tot), int(nf + (nf & 1)), true, true).end) + extra) * sizeof(T);
+}
+
+template <typename T>
+void vc_desc_geometry(VCDesc<T>& D, const Geom& g, const BCDesc& bc, int nl) {
+  D.nl = nl;
+  for (int d = 0; d < 3; ++d) {
+    D.n[d] = g.n[d];
+    D.per[d] = g.periodic[d];
+  }
+  D.dx = T(g.dx);
+  int fo = 0;
+  for (int l = 0; l < nl; ++l) {
+    const Geom gl = l == 0 ? g : coarsen_geom(g, 1 << l);
+    D.off[l + 1] = D.off[l] + int(gl.nvalid());
+    for (int d = 0; d < g.dim; ++d) {
+      D.fo[l][d] = fo;
+      fo += int(gl.nface[d]);
+    }
+  }
+  D.tot = D.off[nl];
+  BCDesc hom = bc;
+  hom.apply = 1;
+  for (auto& d : hom.val)
+    for (auto& s : d)
+      for (auto& v : s) v = 0.0;
+  const GhostForm<T> gf = ghost_form<T>(hom, T(g.dx));
+  for (int d = 0; d < 3; ++d)
+    for (int s = 0; s < 2; ++s) {
+      D.gs[d][s] = gf.s[d][s][0];
+      D.gb[d][s] = gf.b[d][s][0];
+    }
 }
 
 template <typename T>
@@ -1615,6 +1774,7 @@ template hipError_t vc_lambda_mult<double>(const VCArgs<double>&, const double*,
 template hipError_t vc_dot<double>(const Geom&, const double*, const double*, double*, hipStream_t);
 template hipError_t vc_restrict_residual<double>(const VCArgs<double>&, const Geom&, const double*, const double*,
                                                  double*, hipStream_t);
+template void vc_desc_geometry<double>(VCDesc<double>&, const Geom&, const BCDesc&, int);
 template hipError_t vc_coarse_vcycle<double>(const VCDesc<double>*, int, size_t, hipStream_t);
 template size_t vc_coarse_lds_bytes<double>(const Geom*, int, int, bool);
 template hipError_t vc_relax_batch<double>(int, int, const VCRelaxJob<double>*, const unsigned*, int, size_t,

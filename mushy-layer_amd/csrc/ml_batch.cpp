@@ -433,7 +433,7 @@ int build_tables(ml_hc_batch b, double* const* phi, const double* const* src, do
     R.M32 = I.lin[0].M;
     R.slots = slots;
     R.ctl = ctl;
-    R.arrive = b->arrive + i;
+    R.arrive = b->arrive + i * (kArriveBytes / sizeof(unsigned int));
     R.ntiles = unsigned(I.nres);
     R.ntx = I.res_ntx;
     R.nty = I.res_nty;
@@ -728,7 +728,7 @@ int ml_hc_batch_create(ml_ctx ctx, int count, const ml_hc_op ops[], ml_hc_batch*
   if (rc == ML_OK) rc = max_lds(ctx, &maxlds);
   if (rc == ML_OK) rc = dalloc(b, sizeof(SolveCtl) * count, &b->ctl);
   if (rc == ML_OK) rc = dalloc(b, sizeof(unsigned long long) * kBatchSlots * count, &b->slots);
-  if (rc == ML_OK) rc = dalloc(b, sizeof(unsigned int) * count, &b->arrive);
+  if (rc == ML_OK) rc = dalloc(b, kArriveBytes * count, &b->arrive);
   if (rc == ML_OK) {
     if (hipHostMalloc(&v, sizeof(SolveCtl) * count, hipHostMallocDefault) != hipSuccess)
       rc = fail(ctx, ML_ENOMEM, "hipHostMalloc");

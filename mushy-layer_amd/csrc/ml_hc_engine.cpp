@@ -99,9 +99,9 @@ int HCEngine::init() {
   m_hslots = static_cast<unsigned long long*>(p);
   ML_HIP(ctx, hipMalloc(&p, sizeof(SolveCtl)));
   m_ctl = static_cast<SolveCtl*>(p);
-  ML_HIP(ctx, hipMalloc(&p, sizeof(unsigned int)));
+  ML_HIP(ctx, hipMalloc(&p, kArriveBytes));
   m_arrive = static_cast<unsigned int*>(p);
-  ML_HIP(ctx, hipMemsetAsync(m_arrive, 0, sizeof(unsigned int), ctx->stream));
+  ML_HIP(ctx, hipMemsetAsync(m_arrive, 0, kArriveBytes, ctx->stream));
   ML_HIP(ctx, hipHostMalloc(&p, sizeof(SolveCtl), hipHostMallocDefault));
   m_hctl = static_cast<SolveCtl*>(p);
   return ML_OK;

@@ -72,10 +72,21 @@ __device__ inline void ctl_check_step(SolveCtl* c, const unsigned long long* slo
 }
 
 // The stopping rule applied by the last workgroup of the kernel that
-// computes the residual norm (ctl == nullptr: none).  `arrive` counts the
-// workgroups that have added their norm; the last one resets it.  A kernel
-// given no norm pointer writes the norm into slots[ctl->iter + 1] (the
-// iteration it completes), so the same launch serves every iteration.
+// computes the residual norm (ctl == nullptr: none).  `arrive` (kArriveBytes,
+// zero between launches) counts the workgroups that have added their norm;
+// the last one resets it.  A kernel given no norm pointer writes the norm
+// into slots[ctl->iter + 1] (the iteration it completes), so the same launch
+// serves every iteration.
+//
+// Atomics on one address are performed one after another, some 10 ns each:
+// with 4096 workgroups they were 44 of a residual's 54 us.  So a large grid
+// reports in kArriveGroups groups, each with its maximum and its count on a
+// line of its own, and the last workgroup of a group reports for the group;
+// a grid of up to kArriveDirect workgroups, whose atomics take less than
+// the second level's round trips, reports directly.
+constexpr unsigned kArriveGroups = 32, kArriveDirect = 512;
+constexpr unsigned kArriveLine = 128 / sizeof(unsigned int);   // words of a line
+constexpr size_t kArriveBytes = (1 + kArriveGroups) * 128;     // the counter, then the groups (maximum, count)
 struct CtlFuse {
   SolveCtl* ctl;
   const unsigned long long* slots;
@@ -111,25 +122,38 @@ __device__ inline void block_max_atomic(T v, int nan, unsigned long long* out, C
       const double o = wmax[i];
       m = (o != o || m != m) ? __longlong_as_double(0x7ff8000000000000LL) : (o > m ? o : m);
     }
-    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    const unsigned int grid = gridDim.x * gridDim.y * gridDim.z;
+    const bool direct = grid <= kArriveDirect || f.total;
     if (!f.ctl) {
-      atomicMax(out, bits);
-    } else {
-      // Device-scope atomics are performed at the device's coherence point.
-      // The arrival is counted only once this workgroup's maximum has been
-      // performed there: the increment depends on the value the max returns
-      // (the sign bit of a stored norm, always 0), so the wave waits for it.
-      // The last arrival then reads every maximum with device-scope atomic
-      // loads; no fence (and no L2 write-back) is needed in any workgroup.
-      const unsigned long long before =
-          __hip_atomic_fetch_max(out, bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned int inc = 1u + unsigned(before >> 63);
-      const unsigned int total = f.total ? f.total : gridDim.x * gridDim.y * gridDim.z;
-      if (__hip_atomic_fetch_add(f.arrive, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == total - 1) {
-        __hip_atomic_store(f.arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        ctl_check_step(f.ctl, f.slots, f.refined);
-      }
+      // (a maximum already passed needs no atomic)
+      if (direct || bits > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, bits);
+      return;
     }
+    // Device-scope atomics are performed at the device's coherence point.
+    // An arrival is counted only once this workgroup's maximum has been
+    // performed there: the increment depends on the value the max returns
+    // (the sign bit of a stored norm, always 0), so the wave waits for it.
+    // The last arrival then reads every maximum with device-scope atomics;
+    // no fence (and no L2 write-back) is needed in any workgroup.
+    auto report = [](unsigned long long* to, unsigned long long v, unsigned int* count, unsigned int members) {
+      const unsigned long long before = __hip_atomic_fetch_max(to, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned int inc = 1u + unsigned(before >> 63);
+      if (__hip_atomic_fetch_add(count, inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != members - 1) return false;
+      __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return true;
+    };
+    unsigned int members = f.total ? f.total : grid;
+    if (!direct) {
+      const unsigned int id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+      const unsigned int grp = id % kArriveGroups;
+      unsigned int* line = f.arrive + (1 + grp) * kArriveLine;
+      unsigned long long* gmax = reinterpret_cast<unsigned long long*>(line);
+      if (!report(gmax, bits, line + 2, (grid - grp + kArriveGroups - 1) / kArriveGroups)) return;
+      bits = __hip_atomic_exchange(gmax, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      members = kArriveGroups;
+    }
+    if (report(out, bits, f.arrive, members)) ctl_check_step(f.ctl, f.slots, f.refined);
   }
 }
 

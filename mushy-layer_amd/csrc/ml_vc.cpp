@@ -154,9 +154,9 @@ int vc_work_init(ml_vc_op op, ml::VCWork& W, bool own_stream) {
   W.ctl = static_cast<ml::SolveCtl*>(p);
   ML_HIP(ctx, hipHostMalloc(&p, sizeof(ml::SolveCtl), hipHostMallocDefault));
   W.hctl = static_cast<ml::SolveCtl*>(p);
-  ML_HIP(ctx, hipMalloc(&p, sizeof(unsigned int)));
+  ML_HIP(ctx, hipMalloc(&p, ml::kArriveBytes));
   W.arrive = static_cast<unsigned int*>(p);
-  ML_HIP(ctx, hipMemsetAsync(W.arrive, 0, sizeof(unsigned int), ctx->stream));
+  ML_HIP(ctx, hipMemsetAsync(W.arrive, 0, ml::kArriveBytes, ctx->stream));
   ML_HIP(ctx, hipEventCreateWithFlags(&W.joined, hipEventDisableTiming));
   if (own_stream) {
     ML_HIP(ctx, hipStreamCreateWithFlags(&W.stream, hipStreamNonBlocking));

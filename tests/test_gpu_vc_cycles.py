@@ -57,3 +57,33 @@ def test_single_workgroup_cycles(ml, gpu_ctx, name, acoef, ccoef, bicgstab):
     assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     assert HC.bitwise_equal(np.ascontiguousarray(HC.valid(n, dphi.get())), np.ascontiguousarray(HC.valid(n, phi)))
     op.close()
+
+
+@pytest.mark.parametrize("n", [(1024, 128), (1024, 132), (1056, 128), (40, 4360), (1504, 776)])
+def test_residual_norms_of_many_workgroups(ml, gpu_ctx, n):
+    """The stopping rule sees the largest residual of every workgroup: grids
+    of 512 workgroups (which report one by one), just above (in groups of
+    unequal size) and several thousand, the largest value in the first, a
+    middle and the last workgroup, solve after solve on one operator."""
+    dx = 1.0 / n[0]
+    g = O.make_grid(n, dx, [1, 0, 0])
+    b = [np.ones(O.face_shape(g, d, 1)) for d in range(2)]
+    bc = {(1, s, 0): (0, 0.0) for s in (0, 1)}
+    op = ml.VCOp(gpu_ctx, list(n), dx, [1, 0], ml.make_bc(bc))
+    dev = lambda x: ml.DeviceArray(gpu_ctx, x.shape, host=x)
+    db = [dev(x) for x in b]
+    op.set_coefs(None, db, None, 1.0, -1e-7)
+    kw = dict(max_iter=2, nu1=1, nu2=1, bottom=2, eps=1e-15, hang=1e-15, norm_thresh=1e-15)
+    rng = np.random.default_rng(n[1])
+    for spot in ((0, 0), (n[0] // 2, n[1] // 2), (n[0] - 1, n[1] - 1)):
+        rhs = np.zeros(O.cell_shape(g, 1))
+        v = O.valid(g, rhs)
+        v[...] = 1e-3 * rng.standard_normal(v.shape)
+        v[(0,) * (v.ndim - 2) + spot[::-1]] = 7.0
+        phi = np.zeros(O.cell_shape(g, 1))
+        so = O.lin_mg_solve(g, 1, O.make_bc(bc), 1.0, None, -1e-7, None, b, phi, rhs, opts=O.default_opts(**kw))
+        dphi = dev(np.zeros_like(phi))
+        st = op.solve(dphi, dev(rhs), opts=ml.default_opts(**kw))
+        assert st.initial_residual == so.initial_residual == 7.0
+        assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
+    op.close()

@@ -1198,10 +1198,10 @@ __global__ void hc_diffused_var_kernel(HCArgs<T> A, const T* __restrict__ phi, T
   }
 }
 
-// ---- streaming relaxation for large levels -------------------------------
+// ---- streaming relaxation for large 2D levels ----------------------------
 // The (H, Theta) counterpart of the linear operator's streaming kernel: a
-// workgroup owns a block of columns and a segment of planes along the last
-// direction and marches through them with a window of 4 planes in LDS
+// workgroup owns a block of columns and a segment of rows ("planes" below)
+// and marches through them with a window of 4 planes in LDS
 // holding (H, Theta) and their closure (theta, Theta_l).  With plane R just
 // loaded (and its closure taken), colour pass p runs on plane R-1-p, so
 // plane R-P is final and is written.  A cell's pass reads its own state and
@@ -1212,23 +1212,23 @@ __global__ void hc_diffused_var_kernel(HCArgs<T> A, const T* __restrict__ phi, T
 // Per plane and position the face coefficients, rhs (and aCoef) stay in
 // registers in compile-time-indexed sets, loaded two planes ahead; lambda is
 // formed where it is used.  Every input is read once per launch.
-template <typename T, int DIM>
+template <typename T>
 struct HCoef {
-  CellFaces<T, DIM> F;
+  CellFaces<T, 2> F;
   T rr[2], aq[2], v[2];   // rhs, aCoef, state as loaded
 };
 
-template <typename T, int DIM, int TX, int TY, int P, int NT, bool HASA>
+template <typename T, int TX, int P, int NT, bool HASA>
 __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const T* __restrict__ in,
                                                              T* __restrict__ out, const T* __restrict__ rhs,
-                                                             int first, int nbx, int nby, int seg) {
+                                                             int first, int nbx, int seg) {
   if (A.skip && *A.skip) return;
   constexpr int EX = TX + 2 * P;
-  constexpr int EL = EX * (DIM == 3 ? TY + 2 * P : 1);
+  constexpr int EL = EX;
   constexpr int K = (EL + NT - 1) / NT;
   static_assert(P >= 1 && P <= 2, "one or two colour passes per launch");
   constexpr int W = 4;   // planes in the window
-  constexpr int MD = DIM - 1;
+  constexpr int MD = 1;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* su = reinterpret_cast<T*>(smem_raw);
   const Geom& g = A.g;
@@ -1236,12 +1236,8 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
   const bool zper = g.periodic[MD] != 0;
   const T dxinv = T(1) / (T(g.dx) * T(g.dx));
   const T dxg = T(g.dx);
-  int b = blockIdx.x;
-  const int bx = b % nbx;
-  b /= nbx;
-  const int by = DIM == 3 ? b % nby : 0;
-  const int bz = DIM == 3 ? b / nby : b;
-  const int x0 = bx * TX, y0 = by * TY;
+  const int bx = int(blockIdx.x) % nbx, bz = int(blockIdx.x) / nbx;
+  const int x0 = bx * TX;
   const int z0 = bz * seg;
   const int z1 = z0 + seg < nz ? z0 + seg : nz;
   SPos S[K];
@@ -1253,14 +1249,13 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
     gt[kk][0] = gt[kk][1] = 0;
     gval[kk][0] = gval[kk][1] = T(0);
     if (e < EL) {
-      spos_init<DIM, TX, TY, P>(g, x0, y0, e, S[kk]);
-      for (int d = 0; d < DIM - 1; ++d)
-        for (int sd = 0; sd < 2; ++sd)
-          if (S[kk].kind == 2 && S[kk].gd == d && S[kk].gs == sd)
-            for (int n = 0; n < 2; ++n) {
-              gt[kk][n] = A.bc.type[d][sd][n];
-              gval[kk][n] = T(A.bc.val[d][sd][n]);
-            }
+      spos_init<TX, P>(g, x0, e, S[kk]);
+      for (int sd = 0; sd < 2; ++sd)
+        if (S[kk].kind == 2 && S[kk].gs == sd)
+          for (int n = 0; n < 2; ++n) {
+            gt[kk][n] = A.bc.type[0][sd][n];
+            gval[kk][n] = T(A.bc.val[0][sd][n]);
+          }
     } else {
       S[kk].kind = 0;
       S[kk].dist = P;
@@ -1275,32 +1270,31 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
   auto zwrap = [&](int z) { return z < 0 ? z + nz : (z >= nz ? z - nz : z); };
   auto real_plane = [&](int z) { return zper || (z >= 0 && z < nz); };
   // 32-bit element offsets (levels below 2^28 cells per component)
-  const unsigned csz = unsigned(DIM == 3 ? g.sz : g.sy);
+  const unsigned csz = unsigned(g.sy);
   const unsigned cn = unsigned(g.ncell);
-  unsigned fpl[DIM], fup[DIM], fn[DIM];
+  unsigned fpl[2], fup[2], fn[2];
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    fpl[d] = unsigned(g.fn[d][0] * (DIM == 3 ? g.fn[d][1] : 1));
+  for (int d = 0; d < 2; ++d) {
+    fpl[d] = unsigned(g.fn[d][0]);
     fn[d] = unsigned(g.nface[d]);
   }
   fup[0] = 1;
-  if (DIM == 3) fup[1] = unsigned(g.fn[1][0]);
   fup[MD] = fpl[MD];
-  unsigned cl[K], fl[K][DIM];
+  unsigned cl[K], fl[K][2];
 #pragma unroll
   for (int kk = 0; kk < K; ++kk) {
     const SPos& s = S[kk];
-    cl[kk] = unsigned(s.gx + 1) + (DIM == 3 ? unsigned(g.sy) * unsigned(s.gy + 1) : 0u);
+    cl[kk] = unsigned(s.gx + 1);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
-      fl[kk][d] = unsigned(s.gx) + (DIM == 3 ? unsigned(g.fn[d][0]) * unsigned(s.gy) : 0u);
+    for (int d = 0; d < 2; ++d)
+      fl[kk][d] = unsigned(s.gx);
   }
   auto ld = [](const T* p, unsigned i) -> T {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (i * unsigned(sizeof(T))));
   };
   constexpr int NS = P + 3;
-  HCoef<T, DIM> cs[NS][K];
-  auto prefetch = [&](int R, HCoef<T, DIM>(&pf)[K]) {
+  HCoef<T> cs[NS][K];
+  auto prefetch = [&](int R, HCoef<T>(&pf)[K]) {
     const int zw = zper ? zwrap(R) : (R < 0 ? 0 : (R >= nz ? nz - 1 : R));
     const unsigned qz = unsigned(zw + 1) * csz;
 #pragma unroll
@@ -1312,7 +1306,7 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
         pf[kk].rr[n] = ld(rhs, q + unsigned(n) * cn);
         if (HASA) pf[kk].aq[n] = ld(A.a, q + unsigned(n) * cn);
 #pragma unroll
-        for (int d = 0; d < DIM; ++d) {
+        for (int d = 0; d < 2; ++d) {
           const unsigned f = fl[kk][d] + unsigned(zw) * fpl[d] + unsigned(n) * fn[d];
           pf[kk].F.v[n][2 * d] = ld(A.b[d], f);
           pf[kk].F.v[n][2 * d + 1] = ld(A.b[d], f + fup[d]);
@@ -1385,9 +1379,9 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
           const SPos& s = S[kk];
-          if (s.kind != 1 || s.dist > reach || ((s.gx + s.gy + zw + colour) & 1)) continue;
+          if (s.kind != 1 || s.dist > reach || ((s.gx + zw + colour) & 1)) continue;
           const int e = threadIdx.x + kk * NT;
-          const HCoef<T, DIM>& C = cs[jp][kk];
+          const HCoef<T>& C = cs[jp][kk];
           T nv[2];
 #pragma unroll
           for (int n = 0; n < 2; ++n) {
@@ -1396,19 +1390,12 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
             st[0] = lz[e];
             st[1] = lz[e + 1];
             st[2] = lz[e - 1];
-            if (DIM == 3) {
-              st[3] = lz[e + EX];
-              st[4] = lz[e - EX];
-              st[5] = pp[(2 + n) * EL + e];
-              st[6] = pm[(2 + n) * EL + e];
-            } else {
-              st[3] = pp[(2 + n) * EL + e];
-              st[4] = pm[(2 + n) * EL + e];
-            }
+            st[3] = pp[(2 + n) * EL + e];
+            st[4] = pm[(2 + n) * EL + e];
             const T ph = pz[n * EL + e];
             const T aq = HASA ? C.aq[n] : T(1);
-            const T lam = lambda_of<T, DIM>(C.F, n, aq, A.alpha, A.beta, dxinv);
-            const T lof = lof_of<T, DIM>(C.F, n, st, aq, ph, A.alpha, A.beta, dxinv);
+            const T lam = lambda_of<T, 2>(C.F, n, aq, A.alpha, A.beta, dxinv);
+            const T lof = lof_of<T, 2>(C.F, n, st, aq, ph, A.alpha, A.beta, dxinv);
             nv[n] = ph - lam * (lof - C.rr[n]);
           }
           pz[e] = nv[0];
@@ -1421,18 +1408,14 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
           pz[2 * EL + e] = th;
           pz[3 * EL + e] = clv;
           // wall ghosts of this cell: lateral, then along the march
-          const int glc[2] = {s.gx, s.gy};
-#pragma unroll
-          for (int d = 0; d < (DIM == 3 ? 2 : 1); ++d) {
-            if (g.periodic[d]) continue;
-            const int st1 = d == 0 ? 1 : EX;
-            if (glc[d] == 0) {
-              pz[2 * EL + e - st1] = ghost(d, 0, 0, th);
-              pz[3 * EL + e - st1] = ghost(d, 0, 1, clv);
+          if (!g.periodic[0]) {
+            if (s.gx == 0) {
+              pz[2 * EL + e - 1] = ghost(0, 0, 0, th);
+              pz[3 * EL + e - 1] = ghost(0, 0, 1, clv);
             }
-            if (glc[d] == g.n[d] - 1) {
-              pz[2 * EL + e + st1] = ghost(d, 1, 0, th);
-              pz[3 * EL + e + st1] = ghost(d, 1, 1, clv);
+            if (s.gx == g.n[0] - 1) {
+              pz[2 * EL + e + 1] = ghost(0, 1, 0, th);
+              pz[3 * EL + e + 1] = ghost(0, 1, 1, clv);
             }
           }
           if (!zper) {
@@ -1639,42 +1622,171 @@ static hipError_t launch_relax_tile3(const HCArgs<T>& A, TileIO<T> io, hipStream
   return err;
 }
 
-// streaming launch shapes: 2D columns of 252 cells (256 threads), 3D blocks
-// of 12 x 12 columns
-template <int DIM>
-struct HCStream;
-template <>
-struct HCStream<2> {
-  static constexpr int NT = 256, TY = 1, SEGMIN = 8;
+// One colour pass of a 3D level straight from memory (Sweep3).  The closure
+// of the neighbours is worked out again by every cell that reads it: 3.5 of
+// them per cell and pass, some 3 us of the chip's FP64 units at 96 x 64 x 48,
+// against tiles that stage 3.75 positions per cell and leave half their lanes
+// idle in a pass.  MODE 0: in place on `out`; 1: from `in`, every cell written
+// to `out`; 2: no pass, `out` = `in` + prolonged pc - pc0.  Two passes: 69 us
+// at 128^3 (a march along z with planes in LDS: 161), 17.6 at 96 x 64 x 48
+// (tiles: 50.9), 12 from 48 x 32 x 24 down to 16^3 (tiles: 17), so every 3D
+// level takes it that may.
+template <typename T>
+struct HCSweep {
+  Sweep3 S;
+  const int* skip;
+  const T* in;
+  T* out;
+  const T* rhs;
+  const T* a;
+  const T* b[3];
+  const T* pc;
+  const T* pc0;
+  long long ncell, nface[3];
+  T alpha, beta, dxinv, gs[3][2][2], gb[3][2][2];
+  ClosureP<T> cp;
 };
-template <>
-struct HCStream<3> {
-  static constexpr int NT = 256, TY = 12, SEGMIN = 8;
+template <typename T, int MODE>
+__global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T> A, Geom gc) {
+  if (A.skip && *A.skip) return;
+  Sweep3Pos P;
+  if (!sweep3_pos(A.S, P)) return;
+  if constexpr (MODE == 2) {
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      if (!(m ? P.oth : P.act)) continue;
+      const unsigned q = m ? P.qo : P.q;
+      const int i = m ? P.i + 1 - 2 * P.par : P.i;
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        put32(A.out + n * A.ncell, q,
+              prolong_value<T, 3>(gc, i, P.j, P.k, A.pc + n * gc.ncell, A.pc0 ? A.pc0 + n * gc.ncell : nullptr,
+                                  at32(A.in + n * A.ncell, q)));
+    }
+  } else {
+    const T* in = MODE == 1 ? A.in : A.out;
+    if (MODE == 1 && P.oth) {
+      put32(A.out, P.qo, at32(in, P.qo));
+      put32(A.out + A.ncell, P.qo, at32(in + A.ncell, P.qo));
+    }
+    if (!P.act) return;
+    T h[7], c[7];
+    h[0] = at32(in, P.q);
+    c[0] = at32(in + A.ncell, P.q);
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      h[1 + (f ^ 1)] = at32(in, P.nb[f]);
+      c[1 + (f ^ 1)] = at32(in + A.ncell, P.nb[f]);
+    }
+    CellFaces<T, 3> F;
+    T aq[2], rr[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+        sweep3_faces(A.S, P, d, A.b[d] + n * A.nface[d], F.v[n][2 * d], F.v[n][2 * d + 1]);
+      rr[n] = at32(A.rhs + n * A.ncell, P.q);
+      aq[n] = A.a ? at32(A.a + n * A.ncell, P.q) : T(1);
+    }
+    T st[2][7];
+#pragma unroll
+    for (int m = 0; m < 7; ++m) closure<T>(h[m], c[m], A.cp, st[0][m], st[1][m]);
+    if (P.wall) {
+#pragma unroll
+      for (int f = 0; f < 6; ++f)
+        if ((P.wall >> f) & 1)
+#pragma unroll
+          for (int n = 0; n < 2; ++n)
+            st[n][1 + (f ^ 1)] = fma(A.gs[f >> 1][f & 1][n], st[n][0], A.gb[f >> 1][f & 1][n]);
+    }
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const T ph = n ? c[0] : h[0];
+      const T lam = lambda_of<T, 3>(F, n, aq[n], A.alpha, A.beta, A.dxinv);
+      const T lof = lof_of<T, 3>(F, n, st[n], aq[n], ph, A.alpha, A.beta, A.dxinv);
+      put32(A.out + n * A.ncell, P.q, ph - lam * (lof - rr[n]));
+    }
+  }
+}
+
+// npass >= 1 colour passes of a 3D level: the prolongation, or the first
+// pass, from buf[*cur] to the other buffer, the others in place there
+template <typename T>
+hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
+                           const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm) {
+  const Geom& g = A.g;
+  HCSweep<T> V{};
+  V.S = sweep3_make(g);
+  V.skip = A.skip;
+  V.in = buf[*cur];
+  V.out = buf[1 - *cur];
+  V.rhs = rhs;
+  V.a = A.a;
+  V.pc = pc;
+  V.pc0 = pc0;
+  V.ncell = g.ncell;
+  V.alpha = A.alpha;
+  V.beta = A.beta;
+  V.dxinv = T(1) / (T(g.dx) * T(g.dx));
+  V.cp = A.cp;
+  const GhostForm<T> gf = ghost_form<T>(A.bc, T(g.dx));
+  double faces = 0;
+  for (int d = 0; d < 3; ++d) {
+    V.b[d] = A.b[d];
+    V.nface[d] = g.nface[d];
+    faces += double(g.nface[d]);
+    for (int sd = 0; sd < 2; ++sd)
+      for (int n = 0; n < 2; ++n) {
+        V.gs[d][sd][n] = gf.s[d][sd][n];
+        V.gb[d][sd][n] = gf.b[d][sd][n];
+      }
+  }
+  const Geom gcc = gc ? *gc : g;
+  for (int p = pc ? -1 : 0; p < npass; ++p) {
+    V.S.colour = (first + p) & 1;
+    const bool timed = p >= 0 && tm && *tm->n < tm->cap;
+    if (p >= 0 && tm && !timed) ++*tm->missed;
+    auto kern = p < 0 ? hc_sweep3_kernel<T, 2> : (p == 0 && !pc ? hc_sweep3_kernel<T, 1> : hc_sweep3_kernel<T, 0>);
+    hipExtLaunchKernelGGL(kern, dim3(8 * V.S.chunk), dim3(256), 0, s, timed ? tm->start[*tm->n] : nullptr,
+                          timed ? tm->stop[*tm->n] : nullptr, 0, V, gcc);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (timed) {
+      // both components: every state read, rhs and a of the colour, every
+      // face; the colour written (a first pass: every cell)
+      const double cells = double(g.nvalid());
+      *tm->bytes += (2 * cells + cells * (1 + (A.a ? 1 : 0)) + 2 * faces + (p == 0 && !pc ? 2 : 1) * cells) * sizeof(T);
+      ++*tm->n;
+    }
+  }
+  *cur = 1 - *cur;
+  return hipSuccess;
+}
+
+// streaming launch shape: columns of 252 cells (256 threads)
+struct HCStream {
+  static constexpr int NT = 256, SEGMIN = 8;
 };
 
-// levels whose plain relaxations stream (2D above 512^2 cells, 3D above
-// 96^3), with 32-bit offsets for both components of every array
+// 2D levels whose plain relaxations stream (above 512^2 cells), with 32-bit
+// offsets for both components of every array
 constexpr long long kHCStreamCells2 = 512 * 512;
-constexpr long long kHCStreamCells3 = 96LL * 96 * 96;
 inline bool hc_streams(const Geom& g) {
   long long nf = 0;
   for (int d = 0; d < g.dim; ++d) nf = nf > g.nface[d] ? nf : g.nface[d];
   const long long most = 2 * (g.ncell > nf ? g.ncell : nf);
-  return g.nvalid() > (g.dim == 2 ? kHCStreamCells2 : kHCStreamCells3) && g.n[g.dim - 1] >= 8 && most < (1LL << 29);
+  return g.dim == 2 && g.nvalid() > kHCStreamCells2 && g.n[1] >= 8 && most < (1LL << 29);
 }
 
-template <typename T, int DIM, int P, bool HASA>
+template <typename T, int P, bool HASA>
 hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rhs, int first, hipStream_t s,
                             const LaunchTimer* tm) {
-  using D = HCStream<DIM>;
-  constexpr int TX = DIM == 2 ? D::NT - 2 * P : D::TY;
-  constexpr int TY = DIM == 2 ? 1 : D::TY;
-  constexpr int EL = (TX + 2 * P) * (DIM == 3 ? TY + 2 * P : 1);
+  using D = HCStream;
+  constexpr int TX = D::NT - 2 * P, EL = D::NT;
   const Geom& g = A.g;
   const int nbx = (g.n[0] + TX - 1) / TX;
-  const int nby = DIM == 3 ? (g.n[1] + TY - 1) / TY : 1;
   const size_t lds = size_t(4) * 4 * EL * sizeof(T);
-  auto kern = hc_relax_stream_kernel<T, DIM, TX, TY, P, D::NT, HASA>;
+  auto kern = hc_relax_stream_kernel<T, TX, P, D::NT, HASA>;
   // segments sized so that the whole grid is resident at once
   static int resident = 0;
   if (!resident) {
@@ -1688,21 +1800,20 @@ hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rh
     else
       resident = 768;
   }
-  const int nz = g.n[DIM - 1];
-  const int columns = nbx * nby;
-  const int per_column = resident / columns > 1 ? resident / columns : 1;
+  const int nz = g.n[1];
+  const int per_column = resident / nbx > 1 ? resident / nbx : 1;
   int seg = (nz + per_column - 1) / per_column;
   if (seg < D::SEGMIN) seg = D::SEGMIN;
   const int nbz = (nz + seg - 1) / seg;
   const bool timed = tm && *tm->n < tm->cap;
   if (tm && !timed) ++*tm->missed;
-  hipExtLaunchKernelGGL(kern, dim3(nbx * nby * nbz), dim3(D::NT), lds, s, timed ? tm->start[*tm->n] : nullptr,
-                        timed ? tm->stop[*tm->n] : nullptr, 0, A, in, out, rhs, first, nbx, nby, seg);
+  hipExtLaunchKernelGGL(kern, dim3(nbx * nbz), dim3(D::NT), lds, s, timed ? tm->start[*tm->n] : nullptr,
+                        timed ? tm->stop[*tm->n] : nullptr, 0, A, in, out, rhs, first, nbx, seg);
   const hipError_t e = hipGetLastError();
   if (e == hipSuccess && timed) {
     const double cells = double(g.nvalid());
     double faces = 0;
-    for (int d = 0; d < DIM; ++d) faces += double(g.nface[d]);
+    for (int d = 0; d < 2; ++d) faces += double(g.nface[d]);
     const double by = 2 * cells + 2 * cells + (HASA ? 2 * cells : 0) + 2 * faces + 2 * cells;
     *tm->bytes += by * sizeof(T);
     ++*tm->n;
@@ -1710,7 +1821,7 @@ hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rh
   return e;
 }
 
-template <typename T, int DIM>
+template <typename T>
 hipError_t hc_relax_stream(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                            hipStream_t s, const LaunchTimer* tm) {
   int done = 0;
@@ -1719,11 +1830,11 @@ hipError_t hc_relax_stream(const HCArgs<T>& A, T* const buf[2], int* cur, const 
     const int f = (first + done) & 1;
     hipError_t e;
     if (A.a)
-      e = p == 2 ? hc_stream_launch<T, DIM, 2, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
-                 : hc_stream_launch<T, DIM, 1, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
+      e = p == 2 ? hc_stream_launch<T, 2, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
+                 : hc_stream_launch<T, 1, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
     else
-      e = p == 2 ? hc_stream_launch<T, DIM, 2, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
-                 : hc_stream_launch<T, DIM, 1, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
+      e = p == 2 ? hc_stream_launch<T, 2, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
+                 : hc_stream_launch<T, 1, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += p;
@@ -1734,10 +1845,10 @@ hipError_t hc_relax_stream(const HCArgs<T>& A, T* const buf[2], int* cur, const 
 template <typename T>
 hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                           const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm) {
+  if (npass > 0 && sweep3_ok(A.g))
+    return hc_relax_sweeps<T>(A, buf, cur, rhs, npass, first, gc, pc, pc0, s, tm);
   // plain relaxations of large levels stream along the last direction
-  if (!pc && npass > 0 && hc_streams(A.g))
-    return A.g.dim == 2 ? hc_relax_stream<T, 2>(A, buf, cur, rhs, npass, first, s, tm)
-                        : hc_relax_stream<T, 3>(A, buf, cur, rhs, npass, first, s, tm);
+  if (!pc && npass > 0 && hc_streams(A.g)) return hc_relax_stream<T>(A, buf, cur, rhs, npass, first, s, tm);
   const int pmax = relax_passes_per_launch(A.g);
   int done = 0;
   while (done < npass) {

@@ -312,63 +312,137 @@ struct IC {
   static constexpr int value = N;
 };
 
-// lateral position of the extended block: global coordinates (wrapped in
-// periodic directions), kind 1 cell / 2 wall ghost / 0 unused, Chebyshev
-// distance to the core, owner flag, and for a ghost its wall (direction,
-// side) and the LDS offset of its interior neighbour
+// lateral position of the extended column block: global coordinate (wrapped
+// when periodic), kind 1 cell / 2 wall ghost / 0 unused, distance to the core,
+// owner flag, and for a ghost its side (gx: its interior neighbour)
 struct SPos {
-  int gx, gy;
+  int gx;
   int kind, dist, owner;
-  int gd, gs, eint;
+  int gs;
   int gtype;   // a ghost's boundary type (resolved once: a per-thread index
                // into the kernel arguments would be a memory load)
 };
 
-template <int DIM, int TX, int TY, int P>
-__device__ inline void spos_init(const Geom& g, int x0, int y0, int e, SPos& s) {
-  constexpr int EX = TX + 2 * P;
-  const int ex = e % EX, ey = e / EX;
-  const int lc[2] = {ex - P, DIM == 3 ? ey - P : 0};
-  const int org[2] = {x0, y0};
-  const int nl = DIM == 3 ? 2 : 1;
+template <int TX, int P>
+__device__ inline void spos_init(const Geom& g, int x0, int e, SPos& s) {
+  const int l = e - P, n = g.n[0];
+  int v = x0 + l;
+  s.dist = l < 0 ? -l : (l >= TX ? l - TX + 1 : 0);
+  s.owner = s.dist == 0 && v >= 0 && v < n;
   s.kind = 1;
-  s.dist = 0;
-  s.owner = 1;
-  s.gd = -1;
   s.gs = 0;
-  s.eint = e;
-  int gv[2] = {0, 0};
-  int outside = 0;
-  for (int d = 0; d < nl; ++d) {
-    const int ext = d == 0 ? TX : TY;
-    const int l = lc[d];
-    const int dd = l < 0 ? -l : (l >= ext ? l - ext + 1 : 0);
-    if (dd > s.dist) s.dist = dd;
-    int v = org[d] + l;
-    const int n = g.n[d];
-    if (v >= n || v < 0) s.owner = 0;
-    if (v >= 0 && v < n) {
-      gv[d] = v;
-    } else if (g.periodic[d]) {
-      gv[d] = v < 0 ? v + n : v - n;
-    } else if (v == -1 || v == n) {
-      ++outside;
-      s.gd = d;
-      s.gs = v == n ? 1 : 0;
-      gv[d] = v == n ? n - 1 : 0;   // the interior neighbour
-      s.eint = e + (v == n ? -1 : 1) * (d == 0 ? 1 : EX);
+  if (v < 0 || v >= n) {
+    if (g.periodic[0]) {
+      v = v < 0 ? v + n : v - n;
     } else {
-      outside += 2;
+      s.kind = v == -1 || v == n ? 2 : 0;
+      s.gs = v >= n;
     }
   }
-  if (s.dist > 0) s.owner = 0;
-  if (outside == 1) s.kind = 2;
-  else if (outside > 1) s.kind = 0;
-  // every position gets in-domain coordinates (unused ones clamped), so the
+  // every position gets an in-domain coordinate (unused ones clamped), so the
   // prefetch can load unconditionally
-  for (int d = 0; d < nl; ++d) gv[d] = gv[d] < 0 ? 0 : (gv[d] >= g.n[d] ? g.n[d] - 1 : gv[d]);
-  s.gx = gv[0];
-  s.gy = gv[1];
+  s.gx = v < 0 ? 0 : (v >= n ? n - 1 : v);
+}
+
+// ---- 3D colour passes straight from memory --------------------------------
+// One launch updates the cells of one colour: they read the other colour and
+// themselves only, so a pass can work in place, without tiles and halos.  (A
+// 16 x 8 x 4 tile with the halo of two passes stages 3.75 positions per cell
+// it keeps.)  A thread handles a pair of cells (2s, 2s+1) of a row, one of
+// which has the colour: every lane works, and rows are read and written
+// whole.  Blocks of 2^lpx pairs by 256 >> lpx rows; the blocks of one L2
+// (workgroups go round the 8 of them) are neighbours in the level.
+// Byte offsets within one component are 32-bit (sweep3_ok).
+struct Sweep3 {
+  int n[3], per[3];
+  unsigned sy, sz, fx[3], fxy[3];   // cell and face strides (row, plane)
+  int lpx, nbx, nby, nblocks, chunk, colour;
+};
+
+inline bool sweep3_ok(const Geom& g) {
+  long long most = g.ncell;
+  for (int d = 0; d < 3; ++d) {
+    if (g.periodic[d] && (g.n[d] & 1)) return false;   // (the ends of a row would share a colour)
+    most = most > g.nface[d] ? most : g.nface[d];
+  }
+  return g.dim == 3 && most < (1LL << 29);
+}
+
+inline Sweep3 sweep3_make(const Geom& g) {
+  Sweep3 S{};
+  for (int d = 0; d < 3; ++d) {
+    S.n[d] = g.n[d];
+    S.per[d] = g.periodic[d];
+    S.fx[d] = unsigned(g.fn[d][0]);
+    S.fxy[d] = unsigned(g.fn[d][0] * g.fn[d][1]);
+  }
+  S.sy = unsigned(g.sy);
+  S.sz = unsigned(g.sz);
+  const int pairs = (g.n[0] + 1) / 2;
+  // the widest row of a block, up to 64 pairs, that leaves the fewest lanes idle
+  auto blocks = [&](int l) { return ((pairs + (1 << l) - 1) >> l) * ((g.n[1] + (256 >> l) - 1) / (256 >> l)); };
+  S.lpx = 6;
+  for (int l = 5; l >= 3; --l)
+    if (blocks(l) < blocks(S.lpx)) S.lpx = l;
+  S.nbx = (pairs + (1 << S.lpx) - 1) >> S.lpx;
+  S.nby = (g.n[1] + (256 >> S.lpx) - 1) / (256 >> S.lpx);
+  S.nblocks = S.nbx * S.nby * g.n[2];
+  S.chunk = (S.nblocks + 7) / 8;
+  return S;
+}
+
+struct Sweep3Pos {
+  int i, j, k, par;
+  bool act, oth;       // the pair's cell of the colour, its other cell: in the level
+  unsigned q, qo;      // ... their indices
+  unsigned nb[6];      // neighbours of the cell of the colour (-x, +x, ...), itself beyond a wall
+  unsigned wall;       // bit f: neighbour f is a wall's ghost
+};
+
+__device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos& P) {
+  const int l = int(blockIdx.x & 7u) * S.chunk + int(blockIdx.x >> 3);
+  if (l >= S.nblocks || int(blockIdx.x >> 3) >= S.chunk) return false;
+  const int bx = l % S.nbx, r = l / S.nbx, by = r % S.nby;
+  P.k = r / S.nby;
+  const int s = (bx << S.lpx) + (int(threadIdx.x) & ((1 << S.lpx) - 1));
+  P.j = by * (256 >> S.lpx) + (int(threadIdx.x) >> S.lpx);
+  if (2 * s >= S.n[0] || P.j >= S.n[1]) return false;
+  P.par = (P.j + P.k + S.colour) & 1;
+  P.i = 2 * s + P.par;
+  P.act = P.i < S.n[0];
+  P.oth = 2 * s + 1 - P.par < S.n[0];
+  const unsigned row = S.sy * unsigned(P.j + 1) + S.sz * unsigned(P.k + 1);
+  P.q = row + unsigned(P.i + 1);
+  P.qo = row + unsigned(2 * s + 2 - P.par);
+  P.wall = 0;
+  const int iv[3] = {P.i, P.j, P.k};
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const unsigned st = d == 0 ? 1u : (d == 1 ? S.sy : S.sz);
+    const unsigned span = st * unsigned(S.n[d] - 1);
+    const bool lo = iv[d] == 0, hi = iv[d] == S.n[d] - 1;
+    P.nb[2 * d] = lo ? (S.per[d] ? P.q + span : P.q) : P.q - st;
+    P.nb[2 * d + 1] = hi ? (S.per[d] ? P.q - span : P.q) : P.q + st;
+    if (!S.per[d]) P.wall |= (lo ? 1u << (2 * d) : 0u) | (hi ? 2u << (2 * d) : 0u);
+  }
+  return true;
+}
+
+// element i (32-bit byte offset) of p
+template <typename T>
+__device__ __forceinline__ T at32(const T* p, unsigned i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + i * unsigned(sizeof(T)));
+}
+template <typename T>
+__device__ __forceinline__ void put32(T* p, unsigned i, T v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + i * unsigned(sizeof(T))) = v;
+}
+// the six faces of the cell, component array b
+template <typename T>
+__device__ __forceinline__ void sweep3_faces(const Sweep3& S, const Sweep3Pos& P, int d, const T* b, T& lo, T& hi) {
+  const unsigned f = unsigned(P.i) + S.fx[d] * unsigned(P.j) + S.fxy[d] * unsigned(P.k);
+  lo = at32(b, f);
+  hi = at32(b, f + (d == 0 ? 1u : (d == 1 ? S.fx[1] : S.fxy[2])));
 }
 
 }  // namespace ml

@@ -1101,10 +1101,9 @@ hipError_t vc_relax_cfg(const VCArgs<T>& A, T* const buf[2], int* cur, const T* 
   return hipSuccess;
 }
 
-// ---- streaming relaxation for large levels -------------------------------
-// A workgroup owns a block of columns (2D: TX cells in x; 3D: TX x TY cells
-// in (x, y)) and a segment of planes along the last direction, and marches
-// through them with a window of P+2 planes in LDS.  With plane R just
+// ---- streaming relaxation for large 2D levels ----------------------------
+// A workgroup owns TX columns and a segment of rows ("planes" below), and
+// marches through them with a window of P+2 planes in LDS.  With plane R just
 // loaded, colour pass p runs on plane R-1-p (p = 0..P-1), so plane R-P is
 // final and is written: the passes form a pipeline along the march instead
 // of a halo in that direction.  Pass p covers the lateral positions within
@@ -1115,24 +1114,24 @@ hipError_t vc_relax_cfg(const VCArgs<T>& A, T* const buf[2], int* cur, const T* 
 // ahead of their first use, so their loads overlap the previous plane's
 // passes.  Stencil, lambda and update are the tiled kernel's, so results
 // are identical bit for bit.
-template <typename T, int DIM>
+template <typename T>
 struct SCoef {
-  Faces1<T, DIM> F;
+  Faces1<T, 2> F;
   T aq, cq, rr, lam;
 };
 
-template <typename T, int DIM, int TX, int TY, int P, int NT>
+template <typename T, int TX, int P, int NT>
 __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const T* __restrict__ in,
                                                              T* __restrict__ out, const T* __restrict__ rhs,
                                                              int first, int zero_init, Geom gc,
-                                                             const T* __restrict__ pc, int nbx, int nby, int seg) {
+                                                             const T* __restrict__ pc, int nbx, int seg) {
   if (A.skip && *A.skip) return;
   constexpr int EX = TX + 2 * P;
-  constexpr int EL = EX * (DIM == 3 ? TY + 2 * P : 1);
+  constexpr int EL = EX;
   constexpr int K = (EL + NT - 1) / NT;
   static_assert(P >= 1 && P <= 2, "one or two colour passes per launch");
   constexpr int W = 4;   // planes in the window (P+2 <= 4; a power of two)
-  constexpr int MD = DIM - 1;
+  constexpr int MD = 1;
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T* su = reinterpret_cast<T*>(smem_raw);
   const Geom& g = A.g;
@@ -1140,12 +1139,8 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   const bool zper = g.periodic[MD] != 0;
   const T dxinv = T(1) / (T(g.dx) * T(g.dx));
   const bool hasc = A.c != nullptr;
-  int b = blockIdx.x;
-  const int bx = b % nbx;
-  b /= nbx;
-  const int by = DIM == 3 ? b % nby : 0;
-  const int bz = DIM == 3 ? b / nby : b;
-  const int x0 = bx * TX, y0 = by * TY;
+  const int bx = int(blockIdx.x) % nbx, bz = int(blockIdx.x) / nbx;
+  const int x0 = bx * TX;
   const int z0 = bz * seg;
   const int z1 = z0 + seg < nz ? z0 + seg : nz;
   SPos S[K];
@@ -1153,11 +1148,10 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   for (int kk = 0; kk < K; ++kk) {
     const int e = threadIdx.x + kk * NT;
     if (e < EL) {
-      spos_init<DIM, TX, TY, P>(g, x0, y0, e, S[kk]);
+      spos_init<TX, P>(g, x0, e, S[kk]);
       S[kk].gtype = 0;
-      for (int d = 0; d < DIM - 1; ++d)
-        for (int sd = 0; sd < 2; ++sd)
-          if (S[kk].kind == 2 && S[kk].gd == d && S[kk].gs == sd) S[kk].gtype = A.bc.type[d][sd][0];
+      for (int sd = 0; sd < 2; ++sd)
+        if (S[kk].kind == 2 && S[kk].gs == sd) S[kk].gtype = A.bc.type[0][sd][0];
     } else {
       S[kk].kind = 0;
       S[kk].dist = P;
@@ -1168,23 +1162,22 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   auto real_plane = [&](int z) { return zper || (z >= 0 && z < nz); };
   // 32-bit element offsets: a position's lateral part, computed once, plus a
   // plane part common to the workgroup (levels below 2^29 cells per array)
-  const unsigned csz = unsigned(DIM == 3 ? g.sz : g.sy);   // cell stride between planes
-  unsigned fpl[DIM], fup[DIM];                              // face plane stride, offset to the upper face
+  const unsigned csz = unsigned(g.sy);   // cell stride between planes
+  unsigned fpl[2], fup[2];                              // face plane stride, offset to the upper face
 #pragma unroll
-  for (int d = 0; d < DIM; ++d) fpl[d] = unsigned(g.fn[d][0] * (DIM == 3 ? g.fn[d][1] : 1));
+  for (int d = 0; d < 2; ++d) fpl[d] = unsigned(g.fn[d][0]);
   fup[0] = 1;
-  if (DIM == 3) fup[1] = unsigned(g.fn[1][0]);
   fup[MD] = fpl[MD];
-  const unsigned cgsz = unsigned(DIM == 3 ? gc.sz : gc.sy);
-  unsigned cl[K], fl[K][DIM], ccl[K];
+  const unsigned cgsz = unsigned(gc.sy);
+  unsigned cl[K], fl[K][2], ccl[K];
 #pragma unroll
   for (int kk = 0; kk < K; ++kk) {
     const SPos& s = S[kk];
-    cl[kk] = unsigned(s.gx + 1) + (DIM == 3 ? unsigned(g.sy) * unsigned(s.gy + 1) : 0u);
+    cl[kk] = unsigned(s.gx + 1);
 #pragma unroll
-    for (int d = 0; d < DIM; ++d)
-      fl[kk][d] = unsigned(s.gx) + (DIM == 3 ? unsigned(g.fn[d][0]) * unsigned(s.gy) : 0u);
-    ccl[kk] = unsigned(s.gx / 2 + 1) + (DIM == 3 ? unsigned(gc.sy) * unsigned(s.gy / 2 + 1) : 0u);
+    for (int d = 0; d < 2; ++d)
+      fl[kk][d] = unsigned(s.gx);
+    ccl[kk] = unsigned(s.gx / 2 + 1);
   }
   auto ld = [](const T* p, unsigned i) -> T {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (i * unsigned(sizeof(T))));
@@ -1194,7 +1187,7 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   // into their set and are used only at that plane's commit two steps later,
   // so no instruction touches a load in flight.
   constexpr int NS = P + 3;
-  SCoef<T, DIM> cs[NS][K];
+  SCoef<T> cs[NS][K];
   T sv[NS][K], scv[NS][K];   // state and coarse correction as loaded
   // the same loads for every position and plane (in-domain addresses; an
   // absent array is replaced by a duplicate read of rhs), so that the waits
@@ -1203,7 +1196,7 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   const T* ain = A.a ? A.a : rhs;
   const T* cin = hasc ? A.c : rhs;
   const T* cvp = pc ? pc : rhs;
-  auto prefetch = [&](int R, SCoef<T, DIM>(&pf)[K], T(&v)[K], T(&cv)[K]) {
+  auto prefetch = [&](int R, SCoef<T>(&pf)[K], T(&v)[K], T(&cv)[K]) {
     const int zw = zper ? zwrap(R) : (R < 0 ? 0 : (R >= nz ? nz - 1 : R));
     const unsigned qz = unsigned(zw + 1) * csz, cz = unsigned(zw / 2 + 1) * cgsz;
 #pragma unroll
@@ -1212,7 +1205,7 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
       v[kk] = ld(vin, q);
       cv[kk] = ld(cvp, pc ? ccl[kk] + cz : q);
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) {
+      for (int d = 0; d < 2; ++d) {
         const unsigned f = fl[kk][d] + unsigned(zw) * fpl[d];
         pf[kk].F.v[2 * d] = ld(A.b[d], f);
         pf[kk].F.v[2 * d + 1] = ld(A.b[d], f + fup[d]);
@@ -1244,7 +1237,7 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
           if (!A.a) cs[j][kk].aq = T(1);
           if (!hasc) cs[j][kk].cq = T(0);
           if (s.dist <= P - 1)
-            cs[j][kk].lam = vc_lambda<T, DIM>(cs[j][kk].F, cs[j][kk].aq, hasc, cs[j][kk].cq, A.alpha, A.beta, dxinv);
+            cs[j][kk].lam = vc_lambda<T, 2>(cs[j][kk].F, cs[j][kk].aq, hasc, cs[j][kk].cq, A.alpha, A.beta, dxinv);
         } else {
           pl[e] = bc_ghost<T>(s.gtype, T(0), val, s.gs == 0 ? -1 : 1, T(g.dx));
         }
@@ -1277,33 +1270,22 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
           const SPos& s = S[kk];
-          if (s.kind != 1 || s.dist > reach || ((s.gx + s.gy + zw + colour) & 1)) continue;
+          if (s.kind != 1 || s.dist > reach || ((s.gx + zw + colour) & 1)) continue;
           const int e = threadIdx.x + kk * NT;
           T st[7];
           st[0] = pz[e];
           st[1] = pz[e + 1];
           st[2] = pz[e - 1];
-          if (DIM == 3) {
-            st[3] = pz[e + EX];
-            st[4] = pz[e - EX];
-            st[5] = pp[e];
-            st[6] = pm[e];
-          } else {
-            st[3] = pp[e];
-            st[4] = pm[e];
-          }
-          const SCoef<T, DIM>& C = cs[jp][kk];
-          const T lof = vc_lof<T, DIM>(C.F, st, C.aq, hasc, C.cq, A.alpha, A.beta, dxinv);
+          st[3] = pp[e];
+          st[4] = pm[e];
+          const SCoef<T>& C = cs[jp][kk];
+          const T lof = vc_lof<T, 2>(C.F, st, C.aq, hasc, C.cq, A.alpha, A.beta, dxinv);
           const T nv = st[0] - C.lam * (lof - C.rr);
           pz[e] = nv;
           // wall ghosts of this cell: lateral, then along the march
-          const int gl[2] = {s.gx, s.gy};
-#pragma unroll
-          for (int d = 0; d < (DIM == 3 ? 2 : 1); ++d) {
-            if (g.periodic[d]) continue;
-            const int st1 = d == 0 ? 1 : EX;
-            if (gl[d] == 0) pz[e - st1] = bc_ghost<T>(A.bc.type[d][0][0], T(0), nv, -1, T(g.dx));
-            if (gl[d] == g.n[d] - 1) pz[e + st1] = bc_ghost<T>(A.bc.type[d][1][0], T(0), nv, 1, T(g.dx));
+          if (!g.periodic[0]) {
+            if (s.gx == 0) pz[e - 1] = bc_ghost<T>(A.bc.type[0][0][0], T(0), nv, -1, T(g.dx));
+            if (s.gx == g.n[0] - 1) pz[e + 1] = bc_ghost<T>(A.bc.type[0][1][0], T(0), nv, 1, T(g.dx));
           }
           if (!zper) {
             if (zw == 0) slot(-1)[e] = bc_ghost<T>(A.bc.type[MD][0][0], T(0), nv, -1, T(g.dx));
@@ -1343,41 +1325,30 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   }
 }
 
-template <int DIM>
-struct VCStream;
-template <>
-struct VCStream<2> {
-  static constexpr int NT = 256, TY = 1, SEGMIN = 8;
-};
-template <>
-struct VCStream<3> {
-  static constexpr int NT = 256, TY = 12, SEGMIN = 8;
+struct VCStream {
+  static constexpr int NT = 256, SEGMIN = 8;
 };
 
-// levels on which plain relaxation launches stream (2D above 512^2, 3D
-// above 96^3); the tiled kernel keeps the fused restriction / residual
+// 2D levels on which plain relaxation launches stream (above 512^2); the
+// tiled kernel keeps the fused restriction / residual
 constexpr long long kStreamCells2 = 512 * 512;
-constexpr long long kStreamCells3 = 96LL * 96 * 96;
 inline bool vc_streams(const Geom& g) {
   long long nf = 0;
   for (int d = 0; d < g.dim; ++d) nf = nf > g.nface[d] ? nf : g.nface[d];
   const long long most = g.ncell > nf ? g.ncell : nf;
-  return g.nvalid() > (g.dim == 2 ? kStreamCells2 : kStreamCells3) && g.n[g.dim - 1] >= 8 &&
+  return g.dim == 2 && g.nvalid() > kStreamCells2 && g.n[1] >= 8 &&
          most < (1LL << 29);   // byte offsets of every array within 32 bits
 }
 
-template <typename T, int DIM, int P>
+template <typename T, int P>
 hipError_t vc_stream_launch(const VCArgs<T>& A, const T* in, T* out, const T* rhs, int first, bool zero_init,
                             const Geom& gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
-  using D = VCStream<DIM>;
-  constexpr int TX = DIM == 2 ? D::NT - 2 * P : D::TY;
-  constexpr int TY = DIM == 2 ? 1 : D::TY;
-  constexpr int EL = (TX + 2 * P) * (DIM == 3 ? TY + 2 * P : 1);
+  using D = VCStream;
+  constexpr int TX = D::NT - 2 * P, EL = D::NT;
   const Geom& g = A.g;
   const int nbx = (g.n[0] + TX - 1) / TX;
-  const int nby = DIM == 3 ? (g.n[1] + TY - 1) / TY : 1;
   const size_t lds = size_t(4) * EL * sizeof(T);
-  auto kern = vc_relax_stream_kernel<T, DIM, TX, TY, P, D::NT>;
+  auto kern = vc_relax_stream_kernel<T, TX, P, D::NT>;
   // segments sized so that the whole grid is resident at once (one round of
   // workgroups; measured best at 2048^2: a grid that fills every CU's
   // workgroup slots beats both fewer, longer segments and a second round)
@@ -1393,24 +1364,23 @@ hipError_t vc_stream_launch(const VCArgs<T>& A, const T* in, T* out, const T* rh
     else
       resident = 768;
   }
-  const int nz = g.n[DIM - 1];
-  const int columns = nbx * nby;
-  const int per_column = resident / columns > 1 ? resident / columns : 1;
+  const int nz = g.n[1];
+  const int per_column = resident / nbx > 1 ? resident / nbx : 1;
   int seg = (nz + per_column - 1) / per_column;
   if (seg < D::SEGMIN) seg = D::SEGMIN;
   const int nbz = (nz + seg - 1) / seg;
   const bool timed = tm && *tm->n < tm->cap;
   if (tm && !timed) ++*tm->missed;
-  hipExtLaunchKernelGGL(kern, dim3(nbx * nby * nbz), dim3(D::NT), lds, s, timed ? tm->start[*tm->n] : nullptr,
+  hipExtLaunchKernelGGL(kern, dim3(nbx * nbz), dim3(D::NT), lds, s, timed ? tm->start[*tm->n] : nullptr,
                         timed ? tm->stop[*tm->n] : nullptr, 0, A, in, out, rhs, first, zero_init ? 1 : 0, gc, pc, nbx,
-                        nby, seg);
+                        seg);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   if (timed) {
     const double cells = double(g.nvalid());
     double faces = 0;
-    for (int d = 0; d < DIM; ++d) faces += double(g.nface[d]);
-    double by = cells * (zero_init ? 0 : 1) + (pc ? cells / double(DIM == 3 ? 8 : 4) : 0) + cells +
+    for (int d = 0; d < 2; ++d) faces += double(g.nface[d]);
+    double by = cells * (zero_init ? 0 : 1) + (pc ? cells / 4 : 0) + cells +
                 (A.a ? cells : 0) + (A.c ? cells : 0) + faces + cells;
     *tm->bytes += by * sizeof(T);
     ++*tm->n;
@@ -1419,7 +1389,7 @@ hipError_t vc_stream_launch(const VCArgs<T>& A, const T* in, T* out, const T* rh
 }
 
 // npass colour passes by streaming launches of up to 2 passes each
-template <typename T, int DIM>
+template <typename T>
 hipError_t vc_relax_stream(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                            const Geom* gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
   const Geom gcc = gc ? *gc : A.g;
@@ -1428,13 +1398,139 @@ hipError_t vc_relax_stream(const VCArgs<T>& A, T* const buf[2], int* cur, const 
     const int p = (npass - done) >= 2 ? 2 : (npass - done);
     const bool zi = done == 0 && zero_init;
     const T* pcl = done == 0 ? pc : nullptr;
-    hipError_t e = p == 2 ? vc_stream_launch<T, DIM, 2>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s, tm)
-                          : vc_stream_launch<T, DIM, 1>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s,
+    hipError_t e = p == 2 ? vc_stream_launch<T, 2>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s, tm)
+                          : vc_stream_launch<T, 1>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s,
                                                         tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += p;
   }
+  return hipSuccess;
+}
+
+// the homogeneous wall ghosts of a correction
+template <typename T>
+GhostForm<T> vc_ghost_form(BCDesc bc, T dx) {
+  bc.apply = 1;
+  for (auto& d : bc.val)
+    for (auto& s : d)
+      for (auto& v : s) v = 0.0;
+  return ghost_form<T>(bc, dx);
+}
+
+// One colour pass of a 3D level straight from memory (Sweep3).  FIRST: from
+// `in`, or zero, plus the coarse correction pc, every cell written to `out`;
+// otherwise in place on `out`.  Two passes with c: 37 us at 128^3 (98 bytes a
+// cell of required traffic: 5.6 TB/s; a march along z with a window of planes
+// in LDS was 71), 8.5 at 64^3 and 7.5 at 16^3 (16 x 8 x 4 tiles with the halo
+// of both passes: 15.1 and 8.0), so every 3D level takes it that may.
+template <typename T>
+struct VCSweep {
+  Sweep3 S;
+  const int* skip;
+  const T* in;
+  T* out;
+  const T* rhs;
+  const T* a;
+  const T* c;
+  const T* b[3];
+  const T* pc;
+  unsigned csy, csz;   // coarse cell strides
+  T alpha, beta, dxinv, gs[3][2], gb[3][2];
+  int zero;
+};
+template <typename T, bool FIRST>
+__global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
+  if (A.skip && *A.skip) return;
+  Sweep3Pos P;
+  if (!sweep3_pos(A.S, P)) return;
+  auto val = [&](unsigned q, int i, int j, int k) __attribute__((always_inline)) {
+    if (!FIRST) return at32(A.out, q);
+    T v = A.zero ? T(0) : at32(A.in, q);
+    if (A.pc) v = v + at32(A.pc, unsigned((i >> 1) + 1) + A.csy * unsigned((j >> 1) + 1) + A.csz * unsigned((k >> 1) + 1));
+    return v;
+  };
+  if (FIRST && P.oth) put32(A.out, P.qo, val(P.qo, P.i, P.j, P.k));   // (both cells of a pair have one coarse cell)
+  if (!P.act) return;
+  T st[7];
+  st[0] = val(P.q, P.i, P.j, P.k);
+#pragma unroll
+  for (int f = 0; f < 6; ++f) {
+    int iv[3] = {P.i, P.j, P.k};
+    if (FIRST) {
+      const int d = f >> 1, n = A.S.n[d];
+      iv[d] = f & 1 ? (iv[d] == n - 1 ? (A.S.per[d] ? 0 : iv[d]) : iv[d] + 1)
+                    : (iv[d] == 0 ? (A.S.per[d] ? n - 1 : 0) : iv[d] - 1);
+    }
+    st[1 + (f ^ 1)] = val(P.nb[f], iv[0], iv[1], iv[2]);
+  }
+  Faces1<T, 3> F;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) sweep3_faces(A.S, P, d, A.b[d], F.v[2 * d], F.v[2 * d + 1]);
+  const bool hasc = A.c != nullptr;
+  const T aq = A.a ? at32(A.a, P.q) : T(1), cq = hasc ? at32(A.c, P.q) : T(0), rr = at32(A.rhs, P.q);
+  if (P.wall) {
+#pragma unroll
+    for (int f = 0; f < 6; ++f)
+      if ((P.wall >> f) & 1) st[1 + (f ^ 1)] = fma(A.gs[f >> 1][f & 1], st[0], A.gb[f >> 1][f & 1]);
+  }
+  const T lam = vc_lambda<T, 3>(F, aq, hasc, cq, A.alpha, A.beta, A.dxinv);
+  const T lof = vc_lof<T, 3>(F, st, aq, hasc, cq, A.alpha, A.beta, A.dxinv);
+  put32(A.out, P.q, st[0] - lam * (lof - rr));
+}
+
+// npass >= 1 colour passes: the first from buf[*cur] to the other buffer,
+// the others in place there
+template <typename T>
+hipError_t vc_relax_sweeps(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
+                           const Geom* gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
+  const Geom& g = A.g;
+  VCSweep<T> V{};
+  V.S = sweep3_make(g);
+  V.skip = A.skip;
+  V.in = buf[*cur];
+  V.out = buf[1 - *cur];
+  V.rhs = rhs;
+  V.a = A.a;
+  V.c = A.c;
+  for (int d = 0; d < 3; ++d) V.b[d] = A.b[d];
+  V.pc = pc;
+  if (gc) {
+    V.csy = unsigned(gc->sy);
+    V.csz = unsigned(gc->sz);
+  }
+  V.alpha = A.alpha;
+  V.beta = A.beta;
+  V.dxinv = T(1) / (T(g.dx) * T(g.dx));
+  V.zero = zero_init ? 1 : 0;
+  const GhostForm<T> gf = vc_ghost_form<T>(A.bc, T(g.dx));
+  for (int d = 0; d < 3; ++d)
+    for (int sd = 0; sd < 2; ++sd) {
+      V.gs[d][sd] = gf.s[d][sd][0];
+      V.gb[d][sd] = gf.b[d][sd][0];
+    }
+  double faces = 0;
+  for (int d = 0; d < 3; ++d) faces += double(g.nface[d]);
+  for (int p = 0; p < npass; ++p) {
+    V.S.colour = p & 1;
+    const bool timed = tm && *tm->n < tm->cap;
+    if (tm && !timed) ++*tm->missed;
+    auto kern = p == 0 ? vc_sweep3_kernel<T, true> : vc_sweep3_kernel<T, false>;
+    hipExtLaunchKernelGGL(kern, dim3(8 * V.S.chunk), dim3(256), 0, s, timed ? tm->start[*tm->n] : nullptr,
+                          timed ? tm->stop[*tm->n] : nullptr, 0, V);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (timed) {
+      // state, rhs, a and c of the colour and the other colour's state once;
+      // every face; the colour written (the first pass: every cell)
+      const double cells = double(g.nvalid());
+      const double b = cells * (p == 0 && zero_init ? 0 : 1) + (p == 0 && pc ? cells / 8 : 0) +
+                       0.5 * cells * (1 + (A.a ? 1 : 0) + (A.c ? 1 : 0)) + faces + (p == 0 ? 1.0 : 0.5) * cells;
+      *tm->bytes += b * sizeof(T);
+      ++*tm->n;
+    }
+  }
+  *cur = 1 - *cur;
   return hipSuccess;
 }
 
@@ -1456,9 +1552,11 @@ template <typename T, int DIM>
 hipError_t vc_relax_dim(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                         const Geom* gc, const T* pc, hipStream_t s, const Geom* gr = nullptr, T* resc = nullptr,
                         const LaunchTimer* tm = nullptr, const VCFinal<T>* fin = nullptr) {
-  if (!resc && !fin && npass > 0 && vc_streams(A.g))
-    return vc_relax_stream<T, DIM>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
+  if (DIM == 3 && !resc && !fin && npass > 0 && sweep3_ok(A.g))
+    return vc_relax_sweeps<T>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
   if constexpr (DIM == 2) {
+    if (!resc && !fin && npass > 0 && vc_streams(A.g))
+      return vc_relax_stream<T>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
     if (vc_wide(A.g))
       return vc_relax_cfg<T, 2, VCRelaxWide2>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, gr, resc, tm, fin);
   }
@@ -1734,12 +1832,7 @@ void vc_desc_geometry(VCDesc<T>& D, const Geom& g, const BCDesc& bc, int nl) {
     }
   }
   D.tot = D.off[nl];
-  BCDesc hom = bc;
-  hom.apply = 1;
-  for (auto& d : hom.val)
-    for (auto& s : d)
-      for (auto& v : s) v = 0.0;
-  const GhostForm<T> gf = ghost_form<T>(hom, T(g.dx));
+  const GhostForm<T> gf = vc_ghost_form<T>(bc, T(g.dx));
   for (int d = 0; d < 3; ++d)
     for (int s = 0; s < 2; ++s) {
       D.gs[d][s] = gf.s[d][s][0];

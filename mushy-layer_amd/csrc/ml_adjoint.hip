@@ -43,8 +43,7 @@ struct AdjWork {
   double *M = nullptr, *pl = nullptr, *pst = nullptr, *X = nullptr;
   double *x = nullptr, *r = nullptr, *rh = nullptr, *p = nullptr, *v = nullptr, *s = nullptr, *t = nullptr,
          *y = nullptr, *z = nullptr, *rhs = nullptr;
-  double* part = nullptr;    // per-workgroup partial sums (device)
-  double* hpart = nullptr;   // pinned mirror
+  double* hpart = nullptr;   // per-workgroup partial sums (page-locked, written by the kernels)
   int nblk = 0;
   std::vector<void*> owned;
 };
@@ -208,124 +207,11 @@ __device__ inline double stencil(const AdjGeo& G, const double* x, int i, int j,
   return s;
 }
 
-// y = J^T x on valid cells
-__global__ void adj_apply_kernel(AdjGeo G, const double* __restrict__ M, const double* __restrict__ x, double* y) {
-  const Geom& g = G.g;
-  const long long N = g.nvalid();
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
-    int i, j;
-    cell_of(g, c, i, j);
-    const long long q = g.ci(i, j, 0);
-    const double w0 = stencil(G, x, i, j, q, 0), w1 = stencil(G, x, i, j, q, 1);
-    const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
-    y[q] = G.alpha * x[q] - G.bd * (m0 * w0 + m2 * w1);
-    y[q + g.ncell] = G.alpha * x[q + g.ncell] - G.bd * (m1 * w0 + m3 * w1);
-  }
-}
-
-// z = P^{-1} r with P the 2x2 diagonal block of J^T at each cell
-__global__ void adj_jacobi_kernel(AdjGeo G, const double* __restrict__ M, const double* __restrict__ r, double* z) {
-  const Geom& g = G.g;
-  const long long N = g.nvalid();
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
-    int i, j;
-    cell_of(g, c, i, j);
-    const long long q = g.ci(i, j, 0);
-    double sd[2] = {0.0, 0.0};
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-          const double bf = face_b(G, i, j, d, side, n);
-          sd[n] += nbr(g, i, j, d, side) >= 0 ? -bf : bf * (wall_s(G.bc, d, side, n) - 1.0);
-        }
-    const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
-    const double p00 = G.alpha - G.bd * m0 * sd[0], p01 = -G.bd * m2 * sd[1];
-    const double p10 = -G.bd * m1 * sd[0], p11 = G.alpha - G.bd * m3 * sd[1];
-    const double det = p00 * p11 - p01 * p10;
-    const double r0 = r[q], r1 = r[q + g.ncell];
-    z[q] = (p11 * r0 - p01 * r1) / det;
-    z[q + g.ncell] = (p00 * r1 - p10 * r0) / det;
-  }
-}
-
-// One colour of the transposed smoother: block Gauss-Seidel on J^T
-// z = P^{-1} r, updating the cells with (i + j) % 2 == colour from the
-// other colour's current z:  z_q = D_q^{-1} (r_q + bd M_q^T w_q), w_q,n the
-// face-weighted sum of the interior neighbours' z_n (the wall terms sit in
-// D_q, the 2x2 diagonal block of J^T).  The forward smoother relaxes red
-// then black; its transpose relaxes black then red.
-__global__ void adj_gs_kernel(AdjGeo G, const double* __restrict__ M, const double* __restrict__ r, double* z,
-                              int colour) {
-  const Geom& g = G.g;
-  const long long N = g.nvalid();
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
-    int i, j;
-    cell_of(g, c, i, j);
-    if (((i + j) & 1) != colour) continue;
-    const long long q = g.ci(i, j, 0);
-    double sd[2] = {0.0, 0.0}, wn[2] = {0.0, 0.0};
-#pragma unroll
-    for (int n = 0; n < 2; ++n)
-#pragma unroll
-      for (int d = 0; d < 2; ++d)
-#pragma unroll
-        for (int side = 0; side < 2; ++side) {
-          const double bf = face_b(G, i, j, d, side, n);
-          const long long nb = nbr(g, i, j, d, side);
-          if (nb >= 0) {
-            sd[n] += -bf;
-            wn[n] += bf * z[nb + n * g.ncell];
-          } else {
-            sd[n] += bf * (wall_s(G.bc, d, side, n) - 1.0);
-          }
-        }
-    const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
-    const double p00 = G.alpha - G.bd * m0 * sd[0], p01 = -G.bd * m2 * sd[1];
-    const double p10 = -G.bd * m1 * sd[0], p11 = G.alpha - G.bd * m3 * sd[1];
-    const double det = p00 * p11 - p01 * p10;
-    const double r0 = r[q] + G.bd * (m0 * wn[0] + m2 * wn[1]);
-    const double r1 = r[q + g.ncell] + G.bd * (m1 * wn[0] + m3 * wn[1]);
-    z[q] = (p11 * r0 - p01 * r1) / det;
-    z[q + g.ncell] = (p00 * r1 - p10 * r0) / det;
-  }
-}
-
-// out = a x + b y on valid cells (y may be null)
-__global__ void adj_axpby_kernel(Geom g, double a, const double* __restrict__ x, double b, const double* y, double* out) {
-  const long long N = g.nvalid();
-  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
-    int i, j;
-    cell_of(g, c, i, j);
-    const long long q = g.ci(i, j, 0);
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const long long k = q + n * g.ncell;
-      out[k] = y ? a * x[k] + b * y[k] : a * x[k];
-    }
-  }
-}
-
-// per-workgroup partial sums of a.b and c.d over valid cells (c may be
-// null), in a fixed order
-__global__ __launch_bounds__(kT) void adj_dot_kernel(Geom g, const double* __restrict__ a, const double* __restrict__ b,
-                                                     const double* c, const double* d, double* part) {
+// the workgroup's sums of u and w, in a fixed order, to part[2b], part[2b+1]
+// (page-locked host memory: the host adds the workgroups' sums in order once
+// the stream has drained, with no copy in between)
+__device__ __forceinline__ void block_sums(double u, double w, double* part) {
   __shared__ double s0[kT], s1[kT];
-  const long long N = g.nvalid();
-  double u = 0.0, w = 0.0;
-  for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < N; t += (long long)gridDim.x * blockDim.x) {
-    int i, j;
-    cell_of(g, t, i, j);
-    const long long q = g.ci(i, j, 0);
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const long long k = q + n * g.ncell;
-      u += a[k] * b[k];
-      if (c) w += c[k] * d[k];
-    }
-  }
   s0[threadIdx.x] = u;
   s1[threadIdx.x] = w;
   __syncthreads();
@@ -340,6 +226,167 @@ __global__ __launch_bounds__(kT) void adj_dot_kernel(Geom g, const double* __res
     part[2 * blockIdx.x] = s0[0];
     part[2 * blockIdx.x + 1] = s1[0];
   }
+}
+
+// z = P^{-1} r at a cell, P the 2x2 diagonal block of J^T (r of the cell in
+// r0, r1)
+__device__ __forceinline__ void jacobi_cell(const AdjGeo& G, const double* __restrict__ M, int i, int j, long long q,
+                                            double r0, double r1, double* z) {
+  const Geom& g = G.g;
+  double sd[2] = {0.0, 0.0};
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        const double bf = face_b(G, i, j, d, side, n);
+        sd[n] += nbr(g, i, j, d, side) >= 0 ? -bf : bf * (wall_s(G.bc, d, side, n) - 1.0);
+      }
+  const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
+  const double p00 = G.alpha - G.bd * m0 * sd[0], p01 = -G.bd * m2 * sd[1];
+  const double p10 = -G.bd * m1 * sd[0], p11 = G.alpha - G.bd * m3 * sd[1];
+  const double det = p00 * p11 - p01 * p10;
+  z[q] = (p11 * r0 - p01 * r1) / det;
+  z[q + g.ncell] = (p00 * r1 - p10 * r0) / det;
+}
+
+// The transposed smoother at one cell: block Gauss-Seidel on J^T
+// z = P^{-1} r from the other colour's current z (ZERO: from z = 0):
+// z_q = D_q^{-1} (r_q + bd M_q^T w_q), w_q,n the face-weighted sum of the
+// interior neighbours' z_n (the wall terms sit in D_q, the 2x2 diagonal block
+// of J^T).  The forward smoother relaxes red then black; its transpose
+// relaxes black ((i + j) odd) then red.
+template <bool ZERO>
+__device__ __forceinline__ void gs_cell(const AdjGeo& G, const double* __restrict__ M, int i, int j, long long q,
+                                        double rq0, double rq1, double* z) {
+  const Geom& g = G.g;
+  double sd[2] = {0.0, 0.0}, wn[2] = {0.0, 0.0};
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        const double bf = face_b(G, i, j, d, side, n);
+        const long long nb = nbr(g, i, j, d, side);
+        if (nb >= 0) {
+          sd[n] += -bf;
+          wn[n] += bf * (ZERO ? 0.0 : z[nb + n * g.ncell]);
+        } else {
+          sd[n] += bf * (wall_s(G.bc, d, side, n) - 1.0);
+        }
+      }
+  const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
+  const double p00 = G.alpha - G.bd * m0 * sd[0], p01 = -G.bd * m2 * sd[1];
+  const double p10 = -G.bd * m1 * sd[0], p11 = G.alpha - G.bd * m3 * sd[1];
+  const double det = p00 * p11 - p01 * p10;
+  const double r0 = rq0 + G.bd * (m0 * wn[0] + m2 * wn[1]);
+  const double r1 = rq1 + G.bd * (m1 * wn[0] + m3 * wn[1]);
+  z[q] = (p11 * r0 - p01 * r1) / det;
+  z[q + g.ncell] = (p00 * r1 - p10 * r0) / det;
+}
+
+// One colour of the smoother.
+__global__ __launch_bounds__(kT) void adj_gs_kernel(AdjGeo G, const double* __restrict__ M,
+                                                    const double* __restrict__ r, double* z, int colour) {
+  const Geom& g = G.g;
+  const long long N = g.nvalid();
+  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
+    int i, j;
+    cell_of(g, c, i, j);
+    if (((i + j) & 1) != colour) continue;
+    const long long q = g.ci(i, j, 0);
+    gs_cell<false>(G, M, i, j, q, r[q], r[q + g.ncell], z);
+  }
+}
+
+// The vector updates of a BiCGStab iteration, fused with what follows them
+// at the same cell: the sums of their dot products and the start of the
+// preconditioner (the block diagonal, or the black cells of a sweep from
+// z = 0, which reads no neighbour).  On grids of some 10^4 cells a launch of
+// any of these costs its 3-4 us whatever it does: an iteration took 17
+// launches, 5 copies and 5 waits of the host, now 7 launches and 3 waits
+// (adjoint of a 128^2 step, 41 iterations: 6.24 -> 2.94 ms).
+enum AdjStep { ADJ_INIT, ADJ_P, ADJ_S, ADJ_R };
+struct AdjVec {
+  const double* g;
+  double *rhs, *x, *r, *rh, *p, *v, *s, *t, *y, *z;
+  double* part;
+  double a, b;
+  int gs;   // the preconditioner starts with a black half sweep (else: the block diagonal)
+};
+template <int STEP>
+__global__ __launch_bounds__(kT) void adj_vec_kernel(AdjGeo G, const double* __restrict__ M, AdjVec V) {
+  const Geom& g = G.g;
+  const long long N = g.nvalid();
+  double u = 0.0, w = 0.0;
+  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
+    int i, j;
+    cell_of(g, c, i, j);
+    const long long q = g.ci(i, j, 0);
+    double pr[2];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const long long k = q + n * g.ncell;
+      if (STEP == ADJ_INIT) {
+        const double f = 1.0 * V.g[k], zero = 0.0 * f;
+        V.rhs[k] = V.r[k] = V.rh[k] = f;
+        V.x[k] = V.p[k] = V.v[k] = zero;
+        u += f * f;
+      } else if (STEP == ADJ_P) {   // p = r + beta (p - omega v); a = -omega, b = beta
+        const double d = 1.0 * V.p[k] + V.a * V.v[k];
+        pr[n] = 1.0 * V.r[k] + V.b * d;
+        V.p[k] = pr[n];
+      } else if (STEP == ADJ_S) {   // s = r - alpha v, x += alpha y; a = -alpha, b = alpha
+        pr[n] = 1.0 * V.r[k] + V.a * V.v[k];
+        V.s[k] = pr[n];
+        V.x[k] = 1.0 * V.x[k] + V.b * V.y[k];
+        u += pr[n] * pr[n];
+      } else {                      // x += omega z, r = s - omega t; a = -omega, b = omega
+        V.x[k] = 1.0 * V.x[k] + V.b * V.z[k];
+        const double f = 1.0 * V.s[k] + V.a * V.t[k];
+        V.r[k] = f;
+        u += f * f;
+        w += V.rh[k] * f;
+      }
+    }
+    if (STEP == ADJ_P || STEP == ADJ_S) {
+      double* z = STEP == ADJ_P ? V.y : V.z;
+      if (!V.gs)
+        jacobi_cell(G, M, i, j, q, pr[0], pr[1], z);
+      else if ((i + j) & 1)
+        gs_cell<true>(G, M, i, j, q, pr[0], pr[1], z);
+    }
+  }
+  if (STEP != ADJ_P) block_sums(u, w, V.part);
+}
+
+// y = J^T x on valid cells, with the sums of a.y and, with two, of y.y
+__global__ __launch_bounds__(kT) void adj_apply_kernel(AdjGeo G, const double* __restrict__ M,
+                                                       const double* __restrict__ x, double* y,
+                                                       const double* __restrict__ a, int two, double* part) {
+  const Geom& g = G.g;
+  const long long N = g.nvalid();
+  double u = 0.0, w = 0.0;
+  for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < N; c += (long long)gridDim.x * blockDim.x) {
+    int i, j;
+    cell_of(g, c, i, j);
+    const long long q = g.ci(i, j, 0);
+    const double w0 = stencil(G, x, i, j, q, 0), w1 = stencil(G, x, i, j, q, 1);
+    const double m0 = M[q], m1 = M[q + g.ncell], m2 = M[q + 2 * g.ncell], m3 = M[q + 3 * g.ncell];
+    const double y0 = G.alpha * x[q] - G.bd * (m0 * w0 + m2 * w1);
+    const double y1 = G.alpha * x[q + g.ncell] - G.bd * (m1 * w0 + m3 * w1);
+    y[q] = y0;
+    y[q + g.ncell] = y1;
+    u += a[q] * y0;
+    u += a[q + g.ncell] * y1;
+    if (two) {
+      w += y0 * y0;
+      w += y1 * y1;
+    }
+  }
+  block_sums(u, w, part);
 }
 
 // gradients after the solve: dL/dphi^{n-1} (valid cells), the heat-flux
@@ -475,30 +522,22 @@ int adj_init(ml_hc_op op) {
     *a = static_cast<double*>(v);
   }
   void* v = nullptr;
-  ML_HIP(ctx, hipMalloc(&v, sizeof(double) * 2 * kMaxBlk));
-  w->owned.push_back(v);
-  w->part = static_cast<double*>(v);
-  ML_HIP(ctx, hipHostMalloc(&v, sizeof(double) * 2 * kMaxBlk, hipHostMallocDefault));
+  ML_HIP(ctx, hipHostMalloc(&v, sizeof(double) * 4 * kMaxBlk, hipHostMallocDefault));
   w->hpart = static_cast<double*>(v);
   w->nblk = blocks_for(w->g.nvalid());
   return ML_OK;
 }
 
-// a.b (and c.d): partial sums per workgroup, added on the host in order
-int dots(ml_ctx ctx, AdjWork* w, const double* a, const double* b, const double* c, const double* d, double* ab,
-         double* cd) {
-  hipLaunchKernelGGL(adj_dot_kernel, dim3(w->nblk), dim3(kT), 0, ctx->stream, w->g, a, b, c, d, w->part);
-  ML_HIP(ctx, hipGetLastError());
-  ML_HIP(ctx, hipMemcpyAsync(w->hpart, w->part, sizeof(double) * 2 * w->nblk, hipMemcpyDeviceToHost, ctx->stream));
-  ML_HIP(ctx, hipStreamSynchronize(ctx->stream));
+// the sums of the workgroups' part[2b] and part[2b+1], in order (the stream
+// has drained)
+void host_sums(const AdjWork* w, const double* part, double* a, double* b) {
   double s0 = 0.0, s1 = 0.0;
   for (int k = 0; k < w->nblk; ++k) {
-    s0 += w->hpart[2 * k];
-    s1 += w->hpart[2 * k + 1];
+    s0 += part[2 * k];
+    s1 += part[2 * k + 1];
   }
-  *ab = s0;
-  if (cd) *cd = s1;
-  return ML_OK;
+  *a = s0;
+  if (b) *b = s1;
 }
 
 }  // namespace
@@ -528,9 +567,8 @@ int ml_hc_porosity_vjp(ml_hc_op op, const double* phi, const double* g_chi, doub
   if (rc) return rc;
   AdjWork* w = op->adj.get();
   hipLaunchKernelGGL(porosity_vjp_kernel, dim3(w->nblk), dim3(kT), 0, ctx->stream, w->g, op->cp, phi, g_chi, g_phi,
-                     w->part);
+                     w->hpart);
   ML_HIP(ctx, hipGetLastError());
-  ML_HIP(ctx, hipMemcpyAsync(w->hpart, w->part, sizeof(double) * w->nblk, hipMemcpyDeviceToHost, ctx->stream));
   ML_HIP(ctx, hipStreamSynchronize(ctx->stream));
   double st = 0.0;
   for (int k = 0; k < w->nblk; ++k) st += w->hpart[k];
@@ -575,11 +613,6 @@ int ml_hc_adjoint_step(ml_hc_op op, const double* phi_new, const double* phi_old
   G.bd = -dt / (g.dx * g.dx);
   G.DC = op->params.saltDiffusionCoeff;
   for (int d = 0; d < 3; ++d) G.b[d] = op->lev[0].b[d];
-  auto apply = [&](const double* x, double* y) -> int {
-    hipLaunchKernelGGL(adj_apply_kernel, dim3(nb), dim3(kT), 0, s, G, w->M, x, y);
-    ML_HIP(ctx, hipGetLastError());
-    return ML_OK;
-  };
   // preconditioner: o.nu1 sweeps of the transposed smoother (block
   // Gauss-Seidel on J^T, black then red) from z = 0; nu1 == 0: the 2x2
   // block-diagonal (Jacobi)
@@ -588,77 +621,69 @@ int ml_hc_adjoint_step(ml_hc_op op, const double* phi_new, const double* phi_old
   bool odd_seam = false;
   for (int d = 0; d < 2; ++d) odd_seam = odd_seam || (g.periodic[d] && (g.n[d] & 1));
   const int sweeps = (o.nu1 > 0 && !odd_seam) ? o.nu1 : 0;
-  auto prec = [&](const double* r, double* z) -> int {
-    if (sweeps == 0) {
-      hipLaunchKernelGGL(adj_jacobi_kernel, dim3(nb), dim3(kT), 0, s, G, w->M, r, z);
+  double* const part0 = w->hpart;
+  double* const part1 = w->hpart + 2 * kMaxBlk;
+  AdjVec V{g_new, w->rhs, w->x, w->r, w->rh, w->p, w->v, w->s, w->t, w->y, w->z, part0, 0.0, 0.0, sweeps > 0 ? 1 : 0};
+  auto vec = [&](auto kern, double* part, double a, double b) -> int {
+    V.part = part;
+    V.a = a;
+    V.b = b;
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(kT), 0, s, G, w->M, V);
+    ML_HIP(ctx, hipGetLastError());
+    return ML_OK;
+  };
+  // the rest of the preconditioner (the vector update has started it), then
+  // y = J^T z with the sums of a.y (and y.y)
+  auto prec_apply = [&](const double* r, double* z, double* y, const double* a, int two, double* part) -> int {
+    for (int k = 1; k < 2 * sweeps; ++k) {
+      hipLaunchKernelGGL(adj_gs_kernel, dim3(nb), dim3(kT), 0, s, G, w->M, r, z, (k & 1) ? 0 : 1);
       ML_HIP(ctx, hipGetLastError());
-      return ML_OK;
     }
-    hipLaunchKernelGGL(adj_axpby_kernel, dim3(nb), dim3(kT), 0, s, g, 0.0, r, 0.0, nullptr, z);
-    ML_HIP(ctx, hipGetLastError());
-    for (int k = 0; k < sweeps; ++k)
-      for (int colour = 1; colour >= 0; --colour) {
-        hipLaunchKernelGGL(adj_gs_kernel, dim3(nb), dim3(kT), 0, s, G, w->M, r, z, colour);
-        ML_HIP(ctx, hipGetLastError());
-      }
-    return ML_OK;
-  };
-  auto axpby = [&](double a, const double* x, double b, const double* y, double* out) -> int {
-    hipLaunchKernelGGL(adj_axpby_kernel, dim3(nb), dim3(kT), 0, s, g, a, x, b, y, out);
+    hipLaunchKernelGGL(adj_apply_kernel, dim3(nb), dim3(kT), 0, s, G, w->M, z, y, a, two, part);
     ML_HIP(ctx, hipGetLastError());
     return ML_OK;
   };
-  // BiCGStab on J^T lambda = g_new (right block-Jacobi preconditioning),
-  // from lambda = 0
-  double bb;
-  if ((rc = axpby(1.0, g_new, 0.0, nullptr, w->rhs))) return rc;
-  if ((rc = dots(ctx, w, w->rhs, w->rhs, nullptr, nullptr, &bb, nullptr))) return rc;
-  const double bnorm = std::sqrt(bb);
-  if ((rc = axpby(0.0, w->rhs, 0.0, nullptr, w->x))) return rc;
-  if ((rc = axpby(1.0, w->rhs, 0.0, nullptr, w->r))) return rc;
-  if ((rc = axpby(1.0, w->rhs, 0.0, nullptr, w->rh))) return rc;
-  if ((rc = axpby(0.0, w->rhs, 0.0, nullptr, w->p))) return rc;
-  if ((rc = axpby(0.0, w->rhs, 0.0, nullptr, w->v))) return rc;
+  // BiCGStab on J^T lambda = g_new (right preconditioning), from lambda = 0
+  double rho1;   // rh . r of the iteration to come
+  if ((rc = vec(adj_vec_kernel<ADJ_INIT>, part0, 0.0, 0.0))) return rc;
+  ML_HIP(ctx, hipStreamSynchronize(s));
+  host_sums(w, part0, &rho1, nullptr);
+  const double bnorm = std::sqrt(rho1);
   double rho = 1.0, alpha = 1.0, omega = 1.0, rnorm = bnorm;
   int it = 0, status = bnorm == 0.0 ? 8 : 0;
   const double tol = o.eps * bnorm;
   while (status == 0 && it < o.max_iter) {
     ++it;
-    double rho1;
-    if ((rc = dots(ctx, w, w->rh, w->r, nullptr, nullptr, &rho1, nullptr))) return rc;
     if (rho1 == 0.0) {
       status = 4;
       break;
     }
     const double beta = (rho1 / rho) * (alpha / omega);
     rho = rho1;
-    // p = r + beta (p - omega v)
-    if ((rc = axpby(1.0, w->p, -omega, w->v, w->p))) return rc;
-    if ((rc = axpby(1.0, w->r, beta, w->p, w->p))) return rc;
-    if ((rc = prec(w->p, w->y))) return rc;
-    if ((rc = apply(w->y, w->v))) return rc;
+    if ((rc = vec(adj_vec_kernel<ADJ_P>, part0, -omega, beta))) return rc;
+    if ((rc = prec_apply(w->p, w->y, w->v, w->rh, 0, part0))) return rc;
+    ML_HIP(ctx, hipStreamSynchronize(s));
     double rv;
-    if ((rc = dots(ctx, w, w->rh, w->v, nullptr, nullptr, &rv, nullptr))) return rc;
+    host_sums(w, part0, &rv, nullptr);
     alpha = rho / rv;
-    // s = r - alpha v
-    if ((rc = axpby(1.0, w->r, -alpha, w->v, w->s))) return rc;
-    if ((rc = axpby(1.0, w->x, alpha, w->y, w->x))) return rc;
-    double ss;
-    if ((rc = dots(ctx, w, w->s, w->s, nullptr, nullptr, &ss, nullptr))) return rc;
+    // the second half is launched before |s| is looked at: should s end the
+    // solve, z and t are not used
+    if ((rc = vec(adj_vec_kernel<ADJ_S>, part1, -alpha, alpha))) return rc;
+    if ((rc = prec_apply(w->s, w->z, w->t, w->s, 1, part0))) return rc;
+    ML_HIP(ctx, hipStreamSynchronize(s));
+    double ss, ts, tt;
+    host_sums(w, part1, &ss, nullptr);
     if (std::sqrt(ss) <= tol) {
       rnorm = std::sqrt(ss);
       status = 1;
       break;
     }
-    if ((rc = prec(w->s, w->z))) return rc;
-    if ((rc = apply(w->z, w->t))) return rc;
-    double ts, tt;
-    if ((rc = dots(ctx, w, w->t, w->s, w->t, w->t, &ts, &tt))) return rc;
+    host_sums(w, part0, &ts, &tt);
     omega = tt > 0.0 ? ts / tt : 0.0;
-    if ((rc = axpby(1.0, w->x, omega, w->z, w->x))) return rc;
-    if ((rc = axpby(1.0, w->s, -omega, w->t, w->r))) return rc;
+    if ((rc = vec(adj_vec_kernel<ADJ_R>, part0, -omega, omega))) return rc;
+    ML_HIP(ctx, hipStreamSynchronize(s));
     double rr;
-    if ((rc = dots(ctx, w, w->r, w->r, nullptr, nullptr, &rr, nullptr))) return rc;
+    host_sums(w, part0, &rr, &rho1);
     rnorm = std::sqrt(rr);
     if (rnorm <= tol) status = 1;
     if (omega == 0.0 && status == 0) status = 4;
@@ -666,9 +691,8 @@ int ml_hc_adjoint_step(ml_hc_op op, const double* phi_new, const double* phi_old
   if (status == 0) status = 2;
   // gradients
   hipLaunchKernelGGL(adj_grad_kernel, dim3(nb), dim3(kT), 0, s, G, w->x, w->pl, w->pst, w->X, dt, g_old, g_flux,
-                     w->part);
+                     w->hpart);
   ML_HIP(ctx, hipGetLastError());
-  ML_HIP(ctx, hipMemcpyAsync(w->hpart, w->part, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
   ML_HIP(ctx, hipStreamSynchronize(s));
   double gst = 0.0;
   for (int k = 0; k < nb; ++k) gst += w->hpart[k];

@@ -482,7 +482,10 @@ constexpr int kDirect = 16;
 // t + 512; levels whose owners fit one wavefront are relaxed by wave 0
 // alone.  The coarsest level is solved in FP64: exactly (Gauss-Jordan with
 // partial pivoting by one wavefront) when it has at most kDirect unknowns,
-// otherwise by `bottom` block Gauss-Seidel iterations.
+// otherwise by `bottom` block Gauss-Seidel iterations.  Five levels from
+// 32x32, us a launch: 53 before the exact solve worked without LDS and e
+// stayed in registers, 46 now; a colour pass of a small level is 460 cycles,
+// a visit's set-up 3000.
 constexpr int kLL = 6;   // levels one launch handles: 1024 cells coarsen to one cell in 6 (2D), 4 (3D)
 template <int DIM>
 struct LinLevels {
@@ -506,22 +509,23 @@ __device__ __forceinline__ float lc_wsign(int bcw, int d, int s, int n) {
 }
 
 // A thread's cells of one level for the duration of a level visit:
-// coordinates, colour, neighbour indices, faces, a, M, r and the block
-// inverses in registers.
+// coordinates, colour, neighbour indices, faces, a, M, e, r, the block
+// inverses, and per component and face the factor of the neighbour's M e (a
+// wall's ghost: the cell's own, with the wall's sign) in registers.
 template <int DIM>
 struct LCCtx {
-  int pk[2], c[2], col[2], wall[2];
+  int pk[2], c[2], col[2];
   int nb[2][2 * DIM];
+  float sg[2][2][2 * DIM];
   CellFaces<float, DIM> F[2];
-  float aq[2][2], inv[2][4], M[2][4], rr[2][2];
+  float aq[2][2], inv[2][4], M[2][4], rr[2][2], e[2][2];
 };
 
 // inverses: compute the block inverses (and keep them in LDS for the
 // level's next visit) or read them back
 template <int DIM>
 __device__ __forceinline__ void lcx_build(LCCtx<DIM>& X, const CLev& L, const int* per, const LinLds<DIM>& S,
-                                          float alpha, float beta, bool inverses) {
-  const float dxinv = float(1.0 / (L.dx * L.dx));
+                                          float alpha, float beta, float dxinv, int bcw, bool inverses) {
   const int N = L.N;
   const float* sM = S.m(L);
   const float* sr = S.r(L);
@@ -536,7 +540,13 @@ __device__ __forceinline__ void lcx_build(LCCtx<DIM>& X, const CLev& L, const in
     const int c = i + L.nx * j + L.nxy * k;
     X.c[m] = c;
     X.col[m] = (i + j + k) & 1;
-    clev_nbrs<DIM>(L, per, i, j, k, X.nb[m], X.wall[m]);
+    int wall;
+    clev_nbrs<DIM>(L, per, i, j, k, X.nb[m], wall);
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int f = 0; f < 2 * DIM; ++f)
+        X.sg[m][n][f] = ((wall >> f) & 1) ? lc_wsign(bcw, f >> 1, f & 1, n) : 1.0f;
     const int q = L.off + c;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
@@ -560,83 +570,78 @@ __device__ __forceinline__ void lcx_build(LCCtx<DIM>& X, const CLev& L, const in
 
 // (M e) stencil of component n of cell m from the level's su
 template <int DIM>
-__device__ __forceinline__ void lcx_ustencil(const LCCtx<DIM>& X, int m, int n, int bcw, const float* su, float* p) {
+__device__ __forceinline__ void lcx_ustencil(const LCCtx<DIM>& X, int m, int n, const float* su, float* p) {
   p[0] = su[X.c[m]];
 #pragma unroll
-  for (int f = 0; f < 2 * DIM; ++f) {
-    const int d = f >> 1, s = f & 1;
-    float v = su[X.nb[m][f]];
-    if ((X.wall[m] >> f) & 1) v = v * lc_wsign(bcw, d, s, n);
-    p[1 + 2 * d + (1 - s)] = v;
-  }
+  for (int f = 0; f < 2 * DIM; ++f) p[1 + (f ^ 1)] = su[X.nb[m][f]] * X.sg[m][n][f];
 }
 
-// u = M e at the context's cells
-template <int DIM>
-__device__ __forceinline__ void lcx_mvec(const LCCtx<DIM>& X, const CLev& L, const LinLds<DIM>& S) {
-  const int N = L.N;
-  const float* se = S.e(L);
-  float* su = S.u(L);
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    if (X.pk[m] < 0) continue;
-    const int c = X.c[m];
-    const float e0 = se[c], e1 = se[N + c];
-    su[c] = X.M[m][0] * e0 + X.M[m][1] * e1;
-    su[N + c] = X.M[m][2] * e0 + X.M[m][3] * e1;
-  }
-  __syncthreads();
+// a barrier of the threads that visit the level
+__device__ __forceinline__ void lc_sync(bool small) {
+  if (small)
+    wave_sync();
+  else
+    __syncthreads();
 }
 
+// u = M e at cell m
 template <int DIM>
-__device__ __forceinline__ void lcx_relax(const LCCtx<DIM>& X, const CLev& L, int bcw, const LinLds<DIM>& S,
-                                          float alpha, float beta, int npass) {
-  const float dxinv = float(1.0 / (L.dx * L.dx));
+__device__ __forceinline__ void lcx_put(const LCCtx<DIM>& X, int m, int N, float* su) {
+  const int c = X.c[m];
+  su[c] = X.M[m][0] * X.e[m][0] + X.M[m][1] * X.e[m][1];
+  su[N + c] = X.M[m][2] * X.e[m][0] + X.M[m][3] * X.e[m][1];
+}
+
+// M e of the context's cells, npass colour passes, e to LDS
+template <int DIM>
+__device__ __forceinline__ void lcx_relax(LCCtx<DIM>& X, const CLev& L, const LinLds<DIM>& S, float alpha, float beta,
+                                          float dxinv, int npass, bool small) {
   const int N = L.N;
   float* se = S.e(L);
   float* su = S.u(L);
-  auto pass = [&](int p) {
 #pragma unroll
-    for (int m = 0; m < 2; ++m) {
-      if (X.pk[m] < 0 || X.col[m] != (p & 1)) continue;
-      const int c = X.c[m];
-      float u0s[7], u1s[7];
-      lcx_ustencil<DIM>(X, m, 0, bcw, su, u0s);
-      lcx_ustencil<DIM>(X, m, 1, bcw, su + N, u1s);
-      float e0 = se[c], e1 = se[N + c];
-      block_step<float, DIM>(X.F[m], X.aq[m], X.rr[m], X.inv[m], alpha, beta, dxinv, u0s, u1s, e0, e1);
-      se[c] = e0;
-      se[N + c] = e1;
-      su[c] = X.M[m][0] * e0 + X.M[m][1] * e1;
-      su[N + c] = X.M[m][2] * e0 + X.M[m][3] * e1;
-    }
+  for (int m = 0; m < 2; ++m)
+    if (X.pk[m] >= 0) lcx_put<DIM>(X, m, N, su);
+  lc_sync(small);
+  auto update = [&](auto MM) __attribute__((always_inline)) {
+    constexpr int m = decltype(MM)::value;
+    if (X.pk[m] < 0) return;
+    float u0s[7], u1s[7];
+    lcx_ustencil<DIM>(X, m, 0, su, u0s);
+    lcx_ustencil<DIM>(X, m, 1, su + N, u1s);
+    block_step<float, DIM>(X.F[m], X.aq[m], X.rr[m], X.inv[m], alpha, beta, dxinv, u0s, u1s, X.e[m][0], X.e[m][1]);
+    lcx_put<DIM>(X, m, N, su);
   };
-  // levels whose owners fit one wavefront: wave 0 alone with wavefront-scope
-  // syncs (small is uniform, so the workgroup barrier is reached by all
-  // waves or by none)
-  const bool small = cown_active<kWGT>(L) <= 64;
-  if (!small || threadIdx.x < 64) {
+  if ((L.nx & 1) == 0) {   // a thread's cells are one of each colour
+#pragma unroll 1
+    for (int p = 0; p < npass; p += 2) {
+      update(IC<0>{});
+      lc_sync(small);
+      update(IC<1>{});
+      lc_sync(small);
+    }
+  } else {
 #pragma unroll 1
     for (int p = 0; p < npass; ++p) {
-      pass(p);
-      if (small)
-        wave_sync();
-      else
-        __syncthreads();
+      if (X.pk[0] >= 0 && X.col[0] == (p & 1)) update(IC<0>{});
+      if (X.pk[1] >= 0 && X.col[1] == (p & 1)) update(IC<1>{});
+      lc_sync(small);
     }
   }
-  if (small) __syncthreads();
+#pragma unroll
+  for (int m = 0; m < 2; ++m)
+    if (X.pk[m] >= 0) {
+      se[X.c[m]] = X.e[m][0];
+      se[N + X.c[m]] = X.e[m][1];
+    }
 }
 
-// r_c = R(r - J e), M_c = R(M); the coarse correction starts at zero.  The
-// fine level's M e array holds the residual between the two phases (the
+// r_c = R(r - J e), M_c = R(M).  The fine level's M e array holds the residual between the two phases (the
 // next visit of the level recomputes it).
 template <int DIM>
-__device__ __forceinline__ void lcx_restrict(const LCCtx<DIM>& X, const CLev& Lf, const CLev& Lc, int bcw,
-                                             const LinLds<DIM>& S, float alpha, float beta) {
-  const float dxinv = float(1.0 / (Lf.dx * Lf.dx));
+__device__ __forceinline__ void lcx_restrict(const LCCtx<DIM>& X, const CLev& Lf, const CLev& Lc,
+                                             const LinLds<DIM>& S, float alpha, float beta, float dxinv, bool small) {
   const int N = Lf.N;
-  const float* se = S.e(Lf);
   const float* sM = S.m(Lf);
   float* su = S.u(Lf);
   float res[2][2];
@@ -646,24 +651,24 @@ __device__ __forceinline__ void lcx_restrict(const LCCtx<DIM>& X, const CLev& Lf
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       float us[7];
-      lcx_ustencil<DIM>(X, m, n, bcw, su + n * N, us);
-      res[m][n] = X.rr[m][n] - lof_of<float, DIM>(X.F[m], n, us, X.aq[m][n], se[n * N + X.c[m]], alpha, beta, dxinv);
+      lcx_ustencil<DIM>(X, m, n, su + n * N, us);
+      res[m][n] = X.rr[m][n] - lof_of<float, DIM>(X.F[m], n, us, X.aq[m][n], X.e[m][n], alpha, beta, dxinv);
     }
   }
-  __syncthreads();
+  lc_sync(small);
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     if (X.pk[m] < 0) continue;
     su[X.c[m]] = res[m][0];
     su[N + X.c[m]] = res[m][1];
   }
-  __syncthreads();
-  const int NC = Lc.N;
+  lc_sync(small);
+  const int NC = Lc.N, step = small ? 64 : kWGT;
   float* rc = S.r(Lc);
   float* Mc = S.m(Lc);
-  float* ec = S.e(Lc);
   const float w = DIM == 3 ? 0.125f : 0.25f;
-  for (int cc = threadIdx.x; cc < NC; cc += kWGT) {
+#pragma unroll 1
+  for (int cc = threadIdx.x; cc < NC; cc += step) {
     int I, J, K;
     clev_coords(Lc, cc, I, J, K);
     float s0 = 0.f, s1 = 0.f, mm4[4] = {0.f, 0.f, 0.f, 0.f};
@@ -680,85 +685,78 @@ __device__ __forceinline__ void lcx_restrict(const LCCtx<DIM>& X, const CLev& Lf
     rc[NC + cc] = s1 * w;
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm) Mc[mm * NC + cc] = mm4[mm] * w;
-    ec[cc] = 0.f;
-    ec[NC + cc] = 0.f;
   }
-  __syncthreads();
 }
 
-// e_f += P(e_c) (linear prolongation from the coarse level in LDS)
+// e = e_f + P(e_c) (linear prolongation from the coarse level in LDS)
 template <int DIM>
-__device__ __forceinline__ void lcx_prolong(const LCCtx<DIM>& X, const CLev& Lf, const CLev& Lc, const int* per,
+__device__ __forceinline__ void lcx_prolong(LCCtx<DIM>& X, const CLev& Lf, const CLev& Lc, const int* per,
                                             const LinLds<DIM>& S) {
-  float* ef = S.e(Lf);
+  const float* ef = S.e(Lf);
   const float* ec = S.e(Lc);
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     if (X.pk[m] < 0) continue;
     int i, j, k;
     cunpack(X.pk[m], i, j, k);
-    const int c = X.c[m];
-    ef[c] = prolong_value_lds<float, DIM>(Lc.n, per, i, j, k, ec, ef[c]);
-    ef[Lf.N + c] = prolong_value_lds<float, DIM>(Lc.n, per, i, j, k, ec + Lc.N, ef[Lf.N + c]);
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+      X.e[m][n] = prolong_value_lds<float, DIM>(Lc.n, per, i, j, k, ec + n * Lc.N, ef[n * Lf.N + X.c[m]]);
   }
-  __syncthreads();
 }
 
-// Exact FP64 solve of J e = r on a tiny level (U = 2N <= kDirect unknowns)
-// by wave 0: lane R builds row R of J (unknown R = comp*N + cell) from the
-// unit vectors, then Gauss-Jordan elimination with partial pivoting, the
-// rows staying in the lanes' registers.  Returns false (e untouched) on a
-// zero pivot.  bF/bA: the level's FP64 faces and a in LDS; buf and prow:
-// 64 + kDirect + 1 doubles of LDS scratch.
-template <int DIM>
-__device__ __forceinline__ bool lc_direct(const CLev& L, const int* per, int bcw, double alpha, double beta, const double* bF,
-                          const double* bA, const double* dM, const double* dr, double* de, double* buf,
-                          double* prow) {
+// the value of lane `l` (uniform)
+__device__ __forceinline__ double lane_value(double x, int l) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readlane(int(u), l), hi = __builtin_amdgcn_readlane(int(u >> 32), l);
+  return __longlong_as_double((long long)((unsigned long long)lo | ((unsigned long long)hi << 32)));
+}
+
+// Exact FP64 solve of J e = r on a tiny level (U = 2N <= KD unknowns) by wave
+// 0: lane R builds row R of J (unknown R = comp*N + cell) from the unit
+// vectors, then Gauss-Jordan elimination with partial pivoting, the rows
+// staying in the lanes' registers and the pivot row read from its lane.
+// Returns false (e untouched) on a zero pivot.  bF/bA: the level's FP64 faces
+// and a in LDS.  One wave alone issues an operation every 8 cycles, so the
+// count of operations is the time: at 8 unknowns (KD 8) without divisions of
+// indices and without LDS round trips 12.8K cycles of a cycle's 108K, before
+// 26.1K of 121K.
+template <int DIM, int KD>
+__device__ __forceinline__ bool lc_direct(const CLev& L, const int* per, int bcw, double alpha, double beta, double dxinv,
+                                          const double* bF, const double* bA, const double* dM, const double* dr,
+                                          double* de) {
   const int N = L.N, U = 2 * N;
   const int lane = threadIdx.x;
-  const double dxinv = 1.0 / (L.dx * L.dx);
-  double a[kDirect];
+  double a[KD];
   double b = 0.0;
 #pragma unroll
-  for (int t = 0; t < kDirect; ++t) a[t] = 0.0;
+  for (int t = 0; t < KD; ++t) a[t] = 0.0;
   if (lane < U) {
-    const int rc = lane % N, kc = lane / N;
+    const int kc = lane >= N ? 1 : 0, rc = lane - kc * N;
     int i, j, k;
     clev_coords(L, rc, i, j, k);
-    const int iv[3] = {i, j, k};
-    // faces of component kc (held as component 0 of F)
+    int nb[2 * DIM], wall;
+    clev_nbrs<DIM>(L, per, i, j, k, nb, wall);
+    // faces of component kc (held as component 0 of F), the wall's signs
     CellFaces<double, DIM> F;
+    double sg[2 * DIM];
 #pragma unroll
     for (int f = 0; f < 2 * DIM; ++f) {
       F.v[0][f] = bF[(rc * 2 + kc) * 2 * DIM + f];
       F.v[1][f] = 0.0;
+      sg[f] = ((wall >> f) & 1) ? double(lc_wsign(bcw, f >> 1, f & 1, kc)) : 1.0;
     }
     const double aq = bA[rc * 2 + kc];
 #pragma unroll
-    for (int t = 0; t < kDirect; ++t) {
+    for (int t = 0; t < KD; ++t) {
       if (t >= U) continue;
-      const int ct = t % N, nt = t / N;
       // u = M e of the unit vector of unknown t: nonzero only at cell ct
-      auto u_at = [&](int cell) -> double { return cell == ct ? dM[(2 * kc + nt) * N + ct] : 0.0; };
+      const int nt = t >= N ? 1 : 0, ct = t - nt * N;
+      const double mt = dM[(2 * kc + nt) * N + ct];
       double p[7];
-      p[0] = u_at(rc);
+      p[0] = rc == ct ? mt : 0.0;
 #pragma unroll
-      for (int d = 0; d < DIM; ++d) {
-        const int nd = L.n[d];
-        const int st = d == 0 ? 1 : (d == 1 ? L.nx : L.nxy);
-#pragma unroll
-        for (int sd = 0; sd < 2; ++sd) {
-          const int v = iv[d] + (sd ? 1 : -1);
-          double val;
-          if (v >= 0 && v < nd)
-            val = u_at(rc + (sd ? st : -st));
-          else if (per[d])
-            val = u_at(rc + (sd ? -(nd - 1) * st : (nd - 1) * st));
-          else
-            val = p[0] * double(lc_wsign(bcw, d, sd, kc));
-          p[1 + 2 * d + (sd ? 0 : 1)] = val;
-        }
-      }
+      for (int f = 0; f < 2 * DIM; ++f) p[1 + (f ^ 1)] = (nb[f] == ct ? mt : 0.0) * sg[f];
       const double ev = (rc == ct && kc == nt) ? 1.0 : 0.0;
       a[t] = lof_of<double, DIM>(F, 0, p, aq, ev, alpha, beta, dxinv);
     }
@@ -767,40 +765,39 @@ __device__ __forceinline__ bool lc_direct(const CLev& L, const int* per, int bcw
   bool used = false;
   int mycol = -1;
 #pragma unroll
-  for (int c = 0; c < kDirect; ++c) {
+  for (int c = 0; c < KD; ++c) {
     if (c >= U) break;
-    buf[lane] = (lane < U && !used) ? fabs(a[c]) : -1.0;
-    wave_sync();
+    const double key = (lane < U && !used) ? fabs(a[c]) : -1.0;
     int piv = 0;
     double best = -1.0;
-    for (int r = 0; r < U; ++r) {
-      const double v = buf[r];
+#pragma unroll
+    for (int r = 0; r < KD; ++r) {   // (lanes beyond U hold -1)
+      const double v = lane_value(key, r);
       if (v > best) {
         best = v;
         piv = r;
       }
     }
+    piv = __builtin_amdgcn_readfirstlane(piv);
     if (!(best > 0.0)) return false;
     if (lane == piv) {
-#pragma unroll
-      for (int t = 0; t < kDirect; ++t) prow[t] = a[t];
-      prow[kDirect] = b;
       used = true;
       mycol = c;
     }
-    wave_sync();
-    if (lane < U && lane != piv) {
-      const double f = a[c] / prow[c];
+    const double f = a[c] / lane_value(a[c], piv);
+    const bool other = lane < U && lane != piv;
 #pragma unroll
-      for (int t = 0; t < kDirect; ++t) a[t] = a[t] - f * prow[t];
-      b = b - f * prow[kDirect];
+    for (int t = 0; t < KD; ++t) {
+      const double x = a[t] - f * lane_value(a[t], piv);
+      a[t] = other ? x : a[t];
     }
-    wave_sync();
+    const double y = b - f * lane_value(b, piv);
+    b = other ? y : b;
   }
   if (lane < U) {
     double dcol = 1.0;
 #pragma unroll
-    for (int t = 0; t < kDirect; ++t)
+    for (int t = 0; t < KD; ++t)
       if (t == mycol) dcol = a[t];
     de[mycol] = b / dcol;
   }
@@ -856,8 +853,6 @@ __device__ __forceinline__ void linpre_store(const LinPre<DIM>& P, const LinLds<
   }
   if (state) {
     const int N = L.N;
-    S.se[c] = 0.f;
-    S.se[N + c] = 0.f;
     S.sr[c] = P.r[0];
     S.sr[N + c] = P.r[1];
 #pragma unroll
@@ -892,14 +887,15 @@ __global__ __launch_bounds__(kWGT) void lin_coarse_vcycle_kernel(const LinDesc* 
         bcw |= ((D.bc.apply && D.bc.type[d][sd][n] == 0) ? 1 : 0) << (6 * n + 2 * d + sd);
   // level geometry in LDS (uniform reads) rather than registers
   __shared__ CLev G[LL];
+  __shared__ float dxi[LL];
   int tot = 0;
-  for (int l = 0; l < nl && l < LL; ++l) tot += D.lev[l0 + l].g.n[0] * D.lev[l0 + l].g.n[1] * D.lev[l0 + l].g.n[2];
-  if (threadIdx.x == 0) {
-    int off = 0;
-    for (int l = 0; l < nl && l < LL; ++l) {
-      clev_set(G[l], D.lev[l0 + l].g, off);
-      off += G[l].N;
+  for (int l = 0; l < nl && l < LL; ++l) {
+    const Geom& gl = D.lev[l0 + l].g;
+    if (int(threadIdx.x) == l) {   // a lane per level
+      clev_set(G[l], gl, tot);
+      dxi[l] = float(1.0 / (gl.dx * gl.dx));
     }
+    tot += gl.n[0] * gl.n[1] * gl.n[2];
   }
   __syncthreads();
   LinLds<DIM> S;
@@ -916,14 +912,12 @@ __global__ __launch_bounds__(kWGT) void lin_coarse_vcycle_kernel(const LinDesc* 
   const CLev& Lb = G[lb];
   const int Nb = Lb.N;
   const bool direct = 2 * Nb <= kDirect;
-  // exact solve only: FP64 e, M, r, faces [cell][2][2*DIM], a [cell][2] and
-  // 64 + kDirect + 1 scratch
+  // exact solve only: FP64 e, M, r, faces [cell][2][2*DIM], a [cell][2]
   double* de = reinterpret_cast<double*>(smem_raw + ((size_t(16 + 4 * DIM) * tot * sizeof(float) + 15) & ~size_t(15)));
   double* dM = de + 2 * Nb;
   double* dr = dM + 4 * Nb;
   double* bF = dr + 2 * Nb;
   double* bA = bF + 4 * DIM * Nb;
-  double* dbuf = bA + 2 * Nb;
   // operator data of every level (and the coarsest level's FP64 copy for
   // the exact solve), level l0's state: all global loads first (level l0:
   // cells t and t + 512, coarser levels: cell t), then the LDS stores
@@ -941,66 +935,61 @@ __global__ __launch_bounds__(kWGT) void lin_coarse_vcycle_kernel(const LinDesc* 
   for (int l = 1; l < LL; ++l)
     if (l < nl) linpre_store<DIM>(P1[l - 1], S, G[l], threadIdx.x, false, direct && lb == l, bF, bA);
   __syncthreads();
-  // The level visits are runtime loops over one copy of their code (level
+  // The level visits are one runtime loop over one copy of their code (level
   // geometry from LDS): unrolled per level, the kernel's code is several
   // times the instruction cache and a launch spends most of its time
-  // fetching it.
-  // down: pre-smoothing and restriction to the coarsest level
+  // fetching it.  Down: relaxation from zero, restriction; bottom: exact FP64
+  // solve of a tiny level, otherwise (or on a zero pivot) `bottom` block
+  // Gauss-Seidel iterations; up: prolongation and relaxation.
 #pragma unroll 1
-  for (int l = 0; l + 1 < nl; ++l) {
-    LCCtx<DIM> X;
-    lcx_build<DIM>(X, G[l], per, S, alpha, beta, true);
-    lcx_mvec<DIM>(X, G[l], S);
-    lcx_relax<DIM>(X, G[l], bcw, S, alpha, beta, 2 * D.nu1);
-    lcx_restrict<DIM>(X, G[l], G[l + 1], bcw, S, alpha, beta);
-  }
-  // bottom: exact FP64 solve of a tiny coarsest level; otherwise (or on a
-  // zero pivot) `bottom` block Gauss-Seidel iterations
-  {
-    __shared__ int direct_ok;
-    bool solved = false;
-    if (direct) {
-      const float* fr = S.r(Lb);
-      const float* fM = S.m(Lb);
-      for (int c = threadIdx.x; c < Nb; c += kWGT) {
-        de[c] = 0.0;
-        de[Nb + c] = 0.0;
-        dr[c] = double(fr[c]);
-        dr[Nb + c] = double(fr[Nb + c]);
+  for (int v = 0; v < 2 * nl - 1; ++v) {
+    const bool up = v >= nl, bot = v == nl - 1;
+    const int l = up ? 2 * nl - 2 - v : v;
+    const CLev& L = G[l];
+    const bool small = cown_active<kWGT>(L) <= 64;
+    if (!small || threadIdx.x < 64) {
+      bool solved = false;
+      if (bot && direct) {   // (at most kDirect / 2 cells: wave 0)
+        const float* fr = S.r(Lb);
+        const float* fM = S.m(Lb);
+        const int c = threadIdx.x;
+        if (c < Nb) {
+          de[c] = 0.0;
+          de[Nb + c] = 0.0;
+          dr[c] = double(fr[c]);
+          dr[Nb + c] = double(fr[Nb + c]);
 #pragma unroll
-        for (int mm = 0; mm < 4; ++mm) dM[mm * Nb + c] = double(fM[mm * Nb + c]);
-      }
-      __syncthreads();
-      if (threadIdx.x < 64) {
-        const bool ok = lc_direct<DIM>(Lb, per, bcw, D.alpha, D.beta, bF, bA, dM, dr, de, dbuf, dbuf + 64);
-        if (threadIdx.x == 0) direct_ok = ok ? 1 : 0;
-      }
-      __syncthreads();
-      solved = direct_ok != 0;
-      if (solved) {
-        float* fe = S.e(Lb);
-        for (int c = threadIdx.x; c < Nb; c += kWGT) {
+          for (int mm = 0; mm < 4; ++mm) dM[mm * Nb + c] = double(fM[mm * Nb + c]);
+        }
+        wave_sync();
+        const double dxi64 = 1.0 / (Lb.dx * Lb.dx);
+        solved = 2 * Nb <= kDirect / 2
+                     ? lc_direct<DIM, kDirect / 2>(Lb, per, bcw, D.alpha, D.beta, dxi64, bF, bA, dM, dr, de)
+                     : lc_direct<DIM, kDirect>(Lb, per, bcw, D.alpha, D.beta, dxi64, bF, bA, dM, dr, de);
+        if (solved && c < Nb) {
+          float* fe = S.e(Lb);
           fe[c] = float(de[c]);
           fe[Nb + c] = float(de[Nb + c]);
         }
-        __syncthreads();
+      }
+      if (!solved) {
+        const float dxinv = dxi[l];
+        LCCtx<DIM> X;
+        lcx_build<DIM>(X, L, per, S, alpha, beta, dxinv, bcw, !up);
+        X.e[0][0] = X.e[0][1] = X.e[1][0] = X.e[1][1] = 0.f;
+        if (up) lcx_prolong<DIM>(X, L, G[l + 1], per, S);
+        lcx_relax<DIM>(X, L, S, alpha, beta, dxinv, 2 * (bot ? D.bottom : (up ? D.nu2 : D.nu1)), small);
+        if (v < nl - 1) lcx_restrict<DIM>(X, L, G[l + 1], S, alpha, beta, dxinv, small);
       }
     }
-    if (!solved) {
-      LCCtx<DIM> X;
-      lcx_build<DIM>(X, Lb, per, S, alpha, beta, true);
-      lcx_mvec<DIM>(X, Lb, S);
-      lcx_relax<DIM>(X, Lb, bcw, S, alpha, beta, 2 * D.bottom);
-    }
-  }
-  // up: prolongation and post-smoothing
-#pragma unroll 1
-  for (int l = nl - 2; l >= 0; --l) {
-    LCCtx<DIM> X;
-    lcx_build<DIM>(X, G[l], per, S, alpha, beta, false);
-    lcx_prolong<DIM>(X, G[l], G[l + 1], per, S);
-    lcx_mvec<DIM>(X, G[l], S);
-    lcx_relax<DIM>(X, G[l], bcw, S, alpha, beta, 2 * D.nu2);
+    // the next visit reads what this one wrote: wave 0 alone where both are
+    // small, else the workgroup
+    const bool next_small =
+        small && v + 1 < 2 * nl - 1 && cown_active<kWGT>(G[v + 1 >= nl ? 2 * nl - 3 - v : v + 1]) <= 64;
+    if (!next_small)
+      __syncthreads();
+    else if (threadIdx.x < 64)
+      wave_sync();
   }
   const LinLevel<float>& lv = D.lev[l0];
   const float* se = S.e(G[0]);
@@ -1315,7 +1304,7 @@ size_t lin_coarse_lds_bytes(const Geom* g, int l0, int nlev) {
   const long long nb = g[nlev - 1].nvalid();
   const int dim = g[l0].dim;
   const bool direct = 2 * nb <= kDirect;
-  const size_t dbl = direct ? size_t((8 + 4 * dim + 2) * nb + 64 + kDirect + 1) : 0;
+  const size_t dbl = direct ? size_t((8 + 4 * dim + 2) * nb) : 0;
   return ((size_t(16 + 4 * dim) * tot * sizeof(float) + 15) & ~size_t(15)) + dbl * sizeof(double);
 }
 

@@ -107,7 +107,8 @@ def kernel_roofline(ml, ctx, stepper, reps=200):
     ms = ctx.elapsed_ms(0, 1) / reps
     phi.free()
     achieved = bytes_per_cell * cells / (ms * 1e-3) / 1e9
-    return {"kernel": "hc_relax_tile_kernel<double,%d,...> (1 sweep, finest level)" % dim,
+    name = "hc_relax_pair_kernel<double,0,false>" if dim == 2 else "hc_sweep3_kernel<double> (two launches)"
+    return {"kernel": "%s (1 sweep, finest level)" % name,
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": None,
             "avg_launch_us": round(ms * 1e3, 3), "bytes_per_launch": bytes_per_cell * cells}
@@ -135,9 +136,9 @@ def smoother_bandwidth(ml, wl, ctx, n, launches=20):
     n1, ms, nb, _ = ctx.timing_stop()
     gbs = nb / (ms * 1e-3) / 1e9
     # levels above 512^2 cells relax by streaming along y (both colour passes
-    # of a sweep pipelined in one launch), smaller ones in deep-halo tiles
+    # of a sweep pipelined in one launch), smaller ones in deep-halo regions
     hname = ("hc_relax_stream_kernel<double,2,252,1,2,256,false>" if n * n > 512 * 512 else
-             "hc_relax_tile_kernel<double,2,32,8,1,8,512>")
+             "hc_relax_pair_kernel<double,0,false>")
     out["hc_relax"] = {"kernel": "%s (1 sweep per launch)" % hname,
                        "avg_launch_us": round(ms / n1 * 1e3, 2), "bytes_per_launch": nb / n1,
                        "achieved_GBs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4)}
@@ -320,8 +321,8 @@ def timed_steps(ctx, st, steps):
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "vc_relax_tile_256_traffic.json")   # 256x256 workload
 BATCH_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "batch_relax_512_traffic.json")   # 512-instance batch
-# the tiled relaxation of the finest level of the two workloads
-VC_TILE = {2: "vc_relax_tile_kernel<double,2,16,16,1,9,1024>", 3: "vc_relax_tile_kernel<double,3,16,8,4,2,1024>"}
+# the relaxation of the finest level of the two workloads
+VC_TILE = {2: "vc_relax_tile_kernel<double,2,16,16,1,9,1024>", 3: "vc_sweep3_kernel<double> (one colour a launch)"}
 
 
 def vc_relax_roofline(ml, ctx, stepper, steps):

@@ -78,6 +78,8 @@ __device__ inline void tile_diffused_var(const HCArgs<T>& A, const Tile<DIM, TX,
 // io.pc is set, the staged state first receives the linear prolongation of
 // the coarse correction pc - pc0 (prolongIncrement fused with the
 // post-smoother).  Input and output arrays are distinct.
+// 3D levels with an odd periodic length (two cells of a colour meet at the
+// seam) or beyond 32-bit offsets; other levels have faster forms.
 template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
 __global__ __launch_bounds__(NT) void hc_relax_tile_kernel(HCArgs<T> A, TileIO<T> io) {
   if (A.skip && *A.skip) return;

@@ -83,6 +83,8 @@ __device__ inline T vc_lof(const Faces1<T, DIM>& F, const T* p, T aq, bool hasc,
 // homogeneous wall ghosts of the cells it updated, so one barrier per pass.
 // The body works on tile `tile` of the level (a batched launch maps its
 // workgroups to (instance, tile) pairs).
+// 3D plain relaxation comes here with an odd periodic length or beyond 32-bit
+// offsets only.
 template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
 __device__ __forceinline__ void vc_relax_tile_body(const VCArgs<T>& A, const T* __restrict__ in, T* __restrict__ out,
                                                    const T* __restrict__ rhs, int npass, int first, int zero_init,

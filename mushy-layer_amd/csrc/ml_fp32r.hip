@@ -1100,7 +1100,7 @@ struct LinSweep {
 template <int MODE>
 __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
   if (A.skip && *A.skip) return;
-  Sweep3Pos P;
+  Sweep3Pos<false> P;
   if (!sweep3_pos(A.S, P)) return;
   if constexpr (MODE == 2) {
 #pragma unroll
@@ -1112,7 +1112,7 @@ __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
       for (int n = 0; n < 2; ++n) {
         ProlongCorners<float, 3> C;
         prolong_fetch<float, 3>(gc, i, P.j, P.k, A.pc + n * gc.ncell, C);
-        put32(A.out + n * A.ncell, q, prolong_combine<float, 3>(C, A.zero ? 0.0f : at32(A.in + n * A.ncell, q)));
+        put_at(A.out + n * A.ncell, q, prolong_combine<float, 3>(C, A.zero ? 0.0f : get_at(A.in + n * A.ncell, q)));
       }
     }
   } else {
@@ -1120,7 +1120,7 @@ __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
     const bool zero = MODE == 1 && A.zero;
     if (MODE == 1 && P.oth) {
 #pragma unroll
-      for (int n = 0; n < 2; ++n) put32(A.out + n * A.ncell, P.qo, zero ? 0.0f : at32(in + n * A.ncell, P.qo));
+      for (int n = 0; n < 2; ++n) put_at(A.out + n * A.ncell, P.qo, zero ? 0.0f : get_at(in + n * A.ncell, P.qo));
     }
     if (!P.act) return;
     float e[2][7], M[4][7];
@@ -1128,9 +1128,9 @@ __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
     for (int m = 0; m < 7; ++m) {
       const unsigned q = m == 0 ? P.q : P.nb[(m - 1) ^ 1];
 #pragma unroll
-      for (int n = 0; n < 2; ++n) e[n][m] = zero ? 0.0f : at32(in + n * A.ncell, q);
+      for (int n = 0; n < 2; ++n) e[n][m] = zero ? 0.0f : get_at(in + n * A.ncell, q);
 #pragma unroll
-      for (int n = 0; n < 4; ++n) M[n][m] = at32(A.M + n * A.ncell, q);
+      for (int n = 0; n < 4; ++n) M[n][m] = get_at(A.M + n * A.ncell, q);
     }
     CellFaces<float, 3> F;
     float aq[2], rr[2];
@@ -1139,8 +1139,8 @@ __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
 #pragma unroll
       for (int d = 0; d < 3; ++d)
         sweep3_faces(A.S, P, d, A.b[d] + n * A.nface[d], F.v[n][2 * d], F.v[n][2 * d + 1]);
-      rr[n] = at32(A.r + n * A.ncell, P.q);
-      aq[n] = A.a ? at32(A.a + n * A.ncell, P.q) : 1.0f;
+      rr[n] = get_at(A.r + n * A.ncell, P.q);
+      aq[n] = A.a ? get_at(A.a + n * A.ncell, P.q) : 1.0f;
     }
     float u[2][7];
 #pragma unroll
@@ -1160,8 +1160,8 @@ __global__ __launch_bounds__(256) void lin_sweep3_kernel(LinSweep A, Geom gc) {
     block_inverse<float, 3>(F, aq, Mc, A.alpha, A.beta, A.dxinv, inv);
     float e0 = e[0][0], e1 = e[1][0];
     block_step<float, 3>(F, aq, rr, inv, A.alpha, A.beta, A.dxinv, u[0], u[1], e0, e1);
-    put32(A.out, P.q, e0);
-    put32(A.out + A.ncell, P.q, e1);
+    put_at(A.out, P.q, e0);
+    put_at(A.out + A.ncell, P.q, e1);
   }
 }
 
@@ -1207,7 +1207,7 @@ hipError_t lin_relax_sweeps(const LinLevel<float>& L, float* const ebuf[2], int*
 hipError_t lin_relax_impl(const LinLevel<float>& L, float* const ebuf[2], int* cur, const BCDesc& bc, float alpha,
                           float beta, int npass, bool zero_init, const Geom* gc, const float* pc,
                           const LinLevel<float>* C, hipStream_t s) {
-  if (!C && npass > 0 && sweep3_ok(L.g))
+  if (!C && npass > 0 && sweep3_plain(L.g))
     return lin_relax_sweeps(L, ebuf, cur, bc, alpha, beta, npass, zero_init, gc, pc, s);
   int ntx, nty;
   const Geom gcc = gc ? *gc : L.g;

@@ -69,155 +69,12 @@ __device__ inline void tile_diffused_var(const HCArgs<T>& A, const Tile<DIM, TX,
 }
 
 // ---------------------------------------------------------------------------
-// Red/black relaxation of one tile: `npass` colour passes with halo npass
-// staged in LDS (levelGSRB, src/AMRNonLinearMultiCompOp.cpp:815-949, and
-// NONLINEARSMOOTHING, src/AMRNonLinearMultiCompOpF.ChF:125-195: phi_l of
-// every cell as of the start of the pass, frozen within it).  Each thread
-// owns fixed LDS positions whose classification is computed once; a wall
-// ghost's derived value comes from its interior neighbour's state.  When
-// io.pc is set, the staged state first receives the linear prolongation of
-// the coarse correction pc - pc0 (prolongIncrement fused with the
-// post-smoother).  Input and output arrays are distinct.
-// 3D levels with an odd periodic length (two cells of a colour meet at the
-// seam) or beyond 32-bit offsets; other levels have faster forms.
-template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
-__global__ __launch_bounds__(NT) void hc_relax_tile_kernel(HCArgs<T> A, TileIO<T> io) {
-  if (A.skip && *A.skip) return;
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  constexpr int EMAX = (TX + 2 * HMAX) * (TY + 2 * HMAX) * (DIM == 3 ? TZ + 2 * HMAX : 1);
-  constexpr int KMAX = (EMAX + NT - 1) / NT;
-  const Geom& g = A.g;
-  Tile<DIM, TX, TY, TZ> t;
-  t.init(io.npass, io.ntx, io.nty);
-  const int E = t.E;
-  T* sphi = reinterpret_cast<T*>(smem_raw);
-  T* sphl = sphi + 2 * E;
-  const T dxinv = T(1) / (T(g.dx) * T(g.dx));
-  const T scale = dxinv;
-  const Geom gc = io.gc;
-
-  PosRec R[KMAX];
-#pragma unroll
-  for (int kk = 0; kk < KMAX; ++kk) {
-    pos_record<DIM, TX, TY, TZ>(g, t, threadIdx.x + kk * NT, R[kk]);
-  }
-
-  // stage (H, Theta), with the prolonged coarse correction when requested
-#pragma unroll
-  for (int kk = 0; kk < KMAX; ++kk) {
-    const PosRec& r = R[kk];
-    if (r.kind != 1) continue;
-    T h = io.phi[r.q], c = io.phi[r.q + g.ncell];
-    if (io.pc) {
-      h = prolong_value<T, DIM>(gc, r.i, r.j, r.k, io.pc, io.pc0, h);
-      c = prolong_value<T, DIM>(gc, r.i, r.j, r.k, io.pc + gc.ncell, io.pc0 ? io.pc0 + gc.ncell : nullptr, c);
-    }
-    sphi[r.e] = h;
-    sphi[E + r.e] = c;
-  }
-  __syncthreads();
-
-  // closure of every staged cell and wall ghost (computeDiffusedVar,
-  // src/AMRNonLinearMultiCompOp.cpp:57-98); ghosts from their interior
-  // neighbour
-#pragma unroll
-  for (int kk = 0; kk < KMAX; ++kk) {
-    const PosRec& r = R[kk];
-    if (r.kind == 0) continue;
-    const int es = r.kind == 1 ? r.e : r.eint;
-    T th, cl;
-    closure<T>(sphi[es], sphi[E + es], A.cp, th, cl);
-    if (r.kind == 2 && A.bc.apply) {
-      const int isign = r.gs == 0 ? -1 : 1;
-      th = bc_ghost<T>(A.bc.type[r.gd][r.gs][0], T(A.bc.val[r.gd][r.gs][0]), th, isign, T(g.dx));
-      cl = bc_ghost<T>(A.bc.type[r.gd][r.gs][1], T(A.bc.val[r.gd][r.gs][1]), cl, isign, T(g.dx));
-    }
-    sphl[r.e] = th;
-    sphl[E + r.e] = cl;
-  }
-  __syncthreads();
-
-  // Each pass updates one colour and recomputes the closure of exactly the
-  // cells it updated (and of their wall ghosts): the other colour's phi_l is
-  // unchanged, and in this pass a cell reads only its own and the other
-  // colour's phi_l, so one barrier per pass suffices.
-  // operator data of every position this thread may update, in registers
-  CellFaces<T, DIM> F[KMAX];
-  T rr[KMAX][2], aa[KMAX][2], lam[KMAX][2];
-#pragma unroll
-  for (int kk = 0; kk < KMAX; ++kk) {
-    const PosRec& r = R[kk];
-    if (r.kind != 1 || r.dist > t.H - 1) continue;
-    load_faces<T, DIM>(A, r.i, r.j, r.k, F[kk]);
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      rr[kk][n] = io.rhs[r.q + n * g.ncell];
-      aa[kk][n] = A.a ? A.a[r.q + n * g.ncell] : T(1);
-      lam[kk][n] = lambda_of<T, DIM>(F[kk], n, aa[kk][n], A.alpha, A.beta, scale);
-    }
-  }
-  for (int p = 0; p < io.npass; ++p) {
-    const int gext = t.H - p;
-    const int colour = (io.first + p) & 1;
-#pragma unroll
-    for (int kk = 0; kk < KMAX; ++kk) {
-      const PosRec& r = R[kk];
-      if (!(r.kind == 1 && r.dist <= gext - 1 && !((r.i + r.j + r.k + colour) & 1))) continue;
-      const int e = r.e;
-      T nv[2];
-#pragma unroll
-      for (int n = 0; n < 2; ++n) {
-        T st[7];
-        gather_lds<T, DIM>(sphl + n * E, e, t.EX, t.EXY, st);
-        const T ph = sphi[n * E + e];
-        const T lof = lof_of<T, DIM>(F[kk], n, st, aa[kk][n], ph, A.alpha, A.beta, dxinv);
-        nv[n] = ph - lam[kk][n] * (lof - rr[kk][n]);
-      }
-      sphi[e] = nv[0];
-      sphi[E + e] = nv[1];
-      // after the last pass only the state is written out
-      if (p == io.npass - 1) continue;
-      T th, cl;
-      closure<T>(nv[0], nv[1], A.cp, th, cl);
-      sphl[e] = th;
-      sphl[E + e] = cl;
-      // wall ghosts of this cell (it is their interior neighbour)
-      const int iv[3] = {r.i, r.j, r.k};
-#pragma unroll
-      for (int d = 0; d < DIM; ++d) {
-        if (g.periodic[d]) continue;
-        const int stride = d == 0 ? 1 : (d == 1 ? t.EX : t.EXY);
-#pragma unroll
-        for (int sd = 0; sd < 2; ++sd) {
-          if (iv[d] != (sd ? g.n[d] - 1 : 0)) continue;
-          const int ge = sd ? e + stride : e - stride;
-          T gth = th, gcl = cl;
-          if (A.bc.apply) {
-            const int isign = sd ? 1 : -1;
-            gth = bc_ghost<T>(A.bc.type[d][sd][0], T(A.bc.val[d][sd][0]), th, isign, T(g.dx));
-            gcl = bc_ghost<T>(A.bc.type[d][sd][1], T(A.bc.val[d][sd][1]), cl, isign, T(g.dx));
-          }
-          sphl[ge] = gth;
-          sphl[E + ge] = gcl;
-        }
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int kk = 0; kk < KMAX; ++kk) {
-    const PosRec& r = R[kk];
-    if (!r.owner) continue;
-    io.phi_out[r.q] = sphi[r.e];
-    io.phi_out[r.q + g.ncell] = sphi[E + r.e];
-  }
-}
-
-// ---------------------------------------------------------------------------
 // 2D red/black relaxation over regions of 32 x 32 positions: the core of
 // 32 - 2H cells a side that the workgroup owns and a halo of H cells (H = the
-// colour passes, one more where a result of the relaxed state follows).  The
-// passes and values are those of hc_relax_tile_kernel.
+// colour passes, one more where a result of the relaxed state follows).  A
+// pass updates one colour from the closure as of its start, frozen within it
+// (levelGSRB, src/AMRNonLinearMultiCompOp.cpp:815-949, and NONLINEARSMOOTHING,
+// src/AMRNonLinearMultiCompOpF.ChF:125-195).
 //
 // A pass is bound by its chain of some 170 FP64 instructions (stencil and
 // closure), so no lane may idle in it: each of the 512 threads holds the two
@@ -1516,13 +1373,7 @@ static hipError_t launch_tile(const HCArgs<T>& A, TileIO<T> io, hipStream_t s) {
 // the halo's work counts, take one sweep (core 28^2).
 constexpr long long kDeepHaloCells = 512 * 512;
 
-static int relax_passes_per_launch(const Geom& g) { return g.dim == 2 && g.nvalid() <= kDeepHaloCells ? 8 : 2; }
-
-// tiles of the 3D relaxation launch (measured best of 5 shapes at 128^3;
-// the others spill registers)
-struct HCRelaxTile3 {
-  static constexpr int TX = 16, TY = 8, TZ = 4, NT = 512;
-};
+static int relax_passes_per_launch(const Geom& g) { return g.nvalid() <= kDeepHaloCells ? 8 : 2; }
 
 // algorithmic bytes of a relaxation launch: state (2 comps) in and out, rhs,
 // a, faces (2 comps) once each; the coarse state (and its initial copy) when
@@ -1603,36 +1454,15 @@ static hipError_t launch_relax_pair(const HCArgs<T>& A, const TileIO<T>& io, hip
   return err;
 }
 
-template <typename T>
-static hipError_t launch_relax_tile3(const HCArgs<T>& A, TileIO<T> io, hipStream_t s, const LaunchTimer* tm) {
-  using D3 = HCRelaxTile3;
-  if (io.npass < 1 || io.npass > 2) return hipErrorInvalidValue;
-  io.ntx = (A.g.n[0] + D3::TX - 1) / D3::TX;
-  io.nty = (A.g.n[1] + D3::TY - 1) / D3::TY;
-  const int nt = io.ntx * io.nty * ((A.g.n[2] + D3::TZ - 1) / D3::TZ);
-  const size_t lds = 4 * size_t(D3::TX + 2 * io.npass) * (D3::TY + 2 * io.npass) * (D3::TZ + 2 * io.npass) * sizeof(T);
-  if (lds > kMaxLds) return hipErrorInvalidValue;
-  const bool timed = tm && *tm->n < tm->cap;
-  if (tm && !timed) ++*tm->missed;
-  hipExtLaunchKernelGGL((hc_relax_tile_kernel<T, 3, D3::TX, D3::TY, D3::TZ, 2, D3::NT>), dim3(nt), dim3(D3::NT), lds,
-                        s, timed ? tm->start[*tm->n] : nullptr, timed ? tm->stop[*tm->n] : nullptr, 0, A, io);
-  const hipError_t err = hipGetLastError();
-  if (err == hipSuccess && timed) {
-    *tm->bytes += relax_bytes(A, io);
-    ++*tm->n;
-  }
-  return err;
-}
-
 // One colour pass of a 3D level straight from memory (Sweep3).  The closure
 // of the neighbours is worked out again by every cell that reads it: 3.5 of
 // them per cell and pass, some 3 us of the chip's FP64 units at 96 x 64 x 48,
 // against tiles that stage 3.75 positions per cell and leave half their lanes
 // idle in a pass.  MODE 0: in place on `out`; 1: from `in`, every cell written
-// to `out`; 2: no pass, `out` = `in` + prolonged pc - pc0.  Two passes: 69 us
-// at 128^3 (a march along z with planes in LDS: 161), 17.6 at 96 x 64 x 48
-// (tiles: 50.9), 12 from 48 x 32 x 24 down to 16^3 (tiles: 17), so every 3D
-// level takes it that may.
+// to `out` (every pass of the GEN form); 2: no pass, `out` = `in` + prolonged
+// pc - pc0.  Two passes: 69 us at 128^3 (a march along z with planes in LDS:
+// 161), 17.6 at 96 x 64 x 48 (tiles: 50.9), 12 from 48 x 32 x 24 down to 16^3
+// (tiles: 17); GEN 89 us at 129 x 128 x 128, 20 at 97 x 64 x 48.
 template <typename T>
 struct HCSweep {
   Sweep3 S;
@@ -1648,37 +1478,37 @@ struct HCSweep {
   T alpha, beta, dxinv, gs[3][2][2], gb[3][2][2];
   ClosureP<T> cp;
 };
-template <typename T, int MODE>
+template <typename T, int MODE, bool GEN>
 __global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T> A, Geom gc) {
   if (A.skip && *A.skip) return;
-  Sweep3Pos P;
+  Sweep3Pos<GEN> P;
   if (!sweep3_pos(A.S, P)) return;
   if constexpr (MODE == 2) {
 #pragma unroll
     for (int m = 0; m < 2; ++m) {
       if (!(m ? P.oth : P.act)) continue;
-      const unsigned q = m ? P.qo : P.q;
+      const auto q = m ? P.qo : P.q;
       const int i = m ? P.i + 1 - 2 * P.par : P.i;
 #pragma unroll
       for (int n = 0; n < 2; ++n)
-        put32(A.out + n * A.ncell, q,
+        put_at(A.out + n * A.ncell, q,
               prolong_value<T, 3>(gc, i, P.j, P.k, A.pc + n * gc.ncell, A.pc0 ? A.pc0 + n * gc.ncell : nullptr,
-                                  at32(A.in + n * A.ncell, q)));
+                                  get_at(A.in + n * A.ncell, q)));
     }
   } else {
     const T* in = MODE == 1 ? A.in : A.out;
     if (MODE == 1 && P.oth) {
-      put32(A.out, P.qo, at32(in, P.qo));
-      put32(A.out + A.ncell, P.qo, at32(in + A.ncell, P.qo));
+      put_at(A.out, P.qo, get_at(in, P.qo));
+      put_at(A.out + A.ncell, P.qo, get_at(in + A.ncell, P.qo));
     }
     if (!P.act) return;
     T h[7], c[7];
-    h[0] = at32(in, P.q);
-    c[0] = at32(in + A.ncell, P.q);
+    h[0] = get_at(in, P.q);
+    c[0] = get_at(in + A.ncell, P.q);
 #pragma unroll
     for (int f = 0; f < 6; ++f) {
-      h[1 + (f ^ 1)] = at32(in, P.nb[f]);
-      c[1 + (f ^ 1)] = at32(in + A.ncell, P.nb[f]);
+      h[1 + (f ^ 1)] = get_at(in, P.nb[f]);
+      c[1 + (f ^ 1)] = get_at(in + A.ncell, P.nb[f]);
     }
     CellFaces<T, 3> F;
     T aq[2], rr[2];
@@ -1687,8 +1517,8 @@ __global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T> A, Geom gc) {
 #pragma unroll
       for (int d = 0; d < 3; ++d)
         sweep3_faces(A.S, P, d, A.b[d] + n * A.nface[d], F.v[n][2 * d], F.v[n][2 * d + 1]);
-      rr[n] = at32(A.rhs + n * A.ncell, P.q);
-      aq[n] = A.a ? at32(A.a + n * A.ncell, P.q) : T(1);
+      rr[n] = get_at(A.rhs + n * A.ncell, P.q);
+      aq[n] = A.a ? get_at(A.a + n * A.ncell, P.q) : T(1);
     }
     T st[2][7];
 #pragma unroll
@@ -1706,22 +1536,21 @@ __global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T> A, Geom gc) {
       const T ph = n ? c[0] : h[0];
       const T lam = lambda_of<T, 3>(F, n, aq[n], A.alpha, A.beta, A.dxinv);
       const T lof = lof_of<T, 3>(F, n, st[n], aq[n], ph, A.alpha, A.beta, A.dxinv);
-      put32(A.out + n * A.ncell, P.q, ph - lam * (lof - rr[n]));
+      put_at(A.out + n * A.ncell, P.q, ph - lam * (lof - rr[n]));
     }
   }
 }
 
 // npass >= 1 colour passes of a 3D level: the prolongation, or the first
-// pass, from buf[*cur] to the other buffer, the others in place there
-template <typename T>
+// pass, from buf[*cur] to the other buffer, the others in place there (GEN:
+// each on to the other buffer)
+template <typename T, bool GEN>
 hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                            const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm) {
   const Geom& g = A.g;
   HCSweep<T> V{};
   V.S = sweep3_make(g);
   V.skip = A.skip;
-  V.in = buf[*cur];
-  V.out = buf[1 - *cur];
   V.rhs = rhs;
   V.a = A.a;
   V.pc = pc;
@@ -1748,7 +1577,10 @@ hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const 
     V.S.colour = (first + p) & 1;
     const bool timed = p >= 0 && tm && *tm->n < tm->cap;
     if (p >= 0 && tm && !timed) ++*tm->missed;
-    auto kern = p < 0 ? hc_sweep3_kernel<T, 2> : (p == 0 && !pc ? hc_sweep3_kernel<T, 1> : hc_sweep3_kernel<T, 0>);
+    const bool moves = GEN || p < 0 || (p == 0 && !pc);
+    V.in = buf[*cur];
+    V.out = buf[moves ? 1 - *cur : *cur];
+    auto kern = p < 0 ? hc_sweep3_kernel<T, 2, GEN> : (moves ? hc_sweep3_kernel<T, 1, GEN> : hc_sweep3_kernel<T, 0, false>);
     hipExtLaunchKernelGGL(kern, dim3(8 * V.S.chunk), dim3(256), 0, s, timed ? tm->start[*tm->n] : nullptr,
                           timed ? tm->stop[*tm->n] : nullptr, 0, V, gcc);
     const hipError_t e = hipGetLastError();
@@ -1757,11 +1589,11 @@ hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const 
       // both components: every state read, rhs and a of the colour, every
       // face; the colour written (a first pass: every cell)
       const double cells = double(g.nvalid());
-      *tm->bytes += (2 * cells + cells * (1 + (A.a ? 1 : 0)) + 2 * faces + (p == 0 && !pc ? 2 : 1) * cells) * sizeof(T);
+      *tm->bytes += (2 * cells + cells * (1 + (A.a ? 1 : 0)) + 2 * faces + (moves ? 2 : 1) * cells) * sizeof(T);
       ++*tm->n;
     }
+    if (moves) *cur = 1 - *cur;
   }
-  *cur = 1 - *cur;
   return hipSuccess;
 }
 
@@ -1847,8 +1679,9 @@ hipError_t hc_relax_stream(const HCArgs<T>& A, T* const buf[2], int* cur, const 
 template <typename T>
 hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                           const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm) {
-  if (npass > 0 && sweep3_ok(A.g))
-    return hc_relax_sweeps<T>(A, buf, cur, rhs, npass, first, gc, pc, pc0, s, tm);
+  if (npass > 0 && A.g.dim == 3)
+    return sweep3_plain(A.g) ? hc_relax_sweeps<T, false>(A, buf, cur, rhs, npass, first, gc, pc, pc0, s, tm)
+                             : hc_relax_sweeps<T, true>(A, buf, cur, rhs, npass, first, gc, pc, pc0, s, tm);
   // plain relaxations of large levels stream along the last direction
   if (!pc && npass > 0 && hc_streams(A.g)) return hc_relax_stream<T>(A, buf, cur, rhs, npass, first, s, tm);
   const int pmax = relax_passes_per_launch(A.g);
@@ -1865,7 +1698,7 @@ hipError_t hc_relax_tiles(const HCArgs<T>& A, T* const buf[2], int* cur, const T
       io.pc = pc;
       io.pc0 = pc0;
     }
-    hipError_t e = A.g.dim == 2 ? launch_relax_pair<T, RB_PLAIN>(A, io, s, tm) : launch_relax_tile3<T>(A, io, s, tm);
+    const hipError_t e = launch_relax_pair<T, RB_PLAIN>(A, io, s, tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += io.npass;

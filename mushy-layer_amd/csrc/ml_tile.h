@@ -4,6 +4,8 @@
 // L(phi) bracket of the reference's Fortran stencils.
 #pragma once
 
+#include <type_traits>
+
 #include "ml_common.h"
 #include "ml_kernels.h"
 
@@ -352,17 +354,23 @@ __device__ inline void spos_init(const Geom& g, int x0, int e, SPos& s) {
 // which has the colour: every lane works, and rows are read and written
 // whole.  Blocks of 2^lpx pairs by 256 >> lpx rows; the blocks of one L2
 // (workgroups go round the 8 of them) are neighbours in the level.
-// Byte offsets within one component are 32-bit (sweep3_ok).
+// Byte offsets within one component are 32-bit.
+//
+// GEN: any 3D level.  At the seam of an odd periodic length two cells of a
+// colour are neighbours, and each has to see the other as of the start of the
+// pass: so every pass goes from one buffer to the other (a row's pairs still
+// hold one cell of each colour).  Offsets are 64-bit.
 struct Sweep3 {
   int n[3], per[3];
-  unsigned sy, sz, fx[3], fxy[3];   // cell and face strides (row, plane)
+  long long sy, sz, fx[3], fxy[3];   // cell and face strides (row, plane)
   int lpx, nbx, nby, nblocks, chunk, colour;
 };
 
-inline bool sweep3_ok(const Geom& g) {
+// whether level g needs no GEN
+inline bool sweep3_plain(const Geom& g) {
   long long most = g.ncell;
   for (int d = 0; d < 3; ++d) {
-    if (g.periodic[d] && (g.n[d] & 1)) return false;   // (the ends of a row would share a colour)
+    if (g.periodic[d] && (g.n[d] & 1)) return false;
     most = most > g.nface[d] ? most : g.nface[d];
   }
   return g.dim == 3 && most < (1LL << 29);
@@ -373,11 +381,11 @@ inline Sweep3 sweep3_make(const Geom& g) {
   for (int d = 0; d < 3; ++d) {
     S.n[d] = g.n[d];
     S.per[d] = g.periodic[d];
-    S.fx[d] = unsigned(g.fn[d][0]);
-    S.fxy[d] = unsigned(g.fn[d][0] * g.fn[d][1]);
+    S.fx[d] = g.fn[d][0];
+    S.fxy[d] = g.fn[d][0] * g.fn[d][1];
   }
-  S.sy = unsigned(g.sy);
-  S.sz = unsigned(g.sz);
+  S.sy = g.sy;
+  S.sz = g.sz;
   const int pairs = (g.n[0] + 1) / 2;
   // the widest row of a block, up to 64 pairs, that leaves the fewest lanes idle
   auto blocks = [&](int l) { return ((pairs + (1 << l) - 1) >> l) * ((g.n[1] + (256 >> l) - 1) / (256 >> l)); };
@@ -391,15 +399,19 @@ inline Sweep3 sweep3_make(const Geom& g) {
   return S;
 }
 
+template <bool GEN>
 struct Sweep3Pos {
+  using Off = typename std::conditional<GEN, unsigned long long, unsigned>::type;
   int i, j, k, par;
   bool act, oth;       // the pair's cell of the colour, its other cell: in the level
-  unsigned q, qo;      // ... their indices
-  unsigned nb[6];      // neighbours of the cell of the colour (-x, +x, ...), itself beyond a wall
+  Off q, qo;           // ... their indices
+  Off nb[6];           // neighbours of the cell of the colour (-x, +x, ...), itself beyond a wall
   unsigned wall;       // bit f: neighbour f is a wall's ghost
 };
 
-__device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos& P) {
+template <bool GEN>
+__device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos<GEN>& P) {
+  using Off = typename Sweep3Pos<GEN>::Off;
   const int l = int(blockIdx.x & 7u) * S.chunk + int(blockIdx.x >> 3);
   if (l >= S.nblocks || int(blockIdx.x >> 3) >= S.chunk) return false;
   const int bx = l % S.nbx, r = l / S.nbx, by = r % S.nby;
@@ -411,15 +423,15 @@ __device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos& P) {
   P.i = 2 * s + P.par;
   P.act = P.i < S.n[0];
   P.oth = 2 * s + 1 - P.par < S.n[0];
-  const unsigned row = S.sy * unsigned(P.j + 1) + S.sz * unsigned(P.k + 1);
-  P.q = row + unsigned(P.i + 1);
-  P.qo = row + unsigned(2 * s + 2 - P.par);
+  const Off row = Off(S.sy) * Off(P.j + 1) + Off(S.sz) * Off(P.k + 1);
+  P.q = row + Off(P.i + 1);
+  P.qo = row + Off(2 * s + 2 - P.par);
   P.wall = 0;
   const int iv[3] = {P.i, P.j, P.k};
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const unsigned st = d == 0 ? 1u : (d == 1 ? S.sy : S.sz);
-    const unsigned span = st * unsigned(S.n[d] - 1);
+    const Off st = d == 0 ? Off(1) : (d == 1 ? Off(S.sy) : Off(S.sz));
+    const Off span = st * Off(S.n[d] - 1);
     const bool lo = iv[d] == 0, hi = iv[d] == S.n[d] - 1;
     P.nb[2 * d] = lo ? (S.per[d] ? P.q + span : P.q) : P.q - st;
     P.nb[2 * d + 1] = hi ? (S.per[d] ? P.q - span : P.q) : P.q + st;
@@ -428,21 +440,22 @@ __device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos& P) {
   return true;
 }
 
-// element i (32-bit byte offset) of p
-template <typename T>
-__device__ __forceinline__ T at32(const T* p, unsigned i) {
-  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + i * unsigned(sizeof(T)));
+// element i of p
+template <typename T, typename Off>
+__device__ __forceinline__ T get_at(const T* p, Off i) {
+  return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + i * Off(sizeof(T)));
 }
-template <typename T>
-__device__ __forceinline__ void put32(T* p, unsigned i, T v) {
-  *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + i * unsigned(sizeof(T))) = v;
+template <typename T, typename Off>
+__device__ __forceinline__ void put_at(T* p, Off i, T v) {
+  *reinterpret_cast<T*>(reinterpret_cast<char*>(p) + i * Off(sizeof(T))) = v;
 }
 // the six faces of the cell, component array b
-template <typename T>
-__device__ __forceinline__ void sweep3_faces(const Sweep3& S, const Sweep3Pos& P, int d, const T* b, T& lo, T& hi) {
-  const unsigned f = unsigned(P.i) + S.fx[d] * unsigned(P.j) + S.fxy[d] * unsigned(P.k);
-  lo = at32(b, f);
-  hi = at32(b, f + (d == 0 ? 1u : (d == 1 ? S.fx[1] : S.fxy[2])));
+template <typename T, bool GEN>
+__device__ __forceinline__ void sweep3_faces(const Sweep3& S, const Sweep3Pos<GEN>& P, int d, const T* b, T& lo, T& hi) {
+  using Off = typename Sweep3Pos<GEN>::Off;
+  const Off f = Off(P.i) + Off(S.fx[d]) * Off(P.j) + Off(S.fxy[d]) * Off(P.k);
+  lo = get_at(b, f);
+  hi = get_at(b, f + (d == 0 ? Off(1) : (d == 1 ? Off(S.fx[1]) : Off(S.fxy[2]))));
 }
 
 }  // namespace ml

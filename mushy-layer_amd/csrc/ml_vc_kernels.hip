@@ -1444,15 +1444,15 @@ struct VCSweep {
 template <typename T, bool FIRST>
 __global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
   if (A.skip && *A.skip) return;
-  Sweep3Pos P;
+  Sweep3Pos<false> P;
   if (!sweep3_pos(A.S, P)) return;
   auto val = [&](unsigned q, int i, int j, int k) __attribute__((always_inline)) {
-    if (!FIRST) return at32(A.out, q);
-    T v = A.zero ? T(0) : at32(A.in, q);
-    if (A.pc) v = v + at32(A.pc, unsigned((i >> 1) + 1) + A.csy * unsigned((j >> 1) + 1) + A.csz * unsigned((k >> 1) + 1));
+    if (!FIRST) return get_at(A.out, q);
+    T v = A.zero ? T(0) : get_at(A.in, q);
+    if (A.pc) v = v + get_at(A.pc, unsigned((i >> 1) + 1) + A.csy * unsigned((j >> 1) + 1) + A.csz * unsigned((k >> 1) + 1));
     return v;
   };
-  if (FIRST && P.oth) put32(A.out, P.qo, val(P.qo, P.i, P.j, P.k));   // (both cells of a pair have one coarse cell)
+  if (FIRST && P.oth) put_at(A.out, P.qo, val(P.qo, P.i, P.j, P.k));   // (both cells of a pair have one coarse cell)
   if (!P.act) return;
   T st[7];
   st[0] = val(P.q, P.i, P.j, P.k);
@@ -1470,7 +1470,7 @@ __global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
 #pragma unroll
   for (int d = 0; d < 3; ++d) sweep3_faces(A.S, P, d, A.b[d], F.v[2 * d], F.v[2 * d + 1]);
   const bool hasc = A.c != nullptr;
-  const T aq = A.a ? at32(A.a, P.q) : T(1), cq = hasc ? at32(A.c, P.q) : T(0), rr = at32(A.rhs, P.q);
+  const T aq = A.a ? get_at(A.a, P.q) : T(1), cq = hasc ? get_at(A.c, P.q) : T(0), rr = get_at(A.rhs, P.q);
   if (P.wall) {
 #pragma unroll
     for (int f = 0; f < 6; ++f)
@@ -1478,7 +1478,7 @@ __global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
   }
   const T lam = vc_lambda<T, 3>(F, aq, hasc, cq, A.alpha, A.beta, A.dxinv);
   const T lof = vc_lof<T, 3>(F, st, aq, hasc, cq, A.alpha, A.beta, A.dxinv);
-  put32(A.out, P.q, st[0] - lam * (lof - rr));
+  put_at(A.out, P.q, st[0] - lam * (lof - rr));
 }
 
 // npass >= 1 colour passes: the first from buf[*cur] to the other buffer,
@@ -1554,7 +1554,7 @@ template <typename T, int DIM>
 hipError_t vc_relax_dim(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                         const Geom* gc, const T* pc, hipStream_t s, const Geom* gr = nullptr, T* resc = nullptr,
                         const LaunchTimer* tm = nullptr, const VCFinal<T>* fin = nullptr) {
-  if (DIM == 3 && !resc && !fin && npass > 0 && sweep3_ok(A.g))
+  if (DIM == 3 && !resc && !fin && npass > 0 && sweep3_plain(A.g))
     return vc_relax_sweeps<T>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
   if constexpr (DIM == 2) {
     if (!resc && !fin && npass > 0 && vc_streams(A.g))

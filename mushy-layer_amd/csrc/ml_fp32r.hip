@@ -1084,7 +1084,7 @@ namespace {
 // pass, `out` = `in` + prolonged pc.  13.7 us a pass over the levels of a
 // 128^3 cycle (tiles with the halo of two passes: 47 us for two).
 struct LinSweep {
-  Sweep3 S;
+  Sweep3<false> S;
   const int* skip;
   const float* in;
   float* out;
@@ -1171,7 +1171,7 @@ hipError_t lin_relax_sweeps(const LinLevel<float>& L, float* const ebuf[2], int*
                             float beta, int npass, bool zero_init, const Geom* gc, const float* pc, hipStream_t s) {
   const Geom& g = L.g;
   LinSweep V{};
-  V.S = sweep3_make(g);
+  V.S = sweep3_make<false>(g);
   V.skip = L.skip;
   V.in = ebuf[*cur];
   V.out = ebuf[1 - *cur];

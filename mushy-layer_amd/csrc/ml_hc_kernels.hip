@@ -1463,9 +1463,9 @@ static hipError_t launch_relax_pair(const HCArgs<T>& A, const TileIO<T>& io, hip
 // pc - pc0.  Two passes: 69 us at 128^3 (a march along z with planes in LDS:
 // 161), 17.6 at 96 x 64 x 48 (tiles: 50.9), 12 from 48 x 32 x 24 down to 16^3
 // (tiles: 17); GEN 89 us at 129 x 128 x 128, 20 at 97 x 64 x 48.
-template <typename T>
+template <typename T, bool GEN>
 struct HCSweep {
-  Sweep3 S;
+  Sweep3<GEN> S;
   const int* skip;
   const T* in;
   T* out;
@@ -1479,7 +1479,7 @@ struct HCSweep {
   ClosureP<T> cp;
 };
 template <typename T, int MODE, bool GEN>
-__global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T> A, Geom gc) {
+__global__ __launch_bounds__(256) void hc_sweep3_kernel(HCSweep<T, GEN> A, Geom gc) {
   if (A.skip && *A.skip) return;
   Sweep3Pos<GEN> P;
   if (!sweep3_pos(A.S, P)) return;
@@ -1548,8 +1548,8 @@ template <typename T, bool GEN>
 hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                            const Geom* gc, const T* pc, const T* pc0, hipStream_t s, const LaunchTimer* tm) {
   const Geom& g = A.g;
-  HCSweep<T> V{};
-  V.S = sweep3_make(g);
+  HCSweep<T, GEN> V{};
+  V.S = sweep3_make<GEN>(g);
   V.skip = A.skip;
   V.rhs = rhs;
   V.a = A.a;
@@ -1580,7 +1580,7 @@ hipError_t hc_relax_sweeps(const HCArgs<T>& A, T* const buf[2], int* cur, const 
     const bool moves = GEN || p < 0 || (p == 0 && !pc);
     V.in = buf[*cur];
     V.out = buf[moves ? 1 - *cur : *cur];
-    auto kern = p < 0 ? hc_sweep3_kernel<T, 2, GEN> : (moves ? hc_sweep3_kernel<T, 1, GEN> : hc_sweep3_kernel<T, 0, false>);
+    auto kern = p < 0 ? hc_sweep3_kernel<T, 2, GEN> : (moves ? hc_sweep3_kernel<T, 1, GEN> : hc_sweep3_kernel<T, GEN ? 1 : 0, GEN>);
     hipExtLaunchKernelGGL(kern, dim3(8 * V.S.chunk), dim3(256), 0, s, timed ? tm->start[*tm->n] : nullptr,
                           timed ? tm->stop[*tm->n] : nullptr, 0, V, gcc);
     const hipError_t e = hipGetLastError();

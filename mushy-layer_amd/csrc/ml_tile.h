@@ -360,9 +360,11 @@ __device__ inline void spos_init(const Geom& g, int x0, int e, SPos& s) {
 // colour are neighbours, and each has to see the other as of the start of the
 // pass: so every pass goes from one buffer to the other (a row's pairs still
 // hold one cell of each colour).  Offsets are 64-bit.
+template <bool GEN>
 struct Sweep3 {
+  using Off = typename std::conditional<GEN, unsigned long long, unsigned>::type;
   int n[3], per[3];
-  long long sy, sz, fx[3], fxy[3];   // cell and face strides (row, plane)
+  Off sy, sz, fx[3], fxy[3];   // cell and face strides (row, plane)
   int lpx, nbx, nby, nblocks, chunk, colour;
 };
 
@@ -376,16 +378,18 @@ inline bool sweep3_plain(const Geom& g) {
   return g.dim == 3 && most < (1LL << 29);
 }
 
-inline Sweep3 sweep3_make(const Geom& g) {
-  Sweep3 S{};
+template <bool GEN>
+inline Sweep3<GEN> sweep3_make(const Geom& g) {
+  using Off = typename Sweep3<GEN>::Off;
+  Sweep3<GEN> S{};
   for (int d = 0; d < 3; ++d) {
     S.n[d] = g.n[d];
     S.per[d] = g.periodic[d];
-    S.fx[d] = g.fn[d][0];
-    S.fxy[d] = g.fn[d][0] * g.fn[d][1];
+    S.fx[d] = Off(g.fn[d][0]);
+    S.fxy[d] = Off(g.fn[d][0] * g.fn[d][1]);
   }
-  S.sy = g.sy;
-  S.sz = g.sz;
+  S.sy = Off(g.sy);
+  S.sz = Off(g.sz);
   const int pairs = (g.n[0] + 1) / 2;
   // the widest row of a block, up to 64 pairs, that leaves the fewest lanes idle
   auto blocks = [&](int l) { return ((pairs + (1 << l) - 1) >> l) * ((g.n[1] + (256 >> l) - 1) / (256 >> l)); };
@@ -401,7 +405,7 @@ inline Sweep3 sweep3_make(const Geom& g) {
 
 template <bool GEN>
 struct Sweep3Pos {
-  using Off = typename std::conditional<GEN, unsigned long long, unsigned>::type;
+  using Off = typename Sweep3<GEN>::Off;
   int i, j, k, par;
   bool act, oth;       // the pair's cell of the colour, its other cell: in the level
   Off q, qo;           // ... their indices
@@ -410,8 +414,8 @@ struct Sweep3Pos {
 };
 
 template <bool GEN>
-__device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos<GEN>& P) {
-  using Off = typename Sweep3Pos<GEN>::Off;
+__device__ __forceinline__ bool sweep3_pos(const Sweep3<GEN>& S, Sweep3Pos<GEN>& P) {
+  using Off = typename Sweep3<GEN>::Off;
   const int l = int(blockIdx.x & 7u) * S.chunk + int(blockIdx.x >> 3);
   if (l >= S.nblocks || int(blockIdx.x >> 3) >= S.chunk) return false;
   const int bx = l % S.nbx, r = l / S.nbx, by = r % S.nby;
@@ -423,14 +427,14 @@ __device__ __forceinline__ bool sweep3_pos(const Sweep3& S, Sweep3Pos<GEN>& P) {
   P.i = 2 * s + P.par;
   P.act = P.i < S.n[0];
   P.oth = 2 * s + 1 - P.par < S.n[0];
-  const Off row = Off(S.sy) * Off(P.j + 1) + Off(S.sz) * Off(P.k + 1);
+  const Off row = S.sy * Off(P.j + 1) + S.sz * Off(P.k + 1);
   P.q = row + Off(P.i + 1);
   P.qo = row + Off(2 * s + 2 - P.par);
   P.wall = 0;
   const int iv[3] = {P.i, P.j, P.k};
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const Off st = d == 0 ? Off(1) : (d == 1 ? Off(S.sy) : Off(S.sz));
+    const Off st = d == 0 ? Off(1) : (d == 1 ? S.sy : S.sz);
     const Off span = st * Off(S.n[d] - 1);
     const bool lo = iv[d] == 0, hi = iv[d] == S.n[d] - 1;
     P.nb[2 * d] = lo ? (S.per[d] ? P.q + span : P.q) : P.q - st;
@@ -451,11 +455,12 @@ __device__ __forceinline__ void put_at(T* p, Off i, T v) {
 }
 // the six faces of the cell, component array b
 template <typename T, bool GEN>
-__device__ __forceinline__ void sweep3_faces(const Sweep3& S, const Sweep3Pos<GEN>& P, int d, const T* b, T& lo, T& hi) {
-  using Off = typename Sweep3Pos<GEN>::Off;
-  const Off f = Off(P.i) + Off(S.fx[d]) * Off(P.j) + Off(S.fxy[d]) * Off(P.k);
+__device__ __forceinline__ void sweep3_faces(const Sweep3<GEN>& S, const Sweep3Pos<GEN>& P, int d, const T* b, T& lo,
+                                             T& hi) {
+  using Off = typename Sweep3<GEN>::Off;
+  const Off f = Off(P.i) + S.fx[d] * Off(P.j) + S.fxy[d] * Off(P.k);
   lo = get_at(b, f);
-  hi = get_at(b, f + (d == 0 ? Off(1) : (d == 1 ? Off(S.fx[1]) : Off(S.fxy[2]))));
+  hi = get_at(b, f + (d == 0 ? Off(1) : (d == 1 ? S.fx[1] : S.fxy[2])));
 }
 
 }  // namespace ml

@@ -83,8 +83,7 @@ __device__ inline T vc_lof(const Faces1<T, DIM>& F, const T* p, T aq, bool hasc,
 // homogeneous wall ghosts of the cells it updated, so one barrier per pass.
 // The body works on tile `tile` of the level (a batched launch maps its
 // workgroups to (instance, tile) pairs).
-// 3D plain relaxation comes here with an odd periodic length or beyond 32-bit
-// offsets only.
+// In 3D for the fused forms and batches only.
 template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
 __device__ __forceinline__ void vc_relax_tile_body(const VCArgs<T>& A, const T* __restrict__ in, T* __restrict__ out,
                                                    const T* __restrict__ rhs, int npass, int first, int zero_init,
@@ -1420,15 +1419,16 @@ GhostForm<T> vc_ghost_form(BCDesc bc, T dx) {
   return ghost_form<T>(bc, dx);
 }
 
-// One colour pass of a 3D level straight from memory (Sweep3).  FIRST: from
-// `in`, or zero, plus the coarse correction pc, every cell written to `out`;
-// otherwise in place on `out`.  Two passes with c: 37 us at 128^3 (98 bytes a
-// cell of required traffic: 5.6 TB/s; a march along z with a window of planes
-// in LDS was 71), 8.5 at 64^3 and 7.5 at 16^3 (16 x 8 x 4 tiles with the halo
-// of both passes: 15.1 and 8.0), so every 3D level takes it that may.
-template <typename T>
+// One colour pass of a 3D level straight from memory (Sweep3).  MOVE: from
+// `in`, or zero, plus the coarse correction pc, every cell written to `out`
+// (the first pass, and every pass of the GEN form); otherwise in place on
+// `out`.  Two passes with c: 37 us at 128^3 (98 bytes a cell of required
+// traffic: 5.6 TB/s; a march along z with a window of planes in LDS was 71),
+// 8.5 at 64^3 and 7.5 at 16^3 (16 x 8 x 4 tiles with the halo of both passes:
+// 15.1 and 8.0); GEN 50 at 129 x 128 x 128.
+template <typename T, bool GEN>
 struct VCSweep {
-  Sweep3 S;
+  Sweep3<GEN> S;
   const int* skip;
   const T* in;
   T* out;
@@ -1437,29 +1437,30 @@ struct VCSweep {
   const T* c;
   const T* b[3];
   const T* pc;
-  unsigned csy, csz;   // coarse cell strides
+  typename Sweep3<GEN>::Off csy, csz;   // coarse cell strides
   T alpha, beta, dxinv, gs[3][2], gb[3][2];
   int zero;
 };
-template <typename T, bool FIRST>
-__global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
+template <typename T, bool MOVE, bool GEN>
+__global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T, GEN> A) {
+  using Off = typename Sweep3<GEN>::Off;
   if (A.skip && *A.skip) return;
-  Sweep3Pos<false> P;
+  Sweep3Pos<GEN> P;
   if (!sweep3_pos(A.S, P)) return;
-  auto val = [&](unsigned q, int i, int j, int k) __attribute__((always_inline)) {
-    if (!FIRST) return get_at(A.out, q);
+  auto val = [&](Off q, int i, int j, int k) __attribute__((always_inline)) {
+    if (!MOVE) return get_at(A.out, q);
     T v = A.zero ? T(0) : get_at(A.in, q);
-    if (A.pc) v = v + get_at(A.pc, unsigned((i >> 1) + 1) + A.csy * unsigned((j >> 1) + 1) + A.csz * unsigned((k >> 1) + 1));
+    if (A.pc) v = v + get_at(A.pc, Off((i >> 1) + 1) + A.csy * Off((j >> 1) + 1) + A.csz * Off((k >> 1) + 1));
     return v;
   };
-  if (FIRST && P.oth) put_at(A.out, P.qo, val(P.qo, P.i, P.j, P.k));   // (both cells of a pair have one coarse cell)
+  if (MOVE && P.oth) put_at(A.out, P.qo, val(P.qo, P.i, P.j, P.k));   // (both cells of a pair have one coarse cell)
   if (!P.act) return;
   T st[7];
   st[0] = val(P.q, P.i, P.j, P.k);
 #pragma unroll
   for (int f = 0; f < 6; ++f) {
     int iv[3] = {P.i, P.j, P.k};
-    if (FIRST) {
+    if (MOVE) {
       const int d = f >> 1, n = A.S.n[d];
       iv[d] = f & 1 ? (iv[d] == n - 1 ? (A.S.per[d] ? 0 : iv[d]) : iv[d] + 1)
                     : (iv[d] == 0 ? (A.S.per[d] ? n - 1 : 0) : iv[d] - 1);
@@ -1482,29 +1483,26 @@ __global__ __launch_bounds__(256) void vc_sweep3_kernel(VCSweep<T> A) {
 }
 
 // npass >= 1 colour passes: the first from buf[*cur] to the other buffer,
-// the others in place there
-template <typename T>
+// the others in place there (GEN: each on to the other buffer)
+template <typename T, bool GEN>
 hipError_t vc_relax_sweeps(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                            const Geom* gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
   const Geom& g = A.g;
-  VCSweep<T> V{};
-  V.S = sweep3_make(g);
+  using Off = typename Sweep3<GEN>::Off;
+  VCSweep<T, GEN> V{};
+  V.S = sweep3_make<GEN>(g);
   V.skip = A.skip;
-  V.in = buf[*cur];
-  V.out = buf[1 - *cur];
   V.rhs = rhs;
   V.a = A.a;
   V.c = A.c;
   for (int d = 0; d < 3; ++d) V.b[d] = A.b[d];
-  V.pc = pc;
   if (gc) {
-    V.csy = unsigned(gc->sy);
-    V.csz = unsigned(gc->sz);
+    V.csy = Off(gc->sy);
+    V.csz = Off(gc->sz);
   }
   V.alpha = A.alpha;
   V.beta = A.beta;
   V.dxinv = T(1) / (T(g.dx) * T(g.dx));
-  V.zero = zero_init ? 1 : 0;
   const GhostForm<T> gf = vc_ghost_form<T>(A.bc, T(g.dx));
   for (int d = 0; d < 3; ++d)
     for (int sd = 0; sd < 2; ++sd) {
@@ -1517,22 +1515,27 @@ hipError_t vc_relax_sweeps(const VCArgs<T>& A, T* const buf[2], int* cur, const 
     V.S.colour = p & 1;
     const bool timed = tm && *tm->n < tm->cap;
     if (tm && !timed) ++*tm->missed;
-    auto kern = p == 0 ? vc_sweep3_kernel<T, true> : vc_sweep3_kernel<T, false>;
+    const bool moves = GEN || p == 0;
+    V.in = buf[*cur];
+    V.out = buf[moves ? 1 - *cur : *cur];
+    V.zero = p == 0 && zero_init ? 1 : 0;
+    V.pc = p == 0 ? pc : nullptr;
+    auto kern = moves ? vc_sweep3_kernel<T, true, GEN> : vc_sweep3_kernel<T, GEN, GEN>;
     hipExtLaunchKernelGGL(kern, dim3(8 * V.S.chunk), dim3(256), 0, s, timed ? tm->start[*tm->n] : nullptr,
                           timed ? tm->stop[*tm->n] : nullptr, 0, V);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (timed) {
       // state, rhs, a and c of the colour and the other colour's state once;
-      // every face; the colour written (the first pass: every cell)
+      // every face; the colour written (a pass that moves: every cell)
       const double cells = double(g.nvalid());
       const double b = cells * (p == 0 && zero_init ? 0 : 1) + (p == 0 && pc ? cells / 8 : 0) +
-                       0.5 * cells * (1 + (A.a ? 1 : 0) + (A.c ? 1 : 0)) + faces + (p == 0 ? 1.0 : 0.5) * cells;
+                       0.5 * cells * (1 + (A.a ? 1 : 0) + (A.c ? 1 : 0)) + faces + (moves ? 1.0 : 0.5) * cells;
       *tm->bytes += b * sizeof(T);
       ++*tm->n;
     }
+    if (moves) *cur = 1 - *cur;
   }
-  *cur = 1 - *cur;
   return hipSuccess;
 }
 
@@ -1554,8 +1557,9 @@ template <typename T, int DIM>
 hipError_t vc_relax_dim(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                         const Geom* gc, const T* pc, hipStream_t s, const Geom* gr = nullptr, T* resc = nullptr,
                         const LaunchTimer* tm = nullptr, const VCFinal<T>* fin = nullptr) {
-  if (DIM == 3 && !resc && !fin && npass > 0 && sweep3_plain(A.g))
-    return vc_relax_sweeps<T>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
+  if (DIM == 3 && !resc && !fin && npass > 0)
+    return sweep3_plain(A.g) ? vc_relax_sweeps<T, false>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm)
+                             : vc_relax_sweeps<T, true>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);
   if constexpr (DIM == 2) {
     if (!resc && !fin && npass > 0 && vc_streams(A.g))
       return vc_relax_stream<T>(A, buf, cur, rhs, npass, zero_init, gc, pc, s, tm);

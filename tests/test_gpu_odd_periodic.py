@@ -51,3 +51,57 @@ def test_hc_3d_solve(ml, gpu_ctx, wl):
     assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     assert HC.bitwise_equal(HC.valid(case["n"], dn.get()), HC.valid(case["n"], new))
     op.close()
+
+
+def _vc_case(ml, ctx, spec, acoef, ccoef):
+    n = spec["n"]
+    dim, per = len(n), spec.get("periodic", [1] + [0] * (len(n) - 1))
+    dx = 1.0 / max(n)
+    bc = {(d, s, 0): ((d + s) % 2, 0.0) for d in range(dim) if not per[d] for s in (0, 1)}
+    g = O.make_grid(n, dx, list(per) + [0] * (3 - dim))
+    rng = np.random.default_rng(sum(n))
+    b = [rng.uniform(0.5, 1.5, O.face_shape(g, d, 1)) for d in range(dim)]
+    a = rng.uniform(0.5, 1.5, O.cell_shape(g, 1)) if acoef else None
+    c = rng.uniform(0.0, 20.0, O.cell_shape(g, 1)) if ccoef else None
+    phi, rhs = np.zeros(O.cell_shape(g, 1)), np.zeros(O.cell_shape(g, 1))
+    O.valid(g, phi)[...] = rng.standard_normal(O.valid(g, phi).shape)
+    O.valid(g, rhs)[...] = rng.standard_normal(O.valid(g, rhs).shape)
+    op = ml.VCOp(ctx, list(n), dx, list(per), ml.make_bc(bc))
+    dev = lambda x: None if x is None else ml.DeviceArray(ctx, x.shape, host=x)
+    op.set_coefs(dev(a), [dev(x) for x in b], dev(c), 1.0, -2e-3)
+    return n, g, O.make_bc(bc), a, b, c, phi, rhs, op, dev
+
+
+def _vc_relax(ml, ctx, spec, iters, acoef, ccoef):
+    n, g, bc, a, b, c, phi, rhs, op, dev = _vc_case(ml, ctx, spec, acoef, ccoef)
+    ref = O.lin_gsrb(g, 1, bc, 1.0, a, -2e-3, c, b, phi.copy(), rhs, iters=iters)
+    d = dev(phi)
+    op.relax(0, d, dev(rhs), iters)
+    assert HC.bitwise_equal(np.ascontiguousarray(HC.valid(n, d.get())), np.ascontiguousarray(HC.valid(n, ref)))
+    op.close()
+
+
+def _vc_solve(ml, ctx, spec):
+    """A single level of more than 1024 cells, iterations replayed from a
+    graph: the solve is its bottom's relaxations."""
+    n, g, bc, a, b, c, phi, rhs, op, dev = _vc_case(ml, ctx, spec, False, True)
+    kw = dict(max_iter=5, bottom=7, eps=1e-14, hang=1e-14, norm_thresh=1e-14)
+    new = np.zeros_like(phi)
+    so = O.lin_mg_solve(g, 1, bc, 1.0, None, -2e-3, c, b, new, rhs, opts=O.default_opts(**kw))
+    drhs = dev(rhs)
+    for _ in range(2):
+        d = dev(np.zeros_like(phi))
+        st = op.solve(d, drhs, opts=ml.default_opts(**kw))
+        assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
+        assert HC.bitwise_equal(np.ascontiguousarray(HC.valid(n, d.get())), np.ascontiguousarray(HC.valid(n, new)))
+    op.close()
+
+
+@pytest.mark.parametrize("name", sorted(GRIDS3))
+@pytest.mark.parametrize("iters,acoef,ccoef", [(1, False, True), (4, True, False)])
+def test_vc_3d(ml, gpu_ctx, name, iters, acoef, ccoef):
+    _vc_relax(ml, gpu_ctx, GRIDS3[name], iters, acoef, ccoef)
+
+
+def test_vc_3d_solve(ml, gpu_ctx):
+    _vc_solve(ml, gpu_ctx, GRIDS3["y"])

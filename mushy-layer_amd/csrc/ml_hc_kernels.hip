@@ -1070,14 +1070,16 @@ __global__ void hc_diffused_var_kernel(HCArgs<T> A, const T* __restrict__ phi, T
 // (after the launch's last pass nothing reads it, so it is skipped there).
 // Per plane and position the face coefficients, rhs (and aCoef) stay in
 // registers in compile-time-indexed sets, loaded two planes ahead; lambda is
-// formed where it is used.  Every input is read once per launch.
+// formed where it is used.  Every input is read once per launch.  SEAM: the
+// rows are periodic with an odd length, so the two cells at their seam share a
+// colour and read each other as of the start of a pass.
 template <typename T>
 struct HCoef {
   CellFaces<T, 2> F;
   T rr[2], aq[2], v[2];   // rhs, aCoef, state as loaded
 };
 
-template <typename T, int TX, int P, int NT, bool HASA>
+template <typename T, int TX, int P, int NT, bool HASA, bool SEAM>
 __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const T* __restrict__ in,
                                                              T* __restrict__ out, const T* __restrict__ rhs,
                                                              int first, int nbx, int seg) {
@@ -1235,10 +1237,43 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
         T* pz = slot(z);
         const T* pm = slot(z - 1);
         const T* pp = slot(z + 1);
+        auto mine = [&](const SPos& s) __attribute__((always_inline)) {
+          return s.kind == 1 && s.dist <= reach && !((s.gx + zw + colour) & 1);
+        };
+        // an updated cell's closure and its wall ghosts: lateral, then along
+        // the march
+        auto refresh = [&](const SPos& s, int e, T h, T c) __attribute__((always_inline)) {
+          T th, clv;
+          closure<T>(h, c, A.cp, th, clv);
+          pz[2 * EL + e] = th;
+          pz[3 * EL + e] = clv;
+          if (!g.periodic[0]) {
+            if (s.gx == 0) {
+              pz[2 * EL + e - 1] = ghost(0, 0, 0, th);
+              pz[3 * EL + e - 1] = ghost(0, 0, 1, clv);
+            }
+            if (s.gx == g.n[0] - 1) {
+              pz[2 * EL + e + 1] = ghost(0, 1, 0, th);
+              pz[3 * EL + e + 1] = ghost(0, 1, 1, clv);
+            }
+          }
+          if (!zper) {
+            if (zw == 0) {
+              T* gp = slot(-1);
+              gp[2 * EL + e] = ghost(MD, 0, 0, th);
+              gp[3 * EL + e] = ghost(MD, 0, 1, clv);
+            }
+            if (zw == nz - 1) {
+              T* gp = slot(nz);
+              gp[2 * EL + e] = ghost(MD, 1, 0, th);
+              gp[3 * EL + e] = ghost(MD, 1, 1, clv);
+            }
+          }
+        };
 #pragma unroll
         for (int kk = 0; kk < K; ++kk) {
           const SPos& s = S[kk];
-          if (s.kind != 1 || s.dist > reach || ((s.gx + zw + colour) & 1)) continue;
+          if (!mine(s)) continue;
           const int e = threadIdx.x + kk * NT;
           const HCoef<T>& C = cs[jp][kk];
           T nv[2];
@@ -1261,33 +1296,14 @@ __global__ __launch_bounds__(NT) void hc_relax_stream_kernel(HCArgs<T> A, const 
           pz[EL + e] = nv[1];
           // the last pass's closure is never read: its cells' neighbours
           // (the other colour) are not updated again in this launch
-          if constexpr (p == P - 1) continue;
-          T th, clv;
-          closure<T>(nv[0], nv[1], A.cp, th, clv);
-          pz[2 * EL + e] = th;
-          pz[3 * EL + e] = clv;
-          // wall ghosts of this cell: lateral, then along the march
-          if (!g.periodic[0]) {
-            if (s.gx == 0) {
-              pz[2 * EL + e - 1] = ghost(0, 0, 0, th);
-              pz[3 * EL + e - 1] = ghost(0, 0, 1, clv);
-            }
-            if (s.gx == g.n[0] - 1) {
-              pz[2 * EL + e + 1] = ghost(0, 1, 0, th);
-              pz[3 * EL + e + 1] = ghost(0, 1, 1, clv);
-            }
-          }
-          if (!zper) {
-            if (zw == 0) {
-              T* gp = slot(-1);
-              gp[2 * EL + e] = ghost(MD, 0, 0, th);
-              gp[3 * EL + e] = ghost(MD, 0, 1, clv);
-            }
-            if (zw == nz - 1) {
-              T* gp = slot(nz);
-              gp[2 * EL + e] = ghost(MD, 1, 0, th);
-              gp[3 * EL + e] = ghost(MD, 1, 1, clv);
-            }
+          if constexpr (p < P - 1 && !SEAM) refresh(s, e, nv[0], nv[1]);
+        }
+        if constexpr (p < P - 1 && SEAM) {
+          __syncthreads();   // the two cells at the seam read each other's closure
+#pragma unroll
+          for (int kk = 0; kk < K; ++kk) {
+            const int e = threadIdx.x + kk * NT;
+            if (mine(S[kk])) refresh(S[kk], e, pz[e], pz[EL + e]);
           }
         }
       }
@@ -1603,16 +1619,19 @@ struct HCStream {
 };
 
 // 2D levels whose plain relaxations stream (above 512^2 cells), with 32-bit
-// offsets for both components of every array
+// offsets for both components of every array.  Not with an odd periodic
+// length along the march: the rows at its seam share colours, and a pass
+// reaches one of them before the other.
 constexpr long long kHCStreamCells2 = 512 * 512;
 inline bool hc_streams(const Geom& g) {
   long long nf = 0;
   for (int d = 0; d < g.dim; ++d) nf = nf > g.nface[d] ? nf : g.nface[d];
   const long long most = 2 * (g.ncell > nf ? g.ncell : nf);
-  return g.dim == 2 && g.nvalid() > kHCStreamCells2 && g.n[1] >= 8 && most < (1LL << 29);
+  return g.dim == 2 && g.nvalid() > kHCStreamCells2 && g.n[1] >= 8 && !(g.periodic[1] && (g.n[1] & 1)) &&
+         most < (1LL << 29);
 }
 
-template <typename T, int P, bool HASA>
+template <typename T, int P, bool HASA, bool SEAM>
 hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rhs, int first, hipStream_t s,
                             const LaunchTimer* tm) {
   using D = HCStream;
@@ -1620,7 +1639,7 @@ hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rh
   const Geom& g = A.g;
   const int nbx = (g.n[0] + TX - 1) / TX;
   const size_t lds = size_t(4) * 4 * EL * sizeof(T);
-  auto kern = hc_relax_stream_kernel<T, TX, P, D::NT, HASA>;
+  auto kern = hc_relax_stream_kernel<T, TX, P, D::NT, HASA, SEAM>;
   // segments sized so that the whole grid is resident at once
   static int resident = 0;
   if (!resident) {
@@ -1658,17 +1677,17 @@ hipError_t hc_stream_launch(const HCArgs<T>& A, const T* in, T* out, const T* rh
 template <typename T>
 hipError_t hc_relax_stream(const HCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, int first,
                            hipStream_t s, const LaunchTimer* tm) {
+  const bool seam = A.g.periodic[0] && (A.g.n[0] & 1);
   int done = 0;
   while (done < npass) {
     const int p = (npass - done) >= 2 ? 2 : 1;
     const int f = (first + done) & 1;
-    hipError_t e;
-    if (A.a)
-      e = p == 2 ? hc_stream_launch<T, 2, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
-                 : hc_stream_launch<T, 1, true>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
-    else
-      e = p == 2 ? hc_stream_launch<T, 2, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm)
-                 : hc_stream_launch<T, 1, false>(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
+    // (a single pass refreshes no closure, so it has no use for SEAM)
+    auto launch = A.a ? (p == 1 ? hc_stream_launch<T, 1, true, false>
+                                : (seam ? hc_stream_launch<T, 2, true, true> : hc_stream_launch<T, 2, true, false>))
+                      : (p == 1 ? hc_stream_launch<T, 1, false, false>
+                                : (seam ? hc_stream_launch<T, 2, false, true> : hc_stream_launch<T, 2, false, false>));
+    const hipError_t e = launch(A, buf[*cur], buf[1 - *cur], rhs, f, s, tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += p;

@@ -21,6 +21,15 @@ GRIDS3 = {
     "rows_beyond_a_block": dict(n=(131, 9, 3), periodic=[1, 0, 1], bc=WALLS),
 }
 
+# above 512^2 cells rows stream in blocks of 252 columns: the seam inside a
+# block, one cell into the last one, at the march's end (tiles instead)
+STREAMS2 = {
+    "x": dict(n=(1031, 520), periodic=[1, 0], bc=WALLS),
+    "x_last_block_of_one": dict(n=(757, 400), periodic=[1, 1]),
+    "y": dict(n=(600, 601), periodic=[0, 1], bc=WALLS),
+    "both": dict(n=(1031, 517), periodic=[1, 1]),
+}
+
 
 def _hc_relax(ml, ctx, wl, spec, iters, acoef, how="relax"):
     case, g, p, bc, b, a, op = _setup(ml, ctx, wl, spec, acoef)
@@ -51,6 +60,12 @@ def test_hc_3d_solve(ml, gpu_ctx, wl):
     assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     assert HC.bitwise_equal(HC.valid(case["n"], dn.get()), HC.valid(case["n"], new))
     op.close()
+
+
+@pytest.mark.parametrize("name", sorted(STREAMS2))
+@pytest.mark.parametrize("iters,acoef", [(1, True), (3, False)])
+def test_hc_2d_streams(ml, gpu_ctx, wl, name, iters, acoef):
+    _hc_relax(ml, gpu_ctx, wl, STREAMS2[name], iters, acoef)
 
 
 def _vc_case(ml, ctx, spec, acoef, ccoef):

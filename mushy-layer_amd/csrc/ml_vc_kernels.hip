@@ -83,8 +83,11 @@ __device__ inline T vc_lof(const Faces1<T, DIM>& F, const T* p, T aq, bool hasc,
 // homogeneous wall ghosts of the cells it updated, so one barrier per pass.
 // The body works on tile `tile` of the level (a batched launch maps its
 // workgroups to (instance, tile) pairs).
+// ODD: a periodic length is odd, so the two cells at its seam share a colour
+// and read each other: a pass forms its values, then writes them.  (2D and
+// plain relaxation only: a level that coarsens has even lengths.)
 // In 3D for the fused forms and batches only.
-template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
+template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT, bool ODD>
 __device__ __forceinline__ void vc_relax_tile_body(const VCArgs<T>& A, const T* __restrict__ in, T* __restrict__ out,
                                                    const T* __restrict__ rhs, int npass, int first, int zero_init,
                                                    const Geom& gc, const T* __restrict__ pc, int ntx, int nty,
@@ -151,14 +154,26 @@ __device__ __forceinline__ void vc_relax_tile_body(const VCArgs<T>& A, const T* 
   for (int p = 0; p < npass; ++p) {
     const int gext = t.H - p;
     const int colour = (first + p) & 1;
+    auto mine = [&](const PosRec& r) {
+      return r.kind == 1 && r.dist <= gext - 1 && !((r.i + r.j + r.k + colour) & 1);
+    };
+    auto value = [&](int kk) __attribute__((always_inline)) {
+      T st[7];
+      gather_lds<T, DIM>(su, R[kk].e, t.EX, t.EXY, st);
+      const T lof = vc_lof<T, DIM>(F[kk], st, aq[kk], A.c != nullptr, cv[kk], A.alpha, A.beta, dxinv);
+      return st[0] - lam[kk] * (lof - rr[kk]);
+    };
+    if constexpr (ODD) {
+#pragma unroll
+      for (int kk = 0; kk < KMAX; ++kk)
+        if (mine(R[kk])) v[kk] = value(kk);
+      __syncthreads();
+    }
 #pragma unroll
     for (int kk = 0; kk < KMAX; ++kk) {
       const PosRec& r = R[kk];
-      if (!(r.kind == 1 && r.dist <= gext - 1 && !((r.i + r.j + r.k + colour) & 1))) continue;
-      T st[7];
-      gather_lds<T, DIM>(su, r.e, t.EX, t.EXY, st);
-      const T lof = vc_lof<T, DIM>(F[kk], st, aq[kk], A.c != nullptr, cv[kk], A.alpha, A.beta, dxinv);
-      const T nv = st[0] - lam[kk] * (lof - rr[kk]);
+      if (!mine(r)) continue;
+      const T nv = ODD ? v[kk] : value(kk);
       su[r.e] = nv;
       // wall ghosts of this cell (it is their interior neighbour)
       const int iv[3] = {r.i, r.j, r.k};
@@ -251,14 +266,14 @@ __device__ __forceinline__ void vc_relax_tile_body(const VCArgs<T>& A, const T* 
   }
 }
 
-template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT>
+template <typename T, int DIM, int TX, int TY, int TZ, int HMAX, int NT, bool ODD>
 __global__ __launch_bounds__(NT) void vc_relax_tile_kernel(VCArgs<T> A, const T* __restrict__ in,
                                                            T* __restrict__ out, const T* __restrict__ rhs, int npass,
                                                            int first, int zero_init, Geom gc,
                                                            const T* __restrict__ pc, int ntx, int nty, Geom gr,
                                                            T* __restrict__ resc, VCFinal<T> fin) {
-  vc_relax_tile_body<T, DIM, TX, TY, TZ, HMAX, NT>(A, in, out, rhs, npass, first, zero_init, gc, pc, ntx, nty, gr,
-                                                   resc, fin, int(blockIdx.x));
+  vc_relax_tile_body<T, DIM, TX, TY, TZ, HMAX, NT, ODD>(A, in, out, rhs, npass, first, zero_init, gc, pc, ntx, nty,
+                                                        gr, resc, fin, int(blockIdx.x));
 }
 
 // batched form: workgroup w relaxes tile map[w] & mask of job map[w] >> bits
@@ -267,8 +282,9 @@ __global__ __launch_bounds__(NT) void vc_relax_batch_kernel(const VCRelaxJob<T>*
                                                             const unsigned* __restrict__ map) {
   const unsigned w = map[blockIdx.x];
   const VCRelaxJob<T>& J = jobs[w >> kBatchTileBits];
-  vc_relax_tile_body<T, DIM, TX, TY, TZ, HMAX, NT>(J.A, J.in, J.out, J.rhs, J.npass, J.first, J.zero_init, J.gc, J.pc,
-                                                   J.ntx, J.nty, J.gr, J.resc, J.fin, int(w & kBatchTileMask));
+  vc_relax_tile_body<T, DIM, TX, TY, TZ, HMAX, NT, false>(J.A, J.in, J.out, J.rhs, J.npass, J.first, J.zero_init, J.gc,
+                                                          J.pc, J.ntx, J.nty, J.gr, J.resc, J.fin,
+                                                          int(w & kBatchTileMask));
 }
 
 // Residual / operator / restricted residual over a tile with a one-cell halo.
@@ -1062,6 +1078,10 @@ hipError_t vc_relax_cfg(const VCArgs<T>& A, T* const buf[2], int* cur, const T* 
   const Geom gcc = gc ? *gc : A.g;
   const Geom grr = gr ? *gr : A.g;
   if ((resc || fin) && npass + 1 > D::HMAX) return hipErrorInvalidValue;
+  bool odd = false;
+  for (int d = 0; d < DIM; ++d) odd = odd || (A.g.periodic[d] && (A.g.n[d] & 1));
+  odd = odd && npass > 0;
+  if (odd && (DIM != 2 || resc || fin)) return hipErrorInvalidValue;   // (such a level does not coarsen)
   const VCFinal<T> none{};
   int done = 0;
   bool first_launch = true;
@@ -1077,8 +1097,9 @@ hipError_t vc_relax_cfg(const VCArgs<T>& A, T* const buf[2], int* cur, const T* 
     const bool zi = done == 0 && zero_init;
     const T* pcl = done == 0 ? pc : nullptr;
     // a timed launch carries its start and stop events in the dispatch
-    hipExtLaunchKernelGGL((vc_relax_tile_kernel<T, DIM, D::TX, D::TY, D::TZ, D::HMAX, D::NT>), dim3(nt),
-                          dim3(D::NT), lds * sizeof(T), s, timed ? tm->start[*tm->n] : nullptr,
+    auto kern = odd ? vc_relax_tile_kernel<T, DIM, D::TX, D::TY, D::TZ, D::HMAX, D::NT, DIM == 2>
+                    : vc_relax_tile_kernel<T, DIM, D::TX, D::TY, D::TZ, D::HMAX, D::NT, false>;
+    hipExtLaunchKernelGGL(kern, dim3(nt), dim3(D::NT), lds * sizeof(T), s, timed ? tm->start[*tm->n] : nullptr,
                           timed ? tm->stop[*tm->n] : nullptr, 0, A, buf[*cur], buf[1 - *cur], rhs, p, done & 1,
                           zi ? 1 : 0, gcc, pcl, ntx, nty, grr, resc, fin ? *fin : none);
     hipError_t e = hipGetLastError();
@@ -1114,22 +1135,23 @@ hipError_t vc_relax_cfg(const VCArgs<T>& A, T* const buf[2], int* cur, const T* 
 // stay in registers for the P steps that use them and are loaded one plane
 // ahead of their first use, so their loads overlap the previous plane's
 // passes.  Stencil, lambda and update are the tiled kernel's, so results
-// are identical bit for bit.
+// are identical bit for bit.  SEAM: the rows are periodic with an odd length,
+// so the two cells at their seam share a colour and read each other as of the
+// start of a pass.
 template <typename T>
 struct SCoef {
   Faces1<T, 2> F;
   T aq, cq, rr, lam;
 };
 
-template <typename T, int TX, int P, int NT>
+template <typename T, int TX, int P, int NT, bool SEAM>
 __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const T* __restrict__ in,
                                                              T* __restrict__ out, const T* __restrict__ rhs,
                                                              int first, int zero_init, Geom gc,
                                                              const T* __restrict__ pc, int nbx, int seg) {
   if (A.skip && *A.skip) return;
-  constexpr int EX = TX + 2 * P;
-  constexpr int EL = EX;
-  constexpr int K = (EL + NT - 1) / NT;
+  constexpr int EL = NT;   // positions of a plane: one a thread
+  static_assert(TX + 2 * P == NT, "one position a thread");
   static_assert(P >= 1 && P <= 2, "one or two colour passes per launch");
   constexpr int W = 4;   // planes in the window (P+2 <= 4; a power of two)
   constexpr int MD = 1;
@@ -1144,21 +1166,12 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   const int x0 = bx * TX;
   const int z0 = bz * seg;
   const int z1 = z0 + seg < nz ? z0 + seg : nz;
-  SPos S[K];
-#pragma unroll
-  for (int kk = 0; kk < K; ++kk) {
-    const int e = threadIdx.x + kk * NT;
-    if (e < EL) {
-      spos_init<TX, P>(g, x0, e, S[kk]);
-      S[kk].gtype = 0;
-      for (int sd = 0; sd < 2; ++sd)
-        if (S[kk].kind == 2 && S[kk].gs == sd) S[kk].gtype = A.bc.type[0][sd][0];
-    } else {
-      S[kk].kind = 0;
-      S[kk].dist = P;
-      S[kk].owner = 0;
-    }
-  }
+  const int e = int(threadIdx.x);
+  SPos s;
+  spos_init<TX, P>(g, x0, e, s);
+  s.gtype = 0;
+  for (int sd = 0; sd < 2; ++sd)
+    if (s.kind == 2 && s.gs == sd) s.gtype = A.bc.type[0][sd][0];
   auto zwrap = [&](int z) { return z < 0 ? z + nz : (z >= nz ? z - nz : z); };
   auto real_plane = [&](int z) { return zper || (z >= 0 && z < nz); };
   // 32-bit element offsets: a position's lateral part, computed once, plus a
@@ -1170,16 +1183,7 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   fup[0] = 1;
   fup[MD] = fpl[MD];
   const unsigned cgsz = unsigned(gc.sy);
-  unsigned cl[K], fl[K][2], ccl[K];
-#pragma unroll
-  for (int kk = 0; kk < K; ++kk) {
-    const SPos& s = S[kk];
-    cl[kk] = unsigned(s.gx + 1);
-#pragma unroll
-    for (int d = 0; d < 2; ++d)
-      fl[kk][d] = unsigned(s.gx);
-    ccl[kk] = unsigned(s.gx / 2 + 1);
-  }
+  const unsigned cl = unsigned(s.gx + 1), fl = unsigned(s.gx), ccl = unsigned(s.gx / 2 + 1);
   auto ld = [](const T* p, unsigned i) -> T {
     return *reinterpret_cast<const T*>(reinterpret_cast<const char*>(p) + (i * unsigned(sizeof(T))));
   };
@@ -1188,8 +1192,8 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   // into their set and are used only at that plane's commit two steps later,
   // so no instruction touches a load in flight.
   constexpr int NS = P + 3;
-  SCoef<T> cs[NS][K];
-  T sv[NS][K], scv[NS][K];   // state and coarse correction as loaded
+  SCoef<T> cs[NS];
+  T sv[NS], scv[NS];   // state and coarse correction as loaded
   // the same loads for every position and plane (in-domain addresses; an
   // absent array is replaced by a duplicate read of rhs), so that the waits
   // for a set's loads can count the loads issued after it exactly
@@ -1197,24 +1201,21 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
   const T* ain = A.a ? A.a : rhs;
   const T* cin = hasc ? A.c : rhs;
   const T* cvp = pc ? pc : rhs;
-  auto prefetch = [&](int R, SCoef<T>(&pf)[K], T(&v)[K], T(&cv)[K]) {
+  auto prefetch = [&](int R, SCoef<T>& pf, T& v, T& cv) {
     const int zw = zper ? zwrap(R) : (R < 0 ? 0 : (R >= nz ? nz - 1 : R));
     const unsigned qz = unsigned(zw + 1) * csz, cz = unsigned(zw / 2 + 1) * cgsz;
+    const unsigned q = cl + qz;   // a ghost reads its interior neighbour
+    v = ld(vin, q);
+    cv = ld(cvp, pc ? ccl + cz : q);
 #pragma unroll
-    for (int kk = 0; kk < K; ++kk) {
-      const unsigned q = cl[kk] + qz;   // a ghost reads its interior neighbour
-      v[kk] = ld(vin, q);
-      cv[kk] = ld(cvp, pc ? ccl[kk] + cz : q);
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        const unsigned f = fl[kk][d] + unsigned(zw) * fpl[d];
-        pf[kk].F.v[2 * d] = ld(A.b[d], f);
-        pf[kk].F.v[2 * d + 1] = ld(A.b[d], f + fup[d]);
-      }
-      pf[kk].aq = ld(ain, q);
-      pf[kk].cq = ld(cin, q);
-      pf[kk].rr = ld(rhs, q);
+    for (int d = 0; d < 2; ++d) {
+      const unsigned f = fl + unsigned(zw) * fpl[d];
+      pf.F.v[2 * d] = ld(A.b[d], f);
+      pf.F.v[2 * d + 1] = ld(A.b[d], f + fup[d]);
     }
+    pf.aq = ld(ain, q);
+    pf.cq = ld(cin, q);
+    pf.rr = ld(rhs, q);
   };
   const int zl = (!zper && z0 - P < 0) ? 0 : z0 - P;
   const int zend = z1 - 1 + P;   // last step: plane z1 - 1 is final
@@ -1224,32 +1225,22 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
     constexpr int j = decltype(J)::value;
     // A. commit plane R (or the top wall's ghost plane)
     T* pl = slot(R);
-    if (real_plane(R)) {
-#pragma unroll
-      for (int kk = 0; kk < K; ++kk) {
-        const SPos& s = S[kk];
-        const int e = threadIdx.x + kk * NT;
-        if (s.kind == 0) continue;
-        T val = zero_init ? T(0) : sv[j][kk];
-        if (pc) val = val + scv[j][kk];
-        if (s.kind == 1) {
-          pl[e] = val;
-          if (!zper && R == 0) slot(-1)[e] = bc_ghost<T>(A.bc.type[MD][0][0], T(0), val, -1, T(g.dx));
-          if (!A.a) cs[j][kk].aq = T(1);
-          if (!hasc) cs[j][kk].cq = T(0);
-          if (s.dist <= P - 1)
-            cs[j][kk].lam = vc_lambda<T, 2>(cs[j][kk].F, cs[j][kk].aq, hasc, cs[j][kk].cq, A.alpha, A.beta, dxinv);
-        } else {
-          pl[e] = bc_ghost<T>(s.gtype, T(0), val, s.gs == 0 ? -1 : 1, T(g.dx));
-        }
+    if (real_plane(R) && s.kind != 0) {
+      T val = zero_init ? T(0) : sv[j];
+      if (pc) val = val + scv[j];
+      if (s.kind == 1) {
+        pl[e] = val;
+        if (!zper && R == 0) slot(-1)[e] = bc_ghost<T>(A.bc.type[MD][0][0], T(0), val, -1, T(g.dx));
+        if (!A.a) cs[j].aq = T(1);
+        if (!hasc) cs[j].cq = T(0);
+        if (s.dist <= P - 1)
+          cs[j].lam = vc_lambda<T, 2>(cs[j].F, cs[j].aq, hasc, cs[j].cq, A.alpha, A.beta, dxinv);
+      } else {
+        pl[e] = bc_ghost<T>(s.gtype, T(0), val, s.gs == 0 ? -1 : 1, T(g.dx));
       }
-    } else if (!zper && R == nz) {
+    } else if (!zper && R == nz && s.kind == 1) {
       const T* below = slot(nz - 1);
-#pragma unroll
-      for (int kk = 0; kk < K; ++kk) {
-        const int e = threadIdx.x + kk * NT;
-        if (S[kk].kind == 1) pl[e] = bc_ghost<T>(A.bc.type[MD][1][0], T(0), below[e], 1, T(g.dx));
-      }
+      pl[e] = bc_ghost<T>(A.bc.type[MD][1][0], T(0), below[e], 1, T(g.dx));
     }
     // B. loads of plane R+2 into the set of plane R+2-NS, no longer in use
     constexpr int jn = (j + 2) % NS;
@@ -1264,24 +1255,28 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
       const bool run = z >= z0 - reach && z < z1 + reach && real_plane(z);
       if (run) {
         const int zw = zwrap(z);
-        const int colour = (first + p) & 1;
+        const bool mine = s.kind == 1 && s.dist <= reach && !((s.gx + zw + first + p) & 1);
         T* pz = slot(z);
         const T* pm = slot(z - 1);
         const T* pp = slot(z + 1);
-#pragma unroll
-        for (int kk = 0; kk < K; ++kk) {
-          const SPos& s = S[kk];
-          if (s.kind != 1 || s.dist > reach || ((s.gx + zw + colour) & 1)) continue;
-          const int e = threadIdx.x + kk * NT;
+        auto value = [&]() __attribute__((always_inline)) {
           T st[7];
           st[0] = pz[e];
           st[1] = pz[e + 1];
           st[2] = pz[e - 1];
           st[3] = pp[e];
           st[4] = pm[e];
-          const SCoef<T>& C = cs[jp][kk];
+          const SCoef<T>& C = cs[jp];
           const T lof = vc_lof<T, 2>(C.F, st, C.aq, hasc, C.cq, A.alpha, A.beta, dxinv);
-          const T nv = st[0] - C.lam * (lof - C.rr);
+          return st[0] - C.lam * (lof - C.rr);
+        };
+        T nv;
+        if constexpr (SEAM) {
+          if (mine) nv = value();
+          __syncthreads();   // the two cells at the seam read each other
+        }
+        if (mine) {
+          if constexpr (!SEAM) nv = value();
           pz[e] = nv;
           // wall ghosts of this cell: lateral, then along the march
           if (!g.periodic[0]) {
@@ -1300,16 +1295,9 @@ __global__ __launch_bounds__(NT) void vc_relax_stream_kernel(VCArgs<T> A, const 
     if constexpr (P > 1) pass(IC<1>{});
     // D. plane R-P is final
     const int zs = R - P;
-    if (zs >= z0 && zs < z1) {
-      const T* ps = slot(zs);
-#pragma unroll
-      for (int kk = 0; kk < K; ++kk) {
-        const SPos& s = S[kk];
-        if (s.owner)
-          *reinterpret_cast<T*>(reinterpret_cast<char*>(out) + ((cl[kk] + unsigned(zs + 1) * csz) * unsigned(sizeof(T)))) =
-              ps[threadIdx.x + kk * NT];
-      }
-    }
+    if (zs >= z0 && zs < z1 && s.owner)
+      *reinterpret_cast<T*>(reinterpret_cast<char*>(out) + ((cl + unsigned(zs + 1) * csz) * unsigned(sizeof(T)))) =
+          slot(zs)[e];
   };
   prefetch(zl, cs[0], sv[0], scv[0]);
   prefetch(zl + 1, cs[1], sv[1], scv[1]);
@@ -1331,17 +1319,19 @@ struct VCStream {
 };
 
 // 2D levels on which plain relaxation launches stream (above 512^2); the
-// tiled kernel keeps the fused restriction / residual
+// tiled kernel keeps the fused restriction / residual.  Not with an odd
+// periodic length along the march: the rows at its seam share colours, and a
+// pass reaches one of them before the other.
 constexpr long long kStreamCells2 = 512 * 512;
 inline bool vc_streams(const Geom& g) {
   long long nf = 0;
   for (int d = 0; d < g.dim; ++d) nf = nf > g.nface[d] ? nf : g.nface[d];
   const long long most = g.ncell > nf ? g.ncell : nf;
-  return g.dim == 2 && g.nvalid() > kStreamCells2 && g.n[1] >= 8 &&
+  return g.dim == 2 && g.nvalid() > kStreamCells2 && g.n[1] >= 8 && !(g.periodic[1] && (g.n[1] & 1)) &&
          most < (1LL << 29);   // byte offsets of every array within 32 bits
 }
 
-template <typename T, int P>
+template <typename T, int P, bool SEAM>
 hipError_t vc_stream_launch(const VCArgs<T>& A, const T* in, T* out, const T* rhs, int first, bool zero_init,
                             const Geom& gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
   using D = VCStream;
@@ -1349,7 +1339,7 @@ hipError_t vc_stream_launch(const VCArgs<T>& A, const T* in, T* out, const T* rh
   const Geom& g = A.g;
   const int nbx = (g.n[0] + TX - 1) / TX;
   const size_t lds = size_t(4) * EL * sizeof(T);
-  auto kern = vc_relax_stream_kernel<T, TX, P, D::NT>;
+  auto kern = vc_relax_stream_kernel<T, TX, P, D::NT, SEAM>;
   // segments sized so that the whole grid is resident at once (one round of
   // workgroups; measured best at 2048^2: a grid that fills every CU's
   // workgroup slots beats both fewer, longer segments and a second round)
@@ -1394,14 +1384,15 @@ template <typename T>
 hipError_t vc_relax_stream(const VCArgs<T>& A, T* const buf[2], int* cur, const T* rhs, int npass, bool zero_init,
                            const Geom* gc, const T* pc, hipStream_t s, const LaunchTimer* tm) {
   const Geom gcc = gc ? *gc : A.g;
+  const bool seam = A.g.periodic[0] && (A.g.n[0] & 1);
   int done = 0;
   while (done < npass) {
     const int p = (npass - done) >= 2 ? 2 : (npass - done);
     const bool zi = done == 0 && zero_init;
     const T* pcl = done == 0 ? pc : nullptr;
-    hipError_t e = p == 2 ? vc_stream_launch<T, 2>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s, tm)
-                          : vc_stream_launch<T, 1>(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s,
-                                                        tm);
+    auto launch = p == 2 ? (seam ? vc_stream_launch<T, 2, true> : vc_stream_launch<T, 2, false>)
+                         : (seam ? vc_stream_launch<T, 1, true> : vc_stream_launch<T, 1, false>);
+    const hipError_t e = launch(A, buf[*cur], buf[1 - *cur], rhs, done & 1, zi, gcc, pcl, s, tm);
     if (e != hipSuccess) return e;
     *cur = 1 - *cur;
     done += p;

@@ -120,3 +120,28 @@ def test_vc_3d(ml, gpu_ctx, name, iters, acoef, ccoef):
 
 def test_vc_3d_solve(ml, gpu_ctx):
     _vc_solve(ml, gpu_ctx, GRIDS3["y"])
+
+
+TILES2 = {
+    "x": dict(n=(45, 44), periodic=[1, 0], bc=WALLS),
+    "y": dict(n=(44, 45), periodic=[0, 1], bc=WALLS),
+    "both": dict(n=(67, 35), periodic=[1, 1]),
+    "short": dict(n=(3, 400), periodic=[1, 0], bc=WALLS),
+}
+
+
+@pytest.mark.parametrize("name", sorted(TILES2))
+@pytest.mark.parametrize("iters,acoef,ccoef", [(1, False, True), (6, True, False)])
+def test_vc_2d_tiles(ml, gpu_ctx, name, iters, acoef, ccoef):
+    _vc_relax(ml, gpu_ctx, TILES2[name], iters, acoef, ccoef)
+
+
+@pytest.mark.parametrize("name", sorted(STREAMS2))
+@pytest.mark.parametrize("iters,acoef,ccoef", [(1, False, True), (3, True, False)])
+def test_vc_2d_streams(ml, gpu_ctx, name, iters, acoef, ccoef):
+    _vc_relax(ml, gpu_ctx, STREAMS2[name], iters, acoef, ccoef)
+
+
+@pytest.mark.parametrize("spec", [TILES2["both"], STREAMS2["x"]], ids=["tiles", "streams"])
+def test_vc_2d_solve(ml, gpu_ctx, spec):
+    _vc_solve(ml, gpu_ctx, spec)

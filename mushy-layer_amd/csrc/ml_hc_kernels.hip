@@ -99,12 +99,25 @@ __device__ inline void tile_diffused_var(const HCArgs<T>& A, const Tile<DIM, TX,
 // state.  Measured (events around the launch, 256^2 mushy state): 8 passes
 // 14.4 us, 21.2 us with one cell per lane (32x8 tiles, 512 threads); at 512^2
 // 34.7 against 74.3 us; on the way down one launch of 10.5 us replaces
-// relaxation, restriction and operator (9.0 + 7.3 + 8.4 us).  GEN: any grid -- a periodic length below 32 or odd (equal colours
-// then meet at its seam: a pass looks at both slots, and reads neighbours as
-// of its start), arrays beyond 32-bit byte offsets.
+// relaxation, restriction and operator (9.0 + 7.3 + 8.4 us).
+//
+// GEN: any grid -- a periodic length below 32 or odd, arrays beyond 32-bit
+// byte offsets.  Equal colours meet at the seam of an odd length.  A region
+// that holds it reads a pass's neighbours as of its start (the new closures
+// are stored after a barrier), and along x it starts one cell earlier where
+// that keeps the seam from falling inside a pair, whose cells would share a
+// slot's turn; its core is two cells narrower for that.  Only below 32 cells,
+// where a region may hold several seams, a pass looks at both slots.  One
+// sweep of 129 x 128 8.1 us, of 257 x 256 8.3 (11.4 and 11.3 with both slots
+// everywhere; 7.5 and 7.9 with even lengths), of 23 x 500 12; four sweeps of
+// 385 x 384 28.7 us (34.7; even 24.3).
 enum : int { RB_PLAIN = 0, RB_RESTRICT = 1, RB_NORM = 2 };
 constexpr int kRB = 32;            // positions per side
 constexpr int kRBThreads = kRB * kRB / 2;
+// core cells along x
+__host__ __device__ inline int pair_core_x(int nx, int per0, int H) {
+  return kRB - 2 * H - (per0 && (nx & 1) && nx >= kRB ? 2 : 0);
+}
 
 template <typename T>
 struct PairArgs {
@@ -172,13 +185,29 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
   const int nx = A.nx, ny = A.ny, npass = A.npass;
   const int H = npass + (MODE == RB_PLAIN ? 0 : 1);
   const int core = kRB - 2 * H;
+  const int corex = GEN ? pair_core_x(nx, A.per0, H) : core;
   // GEN: the workgroups of all tiles in one dimension
   const int by = GEN ? int(blockIdx.x / unsigned(A.ntx)) : int(blockIdx.y);
   const int bx = GEN ? int(blockIdx.x) - by * A.ntx : int(blockIdx.x);
-  const int x0 = bx * core, y0 = by * core;
+  const int x0 = bx * corex, y0 = by * core;
   const int ey = threadIdx.x >> 4, ex0 = 2 * (threadIdx.x & 15);
-  const int ux0 = x0 - H + ex0, uy = y0 - H + ey;
   const bool per0 = A.per0 != 0, per1 = A.per1 != 0;
+  // GEN: the region holds the seam of an odd length (careful), the pairs'
+  // shift against it, both slots in every pass
+  bool careful = false, both = false;
+  int sh = 0;
+  if constexpr (GEN) {
+    if (per0 && (nx & 1)) {
+      both = nx < kRB;
+      // the seam inside the region, from its first cell (n >= 32: at most one)
+      const int at = x0 < H ? H - x0 : nx - (x0 - H);
+      careful = both || at < kRB;
+      sh = !both && at < kRB ? at & 1 : 0;
+    }
+    if (per1 && (ny & 1)) careful = careful || ny < kRB || y0 < H || ny - (y0 - H) < kRB;
+  }
+  const int Hx = H + sh;   // the core's first column in the region
+  const int ux0 = x0 - Hx + ex0, uy = y0 - H + ey;
   auto wrap = [](int v, int n) {
     if (GEN) {
       v %= n;
@@ -190,18 +219,19 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
   const bool oky = iny || per1;
   const int gj = oky ? wrap(uy, ny) : 0;
   // distance from the core
-  auto beyond = [&](int e) {
-    const int lo = H - e, hi = e - (H + core) + 1;
+  auto beyond = [&](int e, int lo0, int n) {
+    const int lo = lo0 - e, hi = e - (lo0 + n) + 1;
     const int d = lo > hi ? lo : hi;
     return d > 0 ? d : 0;
   };
-  const int dy = beyond(ey);
-  const int swap = (ux0 + uy) & 1;   // parity of the pair's first cell
+  const int dy = beyond(ey, H, core);
   const int wy = per1 ? 0 : ((gj == 0 ? 4 : 0) | (gj == ny - 1 ? 8 : 0));
   // cells of the pair in x order: c = 0, 1; slot m holds cell m ^ swap
   const bool in0 = ux0 >= 0 && ux0 < nx, in1 = ux0 >= -1 && ux0 + 1 < nx;
   const bool ok0 = oky && (in0 || per0), ok1 = oky && (in1 || per0);
   const int gx0 = ok0 ? wrap(ux0, nx) : 0, gx1 = ok1 ? wrap(ux0 + 1, nx) : 0;
+  // parity of the pair's first cell
+  const int swap = (GEN ? (per0 ? gx0 : ux0) + gj : ux0 + uy) & 1;
   const Off row = Off(A.sy) * Off(gj + 1) + Off(1);
   const Off q0 = (row + Off(gx0)) * W, q1 = (row + Off(gx1)) * W;   // byte offsets
 
@@ -283,7 +313,7 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
     cell[m] = second ? ok1 : ok0;
     gi[m] = second ? gx1 : gx0;
     q[m] = second ? q1 : q0;
-    const int dx = beyond(ex);
+    const int dx = beyond(ex, Hx, corex);
     const int dist = dx > dy ? dx : dy;
     owner[m] = (second ? in1 : in0) && iny && dist == 0;
     lim[m] = cell[m] ? H - 1 - dist : -1;   // last pass that updates the cell
@@ -393,17 +423,17 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
 #pragma unroll
     for (int n = 0; n < 2; ++n) ph[m][n] = ph[m][n] - lam[m][n] * (lf[n] - rr[m][n]);
     closure<T>(ph[m][0], ph[m][1], A.cp, pl[m][0], pl[m][1]);
-    if (!GEN) put(m);
+    if (!GEN || !careful) put(m);
   };
 #pragma unroll 1
   for (int p = 0; p < npass; ++p) {
     const int colour = (A.first + p) & 1;
-    if (GEN || colour == 0) update(IC<0>{}, p, colour);
-    if (GEN || colour == 1) update(IC<1>{}, p, colour);
-    if constexpr (GEN) {
+    if (both || colour == 0) update(IC<0>{}, p, colour);
+    if (both || colour == 1) update(IC<1>{}, p, colour);
+    if (careful) {
       __syncthreads();
-      if (runs(0, p, colour)) put(0);
-      if (runs(1, p, colour)) put(1);
+      if ((both || colour == 0) && runs(0, p, colour)) put(0);
+      if ((both || colour == 1) && runs(1, p, colour)) put(1);
     }
     __syncthreads();
   }
@@ -460,7 +490,7 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
     // coarse cells of the core (at most 13 a side), 16 threads a row
     const int cy = threadIdx.x >> 4, cx = threadIdx.x & 15;
     const int I = x0 / 2 + cx, J = y0 / 2 + cy;
-    if (cx >= core / 2 || cy >= core / 2 || I >= A.cnx || J >= A.cny) return;
+    if (cx >= corex / 2 || cy >= core / 2 || I >= A.cnx || J >= A.cny) return;
     const Off qc = (Off(I + 1) + Off(A.csy) * Off(J + 1)) * W;
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
@@ -469,7 +499,7 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
       for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
         for (int ii = 0; ii < 2; ++ii) {
-          const int f = n * NP + (2 * cy + jj + H) * kRB + 2 * cx + ii + H;
+          const int f = n * NP + (2 * cy + jj + H) * kRB + 2 * cx + ii + Hx;
           s = s + sl[f];
           sp = sp + sr[f];
         }
@@ -1450,8 +1480,8 @@ static hipError_t launch_relax_pair(const HCArgs<T>& A, const TileIO<T>& io, hip
         P.gs[d][sd][n] = gf.s[d][sd][n];
         P.gb[d][sd][n] = gf.b[d][sd][n];
       }
-  const int core = kRB - 2 * H;
-  const int ntx = (g.n[0] + core - 1) / core, nty = (g.n[1] + core - 1) / core;
+  const int core = kRB - 2 * H, corex = pair_core_x(g.n[0], g.periodic[0], H);
+  const int ntx = (g.n[0] + corex - 1) / corex, nty = (g.n[1] + core - 1) / core;
   if (g.ncell >= (1LL << 32)) return hipErrorInvalidValue;   // (32-bit component stride)
   P.ntx = ntx;
   // GEN where a grid needs it: more than 2^16 - 1 tiles along y included

@@ -30,6 +30,14 @@ STREAMS2 = {
     "both": dict(n=(1031, 517), periodic=[1, 1]),
 }
 
+# regions of 32 positions: the seam at even and odd places of a region, in the
+# halo of one core and inside the next, more than once in a region (below 32)
+PAIRS2 = {
+    "%dx%d_%d%d" % (n + tuple(per)): dict(n=n, periodic=per, bc=None if per[1] else WALLS)
+    for n, per in [((33, 40), [1, 0]), ((59, 30), [1, 0]), ((81, 64), [1, 0]), ((85, 33), [1, 1]), ((129, 47), [1, 1]),
+                   ((64, 35), [1, 1]), ((48, 53), [0, 1]), ((31, 66), [1, 0]), ((7, 200), [1, 1]), ((200, 9), [1, 1])]
+}
+
 
 def _hc_relax(ml, ctx, wl, spec, iters, acoef, how="relax"):
     case, g, p, bc, b, a, op = _setup(ml, ctx, wl, spec, acoef)
@@ -60,6 +68,12 @@ def test_hc_3d_solve(ml, gpu_ctx, wl):
     assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     assert HC.bitwise_equal(HC.valid(case["n"], dn.get()), HC.valid(case["n"], new))
     op.close()
+
+
+@pytest.mark.parametrize("name", sorted(PAIRS2))
+@pytest.mark.parametrize("iters,acoef", [(1, True), (2, False), (4, True), (5, False)])
+def test_hc_2d_pairs(ml, gpu_ctx, wl, name, iters, acoef):
+    _hc_relax(ml, gpu_ctx, wl, PAIRS2[name], iters, acoef)
 
 
 @pytest.mark.parametrize("name", sorted(STREAMS2))

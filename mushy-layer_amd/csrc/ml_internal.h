@@ -253,6 +253,7 @@ struct VCWork {
   const double* g_rhs = nullptr;
   int g_nu1 = -1, g_nu2 = -1, g_bottom = -1, g_bsolver = -1, g_bimax = -1;
   double g_alpha = 0, g_beta = 0;
+  bool g_has_a = false, g_has_c = false;
 };
 }  // namespace ml
 

@@ -327,7 +327,7 @@ int vc_iteration(ml_vc_op op, ml::VCWork& W, const ml_solve_opts& o, int* ecur, 
 bool vc_capture(ml_vc_op op, ml::VCWork& W, VCSolve& S, const ml_solve_opts& o) {
   if (W.gexec && W.g_phi == S.phi && W.g_rhs == S.rhs && W.g_nu1 == o.nu1 && W.g_nu2 == o.nu2 &&
       W.g_bottom == o.bottom && W.g_bsolver == o.bottom_solver && W.g_bimax == o.bottom_max_iter &&
-      W.g_alpha == op->alpha && W.g_beta == op->beta)
+      W.g_alpha == op->alpha && W.g_beta == op->beta && W.g_has_a == op->has_a && W.g_has_c == op->has_c)
     return true;
   if (W.gexec) hipGraphExecDestroy(W.gexec);
   W.gexec = nullptr;
@@ -355,6 +355,8 @@ bool vc_capture(ml_vc_op op, ml::VCWork& W, VCSolve& S, const ml_solve_opts& o) 
   W.g_bimax = o.bottom_max_iter;
   W.g_alpha = op->alpha;
   W.g_beta = op->beta;
+  W.g_has_a = op->has_a;
+  W.g_has_c = op->has_c;
   return true;
 }
 
@@ -849,8 +851,8 @@ size_t vcb_align(size_t x) { return (x + 255) & ~size_t(255); }
 int vcb_tables(ml_vc_batch b, double* const phi[], const double* const rhs[], const ml_solve_opts& o) {
   ml_ctx ctx = b->ctx;
   const int n = int(b->units.size());
-  // the jobs depend on the state and rhs buffers, alpha and beta (through
-  // the operator arguments) and the smoothing counts
+  // the jobs depend on the state and rhs buffers, alpha, beta, a and c
+  // (through the operator arguments) and the smoothing counts
   std::vector<const void*> key;
   auto bits_of = [](double v) {
     std::uint64_t x;
@@ -862,6 +864,8 @@ int vcb_tables(ml_vc_batch b, double* const phi[], const double* const rhs[], co
     key.push_back(rhs[u]);
     key.push_back(bits_of(b->units[u].op->alpha));
     key.push_back(bits_of(b->units[u].op->beta));
+    key.push_back(b->units[u].op->args(0).a);
+    key.push_back(b->units[u].op->args(0).c);
   }
   key.push_back(reinterpret_cast<const void*>(std::uintptr_t(o.nu1 * 1000 + o.nu2)));
   key.push_back(reinterpret_cast<const void*>(std::uintptr_t(o.max_iter)));

@@ -87,3 +87,35 @@ def test_residual_norms_of_many_workgroups(ml, gpu_ctx, n):
         assert st.initial_residual == so.initial_residual == 7.0
         assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     op.close()
+
+
+def test_replayed_solves_follow_the_coefficients(ml, gpu_ctx):
+    """Solves of one operator on the same arrays replay their iterations, and a
+    batch keeps its tables; the a and c terms may come and go between them with
+    alpha and beta as before."""
+    n, per = (64, 48), (1, 0)
+    dx = 1.0 / n[0]
+    bc = {(1, s, 0): (0, 0.0) for s in (0, 1)}
+    g = O.make_grid(n, dx, list(per) + [0])
+    rng = np.random.default_rng(8)
+    b = [rng.uniform(0.5, 1.5, O.face_shape(g, d, 1)) for d in range(2)]
+    a, c = rng.uniform(0.5, 1.5, O.cell_shape(g, 1)), rng.uniform(0.0, 20.0, O.cell_shape(g, 1))
+    rhs = np.zeros(O.cell_shape(g, 1))
+    O.valid(g, rhs)[...] = rng.standard_normal(O.valid(g, rhs).shape)
+    kw = dict(max_iter=4, nu1=1, nu2=2, bottom=3, eps=1e-14, hang=1e-14, norm_thresh=1e-14)
+    op = ml.VCOp(gpu_ctx, list(n), dx, list(per), ml.make_bc(bc))
+    dev = lambda x: None if x is None else ml.DeviceArray(gpu_ctx, x.shape, host=x)
+    db, drhs, dphi = [dev(x) for x in b], dev(rhs), dev(np.zeros_like(rhs))
+    batch = ml.VCBatch(gpu_ctx, [op])
+    for ac, cc in ((None, None), (None, c), (a, c), (a, None), (None, None)):
+        phi = np.zeros_like(rhs)
+        so = O.lin_mg_solve(g, 1, O.make_bc(bc), 1.0, ac, -2e-3, cc, b, phi, rhs, opts=O.default_opts(**kw))
+        op.set_coefs(dev(ac), db, dev(cc), 1.0, -2e-3)
+        for solve in (op.solve, lambda p, r, opts: batch.solve([p], [r], opts)[0]):
+            dphi.set(np.zeros_like(rhs))
+            st = solve(dphi, drhs, opts=ml.default_opts(**kw))
+            assert (st.iterations, st.exit_status) == (so.iterations, so.exit_status)
+            assert st.final_residual == so.final_residual
+            assert HC.bitwise_equal(np.ascontiguousarray(HC.valid(n, dphi.get())), np.ascontiguousarray(HC.valid(n, phi)))
+    batch.close()
+    op.close()

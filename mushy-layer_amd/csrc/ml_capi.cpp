@@ -338,6 +338,14 @@ int ml_hc_op_create(ml_ctx ctx, int dim, const int lo[], const int hi[], double 
   if (op->lc < depth) {
     void* p = nullptr;
     op->ncfaces += op->ncfaces & 1;
+    size_t mx = 0;
+    int rc = ml::max_lds(ctx, &mx);
+    if (rc == ML_OK && ml::hc_coarse_lds_bytes(op->lev[op->lc].g, depth - op->lc, op->ncfaces) > mx)
+      rc = fail(ctx, ML_ENOTSUP, "the coarse MG levels exceed the workgroup's LDS");
+    if (rc != ML_OK) {
+      ml_hc_op_destroy(op.release());
+      return rc;
+    }
     if (hipMalloc(&p, sizeof(double) * op->ncfaces) != hipSuccess) {
       ml_hc_op_destroy(op.release());
       return fail(ctx, ML_ENOMEM, "hipMalloc bCoef");

@@ -486,7 +486,7 @@ constexpr int kDirect = 16;
 // 32x32, us a launch: 53 before the exact solve worked without LDS and e
 // stayed in registers, 46 now; a colour pass of a small level is 460 cycles,
 // a visit's set-up 3000.
-constexpr int kLL = 6;   // levels one launch handles: 1024 cells coarsen to one cell in 6 (2D), 4 (3D)
+constexpr int kLL = 6;   // levels one launch may hold; 1024 cells make at most 5 (2D) or 3 (3D): no side falls below 2
 template <int DIM>
 struct LinLevels {
   static constexpr int n = DIM == 3 ? 4 : kLL;

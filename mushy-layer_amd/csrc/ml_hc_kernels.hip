@@ -644,9 +644,9 @@ __global__ __launch_bounds__(kThreads) void hc_apply_batch_kernel(const HCApplyJ
 // ---------------------------------------------------------------------------
 // Single-workgroup FAS V-cycle over the small levels (at most kWGCells cells
 // and everything below).  All levels' state, right-hand side, initial state,
-// lambda and faces live in LDS for the whole cycle (at most 156 KB over all
-// shapes; the faces come as one contiguous block), so a level visit waits for
-// no global memory.
+// lambda and faces live in LDS for the whole cycle (hc_coarse_lds_bytes; the
+// faces come as one contiguous block), so a level visit waits for no global
+// memory.
 //
 // A wavefront alone on its SIMD issues an operation every 8 cycles whether it
 // depends on the last one or not, and a branch costs four of them: the count
@@ -1830,6 +1830,19 @@ hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T
 
 int hc_coarse_cells() { return kWGCells; }
 
+// state, right-hand side and (nl > 1) lambda of every level, the initial state
+// below the first, closure and ghosts of one level, the faces; and the ghost
+// rules (static).  At most 156,192 bytes over all shapes of up to 1024 cells
+// (4 x 4 x 64; in 2D 149,504 at 64 x 16).
+static size_t hc_coarse_lds_dyn(int nl, int tot, int n0, size_t nfaces) {
+  return sizeof(double) * ((nl > 1 ? 6 : 4) * size_t(tot) + 2 * size_t(tot - n0) + 4 * kWGCells + nfaces);
+}
+size_t hc_coarse_lds_bytes(const Geom& g, int nl, size_t nfaces) {
+  int tot = 0;
+  for (int l = 0; l < nl; ++l) tot += int(coarsen_geom(g, 1 << l).nvalid());
+  return hc_coarse_lds_dyn(nl, tot, int(g.nvalid()), nfaces) + sizeof(double) * 4 * (2 * g.dim + 1);
+}
+
 template <typename T>
 hipError_t hc_coarse_vcycle(const Geom& g, const BCDesc& bc, HCCoarse<T> A, hipStream_t s) {
   if (g.nvalid() > kWGCells || A.nl < 1 || A.nl > kHCCoarseLevels) return hipErrorInvalidValue;
@@ -1856,12 +1869,12 @@ hipError_t hc_coarse_vcycle(const Geom& g, const BCDesc& bc, HCCoarse<T> A, hipS
         A.gs[d][sd][n] = gf.s[d][sd][n];
         A.gb[d][sd][n] = gf.b[d][sd][n];
       }
-  const size_t elems = (A.nl > 1 ? 6 : 4) * size_t(A.tot) + 2 * size_t(A.tot - A.off[1]) + 4 * kWGCells + size_t(A.nfaces);
-  // (at most 147 KB over all shapes of up to 1024 cells)
+  static_assert(sizeof(T) == sizeof(double), "the LDS map's element");
+  const size_t lds = hc_coarse_lds_dyn(A.nl, A.tot, A.off[1], size_t(A.nfaces));
   if (g.dim == 2)
-    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 2>), dim3(1), dim3(kHCWG), elems * sizeof(T), s, A);
+    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 2>), dim3(1), dim3(kHCWG), lds, s, A);
   else
-    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 3>), dim3(1), dim3(kHCWG), elems * sizeof(T), s, A);
+    hipLaunchKernelGGL((hc_coarse_vcycle_kernel<T, 3>), dim3(1), dim3(kHCWG), lds, s, A);
   return hipGetLastError();
 }
 

@@ -570,6 +570,8 @@ hipError_t hc_relax_final(const HCArgs<T>& A, T* const buf[2], int* cur, const T
                           const T* pc, const T* pc0, unsigned long long* norm, const CtlFuse& fuse, hipStream_t s);
 // FAS V-cycle of the levels from g (at most hc_coarse_cells() cells) down
 int hc_coarse_cells();
+// LDS of its workgroup: levels g .. g / 2^(nl-1), nfaces face values in all
+size_t hc_coarse_lds_bytes(const Geom& g, int nl, size_t nfaces);
 template <typename T>
 hipError_t hc_coarse_vcycle(const Geom& g, const BCDesc& bc, HCCoarse<T> A, hipStream_t s);
 template <typename T>

@@ -450,7 +450,8 @@ __global__ __launch_bounds__(256) void words_batch_kernel(const WordsJob* __rest
 // levels from 44x20 (bottom 22x10) 165 -> 115; a visit is now some 6.5K
 // cycles, half of them its set-up.
 
-constexpr int kVCL = kVCCoarseLevels;   // levels one launch handles: 1024 cells coarsen to one cell in 6 (2D), 4 (3D)
+// levels one launch may hold; 1024 cells make at most 5 (2D) or 3 (3D): no side falls below 2
+constexpr int kVCL = kVCCoarseLevels;
 template <int DIM>
 struct VCLevels {
   static constexpr int n = DIM == 3 ? 4 : kVCL;

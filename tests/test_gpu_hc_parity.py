@@ -189,9 +189,10 @@ WALLS = {(0, 0, 0): (1, 0.3), (0, 1, 0): (0, 0.5), (0, 0, 1): (1, -0.2), (0, 1, 
          (2, 0, 0): (0, -0.5), (2, 1, 0): (1, 0.2), (2, 0, 1): (1, 0.0), (2, 1, 1): (0, -0.8)}
 LARGE = {
     "2d_512": dict(n=(512, 512)),
-    # levels above 512^2 (2D) / 96^3 (3D) cells relax by streaming along the
-    # last direction: walls with inhomogeneous derived-variable values on
-    # every side, periodic march direction, ragged blocks and segments
+    # 2D levels above 512^2 cells relax by streaming along the last direction,
+    # 3D levels by colour passes straight from memory: walls with inhomogeneous
+    # derived-variable values on every side, periodic march direction, ragged
+    # blocks and segments
     "2d_700x600_walls": dict(n=(700, 600), periodic=[0, 0], bc=WALLS),
     "2d_530x520_periodic": dict(n=(530, 520), periodic=[1, 1]),
     "2d_1030x261_no_derived_bc": dict(n=(1030, 261), apply_bc=0),

@@ -1,6 +1,6 @@
 """GPU (FP64) parity of the single-workgroup V-cycle of the linear operator
 over the kinds of level it holds: odd rows (a thread's two cells may share a
-colour), cells with two and more walls, one to six levels, with and without
+colour), cells with two and more walls, one to five levels, with and without
 the a and c coefficients, and BiCGStab bottoms of one wavefront, of two cells
 a thread and in between.  The arithmetic and the order of every sum are the
 oracle's, so solves agree in every bit."""

@@ -74,6 +74,26 @@ def test_fused_cycles(ml, gpu_ctx, wl, n, periodic, nu1, nu2):
     op.close()
 
 
+@pytest.mark.parametrize("n", [(308, 308), (352, 352), (512, 512), (320, 800)])
+@pytest.mark.parametrize("nu2", [4, 2])
+def test_fused_cycles_of_many_workgroups(ml, gpu_ctx, wl, n, nu2):
+    """The last launch of a cycle takes the residual norm and applies the
+    stopping rule: above 512 workgroups (cores of 14 or 22 cells) they report
+    in groups, numbered over both directions of the grid."""
+    case, g, p, bc, b, a, op = _setup(ml, gpu_ctx, wl, dict(n=n), False)
+    old = case["phi"].copy()
+    new = old.copy()
+    kw = dict(max_iter=3, nu2=nu2)
+    so = O.hc_be_step(g, p, bc, a, b, case["dt"], new, old, opts=O.default_opts(**kw))
+    for _ in range(2):
+        dn = ml.DeviceArray(gpu_ctx, old.shape, host=old)
+        st = op.solve_be(dn, ml.DeviceArray(gpu_ctx, old.shape, host=old), case["dt"], opts=ml.default_opts(**kw))
+        assert (st.iterations, st.exit_status) == (so.iterations, so.exit_status)
+        assert (st.initial_residual, st.final_residual) == (so.initial_residual, so.final_residual)
+        assert HC.bitwise_equal(HC.valid(n, dn.get()), HC.valid(n, new))
+    op.close()
+
+
 PARAMS = {
     "default": {},
     "heat_ratio": dict(specificHeatRatio=1.7, thetaEutectic=0.2, ThetaEutectic=0.1, waterDistributionCoeff=0.1),

@@ -86,32 +86,39 @@ def parse():
     return args
 
 
+def hc_relax_name(n):
+    """The kernel of a one-sweep FP64 (H, Theta) relaxation of an n grid."""
+    if len(n) == 3:
+        return "hc_sweep3_kernel<double,...> (one colour a launch)"
+    # levels above 512^2 cells stream along y (both colour passes of a sweep
+    # pipelined in one launch), smaller ones relax in deep-halo regions
+    if np.prod(n) > 512 * 512:
+        return "hc_relax_stream_kernel<double,252,2,256,false,false>"
+    return "hc_relax_pair_kernel<double,0,false>"
+
+
 def kernel_roofline(ml, ctx, stepper, reps=200):
-    """Average duration of the fused closure + smoother sweep on the finest
-    level (HIP events on the library stream) and its algorithmic bandwidth:
-    80 B per cell per red+black sweep in 2D FP64 (state R+W 32, rhs 16,
-    face coefficients 32)."""
+    """Average duration of the launches of the fused closure + smoother sweep
+    on the finest level (start and stop events in every launch, so the copies
+    to and from the partner array do not count) and their algorithmic
+    bandwidth: 80 B per cell per red+black sweep in 2D FP64 (state R+W 32, rhs
+    16, face coefficients 32)."""
     n = stepper.n
-    cells = int(np.prod(n))
-    dim = len(n)
-    bytes_per_cell = 8 * (2 * 2 + 2 + dim * 2)
     phi = ml.DeviceArray(ctx, stepper.phi.shape)
     ctx.check(ctx.lib.ml_buf_copy(ctx.h, phi.ptr, stepper.phi.ptr, phi.nbytes), "copy")
     rhs = stepper.old
     for _ in range(10):
         stepper.op.relax(0, phi, rhs, 1)
-    ctx.record(0)
+    ctx.timing_start(ml.KT_HC_RELAX, 2 * reps)
     for _ in range(reps):
         stepper.op.relax(0, phi, rhs, 1)
-    ctx.record(1)
-    ms = ctx.elapsed_ms(0, 1) / reps
+    launches, ms, nbytes, _ = ctx.timing_stop()
     phi.free()
-    achieved = bytes_per_cell * cells / (ms * 1e-3) / 1e9
-    name = "hc_relax_pair_kernel<double,0,false>" if dim == 2 else "hc_sweep3_kernel<double> (two launches)"
-    return {"kernel": "%s (1 sweep, finest level)" % name,
+    achieved = nbytes / (ms * 1e-3) / 1e9
+    return {"kernel": "%s (1 sweep, finest level)" % hc_relax_name(n),
             "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": None,
-            "avg_launch_us": round(ms * 1e3, 3), "bytes_per_launch": bytes_per_cell * cells}
+            "avg_launch_us": round(ms / launches * 1e3, 3), "bytes_per_launch": round(nbytes / launches, 1)}
 
 
 def smoother_bandwidth(ml, wl, ctx, n, launches=20):
@@ -135,11 +142,7 @@ def smoother_bandwidth(ml, wl, ctx, n, launches=20):
         st.op.relax(0, st.phi, st.old, 1)
     n1, ms, nb, _ = ctx.timing_stop()
     gbs = nb / (ms * 1e-3) / 1e9
-    # levels above 512^2 cells relax by streaming along y (both colour passes
-    # of a sweep pipelined in one launch), smaller ones in deep-halo regions
-    hname = ("hc_relax_stream_kernel<double,2,252,1,2,256,false>" if n * n > 512 * 512 else
-             "hc_relax_pair_kernel<double,0,false>")
-    out["hc_relax"] = {"kernel": "%s (1 sweep per launch)" % hname,
+    out["hc_relax"] = {"kernel": "%s (1 sweep per launch)" % hc_relax_name((n, n)),
                        "avg_launch_us": round(ms / n1 * 1e3, 2), "bytes_per_launch": nb / n1,
                        "achieved_GBs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4)}
     st.op.close()
@@ -155,8 +158,8 @@ def smoother_bandwidth(ml, wl, ctx, n, launches=20):
     # sweep per launch, the whole grid resident), smaller ones in 16x16
     # deep-halo tiles
     wide = n * n > 512 * 512
-    kname, hmax = (("vc_relax_stream_kernel<double,2,252,1,2,256>", 1) if wide else
-                   ("vc_relax_tile_kernel<double,2,16,16,1,9,1024>", 4))
+    kname, hmax = (("vc_relax_stream_kernel<double,252,2,256,false>", 1) if wide else
+                   ("vc_relax_tile_kernel<double,2,16,16,1,9,1024,false>", 4))
     for sweeps in (1, 4):
         op.relax(0, u, r, sweeps)
         ctx.timing_start(ml.KT_VC_RELAX, launches)
@@ -322,7 +325,7 @@ def timed_steps(ctx, st, steps):
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "vc_relax_tile_256_traffic.json")   # 256x256 workload
 BATCH_TRAFFIC_FILE = os.path.join(ROOT, "profiles", "batch_relax_512_traffic.json")   # 512-instance batch
 # the relaxation of the finest level of the two workloads
-VC_TILE = {2: "vc_relax_tile_kernel<double,2,16,16,1,9,1024>", 3: "vc_sweep3_kernel<double> (one colour a launch)"}
+VC_TILE = {2: "vc_relax_tile_kernel<double,2,16,16,1,9,1024,false>", 3: "vc_sweep3_kernel<double> (one colour a launch)"}
 
 
 def vc_relax_roofline(ml, ctx, stepper, steps):

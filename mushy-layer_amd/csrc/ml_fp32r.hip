@@ -1363,14 +1363,16 @@ __global__ __launch_bounds__(kLinThreads) void hc_residual_jacobian_batch_kernel
   const int blk = int(w & kBatchTileMask);
   if (mode == 1) {
     hc_residual_jacobian_body<DIM, TX, TY, TZ>(J.A, J.pb[0], nullptr, J.rhs, nullptr, 1.0, J.r32, J.M32, J.slots,
-                                               J.ntx, J.nty, CtlFuse{}, blk, J.A.skip);
+                                               J.ntx, J.nty, CtlFuse{nullptr, nullptr, nullptr, 1, J.ntiles}, blk,
+                                               J.A.skip);
     return;
   }
   if (mode == 2) {
     const int it = J.ctl->iter + 1;
     const int pc = (it - 1) & 1;
     hc_residual_jacobian_body<DIM, TX, TY, TZ>(J.A, J.pb[pc], J.pb[1 - pc], J.rhs, J.e, omega, J.r32, J.M32,
-                                               J.slots + it, J.ntx, J.nty, CtlFuse{}, blk, nullptr);
+                                               J.slots + it, J.ntx, J.nty,
+                                               CtlFuse{nullptr, nullptr, nullptr, 1, J.ntiles}, blk, nullptr);
     return;
   }
   if (*J.A.skip) return;

@@ -92,7 +92,7 @@ struct CtlFuse {
   const unsigned long long* slots;
   unsigned int* arrive;
   int refined;
-  unsigned int total;   // workgroups that report (0: the whole grid)
+  unsigned int total;   // workgroups that report to this norm (0: the whole grid)
 };
 
 // Max-reduction of a non-negative value over the workgroup, then one
@@ -126,7 +126,8 @@ __device__ inline void block_max_atomic(T v, int nan, unsigned long long* out, C
     const unsigned int grid = gridDim.x * gridDim.y * gridDim.z;
     const bool direct = grid <= kArriveDirect || f.total;
     if (!f.ctl) {
-      // (a maximum already passed needs no atomic)
+      // (a maximum already passed needs no atomic; where a grid reports to
+      // many norms the read would only keep its workgroups waiting)
       if (direct || bits > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, bits);
       return;
     }

@@ -970,6 +970,7 @@ int vcb_tables(ml_vc_batch b, double* const phi[], const double* const rhs[], co
     const int nt = ml::vc_resid_tiles(g0, &ntx, &nty);
     R.io.ntx = ntx;
     R.io.nty = nty;
+    R.io.fuse.total = unsigned(nt);   // (no stopping rule here: the norm alone)
     const unsigned j = unsigned(br.size());
     for (int t = 0; t < nt; ++t) brm.push_back((j << ml::kBatchTileBits) | unsigned(t));
     br.push_back(R);

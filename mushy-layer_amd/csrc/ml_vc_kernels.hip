@@ -1416,8 +1416,8 @@ GhostForm<T> vc_ghost_form(BCDesc bc, T dx) {
 // (the first pass, and every pass of the GEN form); otherwise in place on
 // `out`.  Two passes with c: 37 us at 128^3 (92 bytes a cell needed, 102
 // counted beyond the L2s: 5.8 TB/s; a march along z with a window of planes in
-// LDS was 71), 8.5 at 64^3 and 7.5 at 16^3 (16 x 8 x 4 tiles with the halo of both passes:
-// 15.1 and 8.0); GEN 50 at 129 x 128 x 128.
+// LDS was 71), 8.5 at 64^3 and 7.5 at 16^3 (16 x 8 x 4 tiles with the halo of
+// both passes: 15.1 and 8.0); GEN 50 at 129 x 128 x 128.
 template <typename T, bool GEN>
 struct VCSweep {
   Sweep3<GEN> S;

@@ -55,10 +55,11 @@ def test_hc_3d(ml, gpu_ctx, wl, name, iters, acoef):
     _hc_relax(ml, gpu_ctx, wl, GRIDS3[name], iters, acoef)
 
 
-def test_hc_3d_solve(ml, gpu_ctx, wl):
+@pytest.mark.parametrize("spec", [GRIDS3["x"], PAIRS2["129x47_11"], STREAMS2["x"]], ids=["3d", "pairs", "streams"])
+def test_hc_solve(ml, gpu_ctx, wl, spec):
     """A single level of more than 1024 cells: the solve is its bottom's
     relaxations."""
-    case, g, p, bc, b, a, op = _setup(ml, gpu_ctx, wl, GRIDS3["x"], False)
+    case, g, p, bc, b, a, op = _setup(ml, gpu_ctx, wl, spec, False)
     old = case["phi"].copy()
     new = old.copy()
     kw = dict(max_iter=3, bottom=7)
@@ -68,6 +69,12 @@ def test_hc_3d_solve(ml, gpu_ctx, wl):
     assert (st.iterations, st.exit_status, st.final_residual) == (so.iterations, so.exit_status, so.final_residual)
     assert HC.bitwise_equal(HC.valid(case["n"], dn.get()), HC.valid(case["n"], new))
     op.close()
+
+
+@pytest.mark.parametrize("spec", [GRIDS3["all"], PAIRS2["59x30_10"]], ids=["3d", "pairs"])
+def test_hc_without_allocation(ml, gpu_ctx, wl, spec):
+    for iters in (1, 2, 5):
+        _hc_relax(ml, gpu_ctx, wl, spec, iters, False, "relax_noalloc")
 
 
 @pytest.mark.parametrize("name", sorted(PAIRS2))

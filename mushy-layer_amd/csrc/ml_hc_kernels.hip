@@ -106,17 +106,25 @@ __device__ inline void tile_diffused_var(const HCArgs<T>& A, const Tile<DIM, TX,
 // that holds it reads a pass's neighbours as of its start (the new closures
 // are stored after a barrier), and along x it starts one cell earlier where
 // that keeps the seam from falling inside a pair, whose cells would share a
-// slot's turn; its core is two cells narrower for that.  Only below 32 cells,
-// where a region may hold several seams, a pass looks at both slots.  One
+// slot's turn; its core is narrower for that (pair_core_x).  Only on very short
+// rows, where a region holds several seams, a pass looks at both slots.  One
 // sweep of 129 x 128 8.1 us, of 257 x 256 8.3 (11.4 and 11.3 with both slots
-// everywhere; 7.5 and 7.9 with even lengths), of 23 x 500 12; four sweeps of
-// 385 x 384 28.7 us (34.7; even 24.3).
+// everywhere; 7.5 and 7.9 with even lengths), of 23 x 500 8.6 (11.1), of
+// 17 x 500, with both, 12; four sweeps of 385 x 384 28.7 us (34.7; even 24.3).
 enum : int { RB_PLAIN = 0, RB_RESTRICT = 1, RB_NORM = 2 };
 constexpr int kRB = 32;            // positions per side
 constexpr int kRBThreads = kRB * kRB / 2;
-// core cells along x
-__host__ __device__ inline int pair_core_x(int nx, int per0, int H) {
-  return kRB - 2 * H - (per0 && (nx & 1) && nx >= kRB ? 2 : 0);
+// Core cells along x.  With an odd periodic length the core and its halo are no
+// wider than the row, so that they hold one seam at most, and leave a column for
+// the shift off it; where that would more than halve the core (rows below 18
+// cells in a sweep, 24 in four) the core stays whole and `both` is set.
+__host__ __device__ inline int pair_core_x(int nx, int per0, int H, bool* both) {
+  const int whole = kRB - 2 * H;
+  *both = false;
+  if (!per0 || !(nx & 1)) return whole;
+  const int w = (nx < kRB - 2 ? nx : kRB - 2) - 2 * H;
+  *both = 2 * w < whole;
+  return *both ? whole : w & ~1;
 }
 
 template <typename T>
@@ -185,24 +193,24 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
   const int nx = A.nx, ny = A.ny, npass = A.npass;
   const int H = npass + (MODE == RB_PLAIN ? 0 : 1);
   const int core = kRB - 2 * H;
-  const int corex = GEN ? pair_core_x(nx, A.per0, H) : core;
+  // GEN: both slots in every pass
+  bool both = false;
+  const int corex = GEN ? pair_core_x(nx, A.per0, H, &both) : core;
   // GEN: the workgroups of all tiles in one dimension
   const int by = GEN ? int(blockIdx.x / unsigned(A.ntx)) : int(blockIdx.y);
   const int bx = GEN ? int(blockIdx.x) - by * A.ntx : int(blockIdx.x);
   const int x0 = bx * corex, y0 = by * core;
   const int ey = threadIdx.x >> 4, ex0 = 2 * (threadIdx.x & 15);
   const bool per0 = A.per0 != 0, per1 = A.per1 != 0;
-  // GEN: the region holds the seam of an odd length (careful), the pairs'
-  // shift against it, both slots in every pass
-  bool careful = false, both = false;
+  // GEN: the core and its halo hold the seam of an odd length (careful); the
+  // pairs' shift against it
+  bool careful = false;
   int sh = 0;
   if constexpr (GEN) {
     if (per0 && (nx & 1)) {
-      both = nx < kRB;
-      // the seam inside the region, from its first cell (n >= 32: at most one)
-      const int at = x0 < H ? H - x0 : nx - (x0 - H);
-      careful = both || at < kRB;
-      sh = !both && at < kRB ? at & 1 : 0;
+      const int at = x0 < H ? H - x0 : nx - (x0 - H);   // the seam, from the halo's first cell
+      careful = both || at < corex + 2 * H;
+      sh = !both && careful ? at & 1 : 0;
     }
     if (per1 && (ny & 1)) careful = careful || ny < kRB || y0 < H || ny - (y0 - H) < kRB;
   }
@@ -228,7 +236,8 @@ __global__ __launch_bounds__(kRBThreads, 4) void hc_relax_pair_kernel(PairArgs<T
   const int wy = per1 ? 0 : ((gj == 0 ? 4 : 0) | (gj == ny - 1 ? 8 : 0));
   // cells of the pair in x order: c = 0, 1; slot m holds cell m ^ swap
   const bool in0 = ux0 >= 0 && ux0 < nx, in1 = ux0 >= -1 && ux0 + 1 < nx;
-  const bool ok0 = oky && (in0 || per0), ok1 = oky && (in1 || per0);
+  const bool near = !GEN || ex0 < Hx + corex + H;   // (columns beyond the halo: a narrow core leaves some)
+  const bool ok0 = near && oky && (in0 || per0), ok1 = near && oky && (in1 || per0);
   const int gx0 = ok0 ? wrap(ux0, nx) : 0, gx1 = ok1 ? wrap(ux0 + 1, nx) : 0;
   // parity of the pair's first cell
   const int swap = (GEN ? (per0 ? gx0 : ux0) + gj : ux0 + uy) & 1;
@@ -1480,7 +1489,8 @@ static hipError_t launch_relax_pair(const HCArgs<T>& A, const TileIO<T>& io, hip
         P.gs[d][sd][n] = gf.s[d][sd][n];
         P.gb[d][sd][n] = gf.b[d][sd][n];
       }
-  const int core = kRB - 2 * H, corex = pair_core_x(g.n[0], g.periodic[0], H);
+  bool both = false;
+  const int core = kRB - 2 * H, corex = pair_core_x(g.n[0], g.periodic[0], H, &both);
   const int ntx = (g.n[0] + corex - 1) / corex, nty = (g.n[1] + core - 1) / core;
   if (g.ncell >= (1LL << 32)) return hipErrorInvalidValue;   // (32-bit component stride)
   P.ntx = ntx;

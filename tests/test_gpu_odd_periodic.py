@@ -31,11 +31,13 @@ STREAMS2 = {
 }
 
 # regions of 32 positions: the seam at even and odd places of a region, in the
-# halo of one core and inside the next, more than once in a region (below 32)
+# halo of one core and inside the next, rows hardly wider than core and halo,
+# several seams in a region (rows below 18 cells in a sweep, 24 in four)
 PAIRS2 = {
     "%dx%d_%d%d" % (n + tuple(per)): dict(n=n, periodic=per, bc=None if per[1] else WALLS)
     for n, per in [((33, 40), [1, 0]), ((59, 30), [1, 0]), ((81, 64), [1, 0]), ((85, 33), [1, 1]), ((129, 47), [1, 1]),
-                   ((64, 35), [1, 1]), ((48, 53), [0, 1]), ((31, 66), [1, 0]), ((7, 200), [1, 1]), ((200, 9), [1, 1])]
+                   ((64, 35), [1, 1]), ((48, 53), [0, 1]), ((31, 66), [1, 0]), ((29, 47), [1, 1]), ((25, 48), [1, 0]),
+                   ((23, 90), [1, 0]), ((17, 80), [1, 0]), ((7, 200), [1, 1]), ((200, 9), [1, 1])]
 }
 
 
